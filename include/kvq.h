@@ -361,7 +361,9 @@ KVQ_API int kvq_splitk_reduce(void* out, int out_dtype, float* lse, const float*
  * (cache_kernels.cu:51-55).  A block of the int8 layouts (kvq_cache_geom /
  * kvq_mla_geom: block_bytes = stride_block) holds codes and scales together, so
  * the move is self-contained.  Asynchronous on `stream`; host memory should be
- * pinned.  Pairs must not overlap when src and dst are the same allocation.
+ * pinned: memory the GPU can address is read or written by a kernel, other memory takes a
+ * copy call per block.  The moves of a call are unordered among themselves: each destination block is
+ * named once, and pairs must not overlap when src and dst are the same allocation.
  */
 KVQ_API int kvq_swap_blocks(const void* src, void* dst, int64_t block_bytes,
                     const int64_t* block_mapping, int64_t num_pairs, int64_t map_stride0,

@@ -55,6 +55,27 @@ def test_swap_blocks_gqa_cache(gpu_device, direction, layout, num_mappings):
     assert torch.equal(as_blocks(src).cpu(), src_clone)   # the source is only read
 
 
+@pytest.mark.parametrize("to_host", [True, False], ids=["out", "in"])
+@pytest.mark.parametrize("bs,hkv,d,n", [(16, 8, 128, 1), (16, 1, 64, 480), (16, 1, 64, 481), (64, 2, 128, 7),
+                                        (16, 8, 256, 100)])
+def test_swap_blocks_with_pinned_memory(gpu_device, bs, hkv, d, n, to_host):
+    """Pinned host memory is reached by the copy kernel: blocks of less than, exactly and more than a 16 KB slice,
+    the last pair of a launch's table and the first of the next."""
+    nb = n + 20
+    g = torch.Generator().manual_seed(n)
+    gpu = L.allocate_kv_cache(nb, bs, hkv, d, device=gpu_device, fill=None)
+    host = torch.empty((nb,) + tuple(gpu.shape[1:]), dtype=torch.int8, pin_memory=True)
+    for t in (gpu, host):
+        as_blocks(t).copy_(torch.randint(0, 256, as_blocks(t).shape, generator=g, dtype=torch.uint8))
+    src, dst = (gpu, host) if to_host else (host, gpu)
+    mapping = torch.stack([torch.randperm(nb, generator=g)[:n], torch.randperm(nb, generator=g)[:n]], 1)
+    want = as_blocks(dst).cpu().clone()
+    want[mapping[:, 1]] = as_blocks(src).cpu()[mapping[:, 0]]
+    ops.swap_blocks(src, dst, block_bytes(src), mapping)
+    torch.cuda.synchronize()
+    assert torch.equal(as_blocks(dst).cpu(), want)
+
+
 def test_swap_blocks_same_tensor_and_strided_mapping(gpu_device):
     """Copy inside one allocation (non-overlapping pairs), mapping given as a strided view."""
     nb = 64

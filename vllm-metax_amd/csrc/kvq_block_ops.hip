@@ -2,40 +2,56 @@
 // cache blocks.  A block of this layout carries its codes AND their fp32 scales, so moving
 // `block_bytes` moves a self-contained unit: no scale tensor to keep in step.
 //
-// Device-to-device moves are ONE kernel launch per 128 pairs (the pairs travel in the kernel
-// arguments, 16-byte lane copies, one workgroup per 16 KB slice of a block) instead of one
-// memcpy call per block; moves to or from the host are one asynchronous copy per block on the
-// caller's stream, as in the reference (csrc/libtorch_stable/cache_kernels.cu:33-77).
+// Moves between GPU buffers, and between the GPU and pinned host memory, are ONE kernel launch per 480 pairs
+// (the pairs travel in the kernel arguments, 16-byte lane copies, a workgroup per 16 KB slice of a block).  Host
+// memory that the GPU cannot address takes one asynchronous copy call per block on the caller's stream, as in
+// the reference (csrc/libtorch_stable/cache_kernels.cu:33-77).
 #include "kvq_internal.h"
 
 namespace kvq {
 
-constexpr int kPairsPerLaunch = 128;
-constexpr int kSliceBytes = 16384;  // bytes one workgroup moves
+constexpr int kPairsPerLaunch = 480;   // 3840 bytes of kernel arguments, of the 4 KB a launch can carry
+constexpr int kTriplesPerLaunch = 64;
+constexpr int kSliceBytes = 16384;     // bytes one workgroup moves
+// Workgroups of a launch that crosses PCIe: 64 x 16 KB are requested at a time, several times what the link's
+// latency needs, and three quarters of the compute units stay free for what other streams run meanwhile.  The
+// 2 x 192 blocks above take 300 us with 8 workgroups, 255 with 16, 247 with 32, 239 with 64 or 128, 265 with 1024.
+constexpr int kHostCopyGroups = 64;
 
 struct BlockPairs {
-  int64_t src[kPairsPerLaunch];
-  int64_t dst[kPairsPerLaunch];
+  int32_t src[kPairsPerLaunch];
+  int32_t dst[kPairsPerLaunch];
 };
 
-// grid (slices per block, pairs); 256 threads, each moving 16 bytes per step.
+// A workgroup takes the slices blockIdx.x, blockIdx.x + gridDim.x, ... of the launch's blocks (`slices` each); 256
+// threads, four 16-byte loads per thread in flight.
+// Bound by HBM between GPU buffers and by the link to or from pinned host memory.  192 blocks of 33 KB out and as
+// many back: 3.66 ms as a copy call per block (9.5 us each, whatever the size), 239 us this way = 54 GB/s of the 57
+// that one large copy reaches.
 __global__ __launch_bounds__(256) void move_blocks_kernel(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst,
-                                                          int64_t block_bytes, BlockPairs pairs) {
-  const int64_t s_off = pairs.src[blockIdx.y] * block_bytes;
-  const int64_t d_off = pairs.dst[blockIdx.y] * block_bytes;
-  const int64_t begin = (int64_t)blockIdx.x * kSliceBytes;
-  const int64_t end = begin + kSliceBytes < block_bytes ? begin + kSliceBytes : block_bytes;
-  const u32x4* s = reinterpret_cast<const u32x4*>(src + s_off + begin);
-  u32x4* d = reinterpret_cast<u32x4*>(dst + d_off + begin);
-  const int n = (int)((end - begin) / 16);
-  for (int i = threadIdx.x; i < n; i += 256) d[i] = s[i];
+                                                          int64_t block_bytes, int slices, int items, BlockPairs pairs) {
+  for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    const int pair = item / slices;
+    const int64_t begin = (int64_t)(item - pair * slices) * kSliceBytes;
+    const int64_t left = block_bytes - begin;
+    const int n = (int)((left < kSliceBytes ? left : kSliceBytes) / 16);
+    const u32x4* s = reinterpret_cast<const u32x4*>(src + pairs.src[pair] * block_bytes + begin);
+    u32x4* d = reinterpret_cast<u32x4*>(dst + pairs.dst[pair] * block_bytes + begin);
+    u32x4 v[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if ((int)threadIdx.x + 256 * j < n) v[j] = s[threadIdx.x + 256 * j];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if ((int)threadIdx.x + 256 * j < n) d[threadIdx.x + 256 * j] = v[j];
+  }
 }
 
 // Arbitrary (src pointer, dst pointer, size) triples, all on the device: grid (slices, entries).
 struct CopyTriples {
-  int64_t src[kPairsPerLaunch / 2];
-  int64_t dst[kPairsPerLaunch / 2];
-  int64_t size[kPairsPerLaunch / 2];
+  int64_t src[kTriplesPerLaunch];
+  int64_t dst[kTriplesPerLaunch];
+  int64_t size[kTriplesPerLaunch];
 };
 
 __global__ __launch_bounds__(256) void copy_triples_kernel(CopyTriples t) {
@@ -76,6 +92,20 @@ __global__ __launch_bounds__(256) void copy_blocks_kernel(const int64_t* __restr
   }
 }
 
+// Whether kernels may address the host bytes [first, last] where the host does: pinned memory (hipHostMalloc, or
+// registered) under unified addressing.
+static bool host_range_is_mapped(const uint8_t* first, const uint8_t* last) {
+  for (const uint8_t* p : {first, last}) {
+    hipPointerAttribute_t at{};
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+      (void)hipGetLastError();   // plain memory: not an error of the call
+      return false;
+    }
+    if (at.type != hipMemoryTypeHost || at.devicePointer != p) return false;
+  }
+  return true;
+}
+
 }  // namespace kvq
 
 extern "C" {
@@ -108,22 +138,35 @@ int kvq_swap_blocks(const void* src, void* dst, int64_t block_bytes, const int64
   KVQ_REQUIRE(direction == KVQ_DEVICE_TO_DEVICE || direction == KVQ_DEVICE_TO_HOST || direction == KVQ_HOST_TO_DEVICE,
               "%s: unknown direction %d", op, direction);
   hipStream_t s = as_stream(stream);
+  int64_t lo[2] = {INT64_MAX, INT64_MAX}, hi[2] = {0, 0};   // lowest and highest block number on either side
   for (int64_t i = 0; i < num_pairs; ++i)
-    KVQ_REQUIRE(block_mapping[i * map_stride0] >= 0 && block_mapping[i * map_stride0 + map_stride1] >= 0,
-                "%s: negative block number in pair %lld", op, (long long)i);
-  if (direction == KVQ_DEVICE_TO_DEVICE && block_bytes % 16 == 0 && ((uintptr_t)src % 16) == 0 &&
-      ((uintptr_t)dst % 16) == 0) {
-    const int64_t slices = (block_bytes + kSliceBytes - 1) / kSliceBytes;
-    KVQ_REQUIRE(slices <= 0x7fffffff, "%s: block_bytes out of range", op);
+    for (int side = 0; side < 2; ++side) {
+      const int64_t b = block_mapping[i * map_stride0 + side * map_stride1];
+      KVQ_REQUIRE(b >= 0, "%s: negative block number in pair %lld", op, (long long)i);
+      lo[side] = b < lo[side] ? b : lo[side];
+      hi[side] = b > hi[side] ? b : hi[side];
+    }
+  const int64_t slices = (block_bytes + kSliceBytes - 1) / kSliceBytes;
+  bool by_kernel = block_bytes % 16 == 0 && ((uintptr_t)src % 16) == 0 && ((uintptr_t)dst % 16) == 0 &&
+                   hi[0] <= INT32_MAX && hi[1] <= INT32_MAX && slices <= INT32_MAX / kPairsPerLaunch;
+  if (by_kernel && direction != KVQ_DEVICE_TO_DEVICE) {
+    const int side = direction == KVQ_DEVICE_TO_HOST ? 1 : 0;
+    const uint8_t* host = static_cast<const uint8_t*>(side ? dst : src);
+    by_kernel = host_range_is_mapped(host + lo[side] * block_bytes, host + (hi[side] + 1) * block_bytes - 1);
+  }
+  if (by_kernel) {
     for (int64_t base = 0; base < num_pairs; base += kPairsPerLaunch) {
-      BlockPairs p{};
+      BlockPairs p;
       const int n = (int)(num_pairs - base < kPairsPerLaunch ? num_pairs - base : kPairsPerLaunch);
       for (int i = 0; i < n; ++i) {
-        p.src[i] = block_mapping[(base + i) * map_stride0];
-        p.dst[i] = block_mapping[(base + i) * map_stride0 + map_stride1];
+        p.src[i] = (int32_t)block_mapping[(base + i) * map_stride0];
+        p.dst[i] = (int32_t)block_mapping[(base + i) * map_stride0 + map_stride1];
       }
-      hipLaunchKernelGGL(move_blocks_kernel, dim3((unsigned)slices, (unsigned)n), dim3(256), 0, s,
-                         static_cast<const uint8_t*>(src), static_cast<uint8_t*>(dst), block_bytes, p);
+      for (int i = n; i < kPairsPerLaunch; ++i) p.src[i] = p.dst[i] = 0;
+      const int items = n * (int)slices;
+      const int groups = direction == KVQ_DEVICE_TO_DEVICE || items < kHostCopyGroups ? items : kHostCopyGroups;
+      hipLaunchKernelGGL(move_blocks_kernel, dim3((unsigned)groups), dim3(256), 0, s, static_cast<const uint8_t*>(src),
+                         static_cast<uint8_t*>(dst), block_bytes, (int)slices, items, p);
       if (int rc = check_hip(hipGetLastError(), "swap_blocks launch")) return rc;
     }
     return KVQ_OK;
@@ -154,7 +197,7 @@ int kvq_swap_blocks_batch(const int64_t* src_ptrs, const int64_t* dst_ptrs, cons
                 "%s: entry %lld has a NULL pointer or a negative size", op, (long long)i);
   hipStream_t s = as_stream(stream);
   if (all_on_device) {
-    constexpr int kPer = kPairsPerLaunch / 2;
+    constexpr int kPer = kTriplesPerLaunch;
     for (int64_t base = 0; base < n; base += kPer) {
       CopyTriples t{};
       const int m = (int)(n - base < kPer ? n - base : kPer);
