@@ -7,10 +7,12 @@ STD_TORCH_CHECK the same way, csrc/libtorch_stable/cache_kernels.cu:884-889).
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 import os
 
 _LIB_DIR = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib")
 LIB_PATH = os.path.join(_LIB_DIR, "libkvq_hip.so")
+BINDING_PATH = os.path.join(_LIB_DIR, "kvq_torch.so")   # csrc/kvq_torch.cpp
 
 KVQ_F32, KVQ_BF16, KVQ_F16 = 0, 1, 2
 KVQ_CODE_INT8, KVQ_CODE_FP8_E4M3, KVQ_CODE_INT4 = 0, 1, 2
@@ -92,6 +94,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_binding = None
 
 
 def load() -> ctypes.CDLL:
@@ -118,6 +121,22 @@ def load() -> ctypes.CDLL:
         lib.kvq_set_batch_invariant(1)
     _lib = lib
     return lib
+
+
+def binding():
+    """The extension module through which the per-step ops hand tensors to the library (loaded once)."""
+    global _binding
+    if _binding is not None:
+        return _binding
+    load()
+    if not os.path.exists(BINDING_PATH):
+        raise RuntimeError(f"{BINDING_PATH} is missing: run `make -C vllm-metax_amd/csrc` or __graft_entry__.build()")
+    import torch  # noqa: F401  (its libraries, which the extension links to, are loaded with it)
+    spec = importlib.util.spec_from_file_location("kvq_torch", BINDING_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    _binding = module
+    return module
 
 
 def check(status: int, op: str) -> None:

@@ -142,27 +142,9 @@ def reshape_and_cache_flash_per_token_head_quant(
     INT8_PER_TOKEN_HEAD (scale = absmax / 127, codes rint(x / scale)) or FP8_PER_TOKEN_HEAD
     (scale = absmax / 448, e4m3fn codes) -- the two one-byte modes of this record layout."""
     code_type = code_type_of(kv_quant_mode)   # int8, or the fp8 mode of the same record layout
-    dev = _require_cuda(key, value, key_cache, value_cache, k_scale_cache, v_scale_cache, slot_mapping)
+    _require_cuda(key_cache, value_cache, k_scale_cache, v_scale_cache)
     geom = (geometry or geometry_from_views(key_cache, value_cache, k_scale_cache, v_scale_cache)).with_code_type(code_type)
-    if key.dim() != 3 or value.shape != key.shape or key.dtype != value.dtype:
-        raise RuntimeError("key/value must be [num_tokens, num_kv_heads, head_size] of one dtype")
-    if key.shape[1] != geom.num_kv_heads or key.shape[2] != geom.head_size:
-        raise RuntimeError(f"key shape {tuple(key.shape)} does not match cache (Hkv={geom.num_kv_heads}, D={geom.head_size})")
-    if key.stride(2) != 1 or value.stride(2) != 1:
-        raise RuntimeError("key/value head dim must be contiguous")
-    if slot_mapping.dtype != torch.int64 or slot_mapping.dim() != 1 or not slot_mapping.is_contiguous():
-        raise RuntimeError("slot_mapping must be a contiguous 1-D int64 tensor")
-    num_tokens = slot_mapping.shape[0]
-    if num_tokens > key.shape[0]:
-        raise RuntimeError("slot_mapping is longer than key")
-    lib = _C.load()
-    g = geom.as_struct()
-    with _on_device(dev):
-        rc = lib.kvq_reshape_and_cache_int8(
-            _ptr(key), _ptr(value), _dtype_code(key, "key"), key.stride(0), key.stride(1), value.stride(0),
-            value.stride(1), ctypes.c_void_p(geom.base_ptr), ctypes.byref(g), _ptr(slot_mapping), num_tokens,
-            eps_for_dtype(key.dtype), _stream(dev))
-    _C.check(rc, "reshape_and_cache_flash_per_token_head_quant")
+    _C.binding().cache_update(key, value, key_cache, slot_mapping, geom.struct_addr, geom.base_ptr)
 
 
 # name used at the reference's call site
@@ -352,57 +334,26 @@ def unified_attention(
         raise NotImplementedError("rswa / chunk_lookback are not built")
     if block_table is None or k_scale_cache is None or v_scale_cache is None:
         raise RuntimeError("block_table, k_scale_cache and v_scale_cache are required")
-    dev = _require_cuda(q, k, v, out, cu_seqlens_q, seqused_k, block_table, k_scale_cache, v_scale_cache, workspace, lse)
+    dev = _require_cuda(q, k, v, k_scale_cache, v_scale_cache, workspace)
     geom = (geometry or geometry_from_views(k, v, k_scale_cache, v_scale_cache)).with_code_type(code_type)
-    if q.dim() != 3 or out.shape != q.shape or q.shape[2] != geom.head_size:
-        raise RuntimeError("q/out must be [num_tokens, num_q_heads, head_size] matching the cache head size")
-    if q.stride(2) != 1 or out.stride(2) != 1:
-        raise RuntimeError("q/out head dim must be contiguous")
-    num_seqs = seqused_k.shape[0]
-    if seqused_k.dtype != torch.int32 or cu_seqlens_q.dtype != torch.int32 or block_table.dtype != torch.int32:
-        raise RuntimeError("seqused_k, cu_seqlens_q and block_table must be int32")
-    if cu_seqlens_q.shape[0] != num_seqs + 1 or block_table.shape[0] < num_seqs or block_table.stride(1) != 1:
-        raise RuntimeError("cu_seqlens_q must have num_seqs+1 entries and block_table num_seqs contiguous rows")
-    if not seqused_k.is_contiguous() or not cu_seqlens_q.is_contiguous():
-        raise RuntimeError("seqused_k and cu_seqlens_q must be contiguous")
-    if block_table.shape[1] * geom.block_size < int(max_seqlen_k):
-        raise RuntimeError("block_table rows are too short for max_seqlen_k")
-    if num_seqs == 0 or q.shape[0] == 0:
-        return
-    num_q_heads = q.shape[1]
-    _check_sinks(sinks, num_q_heads, q.device)
-    _check_sinks(alibi_slopes, num_q_heads, q.device, "alibi_slopes")
-    lib = _C.load()
-    if lse is not None and (lse.dtype != torch.float32 or not lse.is_contiguous()
-                            or tuple(lse.shape) != (q.shape[0], num_q_heads)):
-        raise RuntimeError("lse must be a contiguous float32 [num_tokens, num_q_heads] tensor")
-    g = geom.as_struct()
-    head = (_ptr(out), _dtype_code(out, "out"), out.stride(0), out.stride(1),
-            _ptr(q), _dtype_code(q, "q"), q.stride(0), q.stride(1),
-            ctypes.c_void_p(geom.base_ptr), ctypes.byref(g), _ptr(block_table), block_table.stride(0),
-            _ptr(seqused_k), _ptr(cu_seqlens_q), num_seqs, num_q_heads, int(max_seqlen_q),
-            float(softmax_scale), (1 if causal else 0) | (0 if has_decode_rows else 2), window, softcap,
-            _ptr(sinks), _ptr(alibi_slopes), _ptr(lse))
     prefill_splits = int(prefill_splits)
     if not 1 <= prefill_splits <= 8:
         raise RuntimeError("prefill_splits must be 1..8")
+    if q.dim() != 3:
+        raise RuntimeError("q/out must be [num_tokens, num_q_heads, head_size] matching the cache head size")
+    num_seqs = seqused_k.shape[0]
     if static_scratch:
-        with _on_device(dev):
-            rc = lib.kvq_paged_attn_int8_static_scratch(*head, _stream(dev))
-    elif prefill_splits > 1 and int(max_seqlen_q) > 1:
-        need = split_prefill_workspace_bytes(num_seqs, num_q_heads, geom.head_size, q.shape[0], prefill_splits, dev)
-        if workspace is None:
-            workspace = _default_workspace(dev, need)
-        with _on_device(dev):
-            rc = lib.kvq_paged_attn_int8_split_prefill(*head, q.shape[0], prefill_splits, _ptr(workspace),
-                                                       workspace.numel() * workspace.element_size(), _stream(dev))
-    else:
-        if workspace is None:
-            workspace = _default_workspace(dev, paged_attn_workspace_bytes(num_seqs, num_q_heads, geom.head_size, dev))
-        with _on_device(dev):
-            rc = lib.kvq_paged_attn_int8(*head, _ptr(workspace), workspace.numel() * workspace.element_size(),
-                                         _stream(dev))
-    _C.check(rc, "unified_attention")
+        workspace, prefill_splits = None, 1
+    elif workspace is None and num_seqs > 0 and q.shape[0] > 0:
+        if prefill_splits > 1 and int(max_seqlen_q) > 1:
+            need = split_prefill_workspace_bytes(num_seqs, q.shape[1], geom.head_size, q.shape[0], prefill_splits, dev)
+        else:
+            need = paged_attn_workspace_bytes(num_seqs, q.shape[1], geom.head_size, dev)
+        workspace = _default_workspace(dev, need)
+    _C.binding().paged_attention(
+        q, out, -1, 0, k, geom.struct_addr, geom.base_ptr, cu_seqlens_q, seqused_k, block_table, int(max_seqlen_q),
+        int(max_seqlen_k), float(softmax_scale), (1 if causal else 0) | (0 if has_decode_rows else 2), window, softcap,
+        sinks, alibi_slopes, lse, workspace, prefill_splits)
 
 
 def split_prefill_workspace_bytes(max_num_seqs: int, num_q_heads: int, head_size: int, num_tokens: int,
@@ -478,52 +429,16 @@ def decode_attention_with_cache_update(
         window = left + 1
     else:
         raise NotImplementedError(f"window_size {(left, right)}: only (-1, -1) and (W - 1, 0) are built")
-    dev = _require_cuda(q, key, value, k, v, out, seqused_k, block_table, k_scale_cache, v_scale_cache, workspace, lse)
+    dev = _require_cuda(q, k, v, k_scale_cache, v_scale_cache, workspace)
     geom = (geometry or geometry_from_views(k, v, k_scale_cache, v_scale_cache)).with_code_type(code_type)
-    num_seqs = seqused_k.shape[0]
-    if q.dim() != 3 or out.shape != q.shape or q.shape[2] != geom.head_size or q.shape[0] != num_seqs:
-        raise RuntimeError("q/out must be [num_seqs, num_q_heads, head_size] matching the cache head size")
-    if q.stride(2) != 1 or out.stride(2) != 1:
-        raise RuntimeError("q/out head dim must be contiguous")
-    if key.dim() != 3 or value.shape != key.shape or key.dtype != value.dtype or key.shape[0] < num_seqs:
-        raise RuntimeError("key/value must be [num_seqs, num_kv_heads, head_size] of one dtype")
-    if key.shape[1] != geom.num_kv_heads or key.shape[2] != geom.head_size:
-        raise RuntimeError(f"key shape {tuple(key.shape)} does not match cache (Hkv={geom.num_kv_heads}, D={geom.head_size})")
-    if key.stride(2) != 1 or value.stride(2) != 1:
-        raise RuntimeError("key/value head dim must be contiguous")
-    if seqused_k.dtype != torch.int32 or block_table.dtype != torch.int32 or not seqused_k.is_contiguous():
-        raise RuntimeError("seqused_k (contiguous) and block_table must be int32")
-    if block_table.shape[0] < num_seqs or block_table.stride(1) != 1:
-        raise RuntimeError("block_table needs num_seqs contiguous rows")
-    if block_table.shape[1] * geom.block_size < int(max_seqlen_k):
-        raise RuntimeError("block_table rows are too short for max_seqlen_k")
-    if slot_mapping is not None:
-        _require_cuda(slot_mapping)
-        if slot_mapping.dtype != torch.int64 or slot_mapping.dim() != 1 or slot_mapping.shape[0] < num_seqs \
-                or not slot_mapping.is_contiguous():
-            raise RuntimeError("slot_mapping must be a contiguous int64 tensor with one entry per sequence")
-    if num_seqs == 0:
-        return
-    num_q_heads = q.shape[1]
-    if lse is not None and (lse.dtype != torch.float32 or not lse.is_contiguous()
-                            or tuple(lse.shape) != (num_seqs, num_q_heads)):
-        raise RuntimeError("lse must be a contiguous float32 [num_seqs, num_q_heads] tensor")
-    _check_sinks(sinks, num_q_heads, q.device)
-    _check_sinks(alibi_slopes, num_q_heads, q.device, "alibi_slopes")
-    lib = _C.load()
-    g = geom.as_struct()
+    if q.dim() != 3 or key.dim() != 3:
+        raise RuntimeError("q/out must be [num_seqs, num_q_heads, head_size] and key/value [num_seqs, num_kv_heads, head_size]")
     if workspace is None:
-        workspace = _default_workspace(dev, paged_attn_workspace_bytes(num_seqs, num_q_heads, geom.head_size, dev))
-    with _on_device(dev):
-        rc = lib.kvq_paged_attn_int8_fused_write(
-            _ptr(out), _dtype_code(out, "out"), out.stride(0), out.stride(1),
-            _ptr(q), _dtype_code(q, "q"), q.stride(0), q.stride(1),
-            _ptr(key), _ptr(value), _dtype_code(key, "key"), key.stride(0), key.stride(1), value.stride(0),
-            value.stride(1), eps_for_dtype(key.dtype), ctypes.c_void_p(geom.base_ptr), ctypes.byref(g),
-            _ptr(block_table), block_table.stride(0), _ptr(seqused_k), _ptr(slot_mapping), num_seqs, num_q_heads,
-            float(softmax_scale), window, softcap, _ptr(sinks), _ptr(alibi_slopes), _ptr(lse), _ptr(workspace),
-            workspace.numel() * workspace.element_size(), _stream(dev))
-    _C.check(rc, "decode_attention_with_cache_update")
+        workspace = _default_workspace(dev, paged_attn_workspace_bytes(max(seqused_k.shape[0], 1), q.shape[1],
+                                                                       geom.head_size, dev))
+    _C.binding().decode_with_update(
+        q, key, value, out, -1, 0, k, geom.struct_addr, geom.base_ptr, seqused_k, block_table, int(max_seqlen_k),
+        float(softmax_scale), window, softcap, sinks, alibi_slopes, lse, workspace, slot_mapping)
 
 
 def paged_attention_v2(
@@ -738,26 +653,9 @@ def concat_and_cache_mla(kv_c: torch.Tensor, k_pe: torch.Tensor, kv_cache: torch
     kv_c ``[T, R]``, k_pe ``[T, P]``; kv_cache is the int8 latent cache ``(nb, bs, R+P+4)``."""
     if kv_cache_dtype != "int8_per_token":
         raise NotImplementedError(f"kv_cache_dtype {kv_cache_dtype!r}: only int8_per_token is built")
-    dev = _require_cuda(kv_c, k_pe, kv_cache, slot_mapping)
+    _require_cuda(kv_c, kv_cache)
     geom = geometry or mla_geometry(kv_cache, kv_c.shape[-1])
-    if kv_c.dim() != 2 or k_pe.dim() != 2 or kv_c.dtype != k_pe.dtype:
-        raise RuntimeError("kv_c [T, R] and k_pe [T, P] must be 2-D of one dtype")
-    if kv_c.shape[1] != geom.kv_lora_rank or k_pe.shape[1] != geom.rope_dim:
-        raise RuntimeError("kv_c / k_pe widths do not match the cache entry")
-    if kv_c.stride(1) != 1 or k_pe.stride(1) != 1:
-        raise RuntimeError("kv_c / k_pe rows must be contiguous")
-    if slot_mapping.dtype != torch.int64 or not slot_mapping.is_contiguous():
-        raise RuntimeError("slot_mapping must be contiguous int64")
-    T = slot_mapping.shape[0]
-    if T > kv_c.shape[0] or T > k_pe.shape[0]:
-        raise RuntimeError("slot_mapping is longer than kv_c / k_pe")
-    g = geom.as_struct()
-    with _on_device(dev):
-        rc = _C.load().kvq_concat_and_cache_mla_int8(_ptr(kv_c), _ptr(k_pe), _dtype_code(kv_c, "kv_c"),
-                                                     kv_c.stride(0), k_pe.stride(0), ctypes.c_void_p(geom.base_ptr),
-                                                     ctypes.byref(g), _ptr(slot_mapping), T,
-                                                     eps_for_dtype(kv_c.dtype), _stream(dev))
-    _C.check(rc, "concat_and_cache_mla")
+    _C.binding().mla_cache_update(kv_c, k_pe, kv_cache, slot_mapping, geom.struct_addr, geom.base_ptr, 0)
 
 
 def concat_and_cache_mla_rope_fused(positions: torch.Tensor, q_pe: torch.Tensor, k_pe: torch.Tensor,
@@ -949,32 +847,13 @@ def mla_decode_absorb_int8(q_nope: torch.Tensor, W_UK_T: torch.Tensor, q_pe: tor
     (vllm_metax/model_executor/layers/attention/mla_attention.py:835-848) done inside the launch: q_nope
     ``[B, H, P]``, W_UK_T ``[H, P, R]``, q_pe ``[B, H, rope]`` (bf16 or fp16, one dtype); the product is
     written directly as the decode's int8 query operands.  o ``[B, H, R]``, lse ``[B, H]`` fp32 or None."""
-    dev = _require_cuda(q_nope, W_UK_T, q_pe, kv_cache, o, lse, block_table, seq_lens, workspace)
+    dev = _require_cuda(q_nope, kv_cache)
     geom = geometry or mla_geometry(kv_cache, kv_lora_rank)
-    B, H, P = q_nope.shape
-    if tuple(W_UK_T.shape) != (H, P, geom.kv_lora_rank) or tuple(q_pe.shape) != (B, H, geom.rope_dim):
-        raise RuntimeError("W_UK_T must be [H, P, R] and q_pe [B, H, rope]")
-    if not (q_nope.dtype == W_UK_T.dtype == q_pe.dtype):
-        raise RuntimeError("q_nope, W_UK_T and q_pe must share a dtype")
-    if q_nope.stride(2) != 1 or W_UK_T.stride(2) != 1 or q_pe.stride(2) != 1:
-        raise RuntimeError("last dims must be contiguous")
-    if tuple(o.shape) != (B, H, geom.kv_lora_rank) or not o.is_contiguous():
-        raise RuntimeError("o must be contiguous [B, H, R]")
-    if seq_lens.dtype != torch.int32 or block_table.dtype != torch.int32 or block_table.stride(1) != 1:
-        raise RuntimeError("seq_lens and block_table must be int32")
-    if lse is not None and (lse.dtype != torch.float32 or tuple(lse.shape) != (B, H) or not lse.is_contiguous()):
-        raise RuntimeError("lse must be contiguous float32 [B, H]")
     if workspace is None:
+        B, H, _ = q_nope.shape
         workspace = _default_workspace(dev, mla_decode_workspace_bytes(B, H, geom.kv_lora_rank))
-    g = geom.as_struct()
-    with _on_device(dev):
-        rc = _C.load().kvq_mla_decode_absorb_int8(
-            _ptr(o), _dtype_code(o, "o"), _ptr(lse), _ptr(q_nope), _dtype_code(q_nope, "q_nope"), q_nope.stride(0),
-            q_nope.stride(1), P, _ptr(W_UK_T), W_UK_T.stride(0), W_UK_T.stride(1), _ptr(q_pe), q_pe.stride(0),
-            q_pe.stride(1), ctypes.c_void_p(geom.base_ptr), ctypes.byref(g), _ptr(block_table), block_table.stride(0),
-            _ptr(seq_lens), B, H, float(sm_scale), _ptr(workspace), workspace.numel() * workspace.element_size(),
-            _stream(dev))
-    _C.check(rc, "mla_decode_absorb_int8")
+    _C.binding().mla_decode_absorb(q_nope, W_UK_T, q_pe, kv_cache, o, lse, 0, block_table, seq_lens, float(sm_scale),
+                                   workspace, geom.struct_addr, geom.base_ptr)
 
 
 def mla_v_up_proj(x: torch.Tensor, W_UV: torch.Tensor, out: torch.Tensor) -> None:
@@ -982,31 +861,7 @@ def mla_v_up_proj(x: torch.Tensor, W_UV: torch.Tensor, out: torch.Tensor) -> Non
     reference's ``_v_up_proj`` (vllm_metax/model_executor/layers/attention/mla_attention.py:1087-1109)
     for unquantised weights.  x ``[B, H, L]``, W_UV ``[H, L, V]``, out ``[B, H, V]`` or ``[B, H * V]``;
     bf16 or fp16, one dtype; L and V multiples of 128."""
-    dev = _require_cuda(x, W_UV, out)
-    if x.dim() != 3 or W_UV.dim() != 3:
-        raise RuntimeError("mla_v_up_proj takes x [B, H, L] and W_UV [H, L, V]")
-    B, H, L = x.shape
-    V = W_UV.shape[2]
-    if tuple(W_UV.shape) != (H, L, V):
-        raise RuntimeError("W_UV must be [H, L, V]")
-    if out.dim() == 2:
-        if tuple(out.shape) != (B, H * V) or out.stride(1) != 1:
-            raise RuntimeError("out must be [B, H * V] with a contiguous last dim")
-        o_sb, o_sh = out.stride(0), V
-    else:
-        if tuple(out.shape) != (B, H, V) or out.stride(2) != 1:
-            raise RuntimeError("out must be [B, H, V] with a contiguous last dim")
-        o_sb, o_sh = out.stride(0), out.stride(1)
-    if not (x.dtype == W_UV.dtype == out.dtype):
-        raise RuntimeError("x, W_UV and out must share a dtype")
-    if x.stride(2) != 1 or W_UV.stride(2) != 1:
-        raise RuntimeError("last dims must be contiguous")
-    if B == 0:
-        return
-    with _on_device(dev):
-        rc = _C.load().kvq_mla_v_up_proj(_ptr(out), o_sb, o_sh, _ptr(x), _dtype_code(x, "x"), x.stride(0), x.stride(1),
-                                         _ptr(W_UV), W_UV.stride(0), W_UV.stride(1), B, H, L, V, _stream(dev))
-    _C.check(rc, "mla_v_up_proj")
+    _C.binding().mla_v_up_proj(x, -1, W_UV, out)
 
 
 def concat_mla_q(ql_nope: torch.Tensor, q_pe: torch.Tensor, q_out: torch.Tensor) -> None:

@@ -18,6 +18,7 @@ scales, which keeps every row 16-byte aligned and a block opaque-copyable.
 """
 from __future__ import annotations
 
+import ctypes
 import os
 from dataclasses import dataclass
 
@@ -210,6 +211,15 @@ class CacheGeometry:
         return st
 
     @property
+    def struct_addr(self) -> int:
+        """Address of :meth:`as_struct`, as the native op layer takes it (valid while this object lives)."""
+        got = self.__dict__.get("_struct_addr")
+        if got is None:
+            got = ctypes.addressof(self.as_struct())
+            object.__setattr__(self, "_struct_addr", got)
+        return got
+
+    @property
     def record_bytes(self) -> int:
         return 2 * (self.code_bytes + SCALE_BYTES)
 
@@ -330,6 +340,15 @@ class MlaGeometry:
                             self.rope_dim, self.block_size, 0)
             object.__setattr__(self, "_struct", st)
         return st
+
+    @property
+    def struct_addr(self) -> int:
+        """Address of :meth:`as_struct`, as the native op layer takes it (valid while this object lives)."""
+        got = self.__dict__.get("_struct_addr")
+        if got is None:
+            got = ctypes.addressof(self.as_struct())
+            object.__setattr__(self, "_struct_addr", got)
+        return got
 
 
 def mla_geometry(cache: torch.Tensor, kv_lora_rank: int) -> MlaGeometry:

@@ -16,6 +16,7 @@ from typing import ClassVar
 
 import torch
 
+from .... import _C
 from .... import _custom_ops as ops
 from ....kv_cache_interface import KVQuantMode, get_kv_quant_mode, kv_cache_uses_per_token_head_scales
 from ....layout import (
@@ -332,12 +333,13 @@ class Int8AttentionImpl(_ImplBase):
         if sliding_window is not None and sliding_window < 1:
             raise ValueError(f"sliding_window must be >= 1, got {sliding_window}")
         self.sliding_window = (-1, -1) if sliding_window is None else (sliding_window - 1, 0)
+        self._window = self.sliding_window[0] + 1   # keys a query sees; 0 = all
         self.logits_soft_cap = float(logits_soft_cap or 0)
         self._kv_quant_mode = get_kv_quant_mode(kv_cache_dtype)
         self._is_per_token_head_quant = True
         # per-cache views and byte geometry, built when a cache tensor is first seen
         self._filled: dict = {}          # (storage id, offset, shape, strides) -> weak reference to the storage
-        self._views_for = None
+        self._bound = None               # identity of the cache the views below belong to (a native object)
         self._views_storage = None
         self._key_cache = self._value_cache = None
         self._k_scale_cache = self._v_scale_cache = None
@@ -386,10 +388,11 @@ class Int8AttentionImpl(_ImplBase):
         the identity of their storage through weak references, so coming back to a cache never wipes
         the scales written into it, and a new allocation that lands on a freed cache's address is
         filled like any new cache."""
+        native = _C.binding()
+        if native.is_cache(self._bound, kv_cache):
+            return
         storage = kv_cache.untyped_storage()
         key = (storage._cdata, kv_cache.storage_offset(), tuple(kv_cache.shape), tuple(kv_cache.stride()))
-        if self._views_for == key and self._views_storage is storage:
-            return
         seen = self._filled.get(key)
         k_scale, v_scale = scale_views(kv_cache)
         if seen is None or seen() is not storage:
@@ -400,7 +403,8 @@ class Int8AttentionImpl(_ImplBase):
         key_cache, value_cache = key_value_views(kv_cache)
         self._key_cache, self._value_cache, self._k_scale_cache, self._v_scale_cache = key_cache, value_cache, k_scale, v_scale
         self._geometry = geometry_from_views(key_cache, value_cache, k_scale, v_scale, code_type_of(self._kv_quant_mode))
-        self._views_for, self._views_storage = key, storage
+        # the storage is held, so the identity cannot become another allocation's
+        self._bound, self._views_storage = native.cache_ref(kv_cache), storage
 
     def _pth_key_value_caches(self, kv_cache: torch.Tensor):
         """(nb, bs, Hkv, D+4) int8 views of the K and V halves (:729-739)."""
@@ -411,10 +415,9 @@ class Int8AttentionImpl(_ImplBase):
     def do_kv_cache_update(self, layer, key: torch.Tensor, value: torch.Tensor, kv_cache: torch.Tensor,
                            slot_mapping: torch.Tensor) -> None:
         """Quantise-on-write of this step's tokens; mutates ``kv_cache`` in place (:788-815)."""
-        key_cache, value_cache = self._pth_key_value_caches(kv_cache)
-        ops.reshape_and_cache_flash_per_token_head_quant(
-            key, value, key_cache, value_cache, self._k_scale_cache, self._v_scale_cache, slot_mapping,
-            kv_quant_mode=self._kv_quant_mode, geometry=self._geometry)
+        self._ensure_scale_caches(kv_cache)
+        geom = self._geometry
+        _C.binding().cache_update(key, value, kv_cache, slot_mapping, geom.struct_addr, geom.base_ptr)
 
     def do_rope_and_kv_cache_update(self, *args, **kwargs):
         raise NotImplementedError("fused rope + cache update is not built (the reference raises here too)")
@@ -431,20 +434,30 @@ class Int8AttentionImpl(_ImplBase):
             return output.fill_(0)
         if attn_metadata.use_cascade:
             raise NotImplementedError("cascade attention is not supported")
-        n = attn_metadata.num_actual_tokens
-        key_cache, value_cache = self._pth_key_value_caches(kv_cache)
-        q = query[:n].view(n, self.num_heads, self.head_size)
-        out = output[:n].view(n, self.num_heads, self.head_size)
-        ops.unified_attention(
-            q=q, k=key_cache, v=value_cache, out=out, cu_seqlens_q=attn_metadata.query_start_loc,
-            max_seqlen_q=attn_metadata.max_query_len, seqused_k=attn_metadata.seq_lens,
-            max_seqlen_k=attn_metadata.max_seq_len, softmax_scale=self.scale, causal=attn_metadata.causal,
-            window_size=self.sliding_window, block_table=attn_metadata.block_table, softcap=self.logits_soft_cap,
-            kv_quant_mode=self._kv_quant_mode, k_scale_cache=self._k_scale_cache, v_scale_cache=self._v_scale_cache,
-            workspace=attn_metadata.workspace, geometry=self._geometry,
-            has_decode_rows=getattr(attn_metadata, "has_decode_rows", True), sinks=self._sinks_on(q.device),
-            alibi_slopes=self._alibi_on(q.device), prefill_splits=getattr(attn_metadata, "prefill_splits", 1))
+        self._ensure_scale_caches(kv_cache)
+        geom = self._geometry
+        md = attn_metadata
+        workspace = md.workspace
+        if workspace is None:
+            workspace = self._own_workspace(query, md)
+        _C.binding().paged_attention(
+            query, output, md.num_actual_tokens, self.num_heads, kv_cache, geom.struct_addr, geom.base_ptr,
+            md.query_start_loc, md.seq_lens, md.block_table, md.max_query_len, md.max_seq_len, self.scale,
+            (1 if md.causal else 0) | (0 if getattr(md, "has_decode_rows", True) else 2), self._window,
+            self.logits_soft_cap, self._sinks_on(query.device) if self.sinks is not None else None,
+            self._alibi_on(query.device) if self.alibi_slopes is not None else None, None, workspace,
+            getattr(md, "prefill_splits", 1))
         return output
+
+    def _own_workspace(self, query, md):
+        """Scratch for metadata that brings none (the builder's always does): the op layer's per-device buffer."""
+        num_seqs, splits = max(md.seq_lens.shape[0], 1), getattr(md, "prefill_splits", 1)
+        if splits > 1 and md.max_query_len > 1:
+            need = ops.split_prefill_workspace_bytes(num_seqs, self.num_heads, self.head_size, md.num_actual_tokens,
+                                                     splits, query.device)
+        else:
+            need = ops.paged_attn_workspace_bytes(num_seqs, self.num_heads, self.head_size, query.device)
+        return ops._default_workspace(query.device, need)
 
 
 class Int8FusedUpdateAttentionImpl(Int8AttentionImpl):
@@ -469,18 +482,17 @@ class Int8FusedUpdateAttentionImpl(Int8AttentionImpl):
             if key is not None and value is not None:
                 self.do_kv_cache_update(layer, key[:n], value[:n], kv_cache, attn_metadata.slot_mapping[:n])
             return super().forward(layer, query, key, value, kv_cache, attn_metadata, output)
-        key_cache, value_cache = self._pth_key_value_caches(kv_cache)
-        ops.decode_attention_with_cache_update(
-            q=query[:n].view(n, self.num_heads, self.head_size),
-            key=key[:n].view(n, self.num_kv_heads, self.head_size),
-            value=value[:n].view(n, self.num_kv_heads, self.head_size),
-            k=key_cache, v=value_cache, out=output[:n].view(n, self.num_heads, self.head_size),
-            seqused_k=attn_metadata.seq_lens, max_seqlen_k=attn_metadata.max_seq_len, softmax_scale=self.scale,
-            block_table=attn_metadata.block_table, k_scale_cache=self._k_scale_cache, v_scale_cache=self._v_scale_cache,
-            window_size=self.sliding_window, softcap=self.logits_soft_cap, kv_quant_mode=self._kv_quant_mode,
-            workspace=attn_metadata.workspace, geometry=self._geometry,
-            slot_mapping=attn_metadata.slot_mapping[:n] if attn_metadata.slot_mapping is not None else None,
-            sinks=self._sinks_on(query.device), alibi_slopes=self._alibi_on(query.device))
+        self._ensure_scale_caches(kv_cache)
+        geom = self._geometry
+        md = attn_metadata
+        workspace = md.workspace
+        if workspace is None:
+            workspace = self._own_workspace(query, md)
+        _C.binding().decode_with_update(
+            query, key, value, output, n, self.num_heads, kv_cache, geom.struct_addr, geom.base_ptr, md.seq_lens,
+            md.block_table, md.max_seq_len, self.scale, self._window, self.logits_soft_cap,
+            self._sinks_on(query.device) if self.sinks is not None else None,
+            self._alibi_on(query.device) if self.alibi_slopes is not None else None, None, workspace, md.slot_mapping)
         return output
 
 

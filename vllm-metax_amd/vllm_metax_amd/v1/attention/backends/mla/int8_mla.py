@@ -15,6 +15,7 @@ from typing import ClassVar
 
 import torch
 
+from ..... import _C
 from ..... import _custom_ops as ops
 from .....kv_cache_interface import INT8_PER_TOKEN
 from .....layout import mla_cache_shape, mla_geometry
@@ -277,22 +278,27 @@ class Int8MLAImpl(_MLAImplBase):
         self.kv_cache_dtype = kv_cache_dtype
         self.supports_quant_query_input = False
         self._geometry = None
-        self._geometry_for = None
+        self._bound = None       # identity of the cache the geometry belongs to (a native object)
         self._sm_count = None
 
     def _geom(self, cache: torch.Tensor):
-        key = (cache.data_ptr(), tuple(cache.shape))
-        if self._geometry_for != key:
+        native = _C.binding()
+        if not native.is_cache(self._bound, cache):
             self._geometry = mla_geometry(cache, self.kv_lora_rank)
-            self._geometry_for = key
+            self._bound = native.cache_ref(cache)
         return self._geometry
 
     def do_kv_cache_update(self, kv_c_normed: torch.Tensor, k_pe: torch.Tensor, kv_cache: torch.Tensor,
                            slot_mapping: torch.Tensor, kv_cache_dtype: str | None = None, k_scale=None) -> None:
         """Quantise-on-write of the latent rows, call shape of the reference's MLA layer
         (vllm_metax/model_executor/layers/attention/mla_attention.py:633-640)."""
-        ops.concat_and_cache_mla(kv_c_normed, k_pe.reshape(k_pe.shape[0], -1), kv_cache, slot_mapping,
-                                 kv_cache_dtype or self.kv_cache_dtype, k_scale, geometry=self._geom(kv_cache))
+        dtype = kv_cache_dtype or self.kv_cache_dtype
+        if dtype != INT8_PER_TOKEN:
+            raise NotImplementedError(f"kv_cache_dtype {dtype!r}: only int8_per_token is built")
+        if k_pe.dim() != 2 and not (k_pe.dim() == 3 and k_pe.shape[1] == 1):
+            k_pe = k_pe.reshape(k_pe.shape[0], -1)
+        geom = self._geom(kv_cache)
+        _C.binding().mla_cache_update(kv_c_normed, k_pe, kv_cache, slot_mapping, geom.struct_addr, geom.base_ptr, 1)
 
     def forward_mqa(self, q, kv_c_and_k_pe_cache: torch.Tensor, attn_metadata, layer=None, new_rows=None):
         """``q`` [B, H, 576] or ``(ql_nope [B, H, 512], q_pe [B, H, 64])``; returns
@@ -431,38 +437,60 @@ class Int8MLADecodeCaller:
     def v_up_proj(self, x: torch.Tensor, out: torch.Tensor) -> None:
         """``x [B, N, L]`` -> ``out [B, N * V]``."""
         rows = x.numel() // (self.num_heads * self.kv_lora_rank)
-        if x.dtype == torch.float32 or self.kv_lora_rank % 128 != 0 or self.v_head_dim % 128 != 0 \
-                or rows * self.num_heads > self.KERNEL_MAX_ROWS_X_HEADS:
+        if not self._up_proj_kernel_takes(rows, x.dtype):
             self.v_up_proj_library(x, out)
             return
         ops.mla_v_up_proj(x.view(-1, self.num_heads, self.kv_lora_rank), self.W_UV,
                           out.view(-1, self.num_heads, self.v_head_dim))
 
+    def _up_proj_kernel_takes(self, rows: int, dtype: torch.dtype) -> bool:
+        return dtype != torch.float32 and self.kv_lora_rank % 128 == 0 and self.v_head_dim % 128 == 0 \
+            and rows * self.num_heads <= self.KERNEL_MAX_ROWS_X_HEADS
+
+    def _decode_buffers(self, mqa_q_nope: torch.Tensor, attn_metadata):
+        """``(o, lse)`` with at least the batch's rows: the builder's when the metadata carries fitting ones."""
+        B = mqa_q_nope.shape[0]
+        o, lse = getattr(attn_metadata, "decode_out", None), getattr(attn_metadata, "decode_lse", None)
+        if o is not None and lse is not None and o.dtype == mqa_q_nope.dtype and o.shape[0] >= B \
+                and o.shape[1] == self.num_heads and o.shape[2] == self.kv_lora_rank:
+            return o, lse
+        return (torch.empty((B, self.num_heads, self.kv_lora_rank), dtype=mqa_q_nope.dtype, device=mqa_q_nope.device),
+                torch.empty((B, self.num_heads), dtype=torch.float32, device=mqa_q_nope.device))
+
     def decode_absorbed(self, mqa_q_nope: torch.Tensor, mqa_q_pe: torch.Tensor, kv_cache: torch.Tensor, attn_metadata):
         """Absorption + decode in one launch; returns ``(o [B, N, L], lse [B, N])`` like ``forward_mqa``
         (views of the builder's buffers when the metadata carries them: valid until the next decode call on
         this metadata, the next layer's included)."""
-        impl = self.impl
+        o, lse = self._absorb_into_buffers(mqa_q_nope, mqa_q_pe, kv_cache, attn_metadata)
         B = mqa_q_nope.shape[0]
-        o_buf, lse_buf = getattr(attn_metadata, "decode_out", None), getattr(attn_metadata, "decode_lse", None)
-        if o_buf is not None and lse_buf is not None and o_buf.dtype == mqa_q_nope.dtype and o_buf.shape[0] >= B \
-                and o_buf.shape[1] == self.num_heads and o_buf.shape[2] == self.kv_lora_rank:
-            o, lse = o_buf[:B], lse_buf[:B]
-        else:
-            o = torch.empty((B, self.num_heads, self.kv_lora_rank), dtype=mqa_q_nope.dtype, device=mqa_q_nope.device)
-            lse = torch.empty((B, self.num_heads), dtype=torch.float32, device=mqa_q_nope.device)
-        ops.mla_decode_absorb_int8(mqa_q_nope, self.W_UK_T, mqa_q_pe, kv_cache, o, lse, attn_metadata.decode.block_table,
-                                   attn_metadata.decode.seq_lens, impl.scale, self.kv_lora_rank,
-                                   workspace=getattr(attn_metadata, "workspace", None), geometry=impl._geom(kv_cache))
+        return o.narrow(0, 0, B), lse.narrow(0, 0, B)
+
+    def _absorb_into_buffers(self, mqa_q_nope, mqa_q_pe, kv_cache, attn_metadata):
+        """The launch behind ``decode_absorbed``; the buffers it returns may have more rows than the batch."""
+        impl = self.impl
+        o, lse = self._decode_buffers(mqa_q_nope, attn_metadata)
+        workspace = getattr(attn_metadata, "workspace", None)
+        if workspace is None:
+            workspace = ops._default_workspace(mqa_q_nope.device, ops.mla_decode_workspace_bytes(
+                mqa_q_nope.shape[0], self.num_heads, self.kv_lora_rank))
+        geom = impl._geom(kv_cache)
+        _C.binding().mla_decode_absorb(mqa_q_nope, self.W_UK_T, mqa_q_pe, kv_cache, o, lse, 1, attn_metadata.decode.block_table,
+                                       attn_metadata.decode.seq_lens, impl.scale, workspace, geom.struct_addr,
+                                       geom.base_ptr)
         return o, lse
 
     def forward_decode(self, mqa_q_nope: torch.Tensor, mqa_q_pe: torch.Tensor, kv_cache: torch.Tensor,
                        attn_metadata, out: torch.Tensor):
         """q_nope ``[B, N, P]``, q_pe ``[B, N, rope]`` (already rotated), writes ``out [B, N * V]``;
         returns the decode's ``lse [B, N]``."""
-        if mqa_q_nope.dtype == torch.float32 or mqa_q_nope.shape[0] * self.num_heads > self.ABSORB_MAX_ROWS_X_HEADS:
+        B = mqa_q_nope.shape[0]
+        if mqa_q_nope.dtype == torch.float32 or B * self.num_heads > self.ABSORB_MAX_ROWS_X_HEADS:
             attn_out, lse = self.impl.forward_mqa((self.absorb_q(mqa_q_nope), mqa_q_pe), kv_cache, attn_metadata)
+            self.v_up_proj(attn_out, out)
+            return lse
+        attn_out, lse = self._absorb_into_buffers(mqa_q_nope, mqa_q_pe, kv_cache, attn_metadata)
+        if out.dim() == 2 and self._up_proj_kernel_takes(B, attn_out.dtype):
+            _C.binding().mla_v_up_proj(attn_out, B, self.W_UV, out)
         else:
-            attn_out, lse = self.decode_absorbed(mqa_q_nope, mqa_q_pe, kv_cache, attn_metadata)
-        self.v_up_proj(attn_out, out)
-        return lse
+            self.v_up_proj(attn_out.narrow(0, 0, B), out)
+        return lse.narrow(0, 0, B)
