@@ -47,20 +47,29 @@ __device__ __forceinline__ uint32_t bytes_to_half2(uint32_t x, bool upper) {
   return perm(0x64646464u, x, upper ? 0x04030402u : 0x04010400u);
 }
 
-// Two e4m3fn code bytes of x -> two fp16 values code / 2^8: the byte's 7 magnitude bits sit in an fp16
-// pattern at bits 7 .. 13 and the sign at bit 15; as an fp16 number that pattern is the code's value
-// times 2^-8 (the exponent biases differ by 15 - 7), exactly, subnormal codes included.  The 2^8 is put
-// back with the scales.
+// Two e4m3fn code bytes of x -> two fp16 values code / 2^8, exact for every code, subnormal ones included; the 2^8 is
+// put back with the scales.  One conversion instruction, as cheap as the int8 path's byte permute (2.5 ns against
+// 7.6 ns for the same result from shifts and masks, two waves on a SIMD).  It turns the code 0x7f / 0xff, which the
+// writer never stores, into a NaN: GARBAGE = the bytes may be anything (a slot past the end of a sequence), and a NaN
+// must not come out, since 0 x NaN would reach the output.  There the byte's 7 magnitude bits are put at bits 7 .. 13
+// of an fp16 pattern and the sign at bit 15, which is the same number (the exponent biases differ by 15 - 7).
+template <bool GARBAGE = false>
 __device__ __forceinline__ uint32_t fp8_bytes_to_half2(uint32_t x, bool upper) {
-  const uint32_t y = perm(0u, x, upper ? 0x030c020cu : 0x010c000cu);   // the two bytes in the high byte of each half
-  return (y & 0x80008000u) | ((y >> 1) & 0x3f803f80u);
+  if constexpr (GARBAGE) {
+    const uint32_t y = perm(0u, x, upper ? 0x030c020cu : 0x010c000cu);   // the two bytes in the high byte of each half
+    return (y & 0x80008000u) | ((y >> 1) & 0x3f803f80u);
+  }
+  constexpr float kUnit = 1.0f / 256.0f;
+  const half2_t v = upper ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(x, kUnit, true)
+                          : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(x, kUnit, false);
+  return __builtin_bit_cast(uint32_t, v);
 }
 
 // Two code bytes -> the two fp16 numbers the MFMA sees, for either kind of code (int8 bytes are
 // expected already ^ 0x80, see prep_codes).
-template <bool FP8>
+template <bool FP8, bool GARBAGE = false>
 __device__ __forceinline__ uint32_t codes_to_half2(uint32_t x, bool upper) {
-  if constexpr (FP8) return fp8_bytes_to_half2(x, upper);
+  if constexpr (FP8) return fp8_bytes_to_half2<GARBAGE>(x, upper);
   else return bytes_to_half2(x, upper);
 }
 template <bool FP8>
@@ -89,17 +98,23 @@ __device__ __forceinline__ half8_t dequant8(uint32_t lo, uint32_t hi) {
 // so the eight dims of a dword come out in the order 0 4 1 5 2 6 3 7 -- the order in which the query operand of an
 // int4 tile is laid out as well (nibble_order).
 constexpr float kCodeBiasInt4 = 1032.0f;
-__device__ __forceinline__ uint32_t nibbles_to_half2(uint32_t y, int k) {
-  return ((y >> (4 * k)) & 0x000f000fu) | 0x64006400u;
+__device__ __forceinline__ uint32_t nibbles_to_half2(uint32_t y, int k, uint32_t mask = 0x000f000fu) {
+  return ((y >> (4 * k)) & mask) | 0x64006400u;
 }
-__device__ __forceinline__ half8_t dequant8_int4(uint32_t x) {
+__device__ __forceinline__ half8_t dequant8_int4(uint32_t x, uint32_t mask) {
   const uint32_t y = x ^ 0x88888888u;
   u32x4 r;
-  r.x = nibbles_to_half2(y, 0);
-  r.y = nibbles_to_half2(y, 1);
-  r.z = nibbles_to_half2(y, 2);
-  r.w = nibbles_to_half2(y, 3);
+  r.x = nibbles_to_half2(y, 0, mask);
+  r.y = nibbles_to_half2(y, 1, mask);
+  r.z = nibbles_to_half2(y, 2, mask);
+  r.w = nibbles_to_half2(y, 3, mask);
   return __builtin_bit_cast(half8_t, r);
+}
+// A constant the compiler does not see through, in a vector register: an instruction takes one scalar or literal
+// operand, so "x & constant | constant" is one instruction only if a constant lies in a vector register.
+__device__ __forceinline__ uint32_t in_vgpr(uint32_t x) {
+  asm volatile("" : "+v"(x));
+  return x;
 }
 // MFMA k position j of an int4 operand holds dim nibble_order(j) of the dword's eight.
 __host__ __device__ constexpr int nibble_order(int j) { return (j >> 1) + 4 * (j & 1); }
@@ -167,16 +182,32 @@ struct AttnIO {
   float cap_k;        // 2 * log2(e) / cap_c
 };
 
-// cap * tanh(x / cap) for a log2-domain logit x.  Away from zero tanh(u) = 1 - 2 / (exp(2u) + 1), which
-// saturates cleanly at +-cap but whose absolute error is about cap * 2^-23 whatever x is; for |u| < 1/8
-// the odd series u (1 - u^2/3 + 2 u^4/15) takes over (next term 17/315 u^6 < 2e-7), so the result is
-// accurate RELATIVE to x for every cap, and a cap far above the logits is the identity.
-__device__ __forceinline__ float soft_cap(float x, float cap_c, float cap_k) {
-  const float big = cap_c - 2.0f * cap_c * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x * cap_k) + 1.0f);
-  const float u = x * cap_k * 0.34657359f;  // x / cap_c: cap_k = 2 log2(e) / cap_c
-  const float u2 = u * u;
-  const float small = x * (1.0f + u2 * (-0.33333334f + u2 * 0.13333334f));
-  return fabsf(u) < 0.125f ? small : big;
+// cap * tanh(x / cap) of a lane's N log2-domain logits (cap_c = 0: no cap).  For u = |x / cap| < 1/4 the odd series
+// through u^9 (next term 1382/155925 u^10 < 1e-8), beyond it tanh(u) = 1 - 2 / (exp(2u) + 1), which saturates cleanly
+// at +-cap and whose absolute error of about cap * 2^-23 is then small relative to x too; so a cap far above the
+// logits is the identity.  Logits are mostly small next to the cap: the exponentials are only computed when some lane
+// of the wave needs one.
+template <int N>
+__device__ __forceinline__ void soft_cap(float (&x)[N], float cap_c, float cap_k) {
+  if (cap_c == 0.f) return;   // uniform
+  const float inv = cap_k * 0.34657359f;  // 1 / cap_c: cap_k = 2 log2(e) / cap_c
+  const float near = 0.25f * cap_c;
+  float top = 0.f, y[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    top = fmaxf(top, fabsf(x[i]));
+    const float u = x[i] * inv, u2 = u * u;
+    y[i] = x[i] * (1.0f + u2 * (-0.33333334f + u2 * (0.13333334f + u2 * (-0.053968254f + u2 * 0.021869488f))));
+  }
+  if (__builtin_amdgcn_ballot_w64(!(top < near)) != 0) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const float big = cap_c - 2.0f * cap_c * __builtin_amdgcn_rcpf(__builtin_amdgcn_exp2f(x[i] * cap_k) + 1.0f);
+      y[i] = fabsf(x[i]) < near ? y[i] : big;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = y[i];
 }
 
 // First token a decode row of a `len`-token sequence sees.
@@ -243,6 +274,7 @@ struct LaneOffsets {
   uint32_t g_flat;    // HBM: 16 * lane
   uint32_t l_flat[9];
   uint32_t l_flat_split;
+  uint32_t nib_lo, nib_hi;   // int4 codes: 0x000f000f and 0x00f000f0 (see in_vgpr)
 };
 
 // CODE: what a code byte is (KVQ_CODE_INT8 or KVQ_CODE_FP8_E4M3).  An int8 code enters the MFMA as
@@ -283,6 +315,8 @@ struct DecodeTile {
     o.l_v = (uint32_t)(4 * g * PITCH + (DB + 4) + r * VB);
     o.l_sc = (uint32_t)((lane & 31) * PITCH + (lane < 32 ? DB : 2 * DB + 4));
     o.g_flat = (uint32_t)(16 * lane);
+    o.nib_lo = in_vgpr(0x000f000fu);
+    o.nib_hi = in_vgpr(0x00f000f0u);
     o.l_flat_split = 0;
 #pragma unroll
     for (int n = 0; n <= NLD; ++n) {
@@ -376,22 +410,24 @@ struct DecodeTile {
     const uint8_t* p = lds + lo.l_k + mt * 16 * PITCH;
     if constexpr (KSTEPS == 2) {
       const u32x2 w = *reinterpret_cast<const u32x2*>(p);
-      ka[0] = dequant8_int4(w.x);
-      ka[1] = dequant8_int4(w.y);
+      ka[0] = dequant8_int4(w.x, lo.nib_lo);
+      ka[1] = dequant8_int4(w.y, lo.nib_lo);
     } else {
 #pragma unroll
       for (int i = 0; i < KSTEPS / 4; ++i) {
         const u32x4 w = *reinterpret_cast<const u32x4*>(p + 16 * i);
-        ka[4 * i] = dequant8_int4(w.x);
-        ka[4 * i + 1] = dequant8_int4(w.y);
-        ka[4 * i + 2] = dequant8_int4(w.z);
-        ka[4 * i + 3] = dequant8_int4(w.w);
+        ka[4 * i] = dequant8_int4(w.x, lo.nib_lo);
+        ka[4 * i + 1] = dequant8_int4(w.y, lo.nib_lo);
+        ka[4 * i + 2] = dequant8_int4(w.z, lo.nib_lo);
+        ka[4 * i + 3] = dequant8_int4(w.w, lo.nib_lo);
       }
     }
   }
 
   // The V^T operands of the lane's 8 tokens for the four 16-dim tiles that two code bytes hold (unit u = bytes
-  // 2 u, 2 u + 1 of the lane's VB: dims 4 u .. 4 u + 3 of its 2 VB, tile 4 u + n = nibble n), int4 codes.
+  // 2 u, 2 u + 1 of the lane's VB: dims 4 u .. 4 u + 3 of its 2 VB, tile 4 u + n = nibble n), int4 codes.  The odd
+  // nibbles stay where they are in the byte and enter as 1024 + 16 (code ^ 8): their rows of O^T carry 16 (code) +
+  // 1152 instead of code + 1032, which the emission takes out (v_bias, v_unit) -- one shift per dword instead of three.
   __device__ static void v_operands_int4(const LaneOffsets& lo, int u, const uint8_t* lds, half8_t (&va)[4]) {
     uint32_t y[4];
 #pragma unroll
@@ -404,14 +440,19 @@ struct DecodeTile {
     }
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
+      const uint32_t mask = (n & 1) ? lo.nib_hi : lo.nib_lo;
+      const int shift = (n & 2) ? 2 : 0;
       u32x4 av;
-      av.x = nibbles_to_half2(y[0], n);
-      av.y = nibbles_to_half2(y[1], n);
-      av.z = nibbles_to_half2(y[2], n);
-      av.w = nibbles_to_half2(y[3], n);
+      av.x = nibbles_to_half2(y[0], shift, mask);
+      av.y = nibbles_to_half2(y[1], shift, mask);
+      av.z = nibbles_to_half2(y[2], shift, mask);
+      av.w = nibbles_to_half2(y[3], shift, mask);
       va[n] = __builtin_bit_cast(half8_t, av);
     }
   }
+  // What the accumulated rows of output tile dt carry: sum P~ (code x 1 / v_unit + v_bias).
+  __device__ static constexpr float v_bias(int dt) { return FP8 ? 0.f : (INT4 && (dt & 1)) ? kCodeBias : kBias; }
+  __device__ static constexpr float v_unit(int dt) { return INT4 && (dt & 1) ? 1.0f / 16.0f : 1.0f; }
 
   // Token index -> block-table entry / slot, by multiplication (scalar ALU, no divide).
   __device__ static int div_bs(const AttnIO& io, int x) { return (int)__umulhi((uint32_t)x, io.bs_magic); }
@@ -582,11 +623,17 @@ struct DecodeTile {
     const float rel0 = (float)(tok_base - (len - 1));
     float mloc = -INFINITY;
 #pragma unroll
+    for (int j = 0; j < 8; ++j) logit[j] = s[j >> 2][j & 3] * ((j >> 2) ? ks1 : ks0)[j & 3];
+    if constexpr (CAP) {
+      soft_cap(logit, io.cap_c, io.cap_k);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) logit[j] = __builtin_fmaf(ali, rel0 + (float)((j >> 2) * 16 + (j & 3)), logit[j]);
+    }
+#pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        float x = s[mt][i] * (mt ? ks1 : ks0)[i];
-        if constexpr (CAP) x = __builtin_fmaf(ali, rel0 + (float)(mt * 16 + i), soft_cap(x, io.cap_c, io.cap_k));
+        float x = logit[mt * 4 + i];
         if constexpr (MASK) x = ((uint32_t)(tok_base + mt * 16 + i - first) < (uint32_t)(len - first)) ? x : -INFINITY;
         logit[mt * 4 + i] = x;
         mloc = fmaxf(mloc, x);
@@ -629,6 +676,8 @@ struct DecodeTile {
   // Phase 2 of a tile: O^T += (V + 1152)^T . P~^T.  Lane (r, g) reads bytes [r*VB, (r+1)*VB) of
   // tokens 4g+j (j<4) and 16+4g+(j-4) from the LDS window, transposes the 8 x VB byte block in
   // registers (byte permutes), one MFMA per 16-dim tile; sum(P~) comes from a row of ones.
+  // MASK: the tile may hold slots past the end of the sequence, whose bytes may be anything.
+  template <bool MASK>
   __device__ static void pv(const LaneOffsets& lo, half8_t p_op, const uint8_t* lds, State& st) {
     if constexpr (!FP8) {  // fp8 codes carry no bias to take out again
       const half_t one = (half_t)1.0f;
@@ -662,10 +711,10 @@ struct DecodeTile {
       for (int b = 0; b < 4; ++b) {
         u32x4 av;
         const uint32_t* x = (b < 2) ? x0 : x1;
-        av.x = codes_to_half2<FP8>(x[0], b & 1);
-        av.y = codes_to_half2<FP8>(x[1], b & 1);
-        av.z = codes_to_half2<FP8>(x[2], b & 1);
-        av.w = codes_to_half2<FP8>(x[3], b & 1);
+        av.x = codes_to_half2<FP8, MASK>(x[0], b & 1);
+        av.y = codes_to_half2<FP8, MASK>(x[1], b & 1);
+        av.z = codes_to_half2<FP8, MASK>(x[2], b & 1);
+        av.w = codes_to_half2<FP8, MASK>(x[3], b & 1);
         const int dt = 4 * w + b;
         st.o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, av), p_op, st.o[dt], 0, 0, 0);
       }
@@ -676,7 +725,7 @@ struct DecodeTile {
   __device__ static void compute(const AttnIO& io, const LaneOffsets& lo, const half8_t (&qb)[KSTEPS], float s_init, int len,
                                  int first, int t, int lane, const uint8_t* lds, State& st, float ali) {
     const half8_t p = qk_softmax<MASK, CAP>(io, lo, qb, s_init, len, first, t, lane, lds, st, ali);
-    pv(lo, p, lds, st);
+    pv<MASK>(lo, p, lds, st);
   }
   template <bool CAP>
   __device__ static void compute_any(const AttnIO& io, const LaneOffsets& lo, const half8_t (&qb)[KSTEPS], float s_init,
@@ -842,11 +891,10 @@ struct DecodeTile {
   // Lane (c, g) holds O[head c][dim (4g+i)*DT + dt], i = 0..3, dt = 0..DT-1: D/4 contiguous
   // dims starting at g*D/4.  Gather them in order, code bias removed, scaled by `mul`.
   __device__ static void gather_row(const State& st, float mul, float (&v)[D / 4]) {
-    const float corr = FP8 ? 0.f : kBias * st.psum[0];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) v[i * DT + dt] = (st.o[dt][i] - corr) * mul;
+      for (int dt = 0; dt < DT; ++dt) v[i * DT + dt] = (st.o[dt][i] - v_bias(dt) * st.psum[0]) * (mul * v_unit(dt));
   }
 
   // Whole sequence handled by this wave: normalise and write the output row (and lse).

@@ -127,7 +127,6 @@ struct PrefillTile {
     const floatx4 vs0 = *reinterpret_cast<const floatx4*>(sc_lds + 32 + 4 * g);
     const floatx4 vs1 = *reinterpret_cast<const floatx4*>(sc_lds + 48 + 4 * g);
     const int tok_base = t * kTile + 4 * g;
-    const bool capped = io.cap_c != 0.f;  // uniform
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
       float logit[8];
@@ -137,10 +136,7 @@ struct PrefillTile {
 #pragma unroll
         for (int i = 0; i < 4; ++i) logit[mt * 4 + i] = s[nt][mt][i] * (mt ? ks1 : ks0)[i];
       }
-      if (capped) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) logit[j] = soft_cap(logit[j], io.cap_c, io.cap_k);
-      }
+      soft_cap(logit, io.cap_c, io.cap_k);
       if (io.alibi != nullptr) {   // uniform; the column's query stands at limit - 1
         const float rel0 = (float)(tok_base - (limit[nt] - 1));
 #pragma unroll
@@ -191,7 +187,8 @@ struct PrefillTile {
     }
   }
 
-  // O^T += (V + 1152)^T . P~^T: every converted V operand feeds the NT column tiles.
+  // O^T += (V + 1152)^T . P~^T: every converted V operand feeds the NT column tiles.  MASK as in DecodeTile::pv.
+  template <bool MASK>
   __device__ static void pv(const LaneOffsets& lo, const half8_t (&p_op)[NT], const uint8_t* lds, State& st) {
     if constexpr (!FP8) {
       const half_t one = (half_t)1.0f;
@@ -228,10 +225,10 @@ struct PrefillTile {
       for (int b = 0; b < 4; ++b) {
         u32x4 av;
         const uint32_t* x = (b < 2) ? x0 : x1;
-        av.x = codes_to_half2<FP8>(x[0], b & 1);
-        av.y = codes_to_half2<FP8>(x[1], b & 1);
-        av.z = codes_to_half2<FP8>(x[2], b & 1);
-        av.w = codes_to_half2<FP8>(x[3], b & 1);
+        av.x = codes_to_half2<FP8, MASK>(x[0], b & 1);
+        av.y = codes_to_half2<FP8, MASK>(x[1], b & 1);
+        av.z = codes_to_half2<FP8, MASK>(x[2], b & 1);
+        av.w = codes_to_half2<FP8, MASK>(x[3], b & 1);
         const half8_t a_op = __builtin_bit_cast(half8_t, av);
         const int dt = 4 * w + b;
 #pragma unroll
@@ -273,12 +270,11 @@ struct PrefillTile {
     if (l > 0.f) l += sink_term(io.sinks, head, st.m[nt]);   // a row without a visible key keeps its zeros
     const int g = lane >> 4;
     const float mul = l > 0.f ? 1.0f / (l * DTile::kOutDiv) : 0.f;   // no visible key: zeros
-    const float corr = FP8 ? 0.f : DTile::kBias * st.psum[nt][0];
     float v[D / 4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) v[i * DT + dt] = (st.o[nt][dt][i] - corr) * mul;
+      for (int dt = 0; dt < DT; ++dt) v[i * DT + dt] = (st.o[nt][dt][i] - DTile::v_bias(dt) * st.psum[nt][0]) * (mul * DTile::v_unit(dt));
     const int64_t base = row * io.out_stride_t + (int64_t)head * io.out_stride_h + g * (D / 4);
     if constexpr (ODT == KVQ_F32) {
       float* o = reinterpret_cast<float*>(io.out) + base;
@@ -428,13 +424,13 @@ __global__ __launch_bounds__(WPW * 64) void paged_prefill_kernel(PrefillArgs a) 
         PT::template qk_softmax<false>(io, lo, qb, s_init, limit, wspan, t, lane, lds, st, p_op, ali);
       else
         PT::template qk_softmax<true>(io, lo, qb, s_init, limit, wspan, t, lane, lds, st, p_op, ali);
-      PT::pv(lo, p_op, lds, st);
+      PT::template pv<false>(lo, p_op, lds, st);   // not the item's last tile: every slot holds a token
       DTile::phase_fence();
       t += STEP;
     }
     DTile::stage(kv, lo, sc_mul, lane, lds);
     PT::template qk_softmax<true>(io, lo, qb, s_init, limit, wspan, t, lane, lds, st, p_op, ali);
-    PT::pv(lo, p_op, lds, st);
+    PT::template pv<true>(lo, p_op, lds, st);
   }
   if constexpr (SPLIT) {
     // every wave of the workgroup arrives here (the returns above are uniform over it)
@@ -488,8 +484,9 @@ struct Flash32 {
   static constexpr int LDS_BYTES = 2 * RAW_BYTES + 2 * BUF_BYTES;
   static constexpr int COLS = 32 * WAVES;
 
+  template <bool GARBAGE>
   __device__ static __forceinline__ uint32_t to_half2(uint32_t x, bool upper) {
-    if constexpr (FP8) return fp8_bytes_to_half2(x, upper);
+    if constexpr (FP8) return fp8_bytes_to_half2<GARBAGE>(x, upper);
     const half2_t bias = {(half_t)kCodeBias, (half_t)kCodeBias};
     const half2_t v = __builtin_bit_cast(half2_t, bytes_to_half2(x, upper)) - bias;
     return __builtin_bit_cast(uint32_t, v);
@@ -592,7 +589,9 @@ struct Flash32 {
 
   // Raw tile -> fp16 K [token][dim] (codes + 1152) and V^T [dim][position] (codes); token t of the tile sits at position
   // (t/16)*16 + ((t%8)/4)*8 + ((t/8)%2)*4 + t%4, the order in which the 32x32 S accumulator hands a
-  // lane its tokens.  One thread converts one 16-code K chunk and one 4-token x 4-dim V block.
+  // lane its tokens.  One thread converts one 16-code K chunk and one 4-token x 4-dim V block.  GARBAGE: the tile may
+  // hold slots past the end of the sequence.
+  template <bool GARBAGE>
   __device__ static __forceinline__ void expand(const uint8_t* raw, uint8_t* buf, int tid, float sc_mul, uint32_t l_sc) {
     constexpr int KCH = D / 16;
     if constexpr (INT4) {
@@ -628,8 +627,8 @@ struct Flash32 {
       for (int b = 0; b < 4; ++b) {
         const uint32_t p01 = (b < 2) ? a01 : b01, p23 = (b < 2) ? a23 : b23;
         u32x2 o;
-        o.x = to_half2(p01, b & 1);
-        o.y = to_half2(p23, b & 1);
+        o.x = to_half2<GARBAGE>(p01, b & 1);
+        o.y = to_half2<GARBAGE>(p23, b & 1);
         *reinterpret_cast<u32x2*>(vrow + b * V_PITCH) = o;
       }
     }
@@ -683,12 +682,16 @@ struct Flash32 {
     bool capped = false;
     if constexpr (EXT) capped = cap_c != 0.f;  // uniform
     if (capped) {
+      float x[16];
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const floatx4 ksc = *reinterpret_cast<const floatx4*>(sc + 8 * q + 4 * g);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s[4 * q + r] = soft_cap(s[4 * q + r] * ksc[r], cap_c, cap_k) - mref;
+        for (int r = 0; r < 4; ++r) x[4 * q + r] = s[4 * q + r] * ksc[r];
       }
+      soft_cap(x, cap_c, cap_k);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[i] = x[i] - mref;
     } else {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -918,7 +921,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // raw window and refill `next` with tile t+3, ONE barrier, then compute tile t.
     auto step_fn = [&](auto masked, int t, Regs& next) __attribute__((always_inline)) {
       uint8_t* buf = bufs + (t & 1) * FP::BUF_BYTES;
-      FP::expand(raws + (t & 1) * FP::RAW_BYTES, buf, tid, sc_mul, lo.l_sc);
+      FP::template expand<decltype(masked)::value>(raws + (t & 1) * FP::RAW_BYTES, buf, tid, sc_mul, lo.l_sc);
       drop(next, raws + ((t + 1) & 1) * FP::RAW_BYTES);
       issue(nb, t + 3, next);
       lds_barrier();
@@ -936,7 +939,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // loops (every wave runs the same number of steps, hence of barriers, whichever loop a step is
     // in), so that the accumulators keep their registers across the loop instead of being merged
     // at a branch inside it.
-    const int t_plain = min(t_hi, wave_min_limit / kTile) & ~1;
+    // (also for a wave without a valid column: its share of the expansion must expect slots past the sequence's end)
+    const int t_plain = min(t_hi, min(wave_min_limit, len) / kTile) & ~1;
     int t = t_lo;
     if constexpr (EXT) {  // tiles that straddle a column's lower window edge
       const int t_head = min(t_hi, ((wave_max_first + kTile - 1) / kTile + 1) & ~1);
