@@ -266,21 +266,25 @@ struct LaneOffsets {
   uint32_t g_tail;    // HBM: (lane & 15)*stride_slot + 2*D, the record's last 8 bytes
   uint32_t l_chunk;   // LDS: (lane / NCH)*PITCH + 16*(lane % NCH)
   uint32_t l_tail;    // LDS: (lane & 31)*PITCH + 2*D
-  uint32_t l_k;       // LDS: r*PITCH + g*16, K operand chunk of token r
-  uint32_t l_v;       // LDS: 4g*PITCH + (D+4) + r*VB, V operand bytes of token 4g
+  uint32_t l_k;       // LDS: first K operand chunk of the lane's row of M-tile 0
+  uint32_t l_v;       // LDS: first V operand bytes of the lane's first token
   uint32_t l_sc;      // LDS: (lane & 31)*PITCH + (lane < 32 ? D : 2*D+4), the lane's scale
-  // streamed loads: where the 16-byte chunk n*64 + lane of a 16-record run lands in the window (its first 8
-  // bytes; the other 8 follow, or open the next row when bit n of l_flat_split is set)
-  uint32_t g_flat;    // HBM: 16 * lane
-  uint32_t l_flat[9];
-  uint32_t l_flat_split;
+  uint32_t flat;      // streamed loads, HBM and LDS: 16 * lane
   uint32_t nib_lo, nib_hi;   // int4 codes: 0x000f000f and 0x00f000f0 (see in_vgpr)
 };
 
 // CODE: what a code byte is (KVQ_CODE_INT8 or KVQ_CODE_FP8_E4M3).  An int8 code enters the MFMA as
 // code + 1152 and the constant is taken out afterwards; an fp8 code enters as its value / 2^8 (exact in
 // fp16) and the 2^8 is put back with the K scale, while on the V side it cancels the 2^8 that P~ carries.
-template <int D, int QDT, int ODT, int CODE = KVQ_CODE_INT8>
+// STREAM: for a cache in which a head's records of a block lie back to back (the HND order).  A half tile is then ONE run
+// of 16 R bytes, read as aligned 16-byte chunks with the non-temporal hint, scales included -- measured on MI355X, reads of
+// this shape reach 6.8 TB/s against 6.0 without the hint.  (The hint is wrong for the NHD order: there the 128-byte lines
+// at a record's ends belong half to a neighbouring head's wave, a line that is not kept in L2 is fetched by both, and the
+// rate drops by 9 %.)  The run goes into the window as it is, one 16-byte LDS write per chunk, rows R bytes apart; which
+// token, dims and bytes a lane's operands hold is chosen so that reading that unpadded window is free of bank conflicts
+// (see row_token, k_off, v_off).  Re-pitching the rows on the way in, two 8-byte writes per chunk, took longer than the
+// products: 2.9 of the 6.9 us of a tile at head size 256.
+template <int D, int QDT, int ODT, int CODE = KVQ_CODE_INT8, bool STREAM = false>
 struct DecodeTile {
   static constexpr bool FP8 = CODE == KVQ_CODE_FP8_E4M3;
   // int4 codes: a record of head size D has the bytes of an int8 record of head size D / 2, so the tile is loaded
@@ -297,7 +301,7 @@ struct DecodeTile {
   using State = DecodeState<D>;
 
   static constexpr int R = 2 * (DB + 4);     // record bytes
-  static constexpr int PITCH = R + 8;        // LDS row pitch: 16-byte aligned rows, conflict-free operand reads
+  static constexpr int PITCH = STREAM ? R : R + 8;   // LDS row pitch; R + 8: 16-byte aligned rows
   static constexpr int NCH = Tile::NCH;
   static constexpr int NLD = Tile::NLD;
   static constexpr int LDS_TILE = kTile * PITCH;          // bytes of the record window
@@ -311,25 +315,57 @@ struct DecodeTile {
     o.g_tail = (uint32_t)((lane & 15) * G.stride_slot + 2 * DB);
     o.l_chunk = (uint32_t)((lane / NCH) * PITCH + 16 * (lane % NCH));
     o.l_tail = (uint32_t)((lane & 31) * PITCH + 2 * DB);
-    o.l_k = (uint32_t)(r * PITCH + (INT4 ? g * (DB / 4) : g * 16));   // int4: the lane's D / 4 dims are DB / 4 bytes in a row
-    o.l_v = (uint32_t)(4 * g * PITCH + (DB + 4) + r * VB);
+    o.l_k = (uint32_t)(row_token(0, r) * PITCH + k_off(g, 0));
+    o.l_v = (uint32_t)(s_token(g, 0, 0) * PITCH + (DB + 4) + r * (STREAM && VB > 4 ? 4 : VB));
     o.l_sc = (uint32_t)((lane & 31) * PITCH + (lane < 32 ? DB : 2 * DB + 4));
-    o.g_flat = (uint32_t)(16 * lane);
+    o.flat = (uint32_t)(16 * lane);
     o.nib_lo = in_vgpr(0x000f000fu);
     o.nib_hi = in_vgpr(0x00f000f0u);
-    o.l_flat_split = 0;
-#pragma unroll
-    for (int n = 0; n <= NLD; ++n) {
-      const int q = n < NLD ? n * 64 + lane : NLD * 64 + (lane & 7);   // chunk of the run
-      const int rec = (16 * q) / R, off = 16 * q - rec * R;            // its record and the offset inside it
-      o.l_flat[n] = (uint32_t)(rec * PITCH + off);
-      if (off == R - 8) o.l_flat_split |= 1u << n;
-    }
     return o;
   }
 
+  // ---- which token, dims and bytes an operand lane holds ------------------------------------------------------------
+  // Rows of the unpadded window lie R = 2 (DB + 4) bytes apart, 2 dwords modulo the 64 banks for DB = 128 and 256 (34
+  // for DB = 64).  With eight tokens in a row per quarter of the wave, a 4-byte V read of 16 consecutive dwords per
+  // token meets every bank once; an 8-byte K read of a half wave does if its two quarters read 32 bytes apart.
+  // Token of A row r of M-tile mt.
+  __device__ static constexpr int row_token(int mt, int r) { return STREAM ? 8 * (r >> 2) + 4 * mt + (r & 3) : 16 * mt + r; }
+  // Token of S element i of M-tile mt in quarter g (rows 4 g + i), the first of four in a row.
+  __device__ static constexpr int s_token(int g, int mt, int i) { return row_token(mt, 4 * g + i); }
+  // Tokens between the P~ operand's positions 0 and j of a lane.
+  __device__ static constexpr int p_token(int j) { return STREAM ? j : (j >> 2) * 16 + (j & 3); }
+  // Byte offset in a K row of the lane's i-th 16-byte chunk (DB = 32: its only 8 bytes).
+  __device__ static constexpr int k_off(int g, int i) {
+    if (!STREAM) return INT4 ? g * (DB / 4) + 16 * i : 16 * g + 64 * i;
+    if (DB == 32) return 8 * g;
+    if (DB == 64) return 16 * ((g & 1) * 2 + (g >> 1));
+    if (DB == 128) return 16 * (2 * g + i);
+    return 16 * (8 * (g >> 1) + 2 * (g & 1) + (i & 1) + 4 * (i >> 1));
+  }
+  // ... relative to the first chunk's (the same for every g).
+  __device__ static constexpr int k_step(int i) { return k_off(0, i) - k_off(0, 0); }
+  // The lane's i-th K chunk of M-tile mt, and the offset of dword (int4 with two code bytes per lane: half dword) w of
+  // its V bytes of P~ position j.
+  __device__ static u32x4 k_chunk(const LaneOffsets& lo, int mt, int i, const uint8_t* lds) {
+    const uint8_t* p = lds + lo.l_k + (row_token(mt, 0) - row_token(0, 0)) * PITCH + k_step(i);
+    if constexpr (STREAM) {   // rows are 8-byte aligned
+      const u32x2 a = *reinterpret_cast<const u32x2*>(p), b = *reinterpret_cast<const u32x2*>(p + 8);
+      return (u32x4){a.x, a.y, b.x, b.y};
+    } else {
+      return *reinterpret_cast<const u32x4*>(p);
+    }
+  }
+  __device__ static uint32_t v_off(const LaneOffsets& lo, int j, int w) {
+    return lo.l_v + p_token(j) * PITCH + w * (STREAM ? 64 : 4);
+  }
+  // Output tile dt, row 4 g + i of O^T is dim (dt / OG) 16 OG + 4 OG g + OG i + dt % OG: a lane holds runs of 4 OG dims.
+  // gather_row() puts them into v[] in that order; out_dim is where v[p] belongs.
+  static constexpr int OG = !STREAM ? DT : INT4 ? (DT < 8 ? DT : 8) : 4;
+  __device__ static constexpr int out_dim(int g, int p) { return (p / (4 * OG)) * 16 * OG + g * 4 * OG + p % (4 * OG); }
+  __device__ static constexpr int gather_pos(int i, int dt) { return (dt / OG) * 4 * OG + i * OG + dt % OG; }
+
   // ---- Q as the MFMA B operand --------------------------------------------------------------
-  // Lane (c = head in group, g) holds, for k-step kk, dims (kk>>1)*64 + g*16 + (kk&1)*8 + j:
+  // Lane (c = head in group, g) holds, for k-step kk, the dims of its K chunk kk >> 1, half kk & 1 (int8 and fp8):
   // the same dim order in which a K lane holds its code bytes.  Lanes past the group reread
   // head 0 and are zeroed.  Returns -1152 * sum(q) of the lane's head: the QK accumulator's
   // start value that cancels the code bias.
@@ -344,22 +380,21 @@ struct DecodeTile {
   // query row (it must be readable also when !valid; the operand is then zero).
   __device__ static float load_q_row(const AttnIO& io, int64_t elem, bool valid, int lane, half8_t (&qb)[KSTEPS]) {
     const int g = lane >> 4;
-    // int8 / fp8: 16 dims of every 64-dim chunk; int4: the D / 4 dims from g D / 4 on, in a row (the same loads,
-    // chunk `ch` then standing for the ch-th run of 16 of them)
-    constexpr int kChunkStep = INT4 ? 16 : 64;
-    const int64_t base = elem + (INT4 ? g * (D / 4) : g * 16);
+    // int8 / fp8: the 16 dims of the lane's K chunk `ch`; int4: a K chunk holds 32 dims, two runs of 16
+    const int64_t base = elem + (INT4 ? 2 : 1) * k_off(g, 0);
+    auto run_step = [](int ch) { return INT4 ? 2 * k_step(ch >> 1) + 16 * (ch & 1) : k_step(ch); };
     float f[D / 4];
 #pragma unroll
     for (int ch = 0; ch < D / 64; ++ch) {
       if constexpr (QDT == KVQ_F32) {
-        const float* p = reinterpret_cast<const float*>(io.q) + base + ch * kChunkStep;
+        const float* p = reinterpret_cast<const float*>(io.q) + base + run_step(ch);
 #pragma unroll
         for (int i = 0; i < 16; i += 4) {
           const floatx4 v = *reinterpret_cast<const floatx4_a4*>(p + i);
           f[ch * 16 + i] = v.x; f[ch * 16 + i + 1] = v.y; f[ch * 16 + i + 2] = v.z; f[ch * 16 + i + 3] = v.w;
         }
       } else {
-        const uint16_t* p = reinterpret_cast<const uint16_t*>(io.q) + base + ch * kChunkStep;
+        const uint16_t* p = reinterpret_cast<const uint16_t*>(io.q) + base + run_step(ch);
 #pragma unroll
         for (int i = 0; i < 16; i += 8) {
           const u32x4 v = *reinterpret_cast<const u32x4_a4*>(p + i);
@@ -407,15 +442,15 @@ struct DecodeTile {
 
   // The KSTEPS operands of K tokens (M-tile mt) of the lane, int4 codes: DB / 4 bytes in a row, a dword per k-step.
   __device__ static void k_operands_int4(const LaneOffsets& lo, int mt, const uint8_t* lds, half8_t (&ka)[KSTEPS]) {
-    const uint8_t* p = lds + lo.l_k + mt * 16 * PITCH;
     if constexpr (KSTEPS == 2) {
+      const uint8_t* p = lds + lo.l_k + (row_token(mt, 0) - row_token(0, 0)) * PITCH;
       const u32x2 w = *reinterpret_cast<const u32x2*>(p);
       ka[0] = dequant8_int4(w.x, lo.nib_lo);
       ka[1] = dequant8_int4(w.y, lo.nib_lo);
     } else {
 #pragma unroll
       for (int i = 0; i < KSTEPS / 4; ++i) {
-        const u32x4 w = *reinterpret_cast<const u32x4*>(p + 16 * i);
+        const u32x4 w = k_chunk(lo, mt, i, lds);
         ka[4 * i] = dequant8_int4(w.x, lo.nib_lo);
         ka[4 * i + 1] = dequant8_int4(w.y, lo.nib_lo);
         ka[4 * i + 2] = dequant8_int4(w.z, lo.nib_lo);
@@ -425,7 +460,7 @@ struct DecodeTile {
   }
 
   // The V^T operands of the lane's 8 tokens for the four 16-dim tiles that two code bytes hold (unit u = bytes
-  // 2 u, 2 u + 1 of the lane's VB: dims 4 u .. 4 u + 3 of its 2 VB, tile 4 u + n = nibble n), int4 codes.  The odd
+  // 2 u, 2 u + 1 of the lane's VB; tile 4 u + n = nibble n), int4 codes.  The odd
   // nibbles stay where they are in the byte and enter as 1024 + 16 (code ^ 8): their rows of O^T carry 16 (code) +
   // 1152 instead of code + 1032, which the emission takes out (v_bias, v_unit) -- one shift per dword instead of three.
   __device__ static void v_operands_int4(const LaneOffsets& lo, int u, const uint8_t* lds, half8_t (&va)[4]) {
@@ -433,8 +468,8 @@ struct DecodeTile {
 #pragma unroll
     for (int a = 0; a < 4; ++a) {
       const int ja = 2 * a, jb = 2 * a + 1;
-      const uint8_t* pa = lds + lo.l_v + ((ja & 3) + (ja >> 2) * 16) * PITCH + 2 * u;
-      const uint8_t* pb = lds + lo.l_v + ((jb & 3) + (jb >> 2) * 16) * PITCH + 2 * u;
+      const uint8_t* pa = lds + v_off(lo, ja, u >> 1) + 2 * (u & 1);
+      const uint8_t* pb = lds + v_off(lo, jb, u >> 1) + 2 * (u & 1);
       const uint32_t ta = *reinterpret_cast<const uint16_t*>(pa), tb = *reinterpret_cast<const uint16_t*>(pb);
       y[a] = (ta | (tb << 16)) ^ 0x88888888u;   // token ja's two bytes below token jb's
     }
@@ -500,25 +535,17 @@ struct DecodeTile {
 
   // Issue the HBM loads of one tile: 2*NLD chunk loads (lane n*64+l takes chunk (n*64+l) % NCH of
   // record (n*64+l) / NCH of the half) and the two 8-byte record tails.
-  // STREAM: for a cache in which a head's records of a block lie back to back (the HND order).  A half
-  // tile is then ONE run of 16 R bytes, read as aligned 16-byte chunks with the non-temporal hint (scales
-  // included: no 8-byte tail loads) -- measured on MI355X, reads of this shape reach 6.8 TB/s against 6.0
-  // without the hint.  The hint is wrong for the NHD order: there the 128-byte lines at a record's ends
-  // belong half to a neighbouring head's wave, a line that is not kept in L2 is fetched by both, and the
-  // rate drops by 9 %.
-  template <bool STREAM = false>
   __device__ static void load_tile(const AttnIO& io, const Window& w, const LaneOffsets& lo, Tile& kv) {
     constexpr int AUX = STREAM ? 2 : 0;
     if constexpr (STREAM) {
       // the half's 16 records are one run of 16 R bytes: read it as R aligned 16-byte chunks, scales and all
       // (NLD full wave-loads and the last 8 chunks, which every lane names so that the load is unconditional)
-      const uint32_t f = lo.g_flat;
 #pragma unroll
       for (int n = 0; n < NLD; ++n) {
-        kv.c[0][n] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w.r0, f, n * 1024, AUX));
-        kv.c[1][n] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w.r1, f, n * 1024, AUX));
+        kv.c[0][n] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w.r0, lo.flat, n * 1024, AUX));
+        kv.c[1][n] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w.r1, lo.flat, n * 1024, AUX));
       }
-      const uint32_t fe = (f & 127u) + NLD * 1024;
+      const uint32_t fe = (lo.flat & 127u) + NLD * 1024;
       kv.e[0] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w.r0, fe, 0, AUX));
       kv.e[1] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(w.r1, fe, 0, AUX));
       return;
@@ -536,25 +563,16 @@ struct DecodeTile {
   // Drop a loaded tile into the wave's LDS window, one record per PITCH-byte row, then stage the
   // 64 scales (K scales pre-multiplied by scale*log2e, V scales by 2^8, capped so P~ stays finite).
   // After this the tile's registers are free for the next prefetch.
-  template <bool STREAM = false>
   __device__ static void stage(const Tile& kv, const LaneOffsets& lo, float sc_mul, int lane, uint8_t* lds) {
     if constexpr (STREAM) {
-      // a chunk of the run is 8-byte aligned inside its record and may end one record and begin the next:
-      // two 8-byte writes each
-      auto put = [&](const u32x4& v, uint32_t at, bool split) __attribute__((always_inline)) {
-        *reinterpret_cast<u32x2*>(lds + at) = (u32x2){v.x, v.y};
-        *reinterpret_cast<u32x2*>(lds + at + (split ? 8 + (PITCH - R) : 8)) = (u32x2){v.z, v.w};
-      };
 #pragma unroll
       for (int n = 0; n < NLD; ++n) {
-        const bool split = (lo.l_flat_split >> n) & 1;
-        put(kv.c[0][n], lo.l_flat[n], split);
-        put(kv.c[1][n], lo.l_flat[n] + 16 * PITCH, split);
+        *reinterpret_cast<u32x4*>(lds + lo.flat + n * 1024) = kv.c[0][n];
+        *reinterpret_cast<u32x4*>(lds + lo.flat + n * 1024 + 16 * R) = kv.c[1][n];
       }
       if (lane < 8) {
-        const bool split = (lo.l_flat_split >> NLD) & 1;
-        put(kv.e[0], lo.l_flat[NLD], split);
-        put(kv.e[1], lo.l_flat[NLD] + 16 * PITCH, split);
+        *reinterpret_cast<u32x4*>(lds + lo.flat + NLD * 1024) = kv.e[0];
+        *reinterpret_cast<u32x4*>(lds + lo.flat + NLD * 1024 + 16 * R) = kv.e[1];
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
@@ -594,8 +612,8 @@ struct DecodeTile {
                                        int len, int first, int t, int lane, const uint8_t* lds, State& st, float ali) {
     const int g = lane >> 4;
     const float* sc_lds = reinterpret_cast<const float*>(lds + LDS_TILE);
-    const floatx4 ks0 = *reinterpret_cast<const floatx4*>(sc_lds + 4 * g);
-    const floatx4 ks1 = *reinterpret_cast<const floatx4*>(sc_lds + 16 + 4 * g);
+    const floatx4 ks0 = *reinterpret_cast<const floatx4*>(sc_lds + s_token(g, 0, 0));
+    const floatx4 ks1 = *reinterpret_cast<const floatx4*>(sc_lds + s_token(g, 1, 0));
 
     // two 16-token M-tiles, KSTEPS k-steps each; accumulators start at -1152 * sum(q)
     floatx4 s[2];
@@ -610,16 +628,16 @@ struct DecodeTile {
       } else {
 #pragma unroll
       for (int i = 0; i < KSTEPS / 2; ++i) {
-        const u32x4 w = *reinterpret_cast<const u32x4*>(lds + lo.l_k + mt * 16 * PITCH + i * 64);
+        const u32x4 w = k_chunk(lo, mt, i, lds);
         s[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(dequant8<FP8>(w.x, w.y), qb[2 * i], s[mt], 0, 0, 0);
         s[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(dequant8<FP8>(w.z, w.w), qb[2 * i + 1], s[mt], 0, 0, 0);
       }
       }
     }
 
-    // softmax in the log2 domain; lane holds tokens 32t + mt*16 + 4g + i of head (lane & 15)
+    // softmax in the log2 domain; lane holds tokens tok_base + p_token(4 mt + i) of head (lane & 15)
     float logit[8];
-    const int tok_base = t * kTile + 4 * g;
+    const int tok_base = t * kTile + s_token(g, 0, 0);
     const float rel0 = (float)(tok_base - (len - 1));
     float mloc = -INFINITY;
 #pragma unroll
@@ -627,14 +645,14 @@ struct DecodeTile {
     if constexpr (CAP) {
       soft_cap(logit, io.cap_c, io.cap_k);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) logit[j] = __builtin_fmaf(ali, rel0 + (float)((j >> 2) * 16 + (j & 3)), logit[j]);
+      for (int j = 0; j < 8; ++j) logit[j] = __builtin_fmaf(ali, rel0 + (float)p_token(j), logit[j]);
     }
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         float x = logit[mt * 4 + i];
-        if constexpr (MASK) x = ((uint32_t)(tok_base + mt * 16 + i - first) < (uint32_t)(len - first)) ? x : -INFINITY;
+        if constexpr (MASK) x = ((uint32_t)(tok_base + p_token(mt * 4 + i) - first) < (uint32_t)(len - first)) ? x : -INFINITY;
         logit[mt * 4 + i] = x;
         mloc = fmaxf(mloc, x);
       }
@@ -649,8 +667,8 @@ struct DecodeTile {
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) st.o[dt] *= alpha;
     }
-    const floatx4 vs0 = *reinterpret_cast<const floatx4*>(sc_lds + 32 + 4 * g);
-    const floatx4 vs1 = *reinterpret_cast<const floatx4*>(sc_lds + 48 + 4 * g);
+    const floatx4 vs0 = *reinterpret_cast<const floatx4*>(sc_lds + 32 + s_token(g, 0, 0));
+    const floatx4 vs1 = *reinterpret_cast<const floatx4*>(sc_lds + 32 + s_token(g, 1, 0));
     float pt[8];
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
@@ -661,7 +679,7 @@ struct DecodeTile {
         st.l += p;
         float x = p * (mt ? vs1 : vs0)[i];
         if constexpr (MASK)  // garbage scales never enter
-          x = ((uint32_t)(tok_base + mt * 16 + i - first) < (uint32_t)(len - first)) ? x : 0.f;
+          x = ((uint32_t)(tok_base + p_token(mt * 4 + i) - first) < (uint32_t)(len - first)) ? x : 0.f;
         pt[j] = x;
       }
     }
@@ -673,8 +691,8 @@ struct DecodeTile {
     return __builtin_bit_cast(half8_t, pb);
   }
 
-  // Phase 2 of a tile: O^T += (V + 1152)^T . P~^T.  Lane (r, g) reads bytes [r*VB, (r+1)*VB) of
-  // tokens 4g+j (j<4) and 16+4g+(j-4) from the LDS window, transposes the 8 x VB byte block in
+  // Phase 2 of a tile: O^T += (V + 1152)^T . P~^T.  Lane (r, g) reads its VB code bytes of
+  // its eight tokens from the LDS window, transposes the 8 x VB byte block in
   // registers (byte permutes), one MFMA per 16-dim tile; sum(P~) comes from a row of ones.
   // MASK: the tile may hold slots past the end of the sequence, whose bytes may be anything.
   template <bool MASK>
@@ -702,8 +720,8 @@ struct DecodeTile {
 #pragma unroll
       for (int a = 0; a < 4; ++a) {
         const int ja = 2 * a, jb = 2 * a + 1;
-        const uint32_t ta = prep_codes<FP8>(*reinterpret_cast<const uint32_t*>(lds + lo.l_v + ((ja & 3) + (ja >> 2) * 16) * PITCH + 4 * w));
-        const uint32_t tb = prep_codes<FP8>(*reinterpret_cast<const uint32_t*>(lds + lo.l_v + ((jb & 3) + (jb >> 2) * 16) * PITCH + 4 * w));
+        const uint32_t ta = prep_codes<FP8>(*reinterpret_cast<const uint32_t*>(lds + v_off(lo, ja, w)));
+        const uint32_t tb = prep_codes<FP8>(*reinterpret_cast<const uint32_t*>(lds + v_off(lo, jb, w)));
         x0[a] = perm(tb, ta, 0x05010400u);
         x1[a] = perm(tb, ta, 0x07030602u);
       }
@@ -771,7 +789,7 @@ struct DecodeTile {
     st.m = -INFINITY;
     st.l = 0.f;
   }
-  template <bool CAP, bool STREAM = false, bool SPANS = false>
+  template <bool CAP, bool SPANS = false>
   __device__ static void run(const AttnIO& io, int seq, int64_t row, int len, int first, int t_begin, int t_end, int hkv,
                              int lane, uint8_t* lds, State& st, int sub = 0, int nsub = 1, SpanEdges* sp = nullptr) {
     const LaneOffsets lo = lane_offsets(io.g, lane);
@@ -795,7 +813,7 @@ struct DecodeTile {
       Tile a;
       // the first tile's loads go out before anything else of the run is touched
       TileBlocks nb = fetch_blocks(io, bt_row, len, t);
-      load_tile<STREAM>(io, window(io, nb, t, hkv), lo, a);
+      load_tile(io, window(io, nb, t, hkv), lo, a);
       phase_fence();
       nb = fetch_blocks(io, bt_row, len, t + nsub);  // block ids run one tile ahead of the loads
       half8_t qb[KSTEPS];
@@ -808,9 +826,9 @@ struct DecodeTile {
       // steady loop below keeps a single, unmasked body
       if (t + nsub < t_end && t * kTile < first) {
         const Window w = window(io, nb, t + nsub, hkv);
-        stage<STREAM>(a, lo, sc_mul, lane, lds);
+        stage(a, lo, sc_mul, lane, lds);
         phase_fence();
-        load_tile<STREAM>(io, w, lo, a);
+        load_tile(io, w, lo, a);
         phase_fence();
         nb = fetch_blocks(io, bt_row, len, t + 2 * nsub);
         compute<true, CAP>(io, lo, qb, s_init, len, first, t, lane, lds, st, ali);
@@ -839,9 +857,9 @@ struct DecodeTile {
       // end the sequence
       while (t + nsub < t_end) {
         const Window w = window(io, nb, t + nsub, hkv);
-        stage<STREAM>(a, lo, sc_mul, lane, lds);
+        stage(a, lo, sc_mul, lane, lds);
         phase_fence();
-        load_tile<STREAM>(io, w, lo, a);
+        load_tile(io, w, lo, a);
         phase_fence();
         nb = fetch_blocks(io, bt_row, len, t + 2 * nsub);
         compute<false, CAP>(io, lo, qb, s_init, len, first, t, lane, lds, st, ali);
@@ -850,7 +868,7 @@ struct DecodeTile {
         t += nsub;
         rendezvous();
       }
-      stage<STREAM>(a, lo, sc_mul, lane, lds);
+      stage(a, lo, sc_mul, lane, lds);
       compute_any<CAP>(io, lo, qb, s_init, len, first, t, lane, lds, st, ali);
     }
     // the rendezvous count is the same for every wave of the workgroup, whatever its share of the tiles
@@ -888,13 +906,12 @@ struct DecodeTile {
     return l;
   }
 
-  // Lane (c, g) holds O[head c][dim (4g+i)*DT + dt], i = 0..3, dt = 0..DT-1: D/4 contiguous
-  // dims starting at g*D/4.  Gather them in order, code bias removed, scaled by `mul`.
+  // The lane's D / 4 dims of head c in the order of out_dim, code bias removed, scaled by `mul`.
   __device__ static void gather_row(const State& st, float mul, float (&v)[D / 4]) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) v[i * DT + dt] = (st.o[dt][i] - v_bias(dt) * st.psum[0]) * (mul * v_unit(dt));
+      for (int dt = 0; dt < DT; ++dt) v[gather_pos(i, dt)] = (st.o[dt][i] - v_bias(dt) * st.psum[0]) * (mul * v_unit(dt));
   }
 
   // Whole sequence handled by this wave: normalise and write the output row (and lse).
@@ -916,11 +933,11 @@ struct DecodeTile {
     l += sink_term(io.sinks, head, st.m);
     float v[D / 4];
     gather_row(st, 1.0f / (l * kOutDiv), v);
-    const int64_t base = row * io.out_stride_t + (int64_t)head * io.out_stride_h + g * (D / 4);
+    const int64_t base = row * io.out_stride_t + (int64_t)head * io.out_stride_h;
     if constexpr (OT == KVQ_F32) {
       float* o = reinterpret_cast<float*>(io.out) + base;
 #pragma unroll
-      for (int i = 0; i < D / 4; i += 4) *reinterpret_cast<floatx4_a4*>(o + i) = (floatx4){v[i], v[i + 1], v[i + 2], v[i + 3]};
+      for (int i = 0; i < D / 4; i += 4) *reinterpret_cast<floatx4_a4*>(o + out_dim(g, i)) = (floatx4){v[i], v[i + 1], v[i + 2], v[i + 3]};
     } else {
       uint16_t* o = reinterpret_cast<uint16_t*>(io.out) + base;
 #pragma unroll
@@ -936,7 +953,7 @@ struct DecodeTile {
           }
           pk[j] = w;
         }
-        *reinterpret_cast<u32x4_a4*>(o + i) = pk;
+        *reinterpret_cast<u32x4_a4*>(o + out_dim(g, i)) = pk;
       }
     }
     if (io.lse != nullptr && g == 0)
@@ -952,9 +969,9 @@ struct DecodeTile {
     const int head = hkv * io.group + c;
     float v[D / 4];
     gather_row(st, 1.0f / kOutDiv, v);
-    float* o = part_o + (slot * io.num_q_heads + head) * (int64_t)D + g * (D / 4);
+    float* o = part_o + (slot * io.num_q_heads + head) * (int64_t)D;
 #pragma unroll
-    for (int i = 0; i < D / 4; i += 4) *reinterpret_cast<floatx4*>(o + i) = (floatx4){v[i], v[i + 1], v[i + 2], v[i + 3]};
+    for (int i = 0; i < D / 4; i += 4) *reinterpret_cast<floatx4*>(o + out_dim(g, i)) = (floatx4){v[i], v[i + 1], v[i + 2], v[i + 3]};
     if (g == 0) {
       part_ml[(slot * io.num_q_heads + head) * 2 + 0] = st.m;
       part_ml[(slot * io.num_q_heads + head) * 2 + 1] = l;
@@ -971,9 +988,9 @@ struct DecodeTile {
     float v[D / 4];
     gather_row(st, 1.0f / (l * kOutDiv), v);
     const int64_t idx = (seq * io.num_q_heads + head) * (int64_t)max_parts + part;
-    float* o = tmp_out + idx * D + g * (D / 4);
+    float* o = tmp_out + idx * D;
 #pragma unroll
-    for (int i = 0; i < D / 4; i += 4) *reinterpret_cast<floatx4*>(o + i) = (floatx4){v[i], v[i + 1], v[i + 2], v[i + 3]};
+    for (int i = 0; i < D / 4; i += 4) *reinterpret_cast<floatx4*>(o + out_dim(g, i)) = (floatx4){v[i], v[i + 1], v[i + 2], v[i + 3]};
     if (g == 0) {
       max_logits[idx] = st.m * kLn2;
       exp_sums[idx] = l;

@@ -18,12 +18,41 @@
 
 namespace kvq {
 
-extern template int launch_streamk_q<64>(const StreamKArgs& a, int q_dtype, int out_dtype, hipStream_t s);
-extern template int launch_streamk_q<128>(const StreamKArgs& a, int q_dtype, int out_dtype, hipStream_t s);
-extern template int launch_streamk_q<256>(const StreamKArgs& a, int q_dtype, int out_dtype, hipStream_t s);
-extern template int launch_v2_q<64>(const V2Args& a, int num_seqs, int q_dtype, hipStream_t s);
-extern template int launch_v2_q<128>(const V2Args& a, int num_seqs, int q_dtype, hipStream_t s);
-extern template int launch_v2_q<256>(const V2Args& a, int num_seqs, int q_dtype, hipStream_t s);
+#define KVQ_EXTERN(D, Q)                                                             \
+  extern template int launch_streamk<D, Q>(const StreamKArgs& args, hipStream_t s);   \
+  extern template int launch_v2<D, Q>(const V2Args& a, int num_seqs, hipStream_t s);
+KVQ_EXTERN(64, KVQ_F32)
+KVQ_EXTERN(64, KVQ_BF16)
+KVQ_EXTERN(64, KVQ_F16)
+KVQ_EXTERN(128, KVQ_F32)
+KVQ_EXTERN(128, KVQ_BF16)
+KVQ_EXTERN(128, KVQ_F16)
+KVQ_EXTERN(256, KVQ_F32)
+KVQ_EXTERN(256, KVQ_BF16)
+KVQ_EXTERN(256, KVQ_F16)
+#undef KVQ_EXTERN
+
+template <int D>
+static int launch_streamk_q(const StreamKArgs& a, int q_dtype, int out_dtype, hipStream_t s) {
+  if (out_dtype != KVQ_F32 && out_dtype != KVQ_BF16 && out_dtype != KVQ_F16)
+    return fail(KVQ_EINVAL, "paged_attn_int8: unknown out_dtype %d", out_dtype);
+  switch (q_dtype) {
+    case KVQ_F32: return launch_streamk<D, KVQ_F32>(a, s);
+    case KVQ_BF16: return launch_streamk<D, KVQ_BF16>(a, s);
+    case KVQ_F16: return launch_streamk<D, KVQ_F16>(a, s);
+  }
+  return fail(KVQ_EINVAL, "paged_attn_int8: unknown q_dtype %d", q_dtype);
+}
+
+template <int D>
+static int launch_v2_q(const V2Args& a, int num_seqs, int q_dtype, hipStream_t s) {
+  switch (q_dtype) {
+    case KVQ_F32: return launch_v2<D, KVQ_F32>(a, num_seqs, s);
+    case KVQ_BF16: return launch_v2<D, KVQ_BF16>(a, num_seqs, s);
+    case KVQ_F16: return launch_v2<D, KVQ_F16>(a, num_seqs, s);
+  }
+  return fail(KVQ_EINVAL, "paged_attn_v2_int8: unknown q_dtype %d", q_dtype);
+}
 
 // out = sum_j w_j tmp_out_j / sum_j w_j, w_j = exp_sums_j * exp(max_logits_j - max).
 // grid (num_seqs, ceil(Hq/4)), one wave per q head.

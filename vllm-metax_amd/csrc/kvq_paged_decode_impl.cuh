@@ -1,5 +1,5 @@
-// Device code and launch templates of the paged decode kernels, instantiated once per head size in
-// kvq_paged_decode_d64.hip / _d128.hip / _d256.hip (one translation unit each, so they compile in parallel).
+// Device code and launch templates of the paged decode kernels, instantiated once per head size and query type in
+// kvq_paged_decode_d<head size>_<type>.hip (one translation unit each, so they compile in parallel).
 #pragma once
 
 #include <type_traits>
@@ -148,7 +148,7 @@ __device__ __forceinline__ int active_workgroups(int64_t total, int num_wg) {
 // kernel carries none of it: as a run-time branch it cost the headline launch 0.6 us).
 template <int D, int QDT, int HPW, bool CAP, int CODE, bool STREAM, bool FIXED = false>
 __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a) {
-  using DTile = DecodeTile<D, QDT, kRuntimeDtype, CODE>;
+  using DTile = DecodeTile<D, QDT, kRuntimeDtype, CODE, STREAM>;
   constexpr int NSUB = 8 / HPW;
   __shared__ __align__(16) uint8_t lds[8][DTile::LDS_WAVE];
   const int lane = threadIdx.x & 63;
@@ -205,7 +205,7 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
       if constexpr (NSUB > 1) lds_barrier();
     }
     typename DTile::State st;
-    DTile::template run<CAP, STREAM>(a.io, cur, row, len, first, t_begin, t_end, hkv, lane, lds[wave], st, sub, NSUB);
+    DTile::template run<CAP>(a.io, cur, row, len, first, t_begin, t_end, hkv, lane, lds[wave], st, sub, NSUB);
     // the run holds the sequence's first tile: its place on the line, for the reduce kernel (behind the run's loads)
     if (!fixed && t_begin == t0 && blockIdx.y == 0 && wave == 0 && lane == 0) a.seq_first_unit[cur] = cur_start;
     if constexpr (NSUB > 1) {
@@ -240,7 +240,7 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
     }
     typename DTile::State st;
     typename DTile::SpanEdges sp{a.part_o, a.part_ml, (int64_t)cur * kFixedSpans + span, per, per};
-    DTile::template run<CAP, STREAM, true>(a.io, cur, row, len, first, t_begin, t_end, hkv, lane, lds[wave], st, 0, 1, &sp);
+    DTile::template run<CAP, true>(a.io, cur, row, len, first, t_begin, t_end, hkv, lane, lds[wave], st, 0, 1, &sp);
     DTile::emit_partial(a.io, a.part_o, a.part_ml, sp.slot, hkv, lane, st);
   };
 
@@ -844,24 +844,25 @@ __global__ __launch_bounds__(WPW * 64) void paged_decode_v2_kernel(V2Args a) {
   DTile::emit_v2(a.io, a.tmp_out, a.max_logits, a.exp_sums, seq, part, a.max_parts, hkv, lane, st);
 }
 
-// out = sum_j w_j tmp_out_j / sum_j w_j, w_j = exp_sums_j * exp(max_logits_j - max).
+// Main kernel + reduce of the balanced (or batch-invariant) split-K decode.
 template <int D, int QDT>
-static int launch_streamk(const StreamKArgs& args, hipStream_t s) {
+int launch_streamk(const StreamKArgs& args, hipStream_t s) {
   const int hkv = args.io.g.num_kv_heads;
   const int hpw = heads_per_wg(hkv);
   StreamKArgs a = args;
   a.setup_units = setup_units_for(8 / hpw);
   dim3 grid(a.num_wg, (hkv + hpw - 1) / hpw);
+#define KVQ_SK_FORM(H, C, CODE, S)                                                                                \
+  do {                                                                                                            \
+    if (a.fixed_spans)                                                                                            \
+      hipLaunchKernelGGL((paged_decode_streamk_kernel<D, QDT, H, C, CODE, S, true>), grid, dim3(512), 0, s, a);   \
+    else                                                                                                          \
+      hipLaunchKernelGGL((paged_decode_streamk_kernel<D, QDT, H, C, CODE, S>), grid, dim3(512), 0, s, a);         \
+  } while (0)
 #define KVQ_SK_CODE(H, C, CODE)                                                                                   \
   do {                                                                                                            \
-    if (a.fixed_spans && !C && stream)                                                                            \
-      hipLaunchKernelGGL((paged_decode_streamk_kernel<D, QDT, H, false, CODE, true, true>), grid, dim3(512), 0, s, a); \
-    else if (a.fixed_spans)                                                                                       \
-      hipLaunchKernelGGL((paged_decode_streamk_kernel<D, QDT, H, C, CODE, false, true>), grid, dim3(512), 0, s, a); \
-    else if (!C && stream)                                                                                        \
-      hipLaunchKernelGGL((paged_decode_streamk_kernel<D, QDT, H, false, CODE, true>), grid, dim3(512), 0, s, a);  \
-    else                                                                                                          \
-      hipLaunchKernelGGL((paged_decode_streamk_kernel<D, QDT, H, C, CODE, false>), grid, dim3(512), 0, s, a);     \
+    if (stream) KVQ_SK_FORM(H, C, CODE, true);                                                                    \
+    else KVQ_SK_FORM(H, C, CODE, false);                                                                          \
   } while (0)
 #define KVQ_SK(H, C)                                                                                              \
   do {                                                                                                            \
@@ -870,8 +871,7 @@ static int launch_streamk(const StreamKArgs& args, hipStream_t s) {
     else KVQ_SK_CODE(H, C, KVQ_CODE_INT8);                                                                        \
   } while (0)
   // a head's records of a block back to back (HND order): the tile loads may stream past the caches
-  // (not at head size 256, where it measured slower: 293 against 279 us on 64 x 1k-8k tokens)
-  const bool stream = D <= 128 && a.io.g.stride_slot == 2 * (code_bytes(a.io.g) + 4) && a.io.g.block_size >= 16;
+  const bool stream = a.io.g.stride_slot == 2 * (code_bytes(a.io.g) + 4) && a.io.g.block_size >= 16;
   if (a.io.cap_c != 0.f || a.io.alibi != nullptr) {   // the instantiation with the extras: soft cap and ALiBi
     switch (hpw) {
       case 8: KVQ_SK(8, true); break;
@@ -889,6 +889,7 @@ static int launch_streamk(const StreamKArgs& args, hipStream_t s) {
   }
 #undef KVQ_SK
 #undef KVQ_SK_CODE
+#undef KVQ_SK_FORM
   int rc = check_hip(hipGetLastError(), "paged_attn_int8 decode launch");
   if (rc) return rc;
   if (a.fixed_spans) {
@@ -912,20 +913,8 @@ static int launch_streamk(const StreamKArgs& args, hipStream_t s) {
   return check_hip(hipGetLastError(), "paged_attn_int8 reduce launch");
 }
 
-template <int D>
-int launch_streamk_q(const StreamKArgs& a, int q_dtype, int out_dtype, hipStream_t s) {
-  if (out_dtype != KVQ_F32 && out_dtype != KVQ_BF16 && out_dtype != KVQ_F16)
-    return fail(KVQ_EINVAL, "paged_attn_int8: unknown out_dtype %d", out_dtype);
-  switch (q_dtype) {
-    case KVQ_F32: return launch_streamk<D, KVQ_F32>(a, s);
-    case KVQ_BF16: return launch_streamk<D, KVQ_BF16>(a, s);
-    case KVQ_F16: return launch_streamk<D, KVQ_F16>(a, s);
-  }
-  return fail(KVQ_EINVAL, "paged_attn_int8: unknown q_dtype %d", q_dtype);
-}
-
 template <int D, int QDT>
-static int launch_v2(const V2Args& a, int num_seqs, hipStream_t s) {
+int launch_v2(const V2Args& a, int num_seqs, hipStream_t s) {
   const int hkv = a.io.g.num_kv_heads;
   const int wpw = heads_per_wg(hkv);
   dim3 grid(a.max_parts, num_seqs, (hkv + wpw - 1) / wpw);
@@ -948,16 +937,5 @@ static int launch_v2(const V2Args& a, int num_seqs, hipStream_t s) {
 #undef KVQ_V2
   return check_hip(hipGetLastError(), "paged_attn_v2_int8 launch");
 }
-
-template <int D>
-int launch_v2_q(const V2Args& a, int num_seqs, int q_dtype, hipStream_t s) {
-  switch (q_dtype) {
-    case KVQ_F32: return launch_v2<D, KVQ_F32>(a, num_seqs, s);
-    case KVQ_BF16: return launch_v2<D, KVQ_BF16>(a, num_seqs, s);
-    case KVQ_F16: return launch_v2<D, KVQ_F16>(a, num_seqs, s);
-  }
-  return fail(KVQ_EINVAL, "paged_attn_v2_int8: unknown q_dtype %d", q_dtype);
-}
-
 
 }  // namespace kvq
