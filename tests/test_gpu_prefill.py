@@ -378,3 +378,56 @@ def test_context_splits_need_their_workspace(gpu_device):
     with pytest.raises(RuntimeError):
         ops.unified_attention(q, k, v, torch.empty_like(q), cu, 64, sl, 500, 0.1, True, block_table=bt,
                               k_scale_cache=ks, v_scale_cache=vs, prefill_splits=9)
+
+
+@pytest.mark.parametrize("hq,hkv,d,qmax,code,q_dtype", [
+    (32, 8, 128, 8, "int8", torch.bfloat16),    # two column tiles, full
+    (16, 1, 128, 3, "int8", torch.float16),     # one head: eight waves on it, two items per sequence
+    (28, 4, 128, 9, "int4", torch.bfloat16),    # 63 columns, columns that do not fill the tiles
+    (16, 2, 64, 2, "fp8", torch.bfloat16),      # one column tile, full
+    (32, 16, 128, 5, "fp8", torch.float32),     # two workgroups' worth of heads
+    (8, 8, 64, 17, "int4", torch.float16)])
+@pytest.mark.parametrize("extras", [False, True])
+def test_short_run_line(gpu_device, hq, hkv, d, qmax, code, q_dtype, extras):
+    """Short runs on a head-major cache, cut along one line of tiles: lengths at the edges of tiles, runs that cover
+    their sequence, one-token sequences, an empty one, one long enough to be cut dozens of times; with and without
+    window, soft cap, sinks and ALiBi.  Output and lse against the oracle; a workspace without room for the
+    states goes through the other kernels, with the same result."""
+    from vllm_metax_amd.kv_cache_interface import KVQuantMode
+    ct = {"int8": oracle.CODE_INT8, "fp8": oracle.CODE_FP8, "int4": oracle.CODE_INT4}[code]
+    mode = {"int8": KVQuantMode.INT8_PER_TOKEN_HEAD, "fp8": KVQuantMode.FP8_PER_TOKEN_HEAD,
+            "int4": KVQuantMode.INT4_PER_TOKEN_HEAD}[code]
+    dev, bs = gpu_device, 16
+    ctx = [31, 32, 33, 5000, 64, 2, 0, 700, 1, qmax, 129]
+    qls = [min(c, q) for c, q in zip(ctx, [qmax, qmax, 2, qmax, 1, qmax, 0, 3, 1, qmax, 2])]
+    g = torch.Generator().manual_seed(hq + d + qmax)
+    nb = sum((c + bs - 1) // bs for c in ctx) + 5
+    kv_cpu, _, lay = T.cpu_cache(nb, bs, hkv, d, "HND", code_type=ct)
+    T.storage_bytes(kv_cpu).fill_(0xFF)                # NaN scales and codes wherever nothing is written
+    bt = T.make_block_tables(ctx, bs, nb, g)
+    keys = [torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in ctx]
+    vals = [torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in ctx]
+    T.fill_cache_from_sources(kv_cpu, lay, bt, ctx, bs, keys, vals, code_type=ct)
+    q = torch.randn((sum(qls), hq, d), generator=g).to(q_dtype)
+    sl = torch.tensor(ctx, dtype=torch.int32)
+    cu = torch.tensor([0] + torch.tensor(qls).cumsum(0).tolist(), dtype=torch.int32)
+    scale, window, cap = 1 / math.sqrt(d), (900 if extras else 0), (30.0 if extras else 0.0)
+    sinks = (torch.randn(hq, generator=g) * 2).float() if extras else None
+    slopes = torch.tensor([2.0 ** (-8.0 * (i + 1) / hq) for i in range(hq)], dtype=torch.float32) if extras else None
+    want, want_lse = oracle.paged_attn(q, T.storage_bytes(kv_cpu), lay, bt, sl, cu, scale, return_lse=True,
+                                       sliding_window=window, soft_cap=cap, code_type=ct, sinks=sinks, alibi_slopes=slopes)
+    kv = T.to_device_cache(kv_cpu, dev, "HND", code_type=ct)
+    k, v = L.key_value_views(kv)
+    ksc, vsc = L.scale_views(kv)
+    tight = torch.empty(ops.paged_attn_workspace_bytes(len(ctx), hq, d), dtype=torch.uint8, device=dev)
+    for workspace in (None, tight):
+        out = torch.full(q.shape, float("nan"), dtype=q_dtype, device=dev)
+        lse = torch.full(q.shape[:2], float("nan"), dtype=torch.float32, device=dev)
+        ops.unified_attention(q.to(dev), k, v, out, cu.to(dev), max(qls), sl.to(dev), max(ctx), scale, True,
+                              window_size=(window - 1, 0) if window else (-1, -1), softcap=cap, block_table=bt.to(dev),
+                              k_scale_cache=ksc, v_scale_cache=vsc, kv_quant_mode=mode, lse=lse, workspace=workspace,
+                              sinks=None if sinks is None else sinks.to(dev),
+                              alibi_slopes=None if slopes is None else slopes.to(dev))
+        torch.cuda.synchronize()
+        T.assert_close_attn(out, want, what=f"short runs, {code}, workspace {'tight' if workspace is not None else 'default'}")
+        torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)

@@ -560,6 +560,23 @@ struct DecodeTile {
     kv.tail1 = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(w.r1, lo.g_tail, 0, AUX));
   }
 
+  // STREAM only: the same run loaded straight into the window, no registers in between (DB <= 128: the offsets of a
+  // run's pieces fit the instruction).  kDmaLoads instructions; the caller waits for them.
+  static constexpr int kDmaLoads = 2 * NLD + 2;
+  __device__ static void load_tile_to_lds(const Window& w, const LaneOffsets& lo, int lane, uint8_t* lds) {
+    typedef __attribute__((address_space(3))) void* lds_ptr_t;
+    constexpr int AUX = 2;
+#pragma unroll
+    for (int n = 0; n < NLD; ++n) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w.r0, (lds_ptr_t)(lds + n * 1024), 16, lo.flat, n * 1024, 0, AUX);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w.r1, (lds_ptr_t)(lds + 16 * R + n * 1024), 16, lo.flat, n * 1024, 0, AUX);
+    }
+    if (lane < 8) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w.r0, (lds_ptr_t)(lds + NLD * 1024), 16, lo.flat, NLD * 1024, 0, AUX);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(w.r1, (lds_ptr_t)(lds + 16 * R + NLD * 1024), 16, lo.flat, NLD * 1024, 0, AUX);
+    }
+  }
+
   // Drop a loaded tile into the wave's LDS window, one record per PITCH-byte row, then stage the
   // 64 scales (K scales pre-multiplied by scale*log2e, V scales by 2^8, capped so P~ stays finite).
   // After this the tile's registers are free for the next prefetch.

@@ -6,6 +6,7 @@
 #include <mutex>
 
 #include "kvq_attn_core.cuh"
+#include "kvq_short_runs.h"
 
 namespace kvq {
 
@@ -165,6 +166,18 @@ static int paged_attn_launch(const char* op, void* out, int out_dtype, int64_t o
   }
   hipStream_t s = as_stream(stream);
   int rc = KVQ_OK;
+  // a batch of short runs: one launch for all its sequences, where the workspace has room for its states (a caller that
+  // sized it for one-token rows only keeps the kernels below)
+  ShortRunArgs r{};
+  size_t short_bytes = 0;
+  if (short_runs_take(g, num_q_heads, num_seqs, max_query_len, num_wg, &r, &short_bytes) && workspace_bytes >= short_bytes) {
+    r.io = a.io;
+    r.seq_lens = seq_lens;
+    r.cu_seqlens_q = cu_seqlens_q;
+    r.causal = causal;
+    r.q_dtype = q_dtype;
+    return launch_short_runs(r, workspace, out_dtype, s);
+  }
   // a batch that the caller knows to hold no one-row sequence has nothing for the decode kernel and its reduce
   if (!(no_decode_rows && max_query_len > 1)) rc = launch_decode_streamk(a, q_dtype, out_dtype, s);
   if (rc) return rc;

@@ -5,31 +5,11 @@
 #include <type_traits>
 
 #include "kvq_attn_core.cuh"
+#include "kvq_work_line.cuh"
 
 namespace kvq {
 
 int heads_per_wg(int num_kv_heads);
-
-
-
-__device__ __forceinline__ int wave_incl_scan(int v, int lane) {
-#pragma unroll
-  for (int o = 1; o < kWave; o <<= 1) {
-    int u = __shfl_up(v, o, kWave);
-    if (lane >= o) v += u;
-  }
-  return v;
-}
-
-// Starting on a sequence (query row, first tile with nothing in flight, folding and storing the state of the
-// one before) costs a workgroup 4 - 5 us, whatever the number of kv heads it serves; the work line that is cut into
-// equal shares therefore charges every sequence StreamKArgs::setup_units units before its tiles.  A unit is a
-// tile of the workgroup's run, and the 8 / HPW waves of a head take a run's tiles in turn, so a unit lasts
-// 2.9 us / (8 / HPW) and the charge grows with the waves per head (setup_units_for).  Measured on MI355X at batch 64,
-// 1k..8k tokens: with eight kv heads and no charge, workgroups whose share crossed a sequence boundary ran 2.9 us
-// (one tile time) longer than the others and were the last to finish; with one kv head and a charge of one unit
-// they ran 23.0 us against 18.2 us and the launch waited for them.
-constexpr int setup_units_for(int waves_per_head) { return waves_per_head == 1 ? 1 : 3 * waves_per_head / 2; }
 
 // Tiles of a decode sequence: those that hold a token of the row's window,
 // [window_first / 32, ceil(len / 32)).  0 for prefill sequences and empty ones.
@@ -92,7 +72,7 @@ __device__ __forceinline__ int64_t scan_total(const StreamKArgs& a, int lane) {
     for (int j = 0; j < BATCH; ++j)
       n[j] = line_units<FIXED>(a.seq_lens, a.cu_seqlens_q, base + kWave * j + lane, B, a.io.window, a.setup_units);
 #pragma unroll
-    for (int j = 0; j < BATCH; ++j) total += __builtin_amdgcn_readlane(wave_incl_scan(n[j], lane), 63);
+    for (int j = 0; j < BATCH; ++j) total += __builtin_amdgcn_readlane(wave_incl_scan(n[j]), 63);
   }
   return total;
 }
@@ -111,7 +91,7 @@ __device__ __forceinline__ void scan_locate(const StreamKArgs& a, int lane, int6
 #pragma unroll
     for (int j = 0; j < BATCH; ++j) {
       const int n = nn[j];
-      const int incl = wave_incl_scan(n, lane);
+      const int incl = wave_incl_scan(n);
       const int64_t first = cum + incl - n, last = cum + incl;
       const uint64_t hit = __builtin_amdgcn_ballot_w64(n > 0 && first <= lo && lo < last);
       if (hit != 0 && !found) {
@@ -123,21 +103,6 @@ __device__ __forceinline__ void scan_locate(const StreamKArgs& a, int lane, int6
       cum += __builtin_amdgcn_readlane(incl, 63);
     }
   }
-}
-
-__device__ __forceinline__ int64_t wg_tile_begin(int w, int64_t total, int num_wg) {
-  return ((int64_t)w * total) / num_wg;
-}
-
-// Workgroups that take a share of a line of `total` units: all that were launched, unless the line
-// is so short that a share would fall below kMinUnitsPerWg -- a small batch is then spread over
-// fewer workgroups, so that a sequence is not cut into dozens of one-tile partial states for the
-// reduce to merge.  Measured at batch 4 x 512 tokens (main + reduce kernel): 15.6 us with shares of
-// at least 2 units, 18.3 us with 4 (a tile at a time per wave: about 4 us per tile at low load).
-constexpr int kMinUnitsPerWg = 2;
-__device__ __forceinline__ int active_workgroups(int64_t total, int num_wg) {
-  const int64_t want = total / kMinUnitsPerWg;
-  return want >= num_wg ? num_wg : (want < 1 ? 1 : (int)want);
 }
 
 // HPW = kv heads per workgroup (1, 2, 4 or 8).  A workgroup always has eight waves: with fewer than

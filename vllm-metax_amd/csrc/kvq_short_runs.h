@@ -1,0 +1,36 @@
+// Arguments and host entry of the short-run launch (kvq_short_runs_impl.cuh).
+#pragma once
+
+#include "kvq_attn_core.cuh"
+
+namespace kvq {
+
+struct ShortRunArgs {
+  AttnIO io;
+  const int32_t* seq_lens;
+  const int32_t* cu_seqlens_q;
+  int num_seqs;
+  int causal;
+  int q_dtype;
+  int q_tokens;   // query tokens per item
+  int blocks;     // items per sequence: ceil(longest run / q_tokens)
+  int cols;       // columns per item, 16 or 32
+  int num_wg;     // P
+  int setup_units;
+  // Partial states: slot w + item (unique along the staircase of (workgroup, item) pairs) holds [Hkv][cols] rows.
+  float* part_o;
+  float* part_ml;
+  int64_t* line;  // [0] the line's length, [1 + i] item i's first unit
+};
+
+// Longest run x q heads per kv head up to which a batch's runs are short (beyond it the workgroup-shared tile's 128
+// columns are at least half full).
+constexpr int kShortRunCols = 63;
+
+// Fills the run's shape and says whether the launch takes it (a head-major cache whose blocks it can stream) and how many
+// bytes of 16-byte aligned workspace it needs.
+bool short_runs_take(const kvq_cache_geom& g, int num_q_heads, int num_seqs, int max_query_len, int num_wg, ShortRunArgs* a,
+                     size_t* bytes);
+int launch_short_runs(ShortRunArgs& a, void* workspace, int out_dtype, hipStream_t s);
+
+}  // namespace kvq

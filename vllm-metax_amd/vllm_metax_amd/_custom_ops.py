@@ -345,8 +345,9 @@ def unified_attention(
     if static_scratch:
         workspace, prefill_splits = None, 1
     elif workspace is None and num_seqs > 0 and q.shape[0] > 0:
-        if prefill_splits > 1 and int(max_seqlen_q) > 1:
-            need = split_prefill_workspace_bytes(num_seqs, q.shape[1], geom.head_size, q.shape[0], prefill_splits, dev)
+        if int(max_seqlen_q) > 1:   # room for the partial states of the runs' rows as well
+            need = split_prefill_workspace_bytes(num_seqs, q.shape[1], geom.head_size, max(q.shape[0], 2048),
+                                                 max(prefill_splits, 2), dev)
         else:
             need = paged_attn_workspace_bytes(num_seqs, q.shape[1], geom.head_size, dev)
         workspace = _default_workspace(dev, need)
