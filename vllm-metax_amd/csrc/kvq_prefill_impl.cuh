@@ -16,6 +16,8 @@
 
 namespace kvq {
 
+constexpr int kMaxKSplit = 8;   // context splits of a launch at most
+
 struct PrefillArgs {
   AttnIO io;
   const int32_t* seq_lens;
@@ -747,51 +749,57 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     io.lse[row * io.num_q_heads + head] = l > 0.f ? (m + __builtin_amdgcn_logf(l)) * kLn2 : -INFINITY;
 }
 
-// The merge of the context splits: grid (query token of a run, sequence of the plan), 4 waves; a wave takes q heads
-// wave, wave + 4, ... of its row, a lane D / 64 dims.  out = sum_s w_s o_s / sum_s w_s l_s with w_s = 2^(m_s - max m):
-// the algebra of merge_attn_states over the splits' states; the sink's term and the row's lse as in the unsplit kernel.
+// The merge of the context splits: grid (query token of a run, sequence of the plan, ceil(Hq / 4)), a wave per (row, q
+// head), a lane D / 64 dims.  out = sum_s w_s o_s / sum_s w_s l_s with w_s = 2^(m_s - max m): the algebra of
+// merge_attn_states over the splits' states; the sink's term and the row's lse as in the unsplit kernel.
+// A stream of the states, 520 bytes per split at D = 128: every load of a row leaves before the first is used (splits past
+// the last reread it and weigh 0).  One block per row whose four waves went through the heads, and a head's splits, one
+// after the other took 26 us for 512 rows x 32 heads x 4 splits (34 MB), this takes 9.
 template <int D, int ODT>
 __global__ __launch_bounds__(256) void prefill_split_merge_kernel(PrefillArgs a) {
   constexpr int V = D / 64;
+  typedef float vec_t __attribute__((ext_vector_type(V), aligned(4 * V)));
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (blockIdx.y >= (unsigned)a.plan[0]) return;
   const int seq = a.plan[1 + blockIdx.y];
   const int q_begin = a.cu_seqlens_q[seq];
   const int q_len = a.cu_seqlens_q[seq + 1] - q_begin;
   const int qi = blockIdx.x;
-  if (q_len <= 1 || qi >= q_len || a.seq_lens[seq] <= 0) return;
+  const int head = blockIdx.z * 4 + wave;
   const AttnIO& io = a.io;
+  if (q_len <= 1 || qi >= q_len || a.seq_lens[seq] <= 0 || head >= io.num_q_heads) return;
   const int64_t row = q_begin + qi;
   const int S = a.ksplit;
-  for (int head = wave; head < io.num_q_heads; head += 4) {
-    const float* p = a.part + ((row * io.num_q_heads + head) * S) * (D + 2);
-    float mmax = -INFINITY;
-    for (int s = 0; s < S; ++s) mmax = fmaxf(mmax, p[s * (D + 2) + D]);
-    const float mref = mmax == -INFINITY ? 0.f : mmax;
-    float acc[V];
+  const float* p = a.part + ((row * io.num_q_heads + head) * S) * (D + 2);
+  const int mine = min(lane, S - 1);   // lane s takes split s's (m, l)
+  const float ms = p[mine * (D + 2) + D], ls = p[mine * (D + 2) + D + 1];
+  float po[kMaxKSplit][V];
 #pragma unroll
-    for (int i = 0; i < V; ++i) acc[i] = 0.f;
-    float l = 0.f;
-    for (int s = 0; s < S; ++s) {
-      const float* ps = p + s * (D + 2);
-      const float w = __builtin_amdgcn_exp2f(ps[D] - mref);   // an empty range: 2^-inf = 0
-      l += w * ps[D + 1];
+  for (int s = 0; s < kMaxKSplit; ++s) {
+    const vec_t x = *reinterpret_cast<const vec_t*>(p + min(s, S - 1) * (D + 2) + V * lane);
 #pragma unroll
-      for (int i = 0; i < V; ++i) acc[i] += w * ps[V * lane + i];
-    }
-    if (l > 0.f) l += sink_term(io.sinks, head, mmax);   // a row without a visible key keeps its zeros
-    const float mul = l > 0.f ? 1.0f / l : 0.f;
-    const int64_t at = row * io.out_stride_t + (int64_t)head * io.out_stride_h + V * lane;
-#pragma unroll
-    for (int i = 0; i < V; ++i) {
-      const float v = acc[i] * mul;
-      if constexpr (ODT == KVQ_F32) reinterpret_cast<float*>(io.out)[at + i] = v;
-      else if constexpr (ODT == KVQ_BF16) reinterpret_cast<uint16_t*>(io.out)[at + i] = f32_to_bf16_bits(v);
-      else reinterpret_cast<uint16_t*>(io.out)[at + i] = (uint16_t)(pack_half2(v, 0.f) & 0xffffu);
-    }
-    if (io.lse != nullptr && lane == 0)
-      io.lse[row * io.num_q_heads + head] = l > 0.f ? (mmax + __builtin_amdgcn_logf(l)) * kLn2 : -INFINITY;
+    for (int i = 0; i < V; ++i) po[s][i] = x[i];
   }
+  const float mmax = wave_max(ms);
+  const float mref = mmax == -INFINITY ? 0.f : mmax;
+  const float es = lane < S ? __builtin_amdgcn_exp2f(ms - mref) : 0.f;   // an empty range: 2^-inf = 0
+  float l = wave_sum(es * ls);
+  float acc[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) acc[i] = 0.f;
+#pragma unroll
+  for (int s = 0; s < kMaxKSplit; ++s) {
+    const float w = as_f32(__builtin_amdgcn_readlane(as_u32(es), s));
+#pragma unroll
+    for (int i = 0; i < V; ++i) acc[i] += w * po[s][i];
+  }
+  if (l > 0.f) l += sink_term(io.sinks, head, mmax);   // a row without a visible key keeps its zeros
+  const float mul = l > 0.f ? 1.0f / l : 0.f;
+  const int64_t at = row * io.out_stride_t + (int64_t)head * io.out_stride_h + V * lane;
+#pragma unroll
+  for (int i = 0; i < V; ++i) store_act<ODT>(io.out, at + i, acc[i] * mul);
+  if (io.lse != nullptr && lane == 0)
+    io.lse[row * io.num_q_heads + head] = l > 0.f ? (mmax + __builtin_amdgcn_logf(l)) * kLn2 : -INFINITY;
 }
 
 template <int D, int QDT, int ODT, bool EXT, int CODE = KVQ_CODE_INT8>
@@ -806,7 +814,7 @@ static int launch_prefill_flash32(PrefillArgs& a, int max_query_len, hipStream_t
       dim3 grid(blocks * a.ksplit, a.num_seqs, a.io.g.num_kv_heads);
       hipLaunchKernelGGL((paged_prefill_flash32_kernel<D, QDT, ODT, true, CODE, true>), grid, dim3(256), FP::LDS_BYTES, s, a);
       if (int e = check_hip(hipGetLastError(), "paged_prefill_flash32 launch")) return e;
-      dim3 mgrid(max_query_len, a.num_seqs);
+      dim3 mgrid(max_query_len, a.num_seqs, (a.io.num_q_heads + 3) / 4);
       hipLaunchKernelGGL((prefill_split_merge_kernel<D, ODT>), mgrid, dim3(256), 0, s, a);
       return check_hip(hipGetLastError(), "prefill split merge launch");
     }
