@@ -619,7 +619,13 @@ KVQ_API int kvq_mla_v_up_proj(void* out, int64_t out_stride_b, int64_t out_strid
  * with no visible key gets out = 0 and lse = -inf (what mask_empty_context of
  * mla_attention.py:2104-2110 forces).  Built head dims (nope, rope, v):
  * (128, 64, 128), (64, 32, 64), (128, 0, 128).
+ * `causal` is a set of flags: KVQ_MLA_PREFILL_CAUSAL (1), and KVQ_MLA_PREFILL_MERGE
+ * (2): out and lse (then required) already hold the rows' attention over OTHER
+ * keys, and this call's is merged into it, as kvq_merge_attn_states would with
+ * out / lse as one of its two states; rows that see no key here stay as they are.
  */
+#define KVQ_MLA_PREFILL_CAUSAL 1
+#define KVQ_MLA_PREFILL_MERGE 2
 KVQ_API int kvq_mla_prefill_attn(const void* q, int dtype, int64_t q_stride_tok, int64_t q_stride_head,
                          const void* k_nope, int64_t kn_stride_tok, int64_t kn_stride_head,
                          const void* k_pe, int64_t kpe_stride_tok, const void* v,

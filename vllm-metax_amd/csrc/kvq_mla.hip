@@ -151,7 +151,9 @@ __global__ __launch_bounds__(256) void mla_rope_quant_write_kernel(
 // prefill reads its cached context this way).  One wavefront per destination row: lanes 0 .. W/16-1
 // load 16 codes each (one coalesced run of W bytes), every lane reads the row's scale, and the 16
 // products code * scale go out as one or two 16-byte stores per lane.
-template <int DT>
+// WIDE: 16-byte stores (rows of dst 16-byte aligned); element by element the sixteen 2-byte stores per lane took 15.7 us
+// for 7340 rows, against 5 us.
+template <int DT, bool WIDE>
 __global__ __launch_bounds__(256) void mla_gather_dequant_kernel(void* __restrict__ dst, int64_t dst_stride,
                                                                  const uint8_t* __restrict__ cache, kvq_mla_geom g,
                                                                  const int32_t* __restrict__ block_table,
@@ -183,8 +185,29 @@ __global__ __launch_bounds__(256) void mla_gather_dequant_kernel(void* __restric
       for (int j = 0; j < 4; ++j) f[4 * i + j] = (float)(int8_t)(x >> (8 * j)) * scale;
     }
     const int64_t at = t * dst_stride + lane * 16;
+    if constexpr (WIDE) {
+      constexpr int N = DT == KVQ_F32 ? 4 : 8;   // elements per 16-byte store
 #pragma unroll
-    for (int i = 0; i < 16; ++i) store_act<DT>(dst, at + i, f[i]);
+      for (int i = 0; i < 16; i += N) {
+        u32x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if constexpr (DT == KVQ_F32) {
+            v[j] = as_u32(f[i + j]);
+          } else if constexpr (DT == KVQ_BF16) {
+            v[j] = (uint32_t)f32_to_bf16_bits(f[i + 2 * j]) | ((uint32_t)f32_to_bf16_bits(f[i + 2 * j + 1]) << 16);
+          } else {
+            const half2_t h = {(half_t)f[i + 2 * j], (half_t)f[i + 2 * j + 1]};
+            v[j] = __builtin_bit_cast(uint32_t, h);
+          }
+        }
+        constexpr int ESZ = DT == KVQ_F32 ? 4 : 2;
+        *reinterpret_cast<u32x4*>(static_cast<uint8_t*>(dst) + (at + i) * ESZ) = v;
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) store_act<DT>(dst, at + i, f[i]);
+    }
   }
 }
 
@@ -322,10 +345,17 @@ extern "C" int kvq_gather_and_dequant_mla_int8(void* dst, int dst_dtype, int64_t
   hipStream_t s = as_stream(stream);
   const int64_t want = (num_tokens + 3) / 4;
   const unsigned blocks = (unsigned)(want < 65536 ? want : 65536);
-#define KVQ_MLAG(T)                                                                                      \
-  hipLaunchKernelGGL((mla_gather_dequant_kernel<T>), dim3(blocks), dim3(256), 0, s, dst, dst_stride,  \
+#define KVQ_MLAG_W(T, W16)                                                                               \
+  hipLaunchKernelGGL((mla_gather_dequant_kernel<T, W16>), dim3(blocks), dim3(256), 0, s, dst, dst_stride,  \
                      static_cast<const uint8_t*>(cache), g, block_table, bt_stride, cu_seq_lens,       \
                      token_to_seq, seq_starts, (int)num_tokens)
+  const int esz = dst_dtype == KVQ_F32 ? 4 : 2;
+  const bool wide = ((uintptr_t)dst % 16) == 0 && (dst_stride * esz) % 16 == 0;
+#define KVQ_MLAG(T)                \
+  do {                             \
+    if (wide) KVQ_MLAG_W(T, true); \
+    else KVQ_MLAG_W(T, false);     \
+  } while (0)
   switch (dst_dtype) {
     case KVQ_F32: KVQ_MLAG(KVQ_F32); break;
     case KVQ_BF16: KVQ_MLAG(KVQ_BF16); break;
@@ -333,6 +363,7 @@ extern "C" int kvq_gather_and_dequant_mla_int8(void* dst, int dst_dtype, int64_t
     default: return fail(KVQ_EINVAL, "%s: unknown dst_dtype %d", op, dst_dtype);
   }
 #undef KVQ_MLAG
+#undef KVQ_MLAG_W
   return check_hip(hipGetLastError(), "gather_and_dequant_mla_int8 launch");
 }
 

@@ -891,13 +891,15 @@ def concat_mla_q(ql_nope: torch.Tensor, q_pe: torch.Tensor, q_out: torch.Tensor)
 def mla_prefill_attention(q: torch.Tensor, k_nope: torch.Tensor, k_pe: torch.Tensor | None, v: torch.Tensor,
                           cu_seqlens_q: torch.Tensor, cu_seqlens_k: torch.Tensor, max_seqlen_q: int,
                           softmax_scale: float, causal: bool, out: torch.Tensor | None = None,
-                          lse: torch.Tensor | None = None, return_softmax_lse: bool = False):
+                          lse: torch.Tensor | None = None, return_softmax_lse: bool = False, merge_into: bool = False):
     """Varlen attention of the MLA prefill with the LSE the chunked-context merge needs: the role of
     ``flash_attn_varlen_func`` in vllm_metax/v1/attention/backends/mla/prefill/flash_attn.py:128-221 (keyword
     names kept), except that the key comes in the two pieces the layer holds -- ``k_nope [S, H, nope]`` and
     ``k_pe [S, rope]`` or ``[S, 1, rope]``, shared by the heads -- and ``v [S, H, v_dim]`` keeps its own
     head size.  ``q [T, H, nope + rope]``; returns ``out [T, H, v_dim]``, and ``(out, lse [H, T] fp32)`` with
-    ``return_softmax_lse``.  ``out`` / ``lse`` may be passed in to avoid the allocation."""
+    ``return_softmax_lse``.  ``out`` / ``lse`` may be passed in to avoid the allocation.  ``merge_into``: ``out`` and
+    ``lse`` hold the rows' attention over other keys, and this call's is merged into them (:func:`merge_attn_states`
+    without the trip through memory)."""
     dev = _require_cuda(q, k_nope, k_pe, v, cu_seqlens_q, cu_seqlens_k, out, lse)
     if q.dim() != 3 or k_nope.dim() != 3 or v.dim() != 3:
         raise RuntimeError("q, k_nope and v must be [tokens, heads, dim]")
@@ -919,6 +921,8 @@ def mla_prefill_attention(q: torch.Tensor, k_nope: torch.Tensor, k_pe: torch.Ten
     for name, t in (("cu_seqlens_q", cu_seqlens_q), ("cu_seqlens_k", cu_seqlens_k)):
         if t.dtype != torch.int32 or not t.is_contiguous():
             raise RuntimeError(f"{name} must be contiguous int32")
+    if merge_into and (out is None or lse is None):
+        raise RuntimeError("merge_into needs out and lse to merge into")
     B = cu_seqlens_q.numel() - 1
     if cu_seqlens_k.numel() != B + 1:
         raise RuntimeError("cu_seqlens_q and cu_seqlens_k must have the same length")
@@ -935,6 +939,6 @@ def mla_prefill_attention(q: torch.Tensor, k_nope: torch.Tensor, k_pe: torch.Ten
             _ptr(q), _dtype_code(q, "q"), q.stride(0), q.stride(1), _ptr(k_nope), k_nope.stride(0), k_nope.stride(1),
             _ptr(k_pe), k_pe.stride(0) if k_pe is not None else 0, _ptr(v), v.stride(0), v.stride(1),
             _ptr(cu_seqlens_q), _ptr(cu_seqlens_k), B, int(max_seqlen_q), T, H, nope, rope, dv, float(softmax_scale),
-            1 if causal else 0, _ptr(out), out.stride(0), out.stride(1), _ptr(lse), _stream(dev))
+            (1 if causal else 0) | (2 if merge_into else 0), _ptr(out), out.stride(0), out.stride(1), _ptr(lse), _stream(dev))
     _C.check(rc, "mla_prefill_attention")
     return (out, lse) if return_softmax_lse else out

@@ -373,16 +373,12 @@ class Int8MLAImpl(_MLAImplBase):
             prefill.prefill_backend.run_prefill_new_tokens(q=q, k=(k_nope, k_pe2), v=v, return_softmax_lse=False,
                                                            out=out3)
             return output
-        suffix_output, suffix_lse = prefill.prefill_backend.run_prefill_new_tokens(
-            q=q, k=(k_nope, k_pe2), v=v, return_softmax_lse=True)
-        context_output, context_lse = compute_prefill_context(
-            q, kv_c_and_k_pe_cache, prefill, self._kv_up_proj, self.num_heads, self.kv_lora_rank,
-            self.qk_nope_head_dim, self.v_head_dim, geometry=self._geom(kv_c_and_k_pe_cache))
-        if not out3.is_contiguous():
-            raise RuntimeError("output must be contiguous")
-        ops.merge_attn_states(output=out3, prefix_output=context_output, prefix_lse=context_lse,
-                              suffix_output=suffix_output, suffix_lse=suffix_lse,
-                              prefill_tokens_with_context=prefill.chunked_context.prefill_tokens_with_context)
+        # the new tokens' state goes into the output, and the context is merged into it where it lies
+        state = prefill.prefill_backend.run_prefill_new_tokens(q=q, k=(k_nope, k_pe2), v=v, return_softmax_lse=True,
+                                                               out=out3)
+        compute_prefill_context(q, kv_c_and_k_pe_cache, prefill, self._kv_up_proj, self.num_heads, self.kv_lora_rank,
+                                self.qk_nope_head_dim, self.v_head_dim, geometry=self._geom(kv_c_and_k_pe_cache),
+                                into=state)
         return output
 
 

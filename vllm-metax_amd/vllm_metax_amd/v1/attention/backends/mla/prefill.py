@@ -150,22 +150,27 @@ class Int8MLAPrefillBackend:
         return ops.mla_prefill_attention(q, k_nope, k_pe, v, md.query_start_loc, md.query_start_loc, md.max_query_len,
                                          self.scale, causal=True, out=out, return_softmax_lse=return_softmax_lse)
 
-    def run_prefill_context_chunk(self, chunk_idx: int, q: torch.Tensor, k, v: torch.Tensor):
+    def run_prefill_context_chunk(self, chunk_idx: int, q: torch.Tensor, k, v: torch.Tensor, into=None):
+        """``into`` = (out [T, H, v], lse [H, T]): the chunk's result is merged into that state, and it is returned."""
         md = self._prefill_metadata
+        out, lse = into if into is not None else (None, None)
         k_nope, k_pe = _split_k(k, self.qk_nope_head_dim)
         return ops.mla_prefill_attention(q, k_nope, k_pe, v, md.query_start_loc,
                                          md.chunked_context.cu_seq_lens[chunk_idx], md.max_query_len, self.scale,
-                                         causal=False, return_softmax_lse=True)
+                                         causal=False, out=out, lse=lse, return_softmax_lse=True,
+                                         merge_into=into is not None)
 
 
 def compute_prefill_context(q: torch.Tensor, kv_c_and_k_pe_cache: torch.Tensor, prefill: Int8MLAPrefillMetadata,
                             kv_b_proj, num_heads: int, kv_lora_rank: int, qk_nope_head_dim: int, v_head_dim: int,
-                            geometry=None):
+                            geometry=None, into=None):
     """The chunk loop of ``_compute_prefill_context`` (mla_attention.py:2017-2140) over the int8 latent
-    cache; returns the context's ``(output [T, H, v_head_dim], lse [H, T])``."""
+    cache; returns the context's ``(output [T, H, v_head_dim], lse [H, T])``.  The first chunk makes that state, or
+    ``into`` (the new tokens' state) is it from the start; the other chunks' results are merged into it by the
+    attention launch itself."""
     cc = prefill.chunked_context
     backend = prefill.prefill_backend
-    output = output_lse = merge_output = merge_lse = None
+    state = into
     for i in range(len(cc.seq_tot)):
         toks = cc.seq_tot[i]
         ops.gather_and_maybe_dequant_cache(
@@ -181,14 +186,5 @@ def compute_prefill_context(q: torch.Tensor, kv_c_and_k_pe_cache: torch.Tensor, 
         k_pe = rows[..., kv_lora_rank:]
         # a prefill without rows in this chunk comes back with out = 0, lse = -inf from the kernel itself
         # (what mask_empty_context forces, mla_attention.py:2104-2110)
-        attn_output, attn_lse = backend.run_prefill_context_chunk(chunk_idx=i, q=q, k=(k_nope, k_pe), v=v)
-        if output is None:
-            output, output_lse = attn_output, attn_lse
-        else:
-            if merge_output is None:
-                merge_output, merge_lse = torch.empty_like(output), torch.empty_like(output_lse)
-            ops.merge_attn_states(output=merge_output, output_lse=merge_lse, prefix_output=output,
-                                  prefix_lse=output_lse, suffix_output=attn_output, suffix_lse=attn_lse)
-            output, merge_output = merge_output, output
-            output_lse, merge_lse = merge_lse, output_lse
-    return output, output_lse
+        state = backend.run_prefill_context_chunk(chunk_idx=i, q=q, k=(k_nope, k_pe), v=v, into=state)
+    return state
