@@ -28,7 +28,6 @@
 // XCD that prepares its query and reduces it (mla_seq_split_of_block).  Nothing is allocated here,
 // partials and the int8 Q live in the caller's workspace.
 #include <atomic>
-#include <type_traits>
 
 #include "kvq_attn_core.cuh"
 
@@ -153,10 +152,14 @@ __device__ __forceinline__ half8_t mla_code_rows_to_operand(const uint32_t (&x)[
 }
 
 // tokens of a sequence per split, a whole number of tiles
-__device__ __forceinline__ int mla_split_len(int len, int num_splits) {
+// None is shorter than `at_least` tokens: the one-head-tile kernel, whose four waves take a tile each at a time, cuts
+// at 128, so that a short sequence in a small batch leaves a quarter of the states with no wave taking more tiles.
+__host__ __device__ __forceinline__ int mla_split_len(int len, int num_splits, int at_least) {
   const int per = (len + num_splits - 1) / num_splits;
-  return ((per + kTile - 1) / kTile) * kTile;
+  const int tokens = ((per + kTile - 1) / kTile) * kTile;
+  return tokens > at_least ? tokens : at_least;
 }
+constexpr int kMlaMinSplit = kTile, kMlaSmallMinSplit = 4 * kTile;
 
 // 16 values of one head -> the 16 bytes of each of the two int8 terms, q ~ s1 a + s2 b with s2 = s1 / 256:
 // w = rint(q / s2) is a 15-bit integer (|w| <= 16384 because s1 = max|q| / kMlaQ1Max), and w = 256 a + b with
@@ -453,7 +456,7 @@ __global__ __launch_bounds__(kMlaThreads) void mla_decode_kernel(MlaArgs a) {
   int seq, split;
   mla_seq_split_of_block(gridDim.y, a.num_splits, seq, split);
   const int len = a.seq_lens[seq];
-  const int slen = mla_split_len(len > 0 ? len : 0, a.num_splits);
+  const int slen = mla_split_len(len > 0 ? len : 0, a.num_splits, kMlaMinSplit);
   const int tok_begin = split * slen;
   const int tok_end = min(len, tok_begin + slen);
   // head tiles (16 heads each) of this workgroup's 128-head block; wave w < nht owns tile w: it
@@ -921,7 +924,7 @@ __global__ __launch_bounds__(kMlaSmallThreads) void mla_decode_small_kernel(MlaA
   int seq, split;
   mla_seq_split_of_block(gridDim.y, a.num_splits, seq, split);
   const int len = a.seq_lens[seq];
-  const int slen = mla_split_len(len > 0 ? len : 0, a.num_splits);
+  const int slen = mla_split_len(len > 0 ? len : 0, a.num_splits, kMlaSmallMinSplit);
   const int tok_begin = split * slen;
   const int tok_end = min(len, tok_begin + slen);
   const int64_t pblock = ((int64_t)seq * a.num_splits + split) * a.head_groups;
@@ -1282,100 +1285,155 @@ __global__ __launch_bounds__(kMlaSmallThreads) void mla_decode_small_kernel(MlaA
   if (wave == 0 && g == 0) a.part_lse[pblock * 16 + c] = m_all + __builtin_amdgcn_logf(l_all);
 }
 
-// Stage 2: out = sum_j 2^(lse_j - max) o_j / sum_j 2^(lse_j - max); lse = ln 2 * (max + log2 sum).
-// grid (B, ceil(H/16)), 8 waves; wave w combines the d4 = w slice of the block's 16 heads, lane (c, g)
-// as in the split state layout.  RPT = 4: a thread takes its four 4-dim pieces of every split, eight splits per
-// trip to memory.  RPT = 1 (grid.z = 4): one piece per thread and 32 splits per trip, for a few sequences cut
-// into dozens of splits -- their grid is a handful of blocks, and eight splits per trip made 64 splits a chain
-// of eight round trips (20 us for one 32k-token sequence, half as long as its decode kernel).
-template <int ODT, int RPT>
+// Four consecutive dims of a head's finished row.
+template <int ODT>
+__device__ __forceinline__ void mla_store_row4(void* out, int64_t o, floatx4 v) {
+  if constexpr (ODT == KVQ_F32) {
+    *reinterpret_cast<floatx4*>(reinterpret_cast<float*>(out) + o) = v;
+  } else {
+    u32x2 w;
+    if constexpr (ODT == KVQ_BF16) {
+      w.x = (uint32_t)f32_to_bf16_bits(v.x) | ((uint32_t)f32_to_bf16_bits(v.y) << 16);
+      w.y = (uint32_t)f32_to_bf16_bits(v.z) | ((uint32_t)f32_to_bf16_bits(v.w) << 16);
+    } else {
+      w.x = pack_half2(v.x, v.y);
+      w.y = pack_half2(v.z, v.w);
+    }
+    *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(out) + o) = w;
+  }
+}
+
+// Stage 2: out = sum_j 2^(lse_j - max) o_j / sum_j 2^(lse_j - max); lse = ln 2 * (max + log2 sum), for at most
+// kMlaReduceTrip splits.  grid (B, ceil(H/16)), 8 waves; wave w combines the d4 = w slice of the block's 16 heads, lane
+// (c, g) as in the split state layout; every load leaves before anything is computed from them: one trip to memory.
+// N = the splits it requests (2, 4 or 8: the least that holds the launch's).
+// Every load is unconditional and a split that holds nothing (lse = -inf; its state rows were never
+// written) is removed with a bit mask on the loaded words: a select on the value would be turned into
+// a branch around the load, and the loads of successive splits would run one by one.
+constexpr int kMlaReduceTrip = 8;
+template <int ODT, int N>
 __global__ __launch_bounds__(512) void mla_reduce_kernel(void* out, float* lse, const uint16_t* part_o,
                                                          const float* part_lse, const int32_t* seq_lens,
                                                          int num_heads, int head_groups, int num_splits) {
-  constexpr int SPT = RPT == 4 ? 8 : 32;           // splits per trip
-  const int r0 = RPT == 4 ? 0 : (int)blockIdx.z;   // the thread's first piece
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane & 15, g = lane >> 4;
   const int seq = blockIdx.x, hgroup = blockIdx.y;
   const int head = hgroup * 16 + c;
-  const bool head_ok = head < num_heads;
   const int64_t lstride = (int64_t)head_groups * 16;                    // part_lse stride between splits
   const float* pl = part_lse + ((int64_t)seq * num_splits * head_groups + hgroup) * 16 + c;
-  const uint16_t* po = part_o + ((int64_t)seq * num_splits * head_groups + hgroup) * (16 * kMlaR) + (wave * 4 * 64 + lane) * 4 + r0 * 256;
+  const uint16_t* po = part_o + ((int64_t)seq * num_splits * head_groups + hgroup) * (16 * kMlaR) + (wave * 4 * 64 + lane) * 4;
   const int64_t ostride = (int64_t)head_groups * 16 * kMlaR;            // part_o stride between splits
-  floatx4 acc[RPT];
-#pragma unroll
-  for (int r = 0; r < RPT; ++r) acc[r] = (floatx4){0.f, 0.f, 0.f, 0.f};
-  float mx = -INFINITY;
   const bool live = seq_lens[seq] > 0;
+  float lj[N];
+  u32x2 hv[N][4];
+#pragma unroll
+  for (int u = 0; u < N; ++u) {
+    const int j = min(u, num_splits - 1);   // a slot past the last split rereads the last one and weighs 0
+    lj[u] = pl[j * lstride];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) hv[u][r] = *reinterpret_cast<const u32x2*>(po + j * ostride + r * 256);
+  }
+  float mx = -INFINITY;
+#pragma unroll
+  for (int u = 0; u < N; ++u) mx = fmaxf(mx, (live && u < num_splits) ? lj[u] : -INFINITY);
+  const float mref = mx == -INFINITY ? 0.f : mx;
+  floatx4 acc[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) acc[r] = (floatx4){0.f, 0.f, 0.f, 0.f};
   float den = 0.f;
-  // Eight splits at a time, and all loads of a group -- the eight lse values and the eight states -- leave
-  // before anything is computed from them: one trip to memory per group instead of two (the maximum first,
-  // then the states).  The running maximum moves between groups, with the usual rescaling.
-  // Every load is unconditional and a split that holds nothing (lse = -inf; its state rows were never
-  // written) is removed with a bit mask on the loaded words: a select on the value would be turned into
-  // a branch around the load, and the loads of successive splits would run one by one.
-  for (int j0 = 0; j0 < num_splits; j0 += SPT) {
-    float lj[SPT];
-    u32x2 hv[SPT][RPT];
 #pragma unroll
-    for (int u = 0; u < SPT; ++u) {
-      const int j = min(j0 + u, num_splits - 1);   // a slot past the last split rereads the last one and weighs 0
-      lj[u] = pl[j * lstride];
-      const uint16_t* pj = po + j * ostride;
+  for (int u = 0; u < N; ++u) {
+    const bool on = live && u < num_splits && lj[u] != -INFINITY;
+    const float wj = on ? __builtin_amdgcn_exp2f(lj[u] - mref) : 0.f;
+    const uint32_t keep = wj != 0.f ? 0xffffffffu : 0u;
+    den += wj;
 #pragma unroll
-      for (int r = 0; r < RPT; ++r) hv[u][r] = *reinterpret_cast<const u32x2*>(pj + r * 256);
+    for (int r = 0; r < 4; ++r) {
+      const uint32_t h0 = hv[u][r].x & keep, h1 = hv[u][r].y & keep;
+      const half2_t a0 = __builtin_bit_cast(half2_t, h0), a1 = __builtin_bit_cast(half2_t, h1);
+      acc[r] += (floatx4){(float)a0.x, (float)a0.y, (float)a1.x, (float)a1.y} * wj;
     }
-    float cm = -INFINITY;
+  }
+  if (head >= num_heads) return;
+  const float inv = den > 0.f ? 1.0f / den : 0.f;                       // nothing attended: zeros
+  const int64_t obase = ((int64_t)seq * num_heads + head) * kMlaR + 64 * wave + 16 * g;
 #pragma unroll
-    for (int u = 0; u < SPT; ++u) cm = fmaxf(cm, (live && j0 + u < num_splits) ? lj[u] : -INFINITY);
-    const float m_new = fmaxf(mx, cm);
-    const float mref = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = mx == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mx - mref);
-    mx = m_new;
-    den *= alpha;
+  for (int r = 0; r < 4; ++r) mla_store_row4<ODT>(out, obase + 4 * r, acc[r] * inv);
+  if (lse != nullptr && wave == 0 && g == 0)
+    lse[(int64_t)seq * num_heads + head] = den > 0.f ? (mx + __builtin_amdgcn_logf(den)) * kLn2 : -INFINITY;
+}
+
+// The same for a few sequences cut into up to 64 splits: grid (B, ceil(H/16), 8), block z combines the d4 = z slice, its
+// eight waves take the splits in turn (wave w: w, w + 8, ...) and their sums meet in LDS.  Still one trip to memory, and
+// only the splits that the sequence's length fills are read (min_split: what the decode kernel cut by).  With a wave
+// taking every split of its slice, 32 per trip, most of them empty, 7 sequences of 350 - 2400 tokens took 10 us.
+template <int ODT>
+__global__ __launch_bounds__(512) void mla_reduce_wide_kernel(void* out, float* lse, const uint16_t* part_o,
+                                                              const float* part_lse, const int32_t* seq_lens,
+                                                              int num_heads, int head_groups, int num_splits, int min_split) {
+  __shared__ floatx4 sh_acc[8][4][kWave];
+  __shared__ float sh_m[8][kWave], sh_den[8][kWave];
+  constexpr int N = 8;   // splits per wave: 64 / 8
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 15, g = lane >> 4;
+  const int seq = blockIdx.x, hgroup = blockIdx.y, d4 = blockIdx.z;
+  const int head = hgroup * 16 + c;
+  const int len = max(seq_lens[seq], 0);
+  const int slen = mla_split_len(len, num_splits, min_split);
+  const int splits = (len + slen - 1) / slen;   // every one of them holds a token
+  const int64_t block0 = (int64_t)seq * num_splits * head_groups + hgroup;
+  floatx4 acc[4];
 #pragma unroll
-    for (int r = 0; r < RPT; ++r) acc[r] *= alpha;
+  for (int r = 0; r < 4; ++r) acc[r] = (floatx4){0.f, 0.f, 0.f, 0.f};
+  float mx = -INFINITY, den = 0.f;
+  if (wave < splits) {   // uniform over the wave
+    float lj[N];
+    u32x2 hv[N][4];
 #pragma unroll
-    for (int u = 0; u < SPT; ++u) {
-      const bool on = live && j0 + u < num_splits && lj[u] != -INFINITY;
-      const float wj = on ? __builtin_amdgcn_exp2f(lj[u] - mref) : 0.f;
-      const uint32_t keep = wj != 0.f ? 0xffffffffu : 0u;
+    for (int u = 0; u < N; ++u) {
+      const int64_t at = block0 + (int64_t)min(wave + 8 * u, splits - 1) * head_groups;   // past the last: reread, weighs 0
+      lj[u] = part_lse[at * 16 + c];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        hv[u][r] = *reinterpret_cast<const u32x2*>(part_o + at * (16 * kMlaR) + ((d4 * 4 + r) * 64 + lane) * 4);
+    }
+#pragma unroll
+    for (int u = 0; u < N; ++u) mx = fmaxf(mx, wave + 8 * u < splits ? lj[u] : -INFINITY);
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const float wj = wave + 8 * u < splits ? __builtin_amdgcn_exp2f(lj[u] - mx) : 0.f;
       den += wj;
 #pragma unroll
-      for (int r = 0; r < RPT; ++r) {
-        const uint32_t h0 = hv[u][r].x & keep, h1 = hv[u][r].y & keep;
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t h0 = hv[u][r].x, h1 = hv[u][r].y;
         const half2_t a0 = __builtin_bit_cast(half2_t, h0), a1 = __builtin_bit_cast(half2_t, h1);
-        acc[r].x += (float)a0.x * wj;
-        acc[r].y += (float)a0.y * wj;
-        acc[r].z += (float)a1.x * wj;
-        acc[r].w += (float)a1.y * wj;
+        acc[r] += (floatx4){(float)a0.x, (float)a0.y, (float)a1.x, (float)a1.y} * wj;
       }
     }
   }
-  if (!head_ok) return;
-  const float inv = den > 0.f ? 1.0f / den : 0.f;                       // nothing attended: zeros
-  const int64_t obase = ((int64_t)seq * num_heads + head) * kMlaR + 16 * g;
 #pragma unroll
-  for (int r = 0; r < RPT; ++r) {
-    const int64_t o = obase + 64 * wave + 4 * (r0 + r);   // four consecutive dims: one store (rows are 1024 elements apart)
-    const floatx4 v = acc[r] * inv;
-    if constexpr (ODT == KVQ_F32) {
-      *reinterpret_cast<floatx4*>(reinterpret_cast<float*>(out) + o) = v;
-    } else if constexpr (ODT == KVQ_BF16) {
-      u32x2 w;
-      w.x = (uint32_t)f32_to_bf16_bits(v.x) | ((uint32_t)f32_to_bf16_bits(v.y) << 16);
-      w.y = (uint32_t)f32_to_bf16_bits(v.z) | ((uint32_t)f32_to_bf16_bits(v.w) << 16);
-      *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(out) + o) = w;
-    } else {
-      u32x2 w;
-      w.x = pack_half2(v.x, v.y);
-      w.y = pack_half2(v.z, v.w);
-      *reinterpret_cast<u32x2*>(reinterpret_cast<uint16_t*>(out) + o) = w;
-    }
+  for (int r = 0; r < 4; ++r) sh_acc[wave][r][lane] = acc[r];
+  sh_m[wave][lane] = mx;
+  sh_den[wave][lane] = den;
+  __syncthreads();
+  if (wave >= 4 || head >= num_heads) return;   // wave r finishes piece r
+  float m_all = -INFINITY;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) m_all = fmaxf(m_all, sh_m[w][lane]);
+  const float mref = m_all == -INFINITY ? 0.f : m_all;
+  floatx4 sum = {0.f, 0.f, 0.f, 0.f};
+  float total = 0.f;
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    const float e = __builtin_amdgcn_exp2f(sh_m[w][lane] - mref);   // a wave without a split: 0
+    total += sh_den[w][lane] * e;
+    sum += sh_acc[w][wave][lane] * e;
   }
-  if (lse != nullptr && wave == 0 && g == 0 && r0 == 0)
-    lse[(int64_t)seq * num_heads + head] = den > 0.f ? (mx + __builtin_amdgcn_logf(den)) * kLn2 : -INFINITY;
+  const float inv = total > 0.f ? 1.0f / total : 0.f;               // nothing attended: zeros
+  mla_store_row4<ODT>(out, ((int64_t)seq * num_heads + head) * kMlaR + 64 * d4 + 16 * g + 4 * wave, sum * inv);
+  if (lse != nullptr && d4 == 0 && wave == 0 && g == 0)
+    lse[(int64_t)seq * num_heads + head] = total > 0.f ? (m_all + __builtin_amdgcn_logf(total)) * kLn2 : -INFINITY;
 }
 
 // num_kv_splits policy of the reference (vllm_metax/v1/attention/backends/mla/triton_mla.py:45-55),
@@ -1580,19 +1638,21 @@ static int mla_decode_run(const char* op, void* out, int out_dtype, float* lse, 
   int rc = check_hip(hipGetLastError(), "mla_decode_int8 launch");
   if (rc) return rc;
   if (splits == 1) return KVQ_OK;   // the decode kernel wrote the result itself
-  // a few blocks and dozens of splits: a piece per thread, 32 splits per trip, four times the blocks
-  // (never in the batch-invariant mode, whose eight splits are merged in one trip by either kernel: the choice must
-  // not depend on the batch)
-  const bool fine = splits > 8 && 4 * num_seqs * head_groups <= num_cus();
-  dim3 rgrid(num_seqs, head_groups, fine ? 4 : 1);
-#define KVQ_MLAR(T)                                                                                                \
-  do {                                                                                                             \
-    if (fine)                                                                                                      \
-      hipLaunchKernelGGL((mla_reduce_kernel<T, 1>), rgrid, dim3(512), 0, s, out, lse, a.part_o, a.part_lse,        \
-                         seq_lens, num_heads, head_groups, splits);                                                \
-    else                                                                                                           \
-      hipLaunchKernelGGL((mla_reduce_kernel<T, 4>), rgrid, dim3(512), 0, s, out, lse, a.part_o, a.part_lse,        \
-                         seq_lens, num_heads, head_groups, splits);                                                \
+  // more splits than one wave's trip: a few sequences, shared out over the waves and eight times the blocks (never in
+  // the batch-invariant mode, whose eight splits one trip holds: the choice must not depend on the batch)
+  const int min_split = head_groups == 1 ? kMlaSmallMinSplit : kMlaMinSplit;
+  dim3 rgrid(num_seqs, head_groups, splits > kMlaReduceTrip ? 8 : 1);
+#define KVQ_MLAR_N(T, N)                                                                                       \
+  hipLaunchKernelGGL((mla_reduce_kernel<T, N>), rgrid, dim3(512), 0, s, out, lse, a.part_o, a.part_lse, seq_lens, \
+                     num_heads, head_groups, splits)
+#define KVQ_MLAR(T)                                                                                            \
+  do {                                                                                                         \
+    if (splits > kMlaReduceTrip)                                                                               \
+      hipLaunchKernelGGL((mla_reduce_wide_kernel<T>), rgrid, dim3(512), 0, s, out, lse, a.part_o, a.part_lse,  \
+                         seq_lens, num_heads, head_groups, splits, min_split);                                 \
+    else if (splits > 4) KVQ_MLAR_N(T, 8);                                                                     \
+    else if (splits > 2) KVQ_MLAR_N(T, 4);                                                                     \
+    else KVQ_MLAR_N(T, 2);                                                                                     \
   } while (0)
   switch (out_dtype) {
     case KVQ_F32: KVQ_MLAR(KVQ_F32); break;
@@ -1601,6 +1661,7 @@ static int mla_decode_run(const char* op, void* out, int out_dtype, float* lse, 
     default: return fail(KVQ_EINVAL, "%s: unknown out_dtype %d", op, out_dtype);
   }
 #undef KVQ_MLAR
+#undef KVQ_MLAR_N
   return check_hip(hipGetLastError(), "mla_decode_int8 reduce launch");
 }
 
