@@ -19,7 +19,7 @@ int validate_common(const char* op, const void* q, const void* cache, const kvq_
                     const int32_t* block_table, const int32_t* seq_lens, int num_seqs, int num_q_heads);
 int launch_prefill(const AttnIO& io, const int32_t* seq_lens, const int32_t* cu_seqlens_q, int num_seqs,
                    int max_query_len, int causal, int q_dtype, int out_dtype, int32_t* plan, hipStream_t s,
-                   int ksplit, float* part);
+                   int ksplit, int num_tokens, float* part);
 
 // Where the context splits' partial states begin in a workspace, and how many bytes they take.
 static size_t split_part_offset(size_t streamk_bytes) { return (streamk_bytes + 255) & ~(size_t)255; }
@@ -186,7 +186,7 @@ static int paged_attn_launch(const char* op, void* out, int out_dtype, int64_t o
     int32_t* plan = reinterpret_cast<int32_t*>(a.seq_first_unit + num_seqs);
     // (the batch-invariant mode keeps one cut of the context whatever the caller proposes for this launch)
     rc = launch_prefill(a.io, seq_lens, cu_seqlens_q, num_seqs, max_query_len, causal, q_dtype, out_dtype, plan, s,
-                        batch_invariant() ? 1 : prefill_splits,
+                        batch_invariant() ? 1 : prefill_splits, num_tokens,
                         reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + part_at));
   }
   return rc;

@@ -40,9 +40,10 @@ __global__ __launch_bounds__(64) void prefill_plan_kernel(const int32_t* seq_len
 
 int launch_prefill(const AttnIO& io, const int32_t* seq_lens, const int32_t* cu_seqlens_q, int num_seqs,
                    int max_query_len, int causal, int q_dtype, int out_dtype, int32_t* plan, hipStream_t s,
-                   int ksplit, float* part) {
+                   int ksplit, int num_tokens, float* part) {
   PrefillArgs a{};
   a.ksplit = ksplit;
+  a.num_tokens = num_tokens;
   a.part = part;
   a.io = io;
   a.seq_lens = seq_lens;

@@ -34,6 +34,7 @@ struct PrefillArgs {
   // combines them: a launch with few items on a long context (a small prefill chunk of one long request) would
   // otherwise walk the whole context in a handful of workgroups, one tile after the other.
   int ksplit;
+  int num_tokens;   // rows of q, with ksplit > 1
   float* part;
   // Batch-invariant mode: which runs a kernel of this launch takes -- 0 all, 1 only those that fill the
   // workgroup-shared tile by themselves (q_len x group >= 64), 2 only the others.  Without the mode the batch's
@@ -749,8 +750,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     io.lse[row * io.num_q_heads + head] = l > 0.f ? (m + __builtin_amdgcn_logf(l)) * kLn2 : -INFINITY;
 }
 
-// The merge of the context splits: grid (query token of a run, sequence of the plan, ceil(Hq / 4)), a wave per (row, q
-// head), a lane D / 64 dims.  out = sum_s w_s o_s / sum_s w_s l_s with w_s = 2^(m_s - max m): the algebra of
+// The merge of the context splits: grid (query rows, ceil(Hq / 4)), a wave per (row of a run, q head), a lane D / 64 dims.
+// The rows are counted over the plan's runs, a handful where a launch is split (over every sequence of a mixed batch,
+// most of the blocks would find a decode row: 153 us of 330 beside 91 of them).  out = sum_s w_s o_s / sum_s w_s l_s with w_s = 2^(m_s - max m): the algebra of
 // merge_attn_states over the splits' states; the sink's term and the row's lse as in the unsplit kernel.
 // A stream of the states, 520 bytes per split at D = 128: every load of a row leaves before the first is used (splits past
 // the last reread it and weigh 0).  One block per row whose four waves went through the heads, and a head's splits, one
@@ -760,15 +762,21 @@ __global__ __launch_bounds__(256) void prefill_split_merge_kernel(PrefillArgs a)
   constexpr int V = D / 64;
   typedef float vec_t __attribute__((ext_vector_type(V), aligned(4 * V)));
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (blockIdx.y >= (unsigned)a.plan[0]) return;
-  const int seq = a.plan[1 + blockIdx.y];
-  const int q_begin = a.cu_seqlens_q[seq];
-  const int q_len = a.cu_seqlens_q[seq + 1] - q_begin;
-  const int qi = blockIdx.x;
-  const int head = blockIdx.z * 4 + wave;
+  const int head = blockIdx.y * 4 + wave;
   const AttnIO& io = a.io;
-  if (q_len <= 1 || qi >= q_len || a.seq_lens[seq] <= 0 || head >= io.num_q_heads) return;
-  const int64_t row = q_begin + qi;
+  if (head >= io.num_q_heads) return;
+  int qi = blockIdx.x;
+  int64_t row = -1;
+  for (int i = 0; i < a.plan[0]; ++i) {   // uniform: scalar loads
+    const int seq = a.plan[1 + i];
+    const int q_begin = a.cu_seqlens_q[seq], q_len = a.cu_seqlens_q[seq + 1] - q_begin;
+    if (qi < q_len) {
+      row = q_begin + qi;
+      break;
+    }
+    qi -= q_len;
+  }
+  if (row < 0) return;
   const int S = a.ksplit;
   const float* p = a.part + ((row * io.num_q_heads + head) * S) * (D + 2);
   const int mine = min(lane, S - 1);   // lane s takes split s's (m, l)
@@ -814,7 +822,7 @@ static int launch_prefill_flash32(PrefillArgs& a, int max_query_len, hipStream_t
       dim3 grid(blocks * a.ksplit, a.num_seqs, a.io.g.num_kv_heads);
       hipLaunchKernelGGL((paged_prefill_flash32_kernel<D, QDT, ODT, true, CODE, true>), grid, dim3(256), FP::LDS_BYTES, s, a);
       if (int e = check_hip(hipGetLastError(), "paged_prefill_flash32 launch")) return e;
-      dim3 mgrid(max_query_len, a.num_seqs, (a.io.num_q_heads + 3) / 4);
+      dim3 mgrid(a.num_tokens, (a.io.num_q_heads + 3) / 4);
       hipLaunchKernelGGL((prefill_split_merge_kernel<D, ODT>), mgrid, dim3(256), 0, s, a);
       return check_hip(hipGetLastError(), "prefill split merge launch");
     }
