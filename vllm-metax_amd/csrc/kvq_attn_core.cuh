@@ -370,45 +370,56 @@ struct DecodeTile {
   // head 0 and are zeroed.  Returns -1152 * sum(q) of the lane's head: the QK accumulator's
   // start value that cancels the code bias.
   __device__ static float load_q(const AttnIO& io, int64_t row, int hkv, int lane, half8_t (&qb)[KSTEPS]) {
-    const int c = lane & 15;
-    const bool valid = c < io.group;
-    return load_q_row(io, row * io.q_stride_t + (int64_t)(hkv * io.group + (valid ? c : 0)) * io.q_stride_h, valid,
-                      lane, qb);
+    return load_q_row(io, q_elem(io, row, hkv, lane), (lane & 15) < io.group, lane, qb);
   }
 
   // The same for an arbitrary (row, head) per lane: `elem` is the element offset of the lane's
   // query row (it must be readable also when !valid; the operand is then zero).
   __device__ static float load_q_row(const AttnIO& io, int64_t elem, bool valid, int lane, half8_t (&qb)[KSTEPS]) {
+    QRaw raw;
+    load_q_raw(io, elem, lane, raw);
+    return convert_q(raw, valid, lane, qb);
+  }
+  // ... in two steps, the loads and what follows from them.
+  struct QRaw {
+    u32x4 v[D / 64][QDT == KVQ_F32 ? 4 : 2];   // 16 elements per K chunk
+  };
+  __device__ static int64_t q_elem(const AttnIO& io, int64_t row, int hkv, int lane) {
+    const int c = lane & 15;
+    return row * io.q_stride_t + (int64_t)(hkv * io.group + (c < io.group ? c : 0)) * io.q_stride_h;
+  }
+  __device__ static void load_q_raw(const AttnIO& io, int64_t elem, int lane, QRaw& raw) {
     const int g = lane >> 4;
     // int8 / fp8: the 16 dims of the lane's K chunk `ch`; int4: a K chunk holds 32 dims, two runs of 16
     const int64_t base = elem + (INT4 ? 2 : 1) * k_off(g, 0);
-    auto run_step = [](int ch) { return INT4 ? 2 * k_step(ch >> 1) + 16 * (ch & 1) : k_step(ch); };
+    constexpr int ESZ = QDT == KVQ_F32 ? 4 : 2;
+#pragma unroll
+    for (int ch = 0; ch < D / 64; ++ch) {
+      const int step = INT4 ? 2 * k_step(ch >> 1) + 16 * (ch & 1) : k_step(ch);
+      const uint8_t* p = reinterpret_cast<const uint8_t*>(io.q) + (base + step) * ESZ;
+#pragma unroll
+      for (int i = 0; i < ESZ; ++i) raw.v[ch][i] = *reinterpret_cast<const u32x4_a4*>(p + 16 * i);
+    }
+  }
+  __device__ static float convert_q(const QRaw& raw, bool valid, int lane, half8_t (&qb)[KSTEPS]) {
     float f[D / 4];
 #pragma unroll
     for (int ch = 0; ch < D / 64; ++ch) {
-      if constexpr (QDT == KVQ_F32) {
-        const float* p = reinterpret_cast<const float*>(io.q) + base + run_step(ch);
 #pragma unroll
-        for (int i = 0; i < 16; i += 4) {
-          const floatx4 v = *reinterpret_cast<const floatx4_a4*>(p + i);
-          f[ch * 16 + i] = v.x; f[ch * 16 + i + 1] = v.y; f[ch * 16 + i + 2] = v.z; f[ch * 16 + i + 3] = v.w;
-        }
-      } else {
-        const uint16_t* p = reinterpret_cast<const uint16_t*>(io.q) + base + run_step(ch);
+      for (int i = 0; i < (QDT == KVQ_F32 ? 4 : 2); ++i) {
+        const u32x4 v = raw.v[ch][i];
 #pragma unroll
-        for (int i = 0; i < 16; i += 8) {
-          const u32x4 v = *reinterpret_cast<const u32x4_a4*>(p + i);
-#pragma unroll
-          for (int w = 0; w < 4; ++w) {
-            if constexpr (QDT == KVQ_BF16) {
-              f[ch * 16 + i + 2 * w] = as_f32(v[w] << 16);
-              f[ch * 16 + i + 2 * w + 1] = as_f32(v[w] & 0xffff0000u);
-            } else {
-              const uint32_t e = v[w];  // copy the element out first: bit_cast must not see a vector element lvalue
-              const half2_t h = __builtin_bit_cast(half2_t, e);
-              f[ch * 16 + i + 2 * w] = (float)h.x;
-              f[ch * 16 + i + 2 * w + 1] = (float)h.y;
-            }
+        for (int w = 0; w < 4; ++w) {
+          const uint32_t e = v[w];  // copy the element out first: bit_cast must not see a vector element lvalue
+          if constexpr (QDT == KVQ_F32) {
+            f[ch * 16 + 4 * i + w] = as_f32(e);
+          } else if constexpr (QDT == KVQ_BF16) {
+            f[ch * 16 + 8 * i + 2 * w] = as_f32(e << 16);
+            f[ch * 16 + 8 * i + 2 * w + 1] = as_f32(e & 0xffff0000u);
+          } else {
+            const half2_t h = __builtin_bit_cast(half2_t, e);
+            f[ch * 16 + 8 * i + 2 * w] = (float)h.x;
+            f[ch * 16 + 8 * i + 2 * w + 1] = (float)h.y;
           }
         }
       }
@@ -807,9 +818,9 @@ struct DecodeTile {
     st.l = 0.f;
   }
   template <bool CAP, bool SPANS = false>
-  __device__ static void run(const AttnIO& io, int seq, int64_t row, int len, int first, int t_begin, int t_end, int hkv,
-                             int lane, uint8_t* lds, State& st, int sub = 0, int nsub = 1, SpanEdges* sp = nullptr) {
-    const LaneOffsets lo = lane_offsets(io.g, lane);
+  __device__ static void run(const AttnIO& io, const LaneOffsets& lo, int seq, int64_t row, int len, int first, int t_begin,
+                             int t_end, int hkv, int lane, uint8_t* lds, State& st, int sub = 0, int nsub = 1,
+                             SpanEdges* sp = nullptr) {
     const int32_t* bt_row = io.block_table + (int64_t)seq * io.bt_stride;
     const int rounds = (t_end - t_begin + nsub - 1) / nsub;
     const int num_barriers = STREAM ? 0 : rounds / kSyncTiles;
@@ -827,14 +838,17 @@ struct DecodeTile {
     };
     int t = t_begin + sub;
     if (t < t_end) {
+      // the query's loads, then the first tile's: the arithmetic on the query runs while the tile is on its way
+      QRaw qraw;
+      load_q_raw(io, q_elem(io, row, hkv, lane), lane, qraw);
+      phase_fence();
       Tile a;
-      // the first tile's loads go out before anything else of the run is touched
       TileBlocks nb = fetch_blocks(io, bt_row, len, t);
       load_tile(io, window(io, nb, t, hkv), lo, a);
       phase_fence();
       nb = fetch_blocks(io, bt_row, len, t + nsub);  // block ids run one tile ahead of the loads
       half8_t qb[KSTEPS];
-      const float s_init = load_q(io, row, hkv, lane, qb);
+      const float s_init = convert_q(qraw, (lane & 15) < io.group, lane, qb);
       const float sc_mul = lane < 32 ? io.scale_log2 * kKScaleMul : kPScale;
       float ali = 0.f;
       if constexpr (CAP) ali = alibi_slope(io.alibi, hkv * io.group + min(lane & 15, io.group - 1));

@@ -25,6 +25,22 @@ __device__ __forceinline__ int decode_tiles(const int32_t* seq_lens, const int32
   return (s < num_seqs && q_len == 1 && len > 0) ? n : 0;
 }
 
+// A sequence's length and its query rows [q0, q1).
+struct SeqRow {
+  int len, q0, q1;
+};
+__device__ __forceinline__ SeqRow load_seq(const StreamKArgs& a, int s) {
+  SeqRow r;
+  r.len = a.seq_lens[s];
+  r.q0 = a.cu_seqlens_q != nullptr ? a.cu_seqlens_q[s] : s;
+  r.q1 = a.cu_seqlens_q != nullptr ? a.cu_seqlens_q[s + 1] : s + 1;
+  return r;
+}
+// Its tiles as a decode sequence (see decode_tiles).
+__device__ __forceinline__ int seq_tiles(const SeqRow& r, int window) {
+  return r.q1 - r.q0 == 1 && r.len > 0 ? (r.len + kTile - 1) / kTile - window_first(r.len, window) / kTile : 0;
+}
+
 // Batch-invariant cutting (StreamKArgs::fixed_spans): a sequence is cut at places that depend on nothing but its
 // own length -- into at most kFixedSpans spans of equal size, none shorter than kMinSpanTiles tiles.  The spans of
 // all decode sequences form one line (a unit per span) that is cut into equal shares like the balanced line, so
@@ -56,9 +72,15 @@ __device__ __forceinline__ int line_units(const int32_t* seq_lens, const int32_t
   else return decode_units(seq_lens, cu, s, num_seqs, window, setup);
 }
 
-// The scans over the sequences work on chunks of 64 (one per lane).  Large batches take kScanBatch
-// chunks per step so that their loads are in flight together (batch 512: 16 dependent round trips
-// -> 4); a batch that fits one chunk keeps the single-chunk loop, which measured 3 us faster there.
+template <bool FIXED>
+__device__ __forceinline__ int seq_line_units(const SeqRow& r, int window, int setup) {
+  const int n = seq_tiles(r, window);
+  if constexpr (FIXED) return fixed_span_count(n);
+  else return n > 0 ? n + setup : 0;
+}
+
+// The scans over more than 64 sequences work on chunks of 64 (one per lane), kScanBatch chunks per step so that their
+// loads are in flight together (batch 512: 16 dependent round trips -> 4).
 constexpr int kScanBatch = 4;
 
 // Total units of the work line.
@@ -130,13 +152,25 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
 
   constexpr bool fixed = FIXED;
 
+  const LaneOffsets off = DTile::lane_offsets(a.io.g, lane);   // (while the lengths are on their way)
+
   // the balanced cutting: total units of the work line (each wave redoes this tiny scan; no LDS, no barrier)
   const bool one_chunk = B <= kWave;
   int64_t total = 0, lo = 0, hi = 0;
   int seq = 0;
   int64_t seq_start = 0;  // global index of the sequence's first unit
+  SeqRow cur{};           // the sequence's length and row
   {
-    total = one_chunk ? scan_total<1, fixed>(a, lane) : scan_total<kScanBatch, fixed>(a, lane);
+    SeqRow mine{};
+    int n = 0, incl = 0;
+    if (one_chunk) {   // a sequence per lane: one trip to memory for the whole line
+      mine = load_seq(a, min(lane, B - 1));
+      n = lane < B ? seq_line_units<fixed>(mine, a.io.window, a.setup_units) : 0;
+      incl = wave_incl_scan(n);
+      total = __builtin_amdgcn_readlane(incl, 63);
+    } else {
+      total = scan_total<kScanBatch, fixed>(a, lane);
+    }
     // (the batch-invariant line is short -- a unit is a span of at least kMinSpanTiles tiles -- and is always shared
     // out over every workgroup there is a unit for)
     const int num_wg = fixed ? (total < a.num_wg ? (total < 1 ? 1 : (int)total) : a.num_wg) : active_workgroups(total, a.num_wg);
@@ -147,10 +181,17 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
       if (!fixed && w == 0 && blockIdx.y == 0 && wave == 0 && lane == 0) a.wg_info[0] = total;
       return;
     }
-    // locate the sequence holding unit `lo`
-    if (one_chunk) scan_locate<1, fixed>(a, lane, lo, seq, seq_start);
-    else scan_locate<kScanBatch, fixed>(a, lane, lo, seq, seq_start);
-    seq = __builtin_amdgcn_readfirstlane(seq);
+    // the sequence that holds unit `lo`
+    if (one_chunk) {
+      const uint64_t hit = __builtin_amdgcn_ballot_w64(n > 0 && incl - n <= lo && lo < incl);
+      seq = __builtin_ctzll(hit);   // (lo < total: there is one)
+      seq_start = __builtin_amdgcn_readlane(incl - n, seq);
+      cur = {__builtin_amdgcn_readlane(mine.len, seq), __builtin_amdgcn_readlane(mine.q0, seq), __builtin_amdgcn_readlane(mine.q1, seq)};
+    } else {
+      scan_locate<kScanBatch, fixed>(a, lane, lo, seq, seq_start);
+      seq = __builtin_amdgcn_readfirstlane(seq);
+      cur = load_seq(a, seq);
+    }
   }
   // Where the share begins (the reduce kernel's key to the span): noted in the first round of the loop, stored
   // after the last.  A store ahead of the tile loads would sit before them in the wave's in-order memory
@@ -170,7 +211,7 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
       if constexpr (NSUB > 1) lds_barrier();
     }
     typename DTile::State st;
-    DTile::template run<CAP>(a.io, cur, row, len, first, t_begin, t_end, hkv, lane, lds[wave], st, sub, NSUB);
+    DTile::template run<CAP>(a.io, off, cur, row, len, first, t_begin, t_end, hkv, lane, lds[wave], st, sub, NSUB);
     // the run holds the sequence's first tile: its place on the line, for the reduce kernel (behind the run's loads)
     if (!fixed && t_begin == t0 && blockIdx.y == 0 && wave == 0 && lane == 0) a.seq_first_unit[cur] = cur_start;
     if constexpr (NSUB > 1) {
@@ -205,7 +246,8 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
     }
     typename DTile::State st;
     typename DTile::SpanEdges sp{a.part_o, a.part_ml, (int64_t)cur * kFixedSpans + span, per, per};
-    DTile::template run<CAP, true>(a.io, cur, row, len, first, t_begin, t_end, hkv, lane, lds[wave], st, 0, 1, &sp);
+    DTile::template run<CAP, true>(a.io, off, cur, row, len, first, t_begin, t_end, hkv, lane, lds[wave], st, 0, 1,
+                                   &sp);
     DTile::emit_partial(a.io, a.part_o, a.part_ml, sp.slot, hkv, lane, st);
   };
 
@@ -243,17 +285,18 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
     return;
   }
 
+  const int setup = a.setup_units;
   int64_t pos = lo;
-  while (pos < hi && seq < B) {
-    const int units = __builtin_amdgcn_readfirstlane(decode_units(a.seq_lens, a.cu_seqlens_q, seq, B, a.io.window, a.setup_units));
-    if (units == 0) {
-      ++seq;
+  for (; pos < hi && seq < B; ++seq) {
+    const SeqRow nxt = load_seq(a, min(seq + 1, B - 1));   // on its way while this sequence's run is computed
+    const int ntiles = seq_tiles(cur, a.io.window);
+    if (ntiles == 0) {
+      cur = nxt;
       continue;
     }
-    const int setup = a.setup_units;
-    const int ntiles = units - setup;
-    const int len = __builtin_amdgcn_readfirstlane(a.seq_lens[seq]);
-    const int64_t row = a.cu_seqlens_q ? (int64_t)a.cu_seqlens_q[seq] : (int64_t)seq;
+    const int units = ntiles + setup;
+    const int len = cur.len;
+    const int64_t row = cur.q0;
     if (info_seq < 0) {
       info_seq = seq;
       info_start = seq_start;
@@ -265,13 +308,14 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
     const int u_begin = (int)(pos - seq_start);
     const int64_t rem = hi - seq_start;
     const int u_end = rem < units ? (int)rem : units;
-    const int t_begin = __builtin_amdgcn_readfirstlane(t0 + (u_begin > setup ? u_begin - setup : 0));
-    const int t_end = __builtin_amdgcn_readfirstlane(t0 + u_end - setup);
-    if (t_begin < t_end)  // else: this share ends inside the setup charge and holds no tile
-      process(seq, seq_start, row, len, first, t0, ntiles, t_begin, t_end, (int64_t)w + seq);
+    const int t_begin = t0 + (u_begin > setup ? u_begin - setup : 0);
+    const int t_end = t0 + u_end - setup;
+    const int64_t start = seq_start;
     pos = seq_start + u_end;
     seq_start += units;
-    ++seq;
+    if (t_begin < t_end)  // else: this share ends inside the setup charge and holds no tile
+      process(seq, start, row, len, first, t0, ntiles, t_begin, t_end, (int64_t)w + seq);
+    cur = nxt;
   }
   if (blockIdx.y == 0 && wave == 0 && lane == 0) {   // this lane leaves the reduce kernel its notes
     if (w == 0) a.wg_info[0] = total;
@@ -805,7 +849,7 @@ __global__ __launch_bounds__(WPW * 64) void paged_decode_v2_kernel(V2Args a) {
   if (t_begin >= ntiles) return;
   const int t_end = min(ntiles, t_begin + a.partition_tiles);
   typename DTile::State st;
-  DTile::template run<BIAS>(a.io, seq, seq, len, 0, t_begin, t_end, hkv, lane, lds[wave], st);
+  DTile::template run<BIAS>(a.io, DTile::lane_offsets(a.io.g, lane), seq, seq, len, 0, t_begin, t_end, hkv, lane, lds[wave], st);
   DTile::emit_v2(a.io, a.tmp_out, a.max_logits, a.exp_sums, seq, part, a.max_parts, hkv, lane, st);
 }
 
