@@ -196,3 +196,36 @@ def test_backend_serves_fp8_per_token_head(gpu_device):
     want = oracle.paged_attn(q.view(B, hq, d), T.storage_bytes(kv_cpu), lay, bt, torch.tensor(ctx, dtype=torch.int32),
                              torch.arange(B + 1, dtype=torch.int32), 1 / math.sqrt(d), code_type=oracle.CODE_FP8)
     T.assert_close_attn(out.view(B, hq, d), want, what="backend fp8")
+
+
+@pytest.mark.parametrize("hq,hkv,d,layout,qls,splits", [
+    (8, 8, 128, "NHD", [3, 2, 5, 1], 1),       # the per-wave tile
+    (4, 2, 256, "HND", [20, 2, 30, 1], 1),     # the same at the head size that has no other
+    (32, 8, 128, "HND", [3, 2, 5, 1] * 20, 1),  # one launch over the batch's tiles, several of them a share
+    (16, 8, 64, "HND", [3, 2, 5, 1] * 20, 1),
+    (32, 8, 128, "HND", [20, 2, 70, 1], 1),    # the workgroup-shared tile: 80 of its 128 columns, then 128 + 128 + 24
+    (32, 8, 128, "NHD", [20, 2, 70, 1], 2),    # ... in two context splits
+])
+def test_blocks_below_the_window_may_hold_anything(gpu_device, hq, hkv, d, layout, qls, splits):
+    """An engine gives back the blocks that lie wholly below a sequence's window and points their table entries at
+    the null block.  The 32-token tile at the window's lower edge still covers some of their slots: whatever bytes
+    they hold (here the e4m3fn NaN) must not reach a row."""
+    window = 500
+    # the window of the first new token begins 7, 17, 23 or 31 tokens into a 32-token tile
+    ctx = [32 * (9 + i % 7) + edge + window - 1 + n for i, (edge, n) in enumerate(zip([17, 23, 31, 7] * 20, qls))]
+    kv, lay, bt, q, sl, cu = _fp8_case(ctx, qls, hq, hkv, d, 16, seed=hq + d, layout=layout)
+    for i, n in enumerate(qls):
+        bt[i, :(ctx[i] - n + 1 - window) // 16] = 0     # the null block, 0xFF throughout
+    scale = 1 / math.sqrt(d)
+    want = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, scale, sliding_window=window,
+                             code_type=oracle.CODE_FP8)
+    dev = gpu_device
+    kvd = T.to_device_cache(kv, dev, layout)
+    k, v = L.key_value_views(kvd)
+    ks, vs = L.scale_views(kvd)
+    out = torch.full(q.shape, float("nan"), dtype=torch.bfloat16, device=dev)
+    ops.unified_attention(q.to(dev), k, v, out, cu.to(dev), max(qls), sl.to(dev), int(sl.max()), scale, True,
+                          window_size=(window - 1, 0), block_table=bt.to(dev), k_scale_cache=ks, v_scale_cache=vs,
+                          kv_quant_mode=FP8, prefill_splits=splits)
+    torch.cuda.synchronize()
+    T.assert_close_attn(out, want, what=f"null block below the window {hq}/{hkv} d{d} {layout}")

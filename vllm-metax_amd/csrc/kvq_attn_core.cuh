@@ -50,8 +50,8 @@ __device__ __forceinline__ uint32_t bytes_to_half2(uint32_t x, bool upper) {
 // Two e4m3fn code bytes of x -> two fp16 values code / 2^8, exact for every code, subnormal ones included; the 2^8 is
 // put back with the scales.  One conversion instruction, as cheap as the int8 path's byte permute (2.5 ns against
 // 7.6 ns for the same result from shifts and masks, two waves on a SIMD).  It turns the code 0x7f / 0xff, which the
-// writer never stores, into a NaN: GARBAGE = the bytes may be anything (a slot past the end of a sequence), and a NaN
-// must not come out, since 0 x NaN would reach the output.  There the byte's 7 magnitude bits are put at bits 7 .. 13
+// writer never stores, into a NaN: GARBAGE = the bytes may be anything (a slot past the end of a sequence, or below its
+// window in a block that was given back), and a NaN must not come out, since 0 x NaN would reach the output.  There the byte's 7 magnitude bits are put at bits 7 .. 13
 // of an fp16 pattern and the sign at bit 15, which is the same number (the exponent biases differ by 15 - 7).
 template <bool GARBAGE = false>
 __device__ __forceinline__ uint32_t fp8_bytes_to_half2(uint32_t x, bool upper) {
@@ -722,7 +722,7 @@ struct DecodeTile {
   // Phase 2 of a tile: O^T += (V + 1152)^T . P~^T.  Lane (r, g) reads its VB code bytes of
   // its eight tokens from the LDS window, transposes the 8 x VB byte block in
   // registers (byte permutes), one MFMA per 16-dim tile; sum(P~) comes from a row of ones.
-  // MASK: the tile may hold slots past the end of the sequence, whose bytes may be anything.
+  // MASK: the tile may hold slots past the end of the sequence or below its window, whose bytes may be anything.
   template <bool MASK>
   __device__ static void pv(const LaneOffsets& lo, half8_t p_op, const uint8_t* lds, State& st) {
     if constexpr (!FP8) {  // fp8 codes carry no bias to take out again

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(WPW * 64) void paged_prefill_kernel(PrefillArgs a) 
         PT::template qk_softmax<false>(io, lo, qb, s_init, limit, wspan, t, lane, lds, st, p_op, ali);
       else
         PT::template qk_softmax<true>(io, lo, qb, s_init, limit, wspan, t, lane, lds, st, p_op, ali);
-      PT::template pv<false>(lo, p_op, lds, st);   // not the item's last tile: every slot holds a token
+      PT::pv_any(t * kTile < max_first, lo, p_op, lds, st);   // not the item's last tile
       DTile::phase_fence();
       t += STEP;
     }
@@ -329,7 +329,7 @@ struct Flash32 {
   // Raw tile -> fp16 K [token][dim] (codes + 1152) and V^T [dim][position] (codes); token t of the tile sits at position
   // (t/16)*16 + ((t%8)/4)*8 + ((t/8)%2)*4 + t%4, the order in which the 32x32 S accumulator hands a
   // lane its tokens.  One thread converts one 16-code K chunk and one 4-token x 4-dim V block.  GARBAGE: the tile may
-  // hold slots past the end of the sequence.
+  // hold slots past the end of the sequence or below the window.
   template <bool GARBAGE>
   __device__ static __forceinline__ void expand(const uint8_t* raw, uint8_t* buf, int tid, float sc_mul, uint32_t l_sc) {
     constexpr int KCH = D / 16;
@@ -583,12 +583,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   // pair that holds the first query token's lower edge; a wave masks tiles below the latest lower
   // edge among its columns and skips those that end before the earliest.
   uint32_t wspan = 0x7fffffffu;
-  int t_first = 0, wave_min_first = 0, wave_max_first = 0;
+  int t_first = 0, wg_first = 0, wave_min_first = 0, wave_max_first = 0;
   if constexpr (EXT) {
     if (io.window > 0) {
       wspan = (uint32_t)io.window;
-      int wg_first = (a.causal ? ctx + q0 + 1 : len) - io.window;
-      wg_first = wg_first < 0 ? 0 : wg_first;
+      wg_first = max(0, (a.causal ? ctx + q0 + 1 : len) - io.window);
       t_first = (wg_first / kTile) & ~1;
       wave_min_first = max(0, wave_min_limit - io.window);
       wave_max_first = max(0, wave_max_limit - io.window);
@@ -681,8 +680,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // (also for a wave without a valid column: its share of the expansion must expect slots past the sequence's end)
     const int t_plain = min(t_hi, min(wave_min_limit, len) / kTile) & ~1;
     int t = t_lo;
-    if constexpr (EXT) {  // tiles that straddle a column's lower window edge
-      const int t_head = min(t_hi, ((wave_max_first + kTile - 1) / kTile + 1) & ~1);
+    if constexpr (EXT) {
+      // Tiles that straddle a column's lower window edge, and those that hold a slot below every column's (wg_first: also
+      // for a wave without a valid column, which expands its share of them like any other): the blocks there may have
+      // been given back and hold anything.
+      const int t_head = min(t_hi, ((max(wave_max_first, wg_first) + kTile - 1) / kTile + 1) & ~1);
       for (; t < t_head; t += 2) {
         step_fn(std::true_type{}, t, B);
         step_fn(std::true_type{}, t + 1, A);

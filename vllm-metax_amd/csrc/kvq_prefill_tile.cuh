@@ -135,6 +135,14 @@ struct PrefillTile {
     }
   }
 
+  // pv() of a tile whose slots do not all hold a token of the window when `garbage` (uniform): those past the sequence's
+  // end, and those below the window, whose block the engine may have given back.  Only fp8 bytes need the distinction.
+  __device__ __forceinline__ static void pv_any(bool garbage, const LaneOffsets& lo, const half8_t (&p_op)[NT],
+                                                const uint8_t* lds, State& st) {
+    if (FP8 && garbage) pv<true>(lo, p_op, lds, st);
+    else pv<false>(lo, p_op, lds, st);
+  }
+
   // O^T += (V + 1152)^T . P~^T: every converted V operand feeds the NT column tiles.  MASK as in DecodeTile::pv.
   template <bool MASK>
   __device__ __forceinline__ static void pv(const LaneOffsets& lo, const half8_t (&p_op)[NT], const uint8_t* lds, State& st) {

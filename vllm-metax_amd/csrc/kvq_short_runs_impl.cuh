@@ -195,7 +195,7 @@ __global__ __launch_bounds__(512) void short_runs_streamk_kernel(ShortRunArgs a)
         wait_loads<DTile::kDmaLoads>();   // all but those just issued: tile t is there
         DTile::stage_scales(off, sc_mul, lane, cur);
         softmax();
-        PT::template pv<false>(off, p_op, cur, st);   // not the sequence's last tile: every slot holds a token
+        PT::pv_any(t * kTile < max_first, off, p_op, cur, st);   // not the sequence's last tile
         DTile::phase_fence();
         uint8_t* done = cur;
         cur = next;
