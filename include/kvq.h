@@ -362,8 +362,8 @@ KVQ_API int kvq_splitk_reduce(void* out, int out_dtype, float* lse, const float*
  * kvq_mla_geom: block_bytes = stride_block) holds codes and scales together, so
  * the move is self-contained.  Asynchronous on `stream`; host memory should be
  * pinned: memory the GPU can address is read or written by a kernel, other memory takes a
- * copy call per block.  The moves of a call are unordered among themselves: each destination block is
- * named once, and pairs must not overlap when src and dst are the same allocation.
+ * copy call per block.  A destination block that is named more than once ends up with the last pair's
+ * bytes.  When src and dst are the same allocation, no block may be both a source and a destination.
  */
 KVQ_API int kvq_swap_blocks(const void* src, void* dst, int64_t block_bytes,
                     const int64_t* block_mapping, int64_t num_pairs, int64_t map_stride0,

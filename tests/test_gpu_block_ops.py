@@ -76,6 +76,30 @@ def test_swap_blocks_with_pinned_memory(gpu_device, bs, hkv, d, n, to_host):
     assert torch.equal(as_blocks(dst).cpu(), want)
 
 
+@pytest.mark.parametrize("direction", ["out", "in", "on the GPU"])
+@pytest.mark.parametrize("n,distinct", [(2, 1), (480, 479), (481, 480), (700, 90)])
+def test_swap_blocks_last_of_several_pairs_with_one_destination_wins(gpu_device, direction, n, distinct):
+    """Destinations named several times, inside one launch's 480 pairs and across two launches, in either direction:
+    the bytes are those of the moves made one after the other."""
+    nb = n + 5
+    g = torch.Generator().manual_seed(n)
+    gpu = L.allocate_kv_cache(nb, 16, 8, 128, device=gpu_device, fill=None)    # blocks of three slices
+    other = torch.empty((nb,) + tuple(gpu.shape[1:]), dtype=torch.int8, pin_memory=True)
+    if direction == "on the GPU":
+        other = other.to(gpu_device)
+    for t in (gpu, other):
+        as_blocks(t).copy_(torch.randint(0, 256, as_blocks(t).shape, generator=g, dtype=torch.uint8))
+    src, dst = (other, gpu) if direction == "in" else (gpu, other)
+    dsts = torch.randperm(nb, generator=g)[:distinct]
+    mapping = torch.stack([torch.randperm(nb, generator=g)[:n], dsts[torch.arange(n) % distinct]], 1)
+    want, s = as_blocks(dst).cpu().clone(), as_blocks(src).cpu()
+    for a, b in mapping.tolist():
+        want[b] = s[a]
+    ops.swap_blocks(src, dst, block_bytes(src), mapping)
+    torch.cuda.synchronize()
+    assert torch.equal(as_blocks(dst).cpu(), want)
+
+
 def test_swap_blocks_same_tensor_and_strided_mapping(gpu_device):
     """Copy inside one allocation (non-overlapping pairs), mapping given as a strided view."""
     nb = 64

@@ -6,6 +6,8 @@
 // (the pairs travel in the kernel arguments, 16-byte lane copies, a workgroup per 16 KB slice of a block).  Host
 // memory that the GPU cannot address takes one asynchronous copy call per block on the caller's stream, as in
 // the reference (csrc/libtorch_stable/cache_kernels.cu:33-77).
+#include <cstring>
+
 #include "kvq_internal.h"
 
 namespace kvq {
@@ -21,6 +23,31 @@ constexpr int kHostCopyGroups = 64;
 struct BlockPairs {
   int32_t src[kPairsPerLaunch];
   int32_t dst[kPairsPerLaunch];
+};
+
+// The pairs of one launch, each destination once: a launch's workgroups run in any order, and of several pairs that name
+// one destination the last has to win, as it does when the moves run one after the other.  Destinations are kept in an
+// open-addressed table (2.2 - 3.2 ns a pair on the host; launches of a call follow each other, so pairs of different launches need none).
+class PairTable {
+ public:
+  PairTable() { memset(slot_, 0xff, sizeof(slot_)); }
+  bool full() const { return n_ == kPairsPerLaunch; }
+  int size() const { return n_; }
+  void add(BlockPairs& p, int32_t src, int32_t dst) {
+    uint32_t h = ((uint32_t)dst * 2654435761u) >> (32 - kBits);
+    while (slot_[h] >= 0 && p.dst[slot_[h]] != dst) h = (h + 1) & ((1u << kBits) - 1);
+    if (slot_[h] < 0) {
+      slot_[h] = (int16_t)n_;
+      p.dst[n_++] = dst;
+    }
+    p.src[slot_[h]] = src;
+  }
+
+ private:
+  static constexpr int kBits = 10;
+  static_assert((1 << kBits) > 2 * kPairsPerLaunch, "the table is at most half full");
+  int16_t slot_[1 << kBits];
+  int n_ = 0;
 };
 
 // A workgroup takes the slices blockIdx.x, blockIdx.x + gridDim.x, ... of the launch's blocks (`slices` each); 256
@@ -155,13 +182,12 @@ int kvq_swap_blocks(const void* src, void* dst, int64_t block_bytes, const int64
     by_kernel = host_range_is_mapped(host + lo[side] * block_bytes, host + (hi[side] + 1) * block_bytes - 1);
   }
   if (by_kernel) {
-    for (int64_t base = 0; base < num_pairs; base += kPairsPerLaunch) {
+    for (int64_t at = 0; at < num_pairs;) {
       BlockPairs p;
-      const int n = (int)(num_pairs - base < kPairsPerLaunch ? num_pairs - base : kPairsPerLaunch);
-      for (int i = 0; i < n; ++i) {
-        p.src[i] = (int32_t)block_mapping[(base + i) * map_stride0];
-        p.dst[i] = (int32_t)block_mapping[(base + i) * map_stride0 + map_stride1];
-      }
+      PairTable table;
+      for (; at < num_pairs && !table.full(); ++at)
+        table.add(p, (int32_t)block_mapping[at * map_stride0], (int32_t)block_mapping[at * map_stride0 + map_stride1]);
+      const int n = table.size();
       for (int i = n; i < kPairsPerLaunch; ++i) p.src[i] = p.dst[i] = 0;
       const int items = n * (int)slices;
       const int groups = direction == KVQ_DEVICE_TO_DEVICE || items < kHostCopyGroups ? items : kHostCopyGroups;

@@ -521,7 +521,9 @@ def swap_blocks(src: torch.Tensor, dst: torch.Tensor, block_size_in_bytes: int, 
     ``block_mapping[i, 1]`` = src block ``block_mapping[i, 0]``.  ``block_mapping`` is a CPU int64
     ``[n, 2]`` tensor (the reference refuses a GPU one, cache_kernels.cu:51-55); src / dst are cache
     tensors of the int8 layouts (GQA or MLA) on the GPU or in (pinned) host memory, at least one of
-    them on the GPU, both on the same GPU if both are.  Asynchronous on the current stream."""
+    them on the GPU, both on the same GPU if both are.  Of several rows with one destination the last
+    wins; within one allocation no block may be both a source and a destination.  Asynchronous on the
+    current stream."""
     if block_mapping.is_cuda:
         raise RuntimeError("block_mapping must be on CPU")
     if block_mapping.dtype != torch.int64 or block_mapping.dim() != 2 or block_mapping.shape[1] != 2:
