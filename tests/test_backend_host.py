@@ -358,3 +358,23 @@ def test_context_split_proposal_follows_the_launch_shape():
     assert f([2048], 131072, 32, 8, max_split_tokens=4096) == 1
     assert f([1024], 131072, 32, 8, max_split_tokens=4096) == 2    # 256 workgroups: two ranges fill the chip's 512 places
     assert f(torch.tensor([300, 1, 1]), 8192, 28, 4) == 4          # the context allows one split per 2048 tokens
+
+
+def test_native_op_layer_refuses_tensors_without_storage():
+    """A wrapper tensor passes the shape and device checks and has no data pointer (here vmap's, over tensors that only
+    claim to be on a GPU): that is an ordinary error, raised before the call gives up the interpreter's lock or looks for
+    a device."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    native = _C.binding()
+    with FakeTensorMode():
+        x = torch.empty((3, 2, 4, 512), dtype=torch.bfloat16, device="cuda:0")
+        w = torch.empty((4, 512, 128), dtype=torch.bfloat16, device="cuda:0")
+        out = torch.empty((2, 4, 128), dtype=torch.bfloat16, device="cuda:0")
+
+        def one(row):
+            with pytest.raises(RuntimeError, match="data pointer"):
+                native.mla_v_up_proj(row, -1, w, out)
+            return row
+
+        torch.func.vmap(one)(x)

@@ -111,21 +111,37 @@ int device_of(const T&... t) {
   return d.index;
 }
 
-// Calls into the library with the tensors' device current, on its current stream and without the interpreter's lock
-// (a launch may wait for room in the queue).
-template <class F>
-void call(int device, const char* op, F&& f) {
-  int before = device;
-  NEED(hipGetDevice(&before) == hipSuccess, "%s: no current device", op);
-  if (before != device) NEED(hipSetDevice(device) == hipSuccess, "%s: cannot select device %d", op, device);
-  const kvq_stream_t s = reinterpret_cast<kvq_stream_t>(c10::hip::getCurrentHIPStream(device).stream());
+// The interpreter's lock given up, and a device made current, until the end of the block.
+struct Unlocked {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Unlocked() { PyEval_RestoreThread(state); }
+};
+struct OnDevice {
+  int before;
+  OnDevice(int device, const char* op) : before(device) {
+    NEED(hipGetDevice(&before) == hipSuccess, "%s: no current device", op);
+    if (before == device) before = -1;
+    else NEED(hipSetDevice(device) == hipSuccess, "%s: cannot select device %d", op, device);
+  }
+  ~OnDevice() {
+    if (before >= 0) (void)hipSetDevice(before);
+  }
+};
+
+// Calls f, an entry of the library, with the tensors' device current, on its current stream and without the
+// interpreter's lock (a launch may wait for room in the queue).  The arguments are plain values, taken from the tensors
+// by the caller, who holds the lock: a tensor without storage raises there (and may run Python to do so).
+template <class F, class... A>
+void call(int device, const char* op, F f, A... args) {
   int rc;
   char why[512] = "";
-  Py_BEGIN_ALLOW_THREADS;
-  rc = f(s);
-  if (rc != 0) snprintf(why, sizeof(why), "%s", kvq_last_error());
-  if (before != device) (void)hipSetDevice(before);
-  Py_END_ALLOW_THREADS;
+  {
+    const OnDevice on(device, op);
+    const kvq_stream_t s = reinterpret_cast<kvq_stream_t>(c10::hip::getCurrentHIPStream(device).stream());
+    const Unlocked unlocked;
+    rc = f(args..., s);
+    if (rc != 0) snprintf(why, sizeof(why), "%s", kvq_last_error());
+  }
   NEED(rc == 0, "%s failed (status %d): %s", op, rc, why);
 }
 
@@ -168,11 +184,9 @@ PyObject* cache_update(Args& in) {
        "slot_mapping must be a contiguous 1-D int64 tensor");
   NEED(slots.size(0) <= key.size(0), "slot_mapping is longer than key");
   const int dt = dtype_code(key, "key");
-  call(dev, "reshape_and_cache_flash_per_token_head_quant", [&](kvq_stream_t s) {
-    return kvq_reshape_and_cache_int8(ptr(key), ptr(value), dt, key.stride(0), key.stride(1), value.stride(0),
-                                      value.stride(1), base, g, static_cast<const int64_t*>(ptr(slots)), slots.size(0),
-                                      eps_of(dt), s);
-  });
+  call(dev, "reshape_and_cache_flash_per_token_head_quant", kvq_reshape_and_cache_int8, ptr(key), ptr(value), dt,
+       key.stride(0), key.stride(1), value.stride(0), value.stride(1), base, g, static_cast<const int64_t*>(ptr(slots)),
+       slots.size(0), eps_of(dt));
   Py_RETURN_NONE;
 }
 
@@ -218,20 +232,19 @@ PyObject* paged_attention(Args& in) {
              *cq = static_cast<const int32_t*>(ptr(cu));
   const auto *sk = static_cast<const float*>(ptr(sinks)), *al = static_cast<const float*>(ptr(alibi));
   auto* ls = static_cast<float*>(ptr(lse));
-  call(dev, "unified_attention", [&](kvq_stream_t s) {
-    if (ws == nullptr)   // the states live in the library's own array
-      return kvq_paged_attn_int8_static_scratch(ptr(out), odt, ro.stride_t, ro.stride_h, ptr(q), qdt, rq.stride_t,
-                                                rq.stride_h, base, g, bt, table.stride(0), sl, cq, (int)B, (int)rq.heads,
-                                                (int)max_q, (float)scale, flags, window, (float)softcap, sk, al, ls, s);
-    if (splits > 1 && max_q > 1)
-      return kvq_paged_attn_int8_split_prefill(ptr(out), odt, ro.stride_t, ro.stride_h, ptr(q), qdt, rq.stride_t,
-                                               rq.stride_h, base, g, bt, table.stride(0), sl, cq, (int)B, (int)rq.heads,
-                                               (int)max_q, (float)scale, flags, window, (float)softcap, sk, al, ls,
-                                               (int)rq.rows, splits, ptr(ws), ws->nbytes(), s);
-    return kvq_paged_attn_int8(ptr(out), odt, ro.stride_t, ro.stride_h, ptr(q), qdt, rq.stride_t, rq.stride_h, base, g, bt,
-                               table.stride(0), sl, cq, (int)B, (int)rq.heads, (int)max_q, (float)scale, flags, window,
-                               (float)softcap, sk, al, ls, ptr(ws), ws->nbytes(), s);
-  });
+  const char* op = "unified_attention";
+  if (ws == nullptr)   // the states live in the library's own array
+    call(dev, op, kvq_paged_attn_int8_static_scratch, ptr(out), odt, ro.stride_t, ro.stride_h, ptr(q), qdt, rq.stride_t,
+         rq.stride_h, base, g, bt, table.stride(0), sl, cq, (int)B, (int)rq.heads, (int)max_q, (float)scale, flags, window,
+         (float)softcap, sk, al, ls);
+  else if (splits > 1 && max_q > 1)
+    call(dev, op, kvq_paged_attn_int8_split_prefill, ptr(out), odt, ro.stride_t, ro.stride_h, ptr(q), qdt, rq.stride_t,
+         rq.stride_h, base, g, bt, table.stride(0), sl, cq, (int)B, (int)rq.heads, (int)max_q, (float)scale, flags, window,
+         (float)softcap, sk, al, ls, (int)rq.rows, splits, ptr(ws), ws->nbytes());
+  else
+    call(dev, op, kvq_paged_attn_int8, ptr(out), odt, ro.stride_t, ro.stride_h, ptr(q), qdt, rq.stride_t, rq.stride_h, base,
+         g, bt, table.stride(0), sl, cq, (int)B, (int)rq.heads, (int)max_q, (float)scale, flags, window, (float)softcap, sk,
+         al, ls, ptr(ws), ws->nbytes());
   Py_RETURN_NONE;
 }
 
@@ -285,15 +298,12 @@ PyObject* decode_with_update(Args& in) {
   check_heads(sinks, rq.heads, dev, "sinks");
   check_heads(alibi, rq.heads, dev, "alibi_slopes");
   const int odt = dtype_code(out, "out"), qdt = dtype_code(q, "q"), kdt = dtype_code(key, "key");
-  call(dev, "decode_attention_with_cache_update", [&](kvq_stream_t s) {
-    return kvq_paged_attn_int8_fused_write(
-        ptr(out), odt, ro.stride_t, ro.stride_h, ptr(q), qdt, rq.stride_t, rq.stride_h, ptr(key), ptr(value), kdt,
-        rk.stride_t, rk.stride_h, rv.stride_t, rv.stride_h, eps_of(kdt), const_cast<void*>(base), g,
-        static_cast<const int32_t*>(ptr(table)), table.stride(0), static_cast<const int32_t*>(ptr(lens)),
-        static_cast<const int64_t*>(ptr(slots)), (int)B, (int)rq.heads, (float)scale, window, (float)softcap,
-        static_cast<const float*>(ptr(sinks)), static_cast<const float*>(ptr(alibi)), static_cast<float*>(ptr(lse)),
-        ptr(ws), ws.nbytes(), s);
-  });
+  call(dev, "decode_attention_with_cache_update", kvq_paged_attn_int8_fused_write, ptr(out), odt, ro.stride_t, ro.stride_h,
+       ptr(q), qdt, rq.stride_t, rq.stride_h, ptr(key), ptr(value), kdt, rk.stride_t, rk.stride_h, rv.stride_t, rv.stride_h,
+       eps_of(kdt), const_cast<void*>(base), g, static_cast<const int32_t*>(ptr(table)), table.stride(0),
+       static_cast<const int32_t*>(ptr(lens)), static_cast<const int64_t*>(ptr(slots)), (int)B, (int)rq.heads, (float)scale,
+       window, (float)softcap, static_cast<const float*>(ptr(sinks)), static_cast<const float*>(ptr(alibi)),
+       static_cast<float*>(ptr(lse)), ptr(ws), ws.nbytes());
   Py_RETURN_NONE;
 }
 
@@ -315,10 +325,8 @@ PyObject* mla_cache_update(Args& in) {
   const int64_t T = slots.size(0);
   NEED(T <= kv_c.size(0) && T <= k_pe.size(0), "slot_mapping is longer than kv_c / k_pe");
   const int dt = dtype_code(kv_c, "kv_c");
-  call(dev, "concat_and_cache_mla", [&](kvq_stream_t s) {
-    return kvq_concat_and_cache_mla_int8(ptr(kv_c), ptr(k_pe), dt, kv_c.stride(0), k_pe.stride(0), base, g,
-                                         static_cast<const int64_t*>(ptr(slots)), T, eps_of(dt), s);
-  });
+  call(dev, "concat_and_cache_mla", kvq_concat_and_cache_mla_int8, ptr(kv_c), ptr(k_pe), dt, kv_c.stride(0),
+       k_pe.stride(0), base, g, static_cast<const int64_t*>(ptr(slots)), T, eps_of(dt));
   Py_RETURN_NONE;
 }
 
@@ -351,13 +359,10 @@ PyObject* mla_decode_absorb(Args& in) {
              lse->size(1) == H && lse->is_contiguous(),
          "lse must be contiguous float32 [B, H]");
   const int odt = dtype_code(o, "o"), qdt = dtype_code(q, "q_nope");
-  call(dev, "mla_decode_absorb_int8", [&](kvq_stream_t s) {
-    return kvq_mla_decode_absorb_int8(ptr(o), odt, static_cast<float*>(ptr(lse)), ptr(q), qdt, q.stride(0), q.stride(1),
-                                      (int)P, ptr(w), w.stride(0), w.stride(1), ptr(q_pe), q_pe.stride(0), q_pe.stride(1),
-                                      base, g, static_cast<const int32_t*>(ptr(table)), table.stride(0),
-                                      static_cast<const int32_t*>(ptr(lens)), (int)B, (int)H, (float)scale, ptr(ws),
-                                      ws.nbytes(), s);
-  });
+  call(dev, "mla_decode_absorb_int8", kvq_mla_decode_absorb_int8, ptr(o), odt, static_cast<float*>(ptr(lse)), ptr(q), qdt,
+       q.stride(0), q.stride(1), (int)P, ptr(w), w.stride(0), w.stride(1), ptr(q_pe), q_pe.stride(0), q_pe.stride(1), base,
+       g, static_cast<const int32_t*>(ptr(table)), table.stride(0), static_cast<const int32_t*>(ptr(lens)), (int)B, (int)H,
+       (float)scale, ptr(ws), ws.nbytes());
   Py_RETURN_NONE;
 }
 
@@ -380,10 +385,8 @@ PyObject* mla_v_up_proj(Args& in) {
   NEED(x.stride(2) == 1 && w.stride(2) == 1, "last dims must be contiguous");
   if (B == 0) Py_RETURN_NONE;
   const int dt = dtype_code(x, "x");
-  call(dev, "mla_v_up_proj", [&](kvq_stream_t s) {
-    return kvq_mla_v_up_proj(ptr(out), out.stride(0), flat ? V : out.stride(1), ptr(x), dt, x.stride(0), x.stride(1), ptr(w),
-                             w.stride(0), w.stride(1), (int)B, (int)H, (int)L, (int)V, s);
-  });
+  call(dev, "mla_v_up_proj", kvq_mla_v_up_proj, ptr(out), out.stride(0), flat ? V : out.stride(1), ptr(x), dt, x.stride(0),
+       x.stride(1), ptr(w), w.stride(0), w.stride(1), (int)B, (int)H, (int)L, (int)V);
   Py_RETURN_NONE;
 }
 
