@@ -27,7 +27,9 @@
 extern "C" {
 #endif
 
-#define KVQ_ABI_VERSION 19
+/* 20: kvq_mla_prefill_attn takes `causal` as a set of flags (any non-zero value meant causal up to 18; 2 is a flag of
+ * its own since 19, which other builds of 19 may not know). */
+#define KVQ_ABI_VERSION 20
 
 #define KVQ_OK 0
 #define KVQ_EINVAL (-22)
