@@ -254,3 +254,52 @@ def test_mla_forward_mqa_through_the_builder_replays_correctly(gpu_device):
         eo, _ = impl.forward_mqa((ql, qp), cache, md)          # eager work between the replays, same buffers
         torch.cuda.synchronize()
         assert torch.equal(eo, got), f"replay {it}: graph and eager outputs differ"
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(16, 1, 64), (12, 2, 128)])
+def test_short_runs_captured_on_their_first_call(gpu_device, hq, hkv, d):
+    """A batch of short query runs whose first call is the captured one (no warm-up; these head counts with ALiBi appear
+    in no other test): nothing has to be set on the device before its launch.  Replayed on other lengths, each replay
+    against the eager call and the oracle."""
+    dev, bs, B, qlen = gpu_device, 16, 5, 3
+    full = [900, 70, 2100, 333, 16]
+    g = torch.Generator().manual_seed(hq)
+    kv_cpu, _views, lay = T.cpu_cache(240, bs, hkv, d, "HND")
+    bt = T.make_block_tables(full, bs, 240, g)
+    rows = [torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in full]
+    T.fill_cache_from_sources(kv_cpu, lay, bt, full, bs, rows, [r.flip(0) for r in rows])
+    kv = T.to_device_cache(kv_cpu, dev, "HND")
+    k, v = L.key_value_views(kv)
+    ksc, vsc = L.scale_views(kv)
+    geom = L.geometry_from_views(k, v, ksc, vsc)
+    q = torch.zeros((B * qlen, hq, d), dtype=torch.bfloat16, device=dev)
+    out = torch.zeros_like(q)
+    cu = torch.arange(0, B * qlen + 1, qlen, dtype=torch.int32)
+    cu_d, bt_d = cu.to(dev), bt.to(dev)
+    sl = torch.full((B,), qlen, dtype=torch.int32, device=dev)
+    slopes = torch.tensor([2.0 ** (-8.0 * (i + 1) / hq) for i in range(hq)], dtype=torch.float32)
+    slopes_d = slopes.to(dev)
+    ops._default_workspace(dev, 96 << 20)      # grown before the capture
+
+    def step(o):
+        ops.unified_attention(q, k, v, o, cu_d, qlen, sl, max(full), 0.1, True, block_table=bt_d, k_scale_cache=ksc,
+                              v_scale_cache=vsc, geometry=geom, alibi_slopes=slopes_d)
+
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step(out)
+    for it, lens in enumerate((full, [3, 3, 3, 3, 3], [c // 2 for c in full], full)):
+        lens_cpu = torch.tensor(lens, dtype=torch.int32)
+        qh = torch.randn(q.shape, generator=g).to(torch.bfloat16)
+        q.copy_(qh.to(dev))
+        sl.copy_(lens_cpu.to(dev))
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = torch.empty_like(out)
+        step(eager)
+        torch.cuda.synchronize()
+        assert torch.equal(eager, out), f"replay {it}: graph and eager outputs differ"
+        want = oracle.paged_attn(qh, T.storage_bytes(kv_cpu), lay, bt, lens_cpu, cu, 0.1, alibi_slopes=slopes)
+        T.assert_close_attn(out, want, what=f"short runs, graph replay {it}")

@@ -11,8 +11,6 @@
 // of went from 105.8 to 71.3 us.
 #pragma once
 
-#include <atomic>
-
 #include "kvq_prefill_tile.cuh"
 #include "kvq_short_runs.h"
 #include "kvq_work_line.cuh"
@@ -66,7 +64,9 @@ __global__ __launch_bounds__(512) void short_runs_streamk_kernel(ShortRunArgs a)
   // flight in registers the two column tiles' accumulators spilled: 420 against 106 us on the batch named above)
   constexpr int kWindow = DTile::LDS_TILE + 64 * 4;
   constexpr int kLdsWave = short_runs_lds_wave<D, CODE>();
-  extern __shared__ __align__(16) uint8_t lds_all[];
+  // (139 KB at head size 128, one workgroup per compute unit.  A fixed array: dynamic LDS of that size needs a function
+  // attribute that the first call of each instantiation would set, possibly inside a stream capture.)
+  __shared__ __align__(16) uint8_t lds_all[8 * kLdsWave];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = wave % NSUB;
@@ -327,23 +327,9 @@ __global__ __launch_bounds__(256) void short_runs_reduce_kernel(ShortRunArgs a) 
   if (io.lse != nullptr && lane == 0) io.lse[row * Hq + head] = l > 0.f ? (m + __builtin_amdgcn_logf(l)) * kLn2 : -INFINITY;
 }
 
-// A launch of the main kernel; its windows need more dynamic LDS than a kernel gets by default, an attribute that is set
-// the first time a kernel runs on a device.
 template <int D, int NT, int HPW, int CODE, bool EXT>
 static int launch_one(const ShortRunArgs& a, dim3 grid, hipStream_t s) {
-  static std::atomic<uint64_t> done_mask{0};  // one bit per device id < 64
-  auto kernel = &short_runs_streamk_kernel<D, NT, HPW, CODE, EXT>;
-  constexpr int bytes = 8 * short_runs_lds_wave<D, CODE>();
-  int dev = -1;
-  if (int e = check_hip(hipGetDevice(&dev), "hipGetDevice")) return e;
-  const uint64_t bit = dev >= 0 && dev < 64 ? (1ull << dev) : 0;
-  if (bit == 0 || !(done_mask.load(std::memory_order_acquire) & bit)) {
-    if (int e = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, bytes),
-                          "hipFuncSetAttribute(short_runs_streamk_kernel)"))
-      return e;
-    done_mask.fetch_or(bit, std::memory_order_release);
-  }
-  hipLaunchKernelGGL(kernel, grid, dim3(512), bytes, s, a);
+  hipLaunchKernelGGL((short_runs_streamk_kernel<D, NT, HPW, CODE, EXT>), grid, dim3(512), 0, s, a);
   return check_hip(hipGetLastError(), "paged_attn_int8 short runs launch");
 }
 
