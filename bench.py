@@ -600,6 +600,10 @@ def mixed_main(args, cfg, dev, ops):
     splits = ops.prefill_context_splits(qls, max(ctx), hq, hkv) if cfg.get("chunk") else 1
     if splits > 1:
         ws = torch.empty(ops.split_prefill_workspace_bytes(B, hq, d, n_tok, splits), dtype=torch.uint8, device=dev)
+    # a batch of short runs: the launch that serves it, as the layer asks for it with the builder's workspace
+    short = ops.short_runs_workspace_bytes(B, hq, hkv, d, max(qls))
+    if short > ws.numel():
+        ws = torch.empty(short, dtype=torch.uint8, device=dev)
 
     def step(layer, write=True, attn=True, splits=splits):
         c = caches[layer]
@@ -609,7 +613,7 @@ def mixed_main(args, cfg, dev, ops):
         if attn:
             ops.unified_attention(q, c["k"], c["v"], out, cu_d, max(qls), sl_d, max(ctx), scale, True, block_table=bt_d,
                                   k_scale_cache=c["ks"], v_scale_cache=c["vs"], workspace=ws, geometry=c["geom"],
-                                  kv_quant_mode=mode, prefill_splits=splits,
+                                  kv_quant_mode=mode, prefill_splits=splits, short_runs=short > 0,
                                   **_window_kwargs(dict(window=args.sliding_window, softcap=args.soft_cap)))
 
     Lr = args.layers

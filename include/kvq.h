@@ -28,8 +28,8 @@ extern "C" {
 #endif
 
 /* 20: kvq_mla_prefill_attn takes `causal` as a set of flags (any non-zero value meant causal up to 18; 2 is a flag of
- * its own since 19, which other builds of 19 may not know). */
-#define KVQ_ABI_VERSION 20
+ * its own since 19, which other builds of 19 may not know).  21: KVQ_ATTN_SHORT_RUNS and its workspace query. */
+#define KVQ_ABI_VERSION 21
 
 #define KVQ_OK 0
 #define KVQ_EINVAL (-22)
@@ -89,9 +89,10 @@ typedef struct kvq_cache_geom {
 #define KVQ_CODE_FP8_E4M3 1
 #define KVQ_CODE_INT4 2
 
-/* flags of the `causal` argument of kvq_paged_attn_int8 and its static-scratch form */
+/* flags of the `causal` argument of kvq_paged_attn_int8, its split-prefill form and its static-scratch form */
 #define KVQ_ATTN_CAUSAL 1
 #define KVQ_ATTN_NO_DECODE_ROWS 2
+#define KVQ_ATTN_SHORT_RUNS 4
 
 /* Byte geometry of the int8 MLA latent cache: per block, block_size code rows
  * of (kv_lora_rank + rope_dim) bytes followed by block_size fp32 scales. */
@@ -149,6 +150,16 @@ KVQ_API int kvq_reshape_and_cache_int8(const void* key, const void* value, int s
  * vllm_metax/v1/attention/backends/triton_attn.py:155-176.
  */
 KVQ_API size_t kvq_paged_attn_workspace_bytes(int max_num_seqs, int num_q_heads, int head_size);
+
+/*
+ * Workspace for kvq_paged_attn_int8 with KVQ_ATTN_SHORT_RUNS: enough for any batch of at most max_num_seqs
+ * sequences whose runs have at most max_query_len tokens (0: as many as the flag serves), and at least
+ * kvq_paged_attn_workspace_bytes().  0 where the flag changes nothing.
+ * The states are at most two per workgroup, [num_kv_heads][columns][head_size + 2] floats each, however many
+ * sequences there are: 68 MB at 8 kv heads of 128 dims with 32 columns, 34 MB with 16.
+ */
+KVQ_API size_t kvq_paged_attn_short_runs_workspace_bytes(int max_num_seqs, int num_q_heads, int num_kv_heads,
+                                                         int head_size, int max_query_len);
 
 /*
  * Rotary embedding of the step's query and key rows fused with the quantise-on-write of the step's K / V:
@@ -213,6 +224,14 @@ KVQ_API int kvq_rope_and_cache_int8(const int64_t* positions, void* query, int64
  * row (a pure prefill batch; a metadata builder knows it from the host copy of query_start_loc).  The
  * split-K decode kernel and its reduce are then not launched at all; with a one-row sequence in the batch
  * after all, that row's output is left unwritten.
+ *
+ * KVQ_ATTN_SHORT_RUNS (4): a batch whose longest run is short (2 .. 63 columns, a column being a query token of
+ * one q head of a kv group; a speculative-decoding step) is served by one launch over all its sequences where
+ * that launch is built: head sizes 64 and 128, a cache in which a head's records of a block lie back to back,
+ * not in the batch-invariant mode.  Its partial states need more room: the workspace must then hold
+ * kvq_paged_attn_short_runs_workspace_bytes(num_seqs, ..., max_query_len) bytes, and a smaller one is refused.
+ * For any other batch the flag changes nothing.  Without it such a batch goes through the decode and prefill
+ * kernels, whatever the workspace's size; the results agree within the tolerance, not bit for bit.
  *
  * Value range: the weights enter the second product as fp16 numbers
  * p * v_scale * 2^8, so a V row whose scale exceeds 255.8 (int8 codes: absmax
@@ -297,7 +316,8 @@ KVQ_API int kvq_paged_attn_int8_fused_write(void* out, int out_dtype, int64_t ou
  * kvq_paged_attn_workspace_bytes(num_seqs, num_q_heads, head_size) <=
  * KVQ_STATIC_SCRATCH_BYTES (the partial states plus the kernels' notes: 32 q
  * heads of 128 dims on 256 compute units: up to 1255 sequences); a larger one
- * is rejected with KVQ_EINVAL and nothing is launched.  All calls on one GPU
+ * is rejected with KVQ_EINVAL and nothing is launched (with KVQ_ATTN_SHORT_RUNS the
+ * size of that flag's query decides).  All calls on one GPU
  * share that GPU's array: calls that overlap in time on one GPU (different
  * streams, different threads) race and must be serialised by the caller.
  * kvq_paged_attn_static_scratch_bytes() returns the array's size and is the

@@ -157,3 +157,48 @@ def test_small_chunk_on_a_long_context_goes_through_context_splits(gpu_device):
     want = oracle.paged_attn(q.view(n, hq, d), T.storage_bytes(kv_cpu), lay, bt, torch.tensor(ctx, dtype=torch.int32),
                              cu, 1 / math.sqrt(d))
     T.assert_close_attn(out.view(n, hq, d), want, what="chunk on a long context through the backend")
+
+
+@pytest.mark.parametrize("hq,hkv,qlen", [(32, 32, 3), (32, 16, 9), (32, 8, 15)])
+@pytest.mark.parametrize("n", [8, 40, 200])
+def test_verify_steps_through_the_builder_take_one_launch_at_every_batch_size(gpu_device, hq, hkv, qlen, n):
+    """A speculative-decoding step through the metadata builder and the layer's forward: whatever the batch size, the
+    builder's workspace holds what the launch for short runs needs, and the layer asks for it (the same bits as that
+    launch in a workspace of its own)."""
+    dev, d, bs, nb = gpu_device, 128, 16, 1700
+    g = torch.Generator().manual_seed(n + hq)
+    ctx = [qlen + int(x) for x in torch.randint(0, 100, (n,), generator=g)]
+    layout = "NHD" if Int8AttentionBackend.get_kv_cache_stride_order() == (0, 2, 1, 3) else "HND"
+    kv_cpu, _, lay = T.cpu_cache(nb, bs, hkv, d, layout)
+    bt = T.make_block_tables(ctx, bs, nb, g)
+    rows = [torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in ctx]
+    T.fill_cache_from_sources(kv_cpu, lay, bt, ctx, bs, rows, [r.flip(0) for r in rows])
+    impl = Int8AttentionBackend.get_impl_cls()(hq, d, 0.09, hkv, kv_cache_dtype="int8_per_token_head")
+    spec = types.SimpleNamespace(block_size=bs, num_kv_heads=hkv, head_size=d, num_q_heads=hq)
+    cfg = types.SimpleNamespace(scheduler_config=types.SimpleNamespace(max_num_seqs=256))
+    builder = Int8AttentionBackend.get_builder_cls()(spec, ["layer.0"], cfg, dev)
+    kv_cache = L.allocate_kv_cache(nb, bs, hkv, d, device=dev, layout=layout)
+    impl._ensure_scale_caches(kv_cache)                  # fills the scales once, as at first use
+    T.storage_bytes(kv_cache).copy_(T.storage_bytes(kv_cpu).to(dev))
+    cu = torch.arange(0, n * qlen + 1, qlen, dtype=torch.int32)
+    common = types.SimpleNamespace(
+        num_reqs=n, num_actual_tokens=n * qlen, max_query_len=qlen, max_seq_len=max(ctx), query_start_loc=cu.to(dev),
+        query_start_loc_cpu=cu, seq_lens=torch.tensor(ctx, dtype=torch.int32, device=dev),
+        block_table_tensor=bt.to(dev), slot_mapping=torch.zeros(n * qlen, dtype=torch.int64, device=dev), causal=True)
+    md = builder.build(0, common)
+    q = torch.randn((n * qlen, hq * d), generator=g).to(torch.bfloat16)
+    out = torch.zeros((n * qlen, hq * d), dtype=torch.bfloat16, device=dev)
+    impl.forward(types.SimpleNamespace(), q.to(dev), None, None, kv_cache, md, out)
+    k, v = L.key_value_views(kv_cache)
+    ks, vs = L.scale_views(kv_cache)
+    own = torch.empty_like(out)
+    ops.unified_attention(q.to(dev).view(-1, hq, d), k, v, own.view(-1, hq, d), cu.to(dev), qlen, common.seq_lens, max(ctx),
+                          0.09, True, block_table=bt.to(dev), k_scale_cache=ks, v_scale_cache=vs, short_runs=True,
+                          workspace=torch.empty(ops.short_runs_workspace_bytes(n, hq, hkv, d, qlen), dtype=torch.uint8,
+                                                device=dev))
+    torch.cuda.synchronize()
+    assert md.short_runs is True
+    same = torch.equal(out, own)
+    assert same, "not the launch that was asked for"
+    want = oracle.paged_attn(q.view(-1, hq, d), T.storage_bytes(kv_cpu), lay, bt, torch.tensor(ctx, dtype=torch.int32), cu, 0.09)
+    T.assert_close_attn(out.view(-1, hq, d), want, what=f"verify step of {n} sequences")

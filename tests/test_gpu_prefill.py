@@ -431,3 +431,40 @@ def test_short_run_line(gpu_device, hq, hkv, d, qmax, code, q_dtype, extras):
         torch.cuda.synchronize()
         T.assert_close_attn(out, want, what=f"short runs, {code}, workspace {'tight' if workspace is not None else 'default'}")
         torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("hq,hkv,d,qmax", [(32, 8, 128, 4), (16, 16, 64, 30), (28, 4, 128, 9)])
+def test_short_runs_are_asked_for_and_do_not_depend_on_the_workspace(gpu_device, hq, hkv, d, qmax):
+    """The launch for batches of short runs is taken when the caller asks for it, never because its states happen to fit:
+    the bits of a call are the same in a workspace of exactly the stated size and in a larger one, asked for or not, and
+    a workspace one byte short is refused.  The workspaces hold NaN patterns, which no state that was not written may
+    bring into a row."""
+    ctx = [700, 33, 2100, 64, 257, 5, 31] * 6
+    qls = [min(c, 1 + i % qmax) for i, c in enumerate(ctx)]
+    qls[0] = qmax
+    kv, lay, bt, q, sl, cu = build(ctx, qls, hq, hkv, d, 16, layout="HND", seed=hq + qmax)
+    dev, scale = gpu_device, 1 / math.sqrt(d)
+    want = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, scale)
+    kvd = T.to_device_cache(kv, dev, "HND")
+    k, v = L.key_value_views(kvd)
+    ks, vs = L.scale_views(kvd)
+    qd, cu_d, sl_d, bt_d = q.to(dev), cu.to(dev), sl.to(dev), bt.to(dev)
+
+    def call(nbytes, **kw):
+        out = torch.full(q.shape, float("nan"), dtype=q.dtype, device=dev)
+        ops.unified_attention(qd, k, v, out, cu_d, qmax, sl_d, max(ctx), scale, True, block_table=bt_d, k_scale_cache=ks,
+                              v_scale_cache=vs, workspace=torch.full((nbytes,), 0xFF, dtype=torch.uint8, device=dev), **kw)
+        torch.cuda.synchronize()
+        return out
+
+    for kw in ({}, dict(short_runs=True)):
+        exact = ops.paged_attn_workspace_bytes(len(ctx), hq, d)
+        if kw:
+            exact, smaller = ops.short_runs_workspace_bytes(len(ctx), hq, hkv, d, qmax), exact
+            assert smaller <= exact <= ops.short_runs_workspace_bytes(len(ctx) + 100, hq, hkv, d)
+        out = call(exact, **kw)
+        T.assert_close_attn(out, want, what=f"short runs {hq}/{hkv} d{d} q<={qmax} {kw}")
+        same = torch.equal(out, call(256 << 20, **kw))
+        assert same, f"the bits depend on the workspace's size {kw}"
+        with pytest.raises(RuntimeError, match="workspace"):
+            call(exact - 1, **kw)

@@ -81,8 +81,10 @@ static int paged_attn_launch(const char* op, void* out, int out_dtype, int64_t o
                              int num_tokens = 0) {
   int rc0 = validate_common(op, q, cache, geom, block_table, seq_lens, num_seqs, num_q_heads);
   if (rc0) return rc0;
-  KVQ_REQUIRE((causal & ~(KVQ_ATTN_CAUSAL | KVQ_ATTN_NO_DECODE_ROWS)) == 0, "%s: unknown flag in causal (%d)", op, causal);
+  KVQ_REQUIRE((causal & ~(KVQ_ATTN_CAUSAL | KVQ_ATTN_NO_DECODE_ROWS | KVQ_ATTN_SHORT_RUNS)) == 0,
+              "%s: unknown flag in causal (%d)", op, causal);
   const bool no_decode_rows = (causal & KVQ_ATTN_NO_DECODE_ROWS) != 0;
+  const bool want_short_runs = (causal & KVQ_ATTN_SHORT_RUNS) != 0;
   causal &= KVQ_ATTN_CAUSAL;
   KVQ_REQUIRE(out != nullptr, "%s: out is NULL", op);
   KVQ_REQUIRE(max_query_len >= 1, "%s: max_query_len must be >= 1", op);
@@ -105,6 +107,12 @@ static int paged_attn_launch(const char* op, void* out, int out_dtype, int64_t o
     KVQ_REQUIRE(num_tokens >= 1, "%s: num_tokens (the rows of q) is required with prefill_splits > 1", op);
     need = part_at + split_part_bytes(num_tokens, num_q_heads, g.head_size, prefill_splits);
   }
+  // a batch of short runs: one launch for all its sequences, where the caller asked for it
+  ShortRunArgs r{};
+  size_t short_bytes = 0;
+  const bool short_runs = want_short_runs && short_runs_cache(g) &&
+                          short_runs_shape(num_q_heads, g.num_kv_heads, g.head_size, num_seqs, max_query_len, num_wg, &r, &short_bytes);
+  if (short_runs && short_bytes > need) need = short_bytes;
   KVQ_REQUIRE(workspace != nullptr && workspace_bytes >= need && ((uintptr_t)workspace % 16) == 0,
               "%s: %s of %zu bytes (16-byte aligned) required, got %zu", op, workspace_what, need, workspace_bytes);
 
@@ -166,11 +174,7 @@ static int paged_attn_launch(const char* op, void* out, int out_dtype, int64_t o
   }
   hipStream_t s = as_stream(stream);
   int rc = KVQ_OK;
-  // a batch of short runs: one launch for all its sequences, where the workspace has room for its states (a caller that
-  // sized it for one-token rows only keeps the kernels below)
-  ShortRunArgs r{};
-  size_t short_bytes = 0;
-  if (short_runs_take(g, num_q_heads, num_seqs, max_query_len, num_wg, &r, &short_bytes) && workspace_bytes >= short_bytes) {
+  if (short_runs) {
     r.io = a.io;
     r.seq_lens = seq_lens;
     r.cu_seqlens_q = cu_seqlens_q;

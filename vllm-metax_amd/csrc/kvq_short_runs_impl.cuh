@@ -59,7 +59,6 @@ __global__ __launch_bounds__(512) void short_runs_streamk_kernel(ShortRunArgs a)
   using PT = PrefillTile<D, KVQ_BF16, kRuntimeDtype, NT, CODE, true>;   // (the query's type is read at run time)
   using DTile = typename PT::DTile;
   constexpr int NSUB = 8 / HPW;
-  constexpr int NC = 16 * NT;
   // two windows per wave: a tile streams into one, past the registers, while the other is computed (with a tile in
   // flight in registers the two column tiles' accumulators spilled: 420 against 106 us on the batch named above)
   constexpr int kWindow = DTile::LDS_TILE + 64 * 4;
@@ -237,7 +236,8 @@ __global__ __launch_bounds__(512) void short_runs_streamk_kernel(ShortRunArgs a)
         }
         const float l = PT::total_l(st, nt);
         if (!valid) continue;
-        const int64_t at = (((int64_t)w + item) * io.g.num_kv_heads + hkv) * NC + nt * 16 + c;
+        const int slot = 2 * w + (tb == it.t0 ? 1 : 0);
+        const int64_t at = (uint32_t)((slot * io.g.num_kv_heads + hkv) * a.rows + nt * 16 + c);
         float v[D / 4];
         PT::gather_row(st, nt, 1.0f / DTile::kOutDiv, v);
         const int g = lane >> 4;
@@ -261,7 +261,7 @@ template <int D>
 __global__ __launch_bounds__(256) void short_runs_reduce_kernel(ShortRunArgs a) {
   constexpr int V = D / 64;
   const int lane = threadIdx.x & 63;
-  const int r = blockIdx.y * 4 + (threadIdx.x >> 6);
+  const int r = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const AttnIO& io = a.io;
   const int Hq = io.num_q_heads;
   const int qt = r / Hq, head = r - qt * Hq;
@@ -282,18 +282,20 @@ __global__ __launch_bounds__(256) void short_runs_reduce_kernel(ShortRunArgs a) 
     const int w_last = (int)(((start + a.setup_units + ntiles) * P - 1) / total);
     if (w_first == w_last) return;  // written by the main kernel
     const int hkv = head / io.group, n = qt * io.group + head - hkv * io.group;
-    const int64_t stride = (int64_t)io.g.num_kv_heads * a.cols;   // rows between two slots
-    const int64_t at0 = ((int64_t)item * io.g.num_kv_heads + hkv) * a.cols + n;   // slot w lies at at0 + w * stride
+    const int64_t stride = (int64_t)io.g.num_kv_heads * a.rows;   // rows between two slots
+    const int64_t at0 = (int64_t)hkv * a.rows + n;
+    // workgroup w's state of this item lies at at0 + 2 w stride, the first one's (it begins with the item) a stride further
     auto pass = [&](int wb, auto n_tag) __attribute__((always_inline)) {
       constexpr int N = decltype(n_tag)::value;
       const int wj = wb + lane;
       const bool live = lane < N && wj <= w_last && wg_tile_begin(wj, total, P) < wg_tile_begin(wj + 1, total, P);
-      const int64_t mine = at0 + (int64_t)min(wj, w_last) * stride;
+      const int64_t mine = at0 + (2 * (int64_t)min(wj, w_last) + (wj == w_first ? 1 : 0)) * stride;
       const float mj_raw = a.part_ml[2 * mine], lj_raw = a.part_ml[2 * mine + 1];
       float po[N][V];
 #pragma unroll
       for (int k = 0; k < N; ++k) {
-        const float* p = a.part_o + (at0 + (int64_t)min(wb + k, w_last) * stride) * D + lane * V;
+        const int64_t at = at0 + 2 * (int64_t)min(wb + k, w_last) * stride + (k == 0 && wb == w_first ? stride : 0);
+        const float* p = a.part_o + at * D + lane * V;
 #pragma unroll
         for (int i = 0; i < V; ++i) po[k][i] = p[i];
       }

@@ -16,7 +16,8 @@ BINDING_PATH = os.path.join(_LIB_DIR, "kvq_torch.so")   # csrc/kvq_torch.cpp
 
 KVQ_F32, KVQ_BF16, KVQ_F16 = 0, 1, 2
 KVQ_CODE_INT8, KVQ_CODE_FP8_E4M3, KVQ_CODE_INT4 = 0, 1, 2
-ABI_VERSION = 20
+KVQ_ATTN_CAUSAL, KVQ_ATTN_NO_DECODE_ROWS, KVQ_ATTN_SHORT_RUNS = 1, 2, 4
+ABI_VERSION = 21
 
 
 class CacheGeom(ctypes.Structure):
@@ -55,6 +56,7 @@ SIGNATURES = {
     "kvq_get_batch_invariant": (_i, []),
     "kvq_reshape_and_cache_int8": (_i, [_vp, _vp, _i, _i64, _i64, _i64, _i64, _vp, _geom_p, _vp, _i64, _f, _vp]),
     "kvq_paged_attn_workspace_bytes": (_sz, [_i, _i, _i]),
+    "kvq_paged_attn_short_runs_workspace_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "kvq_paged_attn_int8": (_i, [_vp, _i, _i64, _i64, _vp, _i, _i64, _i64, _vp, _geom_p, _vp, _i64, _vp, _vp,
                                  _i, _i, _i, _f, _i, _i, _f, _vp, _vp, _vp, _vp, _sz, _vp]),
     "kvq_paged_attn_int8_fused_write": (_i, [_vp, _i, _i64, _i64, _vp, _i, _i64, _i64, _vp, _vp, _i, _i64, _i64, _i64, _i64,

@@ -231,6 +231,22 @@ def paged_attn_workspace_bytes(max_num_seqs: int, num_q_heads: int, head_size: i
     return got
 
 
+def short_runs_workspace_bytes(max_num_seqs: int, num_q_heads: int, num_kv_heads: int, head_size: int,
+                               max_query_len: int = 0, device: torch.device | None = None) -> int:
+    """Workspace with which a batch of short query runs (at most ``max_query_len`` tokens each; 0 = as many as count as
+    short) is served by one launch, see ``unified_attention(..., short_runs=True)``.  Enough for the decode kernels as
+    well; 0 where that launch is not built for these sizes."""
+    idx = torch.cuda.current_device() if device is None or device.index is None else device.index
+    key = (idx, max_num_seqs, num_q_heads, head_size, num_kv_heads, max_query_len)
+    got = _ws_bytes_cache.get(key)
+    if got is None:
+        with torch.cuda.device(idx):
+            got = int(_C.load().kvq_paged_attn_short_runs_workspace_bytes(max_num_seqs, num_q_heads, num_kv_heads,
+                                                                          head_size, max_query_len))
+        _ws_bytes_cache[key] = got
+    return got
+
+
 _ws_cache: dict = {}
 _ws_retired: list = []
 
@@ -251,6 +267,19 @@ def _default_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
         cur = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=dev)
         _ws_cache[dev] = cur
     return cur
+
+
+def _attention_workspace(dev: torch.device, num_seqs: int, num_rows: int, num_q_heads: int, geom: CacheGeometry,
+                         max_seqlen_q: int, prefill_splits: int) -> tuple[torch.Tensor, bool]:
+    """Scratch for an attention call that brought none, and whether the call is one of short runs (for which it then has
+    the room)."""
+    if max_seqlen_q == 1:
+        return _default_workspace(dev, paged_attn_workspace_bytes(num_seqs, num_q_heads, geom.head_size, dev)), False
+    need = split_prefill_workspace_bytes(num_seqs, num_q_heads, geom.head_size, num_rows, prefill_splits, dev)
+    short = 0
+    if geom.stride_slot == geom.record_bytes:
+        short = short_runs_workspace_bytes(num_seqs, num_q_heads, geom.num_kv_heads, geom.head_size, max_seqlen_q, dev)
+    return _default_workspace(dev, max(need, short)), short > 0
 
 
 def unified_attention(
@@ -284,6 +313,7 @@ def unified_attention(
     static_scratch: bool = False,
     has_decode_rows: bool = True,
     prefill_splits: int = 1,
+    short_runs: bool = False,
     **unused,
 ) -> None:
     """Drop-in for ``unified_attention`` as called at
@@ -306,7 +336,11 @@ def unified_attention(
     ``prefill_splits`` (1..8): the context of the long query runs is cut into that many ranges, each a workgroup of
     its own, and merged (``prefill_context_splits`` proposes a value): for launches whose long runs make few
     workgroups on a long context, e.g. one request's small prefill chunk.  The workspace must then hold
-    ``split_prefill_workspace_bytes(...)``; the default workspace is grown as needed."""
+    ``split_prefill_workspace_bytes(...)``; the default workspace is grown as needed.
+    ``short_runs=True``, for a caller that brings a workspace: a batch whose longest run is short (a
+    speculative-decoding step) is served by one launch over all its sequences, on a head-major cache.  The workspace
+    must then hold ``short_runs_workspace_bytes(...)``; a smaller one is refused.  Other batches are served as without
+    it.  Without a workspace such a batch always takes that launch."""
     code_type = code_type_of(kv_quant_mode)
     if output_scale is not None or mm_prefix_range is not None:
         raise NotImplementedError("fused output quantisation and mm-prefix ranges are not built")
@@ -343,18 +377,16 @@ def unified_attention(
         raise RuntimeError("q/out must be [num_tokens, num_q_heads, head_size] matching the cache head size")
     num_seqs = seqused_k.shape[0]
     if static_scratch:
-        workspace, prefill_splits = None, 1
+        workspace, prefill_splits, short_runs = None, 1, False
     elif workspace is None and num_seqs > 0 and q.shape[0] > 0:
-        if int(max_seqlen_q) > 1:   # room for the partial states of the runs' rows as well
-            need = split_prefill_workspace_bytes(num_seqs, q.shape[1], geom.head_size, max(q.shape[0], 2048),
-                                                 max(prefill_splits, 2), dev)
-        else:
-            need = paged_attn_workspace_bytes(num_seqs, q.shape[1], geom.head_size, dev)
-        workspace = _default_workspace(dev, need)
+        workspace, short_runs = _attention_workspace(dev, num_seqs, q.shape[0], q.shape[1], geom, int(max_seqlen_q),
+                                                     prefill_splits)
+    flags = (_C.KVQ_ATTN_CAUSAL if causal else 0) | (0 if has_decode_rows else _C.KVQ_ATTN_NO_DECODE_ROWS) \
+        | (_C.KVQ_ATTN_SHORT_RUNS if short_runs else 0)
     _C.binding().paged_attention(
         q, out, -1, 0, k, geom.struct_addr, geom.base_ptr, cu_seqlens_q, seqused_k, block_table, int(max_seqlen_q),
-        int(max_seqlen_k), float(softmax_scale), (1 if causal else 0) | (0 if has_decode_rows else 2), window, softcap,
-        sinks, alibi_slopes, lse, workspace, prefill_splits)
+        int(max_seqlen_k), float(softmax_scale), flags, window, softcap, sinks, alibi_slopes, lse, workspace,
+        prefill_splits)
 
 
 def split_prefill_workspace_bytes(max_num_seqs: int, num_q_heads: int, head_size: int, num_tokens: int,

@@ -86,6 +86,8 @@ class Int8AttentionMetadata:
     # False when the builder KNOWS (from the host copy of query_start_loc) that no sequence has exactly one query
     # row: the attention call then skips its decode kernels
     has_decode_rows: bool = True
+    # the workspace has the room of the launch that serves a batch of short query runs (a speculative-decoding step)
+    short_runs: bool = False
 
 
 def _first_attr(obj, *names, default=None):
@@ -125,6 +127,7 @@ class Int8AttentionMetadataBuilder(_BuilderBase):
         sched = getattr(vllm_config, "scheduler_config", None)
         self.max_num_seqs = int(_first_attr(sched, "max_num_seqs", default=256)) if sched is not None else 256
         self._workspace: torch.Tensor | None = None
+        self._short_runs = False
 
     # query rows x context splits whose partial states the workspace has room for (a launch is split only when its
     # long runs are few: a small prefill chunk of a long request)
@@ -132,10 +135,14 @@ class Int8AttentionMetadataBuilder(_BuilderBase):
 
     def _get_workspace(self) -> torch.Tensor | None:
         if self._workspace is None and self.device.type == "cuda":
-            # the plain workspace + the partial states of MAX_SPLIT_TOKENS (rows x splits)
+            # the plain workspace + the partial states of MAX_SPLIT_TOKENS (rows x splits), or those of any batch of
+            # short runs: every batch this builder takes is then served the same way whatever its size
             nbytes = ops.split_prefill_workspace_bytes(self.max_num_seqs, self.num_heads_q, self.headdim,
-                                                       self.MAX_SPLIT_TOKENS // 2, 2)
-            self._workspace = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=self.device)
+                                                       self.MAX_SPLIT_TOKENS // 2, 2, self.device)
+            short = ops.short_runs_workspace_bytes(self.max_num_seqs, self.num_heads_q, self.num_heads_kv, self.headdim,
+                                                   device=self.device)
+            self._short_runs = short > 0
+            self._workspace = torch.empty(max(nbytes, short, 16), dtype=torch.uint8, device=self.device)
         return self._workspace
 
     def build_for_cudagraph_capture(self, common_attn_metadata) -> Int8AttentionMetadata:
@@ -162,9 +169,11 @@ class Int8AttentionMetadataBuilder(_BuilderBase):
                                                         max_split_tokens=self.MAX_SPLIT_TOKENS)
             while prefill_splits > 1 and prefill_splits * int(c.num_actual_tokens) > self.MAX_SPLIT_TOKENS:
                 prefill_splits -= 1
+        workspace = self._get_workspace()
         return Int8AttentionMetadata(
             has_decode_rows=has_decode_rows,
             prefill_splits=prefill_splits,
+            short_runs=self._short_runs,
             num_actual_tokens=c.num_actual_tokens,
             max_query_len=c.max_query_len,
             query_start_loc=c.query_start_loc,
@@ -172,7 +181,7 @@ class Int8AttentionMetadataBuilder(_BuilderBase):
             seq_lens=c.seq_lens,
             block_table=c.block_table_tensor,
             slot_mapping=c.slot_mapping,
-            workspace=self._get_workspace(),
+            workspace=workspace,
             causal=bool(getattr(c, "causal", True)),
         )
 
@@ -437,13 +446,14 @@ class Int8AttentionImpl(_ImplBase):
         self._ensure_scale_caches(kv_cache)
         geom = self._geometry
         md = attn_metadata
-        workspace = md.workspace
+        workspace, short_runs = md.workspace, getattr(md, "short_runs", False)
         if workspace is None:
-            workspace = self._own_workspace(query, md)
+            workspace, short_runs = self._own_workspace(query, md)
+        flags = (_C.KVQ_ATTN_CAUSAL if md.causal else 0) | (_C.KVQ_ATTN_SHORT_RUNS if short_runs else 0) \
+            | (0 if getattr(md, "has_decode_rows", True) else _C.KVQ_ATTN_NO_DECODE_ROWS)
         _C.binding().paged_attention(
             query, output, md.num_actual_tokens, self.num_heads, kv_cache, geom.struct_addr, geom.base_ptr,
-            md.query_start_loc, md.seq_lens, md.block_table, md.max_query_len, md.max_seq_len, self.scale,
-            (1 if md.causal else 0) | (0 if getattr(md, "has_decode_rows", True) else 2), self._window,
+            md.query_start_loc, md.seq_lens, md.block_table, md.max_query_len, md.max_seq_len, self.scale, flags, self._window,
             self.logits_soft_cap, self._sinks_on(query.device) if self.sinks is not None else None,
             self._alibi_on(query.device) if self.alibi_slopes is not None else None, None, workspace,
             getattr(md, "prefill_splits", 1))
@@ -451,13 +461,8 @@ class Int8AttentionImpl(_ImplBase):
 
     def _own_workspace(self, query, md):
         """Scratch for metadata that brings none (the builder's always does): the op layer's per-device buffer."""
-        num_seqs, splits = max(md.seq_lens.shape[0], 1), getattr(md, "prefill_splits", 1)
-        if splits > 1 and md.max_query_len > 1:
-            need = ops.split_prefill_workspace_bytes(num_seqs, self.num_heads, self.head_size, md.num_actual_tokens,
-                                                     splits, query.device)
-        else:
-            need = ops.paged_attn_workspace_bytes(num_seqs, self.num_heads, self.head_size, query.device)
-        return ops._default_workspace(query.device, need)
+        return ops._attention_workspace(query.device, max(md.seq_lens.shape[0], 1), md.num_actual_tokens, self.num_heads,
+                                        self._geometry, md.max_query_len, getattr(md, "prefill_splits", 1))
 
 
 class Int8FusedUpdateAttentionImpl(Int8AttentionImpl):
@@ -487,7 +492,7 @@ class Int8FusedUpdateAttentionImpl(Int8AttentionImpl):
         md = attn_metadata
         workspace = md.workspace
         if workspace is None:
-            workspace = self._own_workspace(query, md)
+            workspace, _ = self._own_workspace(query, md)
         _C.binding().decode_with_update(
             query, key, value, output, n, self.num_heads, kv_cache, geom.struct_addr, geom.base_ptr, md.seq_lens,
             md.block_table, md.max_seq_len, self.scale, self._window, self.logits_soft_cap,
