@@ -303,3 +303,48 @@ def test_short_runs_captured_on_their_first_call(gpu_device, hq, hkv, d):
         assert torch.equal(eager, out), f"replay {it}: graph and eager outputs differ"
         want = oracle.paged_attn(qh, T.storage_bytes(kv_cpu), lay, bt, lens_cpu, cu, 0.1, alibi_slopes=slopes)
         T.assert_close_attn(out, want, what=f"short runs, graph replay {it}")
+
+
+@pytest.mark.parametrize("layout", ["NHD", "HND"])
+@pytest.mark.parametrize("qlen", [3, 40])
+def test_capture_after_a_decode_only_warm_up_keeps_the_default_workspace(gpu_device, monkeypatch, layout, qlen):
+    """Without a workspace of its own a call uses the op layer's buffer, which does not grow inside a capture.  What a
+    decode step needs is enough for a captured batch of query runs, short or long, of as many sequences."""
+    dev, hq, hkv, d, bs = gpu_device, 32, 8, 128, 16
+    full = [300, 70, 129, qlen]
+    B = len(full)
+    g = torch.Generator().manual_seed(qlen)
+    kv_cpu, _views, lay = T.cpu_cache(60, bs, hkv, d, layout)
+    bt = T.make_block_tables(full, bs, 60, g)
+    rows = [torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in full]
+    T.fill_cache_from_sources(kv_cpu, lay, bt, full, bs, rows, [r.flip(0) for r in rows])
+    kv = T.to_device_cache(kv_cpu, dev, layout)
+    k, v = L.key_value_views(kv)
+    ksc, vsc = L.scale_views(kv)
+    geom = L.geometry_from_views(k, v, ksc, vsc)
+    cu = torch.arange(0, B * qlen + 1, qlen, dtype=torch.int32)
+    sl = torch.tensor(full, dtype=torch.int32)
+    cu_d, ones_d, bt_d, sl_d = cu.to(dev), torch.arange(B + 1, dtype=torch.int32, device=dev), bt.to(dev), sl.to(dev)
+    q = torch.zeros((B * qlen, hq, d), dtype=torch.bfloat16, device=dev)
+    out = torch.zeros_like(q)
+    monkeypatch.setattr(ops, "_ws_cache", {})
+
+    def step(qq, oo, cuu, n):
+        ops.unified_attention(qq, k, v, oo, cuu, n, sl_d, max(full), 0.1, True, block_table=bt_d, k_scale_cache=ksc,
+                              v_scale_cache=vsc, geometry=geom)
+
+    step(q[:B], torch.empty_like(q[:B]), ones_d, 1)
+    torch.cuda.synchronize()
+    held = ops._ws_cache[q.device].numel()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step(q, out, cu_d, qlen)
+    assert ops._ws_cache[q.device].numel() == held
+    for it in range(3):
+        qh = torch.randn(q.shape, generator=g).to(torch.bfloat16)
+        q.copy_(qh.to(dev))
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        want = oracle.paged_attn(qh, T.storage_bytes(kv_cpu), lay, bt, sl, cu, 0.1)
+        T.assert_close_attn(out, want, what=f"replay {it}")

@@ -272,13 +272,17 @@ def _default_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
 def _attention_workspace(dev: torch.device, num_seqs: int, num_rows: int, num_q_heads: int, geom: CacheGeometry,
                          max_seqlen_q: int, prefill_splits: int) -> tuple[torch.Tensor, bool]:
     """Scratch for an attention call that brought none, and whether the call is one of short runs (for which it then has
-    the room)."""
+    the room).  A capture whose warm-up left too small a buffer for those (decode steps only) keeps the buffer, and the
+    kernels that it is enough for."""
     if max_seqlen_q == 1:
         return _default_workspace(dev, paged_attn_workspace_bytes(num_seqs, num_q_heads, geom.head_size, dev)), False
     need = split_prefill_workspace_bytes(num_seqs, num_q_heads, geom.head_size, num_rows, prefill_splits, dev)
     short = 0
     if geom.stride_slot == geom.record_bytes:
         short = short_runs_workspace_bytes(num_seqs, num_q_heads, geom.num_kv_heads, geom.head_size, max_seqlen_q, dev)
+    have = _ws_cache.get(dev)
+    if short > need and (have is None or have.numel() < short) and torch.cuda.is_current_stream_capturing():
+        short = 0
     return _default_workspace(dev, max(need, short)), short > 0
 
 
@@ -340,7 +344,8 @@ def unified_attention(
     ``short_runs=True``, for a caller that brings a workspace: a batch whose longest run is short (a
     speculative-decoding step) is served by one launch over all its sequences, on a head-major cache.  The workspace
     must then hold ``short_runs_workspace_bytes(...)``; a smaller one is refused.  Other batches are served as without
-    it.  Without a workspace such a batch always takes that launch."""
+    it.  Without a workspace such a batch takes that launch (inside a stream capture: if the default workspace has
+    grown to its size before)."""
     code_type = code_type_of(kv_quant_mode)
     if output_scale is not None or mm_prefix_range is not None:
         raise NotImplementedError("fused output quantisation and mm-prefix ranges are not built")
