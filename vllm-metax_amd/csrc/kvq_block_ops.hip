@@ -16,8 +16,9 @@ constexpr int kPairsPerLaunch = 480;   // 3840 bytes of kernel arguments, of the
 constexpr int kTriplesPerLaunch = 64;
 constexpr int kSliceBytes = 16384;     // bytes one workgroup moves
 // Workgroups of a launch that crosses PCIe: 64 x 16 KB are requested at a time, several times what the link's
-// latency needs, and three quarters of the compute units stay free for what other streams run meanwhile.  The
-// 2 x 192 blocks above take 300 us with 8 workgroups, 255 with 16, 247 with 32, 239 with 64 or 128, 265 with 1024.
+// latency needs, and three quarters of the compute units stay free for what other streams run meanwhile.  192
+// blocks of 33 KB out and as many back take 300 us with 8 workgroups, 255 with 16, 247 with 32, 239 with 64 or 128,
+// 265 with 1024.
 constexpr int kHostCopyGroups = 64;
 
 struct BlockPairs {

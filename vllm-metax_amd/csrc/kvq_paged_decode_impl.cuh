@@ -11,18 +11,10 @@ namespace kvq {
 
 int heads_per_wg(int num_kv_heads);
 
-// Tiles of a decode sequence: those that hold a token of the row's window,
-// [window_first / 32, ceil(len / 32)).  0 for prefill sequences and empty ones.
-__device__ __forceinline__ int decode_tiles(const int32_t* seq_lens, const int32_t* cu, int s, int num_seqs,
-                                            int window) {
-  // no data-dependent branches: the loads of a lane (and of the lanes' next chunks) all go out
-  // together; a lane past the last sequence rereads the last one and its result is dropped
-  const int sc = s < num_seqs ? s : num_seqs - 1;
-  const int len = seq_lens[sc];
-  int q_len = 1;
-  if (cu != nullptr) q_len = cu[sc + 1] - cu[sc];
-  const int n = (len + kTile - 1) / kTile - window_first(len, window) / kTile;
-  return (s < num_seqs && q_len == 1 && len > 0) ? n : 0;
+// Tiles of a decode sequence of `len` > 0 tokens: those that hold a token of the row's window,
+// [window_first / 32, ceil(len / 32)).
+__device__ __forceinline__ int decode_tiles(int len, int window) {
+  return (len + kTile - 1) / kTile - window_first(len, window) / kTile;
 }
 
 // A sequence's length and its query rows [q0, q1).
@@ -36,9 +28,9 @@ __device__ __forceinline__ SeqRow load_seq(const StreamKArgs& a, int s) {
   r.q1 = a.cu_seqlens_q != nullptr ? a.cu_seqlens_q[s + 1] : s + 1;
   return r;
 }
-// Its tiles as a decode sequence (see decode_tiles).
+// Its tiles as a decode sequence: 0 for query runs and empty ones (the former are the prefill kernels').
 __device__ __forceinline__ int seq_tiles(const SeqRow& r, int window) {
-  return r.q1 - r.q0 == 1 && r.len > 0 ? (r.len + kTile - 1) / kTile - window_first(r.len, window) / kTile : 0;
+  return r.q1 - r.q0 == 1 && r.len > 0 ? decode_tiles(r.len, window) : 0;
 }
 
 // Batch-invariant cutting (StreamKArgs::fixed_spans): a sequence is cut at places that depend on nothing but its
@@ -58,20 +50,7 @@ __device__ __forceinline__ int fixed_span_count(int ntiles) {
   return (ntiles + per - 1) / per;   // 0 for no tiles
 }
 
-// Units a sequence takes on the work line: its setup charge, then one unit per tile.
-__device__ __forceinline__ int decode_units(const int32_t* seq_lens, const int32_t* cu, int s, int num_seqs,
-                                            int window, int setup) {
-  const int n = decode_tiles(seq_lens, cu, s, num_seqs, window);
-  return n > 0 ? n + setup : 0;
-}
-// Units of a sequence on the line the launch cuts: tiles + setup charge, or (FIXED) its spans.
-template <bool FIXED>
-__device__ __forceinline__ int line_units(const int32_t* seq_lens, const int32_t* cu, int s, int num_seqs, int window,
-                                          int setup) {
-  if constexpr (FIXED) return fixed_span_count(decode_tiles(seq_lens, cu, s, num_seqs, window));
-  else return decode_units(seq_lens, cu, s, num_seqs, window, setup);
-}
-
+// Units of a sequence on the line the launch cuts: its setup charge, then one per tile, or (FIXED) its spans.
 template <bool FIXED>
 __device__ __forceinline__ int seq_line_units(const SeqRow& r, int window, int setup) {
   const int n = seq_tiles(r, window);
@@ -79,39 +58,47 @@ __device__ __forceinline__ int seq_line_units(const SeqRow& r, int window, int s
   else return n > 0 ? n + setup : 0;
 }
 
+// The same for sequence s, 0 past the last.  No branch on it: a lane past the last sequence rereads the last one and drops
+// the result, so that the loads of a lane's chunks all go out together.
+template <bool FIXED>
+__device__ __forceinline__ int line_units(const StreamKArgs& a, int s) {
+  const int n = seq_line_units<FIXED>(load_seq(a, min(s, a.num_seqs - 1)), a.io.window, a.setup_units);
+  return s < a.num_seqs ? n : 0;
+}
+
 // The scans over more than 64 sequences work on chunks of 64 (one per lane), kScanBatch chunks per step so that their
 // loads are in flight together (batch 512: 16 dependent round trips -> 4).
 constexpr int kScanBatch = 4;
 
 // Total units of the work line.
-template <int BATCH, bool FIXED = false>
+template <bool FIXED>
 __device__ __forceinline__ int64_t scan_total(const StreamKArgs& a, int lane) {
   const int B = a.num_seqs;
   int64_t total = 0;
-  for (int base = 0; base < B; base += kWave * BATCH) {
-    int n[BATCH];
+  for (int base = 0; base < B; base += kWave * kScanBatch) {
+    int n[kScanBatch];
 #pragma unroll
-    for (int j = 0; j < BATCH; ++j)
-      n[j] = line_units<FIXED>(a.seq_lens, a.cu_seqlens_q, base + kWave * j + lane, B, a.io.window, a.setup_units);
+    for (int j = 0; j < kScanBatch; ++j)
+      n[j] = line_units<FIXED>(a, base + kWave * j + lane);
 #pragma unroll
-    for (int j = 0; j < BATCH; ++j) total += __builtin_amdgcn_readlane(wave_incl_scan(n[j]), 63);
+    for (int j = 0; j < kScanBatch; ++j) total += __builtin_amdgcn_readlane(wave_incl_scan(n[j]), 63);
   }
   return total;
 }
 
 // The sequence that holds unit `lo` and the index of its first unit.
-template <int BATCH, bool FIXED = false>
+template <bool FIXED>
 __device__ __forceinline__ void scan_locate(const StreamKArgs& a, int lane, int64_t lo, int& seq, int64_t& seq_start) {
   const int B = a.num_seqs;
   int64_t cum = 0;
   bool found = false;
-  for (int base = 0; base < B && !found; base += kWave * BATCH) {
-    int nn[BATCH];
+  for (int base = 0; base < B && !found; base += kWave * kScanBatch) {
+    int nn[kScanBatch];
 #pragma unroll
-    for (int j = 0; j < BATCH; ++j)
-      nn[j] = line_units<FIXED>(a.seq_lens, a.cu_seqlens_q, base + kWave * j + lane, B, a.io.window, a.setup_units);
+    for (int j = 0; j < kScanBatch; ++j)
+      nn[j] = line_units<FIXED>(a, base + kWave * j + lane);
 #pragma unroll
-    for (int j = 0; j < BATCH; ++j) {
+    for (int j = 0; j < kScanBatch; ++j) {
       const int n = nn[j];
       const int incl = wave_incl_scan(n);
       const int64_t first = cum + incl - n, last = cum + incl;
@@ -169,7 +156,7 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
       incl = wave_incl_scan(n);
       total = __builtin_amdgcn_readlane(incl, 63);
     } else {
-      total = scan_total<kScanBatch, fixed>(a, lane);
+      total = scan_total<fixed>(a, lane);
     }
     // (the batch-invariant line is short -- a unit is a span of at least kMinSpanTiles tiles -- and is always shared
     // out over every workgroup there is a unit for)
@@ -188,7 +175,7 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
       seq_start = __builtin_amdgcn_readlane(incl - n, seq);
       cur = {__builtin_amdgcn_readlane(mine.len, seq), __builtin_amdgcn_readlane(mine.q0, seq), __builtin_amdgcn_readlane(mine.q1, seq)};
     } else {
-      scan_locate<kScanBatch, fixed>(a, lane, lo, seq, seq_start);
+      scan_locate<fixed>(a, lane, lo, seq, seq_start);
       seq = __builtin_amdgcn_readfirstlane(seq);
       cur = load_seq(a, seq);
     }
@@ -255,7 +242,7 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
     // the spans [lo, hi) of the span line, sequence by sequence
     int64_t at = lo;
     while (at < hi && seq < B) {
-      const int ntiles = __builtin_amdgcn_readfirstlane(decode_tiles(a.seq_lens, a.cu_seqlens_q, seq, B, a.io.window));
+      const int ntiles = __builtin_amdgcn_readfirstlane(seq_tiles(load_seq(a, seq), a.io.window));
       const int spans = fixed_span_count(ntiles);
       const int span = (int)(at - seq_start);
       if (span >= spans) {   // also: a sequence without tiles
@@ -343,7 +330,7 @@ __global__ __launch_bounds__(256) void paged_decode_fixed_spans_reduce_kernel(St
   const int len = a.seq_lens[seq];
   if (q1 - q0 != 1) return;
   const int64_t row = q0;
-  const int ntiles = len > 0 ? (len + kTile - 1) / kTile - window_first(len, a.io.window) / kTile : 0;
+  const int ntiles = len > 0 ? decode_tiles(len, a.io.window) : 0;
   if (ntiles == 0) {  // empty sequence: defined output (zeros, lse = -inf)
     for (int i = 0; i < V; ++i)
       store_act_rt(a.io.out_dtype, a.io.out, row * a.io.out_stride_t + (int64_t)head * a.io.out_stride_h + lane * V + i, 0.f);
@@ -439,7 +426,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_kernel(Stream
   if (w == 0 || w >= P) return;
   const int len = a.seq_lens[seq];
   const int64_t row = a.cu_seqlens_q ? a.cu_seqlens_q[seq] : seq;
-  const int ntiles = (len + kTile - 1) / kTile - window_first(len, a.io.window) / kTile;   // a decode sequence with tiles
+  const int ntiles = decode_tiles(len, a.io.window);   // a decode sequence with tiles
   // workgroup holding unit x: the largest w with floor(w*T/P) <= x; the sequence's tiles are units
   // start + setup_units .. start + setup_units + ntiles - 1
   const int w_first = (int)(((start + a.setup_units + 1) * P - 1) / total);
@@ -595,7 +582,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_by_seq_kernel
   const int64_t start = a.seq_first_unit[seq];   // defined for every decode sequence that has a tile
   if (q1 - q0 != 1) return;
   const int64_t row = q0;
-  const int ntiles = len > 0 ? (len + kTile - 1) / kTile - window_first(len, a.io.window) / kTile : 0;
+  const int ntiles = len > 0 ? decode_tiles(len, a.io.window) : 0;
   if (ntiles == 0) {  // empty sequence: defined output (zeros, lse = -inf)
     for (int i = 0; i < V; ++i)
       store_act_rt(a.io.out_dtype, a.io.out, row * a.io.out_stride_t + (int64_t)head * a.io.out_stride_h + lane * V + i, 0.f);
@@ -730,7 +717,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_split4_kernel
   const int64_t start = a.seq_first_unit[seq];   // defined for every decode sequence that has a tile
   if (q1 - q0 != 1) return;                      // every branch down to the barrier is uniform over the block
   const int64_t row = q0;
-  const int ntiles = len > 0 ? (len + kTile - 1) / kTile - window_first(len, a.io.window) / kTile : 0;
+  const int ntiles = len > 0 ? decode_tiles(len, a.io.window) : 0;
   if (ntiles == 0) {  // empty sequence: defined output (zeros, lse = -inf)
     if (part == 0) {
       for (int i = 0; i < V; ++i)
