@@ -644,7 +644,8 @@ KVQ_API int kvq_mla_v_up_proj(void* out, int64_t out_stride_b, int64_t out_strid
  * `causal` is a set of flags: KVQ_MLA_PREFILL_CAUSAL (1), and KVQ_MLA_PREFILL_MERGE
  * (2): out and lse (then required) already hold the rows' attention over OTHER
  * keys, and this call's is merged into it, as kvq_merge_attn_states would with
- * out / lse as one of its two states; rows that see no key here stay as they are.
+ * out / lse as one of its two states (an infinite lse of either sign: no keys);
+ * rows that see no key here stay as they are.
  */
 #define KVQ_MLA_PREFILL_CAUSAL 1
 #define KVQ_MLA_PREFILL_MERGE 2

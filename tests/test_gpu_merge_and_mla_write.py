@@ -135,6 +135,30 @@ def test_mla_gather_and_dequant_bit_exact(gpu_device, dst_dtype, use_starts):
     assert bool(((want - src).abs() <= amax / 127 * 0.5 * (1 + 1e-4)).all())
 
 
+@pytest.mark.parametrize("dst_dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("lead,pad", [(0, 1), (1, 7), (4, 4)])
+def test_mla_gather_into_rows_of_any_alignment(gpu_device, dst_dtype, lead, pad):
+    """Rows that do not begin on 16 bytes are stored element by element: the same values, and nothing beside them."""
+    dev, R, P, bs, nb, ctx = gpu_device, 512, 64, 16, 12, [33, 1, 70]
+    g = torch.Generator().manual_seed(lead)
+    bt = T.make_block_tables(ctx, bs, nb, g)
+    cpu = L.allocate_mla_cache(nb, bs, R + P, device="cpu")
+    codes, scales = L.mla_cache_views(cpu)
+    lay = oracle.MlaLayout.from_views(cpu, codes, scales, R)
+    for c, slots in zip(ctx, T.slots_for(bt, ctx, bs)):
+        oracle.mla_cache_write(torch.randn((c, R), generator=g).to(torch.bfloat16),
+                               torch.randn((c, P), generator=g).to(torch.bfloat16), cpu, lay, slots)
+    cu = torch.tensor([0, 33, 34, 104], dtype=torch.int32)
+    t2s = torch.repeat_interleave(torch.arange(3, dtype=torch.int32), torch.tensor(ctx))
+    want = oracle.mla_gather_dequant(cpu, lay, bt, cu, t2s, 104, None)
+    whole = torch.full((105, lead + R + P + pad), 7.0, dtype=dst_dtype, device=dev)
+    ops.gather_and_maybe_dequant_cache(cpu.to(dev), whole[:, lead:lead + R + P], bt.to(dev), cu.to(dev), t2s.to(dev), 104)
+    torch.cuda.synchronize()
+    got = whole.cpu()
+    assert torch.equal(got[:104, lead:lead + R + P], want.to(dst_dtype))
+    assert bool((got[104] == 7.0).all() and (got[:, :lead] == 7.0).all() and (got[:, lead + R + P:] == 7.0).all())
+
+
 @pytest.mark.parametrize("use_starts", [False, True])
 def test_mla_cp_gather_bit_exact(gpu_device, use_starts):
     """cp_gather_cache over the int8 latent cache (pattern of the reference's

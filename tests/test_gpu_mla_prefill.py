@@ -69,6 +69,54 @@ def test_varlen_attention_matches_fp32_statement(gpu_device, dtype, H, nope, rop
     _check(out, lse, want, want_lse, "varlen attention")
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,nope,rope,dv", [(16, 128, 64, 128), (4, 64, 32, 64)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_merge_into_a_given_state(gpu_device, dtype, H, nope, rope, dv, causal):
+    """``merge_into`` by itself, into rows of a wider buffer: prior states of every weight beside this call's, rows whose
+    prior saw no key (lse -inf, or +inf as some kernels report it) and rows that see none here (no keys, or all above the
+    diagonal), which stay as they are."""
+    dev = gpu_device
+    qlens, klens = [70, 5, 33, 130], [100, 0, 1, 257]
+    q, kv, kpe = _inputs(qlens, klens, H, nope, rope, dv, dtype, seed=14)
+    g = torch.Generator().manual_seed(15)
+    n, scale = sum(qlens), 1.0 / math.sqrt(nope + rope)
+    cu_q, cu_k = _cu(qlens), _cu(klens)
+    here, here_lse = TR.varlen_attn_lse(q, kv[..., :nope], kpe, kv[..., nope:], cu_q, cu_k, scale, causal)
+    prior = torch.randn((n, H, dv), generator=g).to(dtype)
+    prior_lse = torch.randn((H, n), generator=g) * 4 + 3
+    prior_lse[:, ::7] += torch.tensor([-200.0, 200.0])[torch.arange((n + 6) // 7) % 2]     # one side's weight is 0
+    prior_lse[:, 3::11] = -torch.inf
+    prior_lse[:, 4::11] = torch.inf
+    prior[3::11] = 0
+    prior[4::11] = 0
+    # float64: sum of the two states by their weights
+    a, b = prior_lse.double(), here_lse.double()
+    a = torch.where(torch.isinf(a), torch.full_like(a, -torch.inf), a)
+    want_lse = torch.logaddexp(a, b)
+    none = torch.isinf(want_lse)
+    wa = torch.where(none, torch.zeros_like(a), torch.exp(a - want_lse))
+    wb = torch.where(none, torch.zeros_like(a), torch.exp(b - want_lse))
+    want = prior.double() * wa.T[..., None] + here.double() * wb.T[..., None]
+    wide = torch.full((n, H + 1, dv + 8), 5.0, dtype=dtype, device=dev)
+    out = wide[:, 1:, 8:]
+    out.copy_(prior.to(dev))
+    lse = prior_lse.to(dev)
+    kvd = kv.to(dev)
+    ops.mla_prefill_attention(
+        q.to(dev), kvd[..., :nope], kpe.to(dev), kvd[..., nope:], torch.tensor(cu_q, dtype=torch.int32, device=dev),
+        torch.tensor(cu_k, dtype=torch.int32, device=dev), max(qlens), scale, causal, out=out, lse=lse, merge_into=True)
+    torch.cuda.synchronize()
+    T.assert_close_attn(out, want.float(), what="merged state")
+    got_lse = lse.cpu()
+    seen = torch.isfinite(here_lse)
+    torch.testing.assert_close(got_lse[seen].double(), want_lse[seen], atol=5e-3, rtol=1e-3)
+    stay = ~seen
+    assert bool(stay.any()) and torch.equal(got_lse[stay], prior_lse[stay])
+    assert torch.equal(out.cpu().permute(1, 0, 2)[stay], prior.permute(1, 0, 2)[stay])
+    assert bool((wide[:, 0] == 5.0).all() and (wide[:, :, :8] == 5.0).all())
+
+
 def test_prefill_backend_calls_and_given_buffers(gpu_device):
     """run_prefill_new_tokens / run_prefill_context_chunk (prefill/base.py:154-176) with the key as a pair and
     as the concatenated tensor; ``out`` given; many heads and long rows of keys."""

@@ -322,7 +322,8 @@ __global__ __launch_bounds__(256) void varlen_attn_kernel(VarlenArgs a) {
       // The algebra of merge_attn_states, in the epilogue: the other keys' rows are read and the sum is written once.
       // (As a launch of its own the merge read both states and wrote the rows: 46 us of 1352 for 2765 rows x 128 heads.)
       float* const lp = a.lse + (int64_t)head * a.total_q + tok;
-      const float prior = *lp;
+      const float given = *lp;
+      const float prior = given == INFINITY ? -INFINITY : given;   // +inf: no key either, as merge_attn_states reads it
       const float mx = fmaxf(prior, lse);
       if (lse == -INFINITY) continue;   // nothing visible here: the row stands
       const float wp = prior == -INFINITY ? 0.f : __expf(prior - mx), wn = __expf(lse - mx);
