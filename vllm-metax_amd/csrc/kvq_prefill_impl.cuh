@@ -793,15 +793,16 @@ __global__ __launch_bounds__(256) void prefill_split_merge_kernel(PrefillArgs a)
   const float mmax = wave_max(ms);
   const float mref = mmax == -INFINITY ? 0.f : mmax;
   const float es = lane < S ? __builtin_amdgcn_exp2f(ms - mref) : 0.f;   // an empty range: 2^-inf = 0
-  float l = wave_sum(es * ls);
+  float l = wave_sum(es != 0.f ? es * ls : 0.f);
   float acc[V];
 #pragma unroll
   for (int i = 0; i < V; ++i) acc[i] = 0.f;
 #pragma unroll
   for (int s = 0; s < kMaxKSplit; ++s) {
     const float w = as_f32(__builtin_amdgcn_readlane(as_u32(es), s));
+    const uint32_t keep = w != 0.f ? 0xffffffffu : 0u;   // a weight of 0 takes the words out, whatever they hold
 #pragma unroll
-    for (int i = 0; i < V; ++i) acc[i] += w * po[s][i];
+    for (int i = 0; i < V; ++i) acc[i] += w * as_f32(as_u32(po[s][i]) & keep);
   }
   if (l > 0.f) l += sink_term(io.sinks, head, mmax);   // a row without a visible key keeps its zeros
   const float mul = l > 0.f ? 1.0f / l : 0.f;
