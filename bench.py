@@ -675,7 +675,9 @@ def mixed_main(args, cfg, dev, ops):
             "roofline": {"bound": "hbm", "achieved": round(pre_bytes / attn_s / 1e9, 1), "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                          "frac": round(pre_bytes / attn_s / 1e9 / HBM_PEAK_GBPS, 4), "traffic": None,
                          "timing": f"{n_ev} attention launches back to back between two events on the launch stream",
-                         "kernel": "varlen attention launch = prefill_plan_kernel + paged_prefill_kernel (an item's tiles spread over a workgroup's waves)",
+                         "kernel": "varlen attention launch = " + (
+                             "short_runs_streamk_kernel + short_runs_reduce_kernel" if short and args.kv_layout == "HND" else
+                             "prefill_plan_kernel + paged_prefill_kernel (an item's tiles spread over a workgroup's waves)"),
                          "algorithmic_bytes_per_launch": pre_bytes},
         }
         print(json.dumps(res))

@@ -281,8 +281,9 @@ struct LaneOffsets {
 // this shape reach 6.8 TB/s against 6.0 without the hint.  (The hint is wrong for the NHD order: there the 128-byte lines
 // at a record's ends belong half to a neighbouring head's wave, a line that is not kept in L2 is fetched by both, and the
 // rate drops by 9 %.)  The run goes into the window as it is, one 16-byte LDS write per chunk, rows R bytes apart; which
-// token, dims and bytes a lane's operands hold is chosen so that reading that unpadded window is free of bank conflicts
-// (see row_token, k_off, v_off).  Re-pitching the rows on the way in, two 8-byte writes per chunk, took longer than the
+// token, dims and bytes a lane's operands hold is chosen so that reading that unpadded window has few bank conflicts
+// (see row_token, k_off, v_off): SQ_LDS_BANK_CONFLICT counts 34 of the 198 LDS cycles of a wave's tile at head size 128,
+// against 56 of 192 with the padded rows.  Re-pitching the rows on the way in, two 8-byte writes per chunk, took longer than the
 // products: 2.9 of the 6.9 us of a tile at head size 256.
 template <int D, int QDT, int ODT, int CODE = KVQ_CODE_INT8, bool STREAM = false>
 struct DecodeTile {
@@ -327,7 +328,9 @@ struct DecodeTile {
   // ---- which token, dims and bytes an operand lane holds ------------------------------------------------------------
   // Rows of the unpadded window lie R = 2 (DB + 4) bytes apart, 2 dwords modulo the 64 banks for DB = 128 and 256 (34
   // for DB = 64).  With eight tokens in a row per quarter of the wave, a 4-byte V read of 16 consecutive dwords per
-  // token meets every bank once; an 8-byte K read of a half wave does if its two quarters read 32 bytes apart.
+  // token meets every bank once.  An 8-byte K read would if it were served a half wave at a time, whose two quarters read
+  // 32 bytes apart; the counter shows it is not: four conflict cycles per K read (eight of them per tile, four with int4
+  // codes, which counts 18), and none but two more per tile.
   // Token of A row r of M-tile mt.
   __device__ static constexpr int row_token(int mt, int r) { return STREAM ? 8 * (r >> 2) + 4 * mt + (r & 3) : 16 * mt + r; }
   // Token of S element i of M-tile mt in quarter g (rows 4 g + i), the first of four in a row.
