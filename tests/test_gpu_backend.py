@@ -202,3 +202,30 @@ def test_verify_steps_through_the_builder_take_one_launch_at_every_batch_size(gp
     assert same, "not the launch that was asked for"
     want = oracle.paged_attn(q.view(-1, hq, d), T.storage_bytes(kv_cpu), lay, bt, torch.tensor(ctx, dtype=torch.int32), cu, 0.09)
     T.assert_close_attn(out.view(-1, hq, d), want, what=f"verify step of {n} sequences")
+
+
+@pytest.mark.parametrize("flat", [True, False])
+def test_layer_rotates_and_updates_the_cache_in_one_call(gpu_device, flat):
+    """do_rope_and_kv_cache_update, which fused_rope_kvcache_supported announces: the layer's tensors as it holds them,
+    rotated in place and written as the op does (which is tested against the oracle)."""
+    dev, hq, hkv, d, bs, n = gpu_device, 32, 8, 128, 16, 21
+    g = torch.Generator().manual_seed(3)
+    impl = Int8AttentionBackend.get_impl_cls()(hq, d, 0.09, hkv, kv_cache_dtype="int8_per_token_head")
+    assert impl.fused_rope_kvcache_supported()
+    q, k, v = (torch.randn((n, h, d), generator=g).to(torch.bfloat16).to(dev) for h in (hq, hkv, hkv))
+    ang = torch.rand((50, 64), generator=g) * 6.283
+    cos_sin = torch.cat([ang.cos(), ang.sin()], dim=1).to(torch.bfloat16).to(dev)
+    positions = torch.randint(0, 50, (n,), generator=g).to(dev)
+    slots = torch.randperm(4 * bs, generator=g)[:n].to(dev)
+    caches = [L.allocate_kv_cache(4, bs, hkv, d, device=dev, fill=0) for _ in range(2)]
+    impl._ensure_scale_caches(caches[1])
+    kc, vc = L.key_value_views(caches[1])
+    ks, vs = L.scale_views(caches[1])
+    q2, k2 = q.clone(), k.clone()
+    ops.rope_and_cache_per_token_head_quant(positions, q2, k2, v, cos_sin, True, kc, vc, ks, vs, slots)
+    args = [t.view(n, -1) if flat else t for t in (q, k, v)]
+    impl.do_rope_and_kv_cache_update(types.SimpleNamespace(), *args, positions, cos_sin, True, caches[0], slots)
+    torch.cuda.synchronize()
+    assert torch.equal(q, q2) and torch.equal(k, k2)
+    same = torch.equal(T.storage_bytes(caches[0]), T.storage_bytes(caches[1]))
+    assert same, "cache bytes differ"

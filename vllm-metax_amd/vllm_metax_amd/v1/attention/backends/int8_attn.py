@@ -362,11 +362,17 @@ class Int8AttentionImpl(_ImplBase):
         embedding and the cache update are one launch."""
         return True
 
-    def do_rope_and_kv_cache_update(self, layer, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor,
-                                    positions: torch.Tensor, cos_sin_cache: torch.Tensor, is_neox: bool,
-                                    kv_cache: torch.Tensor, layer_slot_mapping: torch.Tensor) -> None:
+    def do_rope_and_kv_cache_update(self, layer=None, query: torch.Tensor | None = None, key: torch.Tensor | None = None,
+                                    value: torch.Tensor | None = None, positions: torch.Tensor | None = None,
+                                    cos_sin_cache: torch.Tensor | None = None, is_neox: bool = True,
+                                    kv_cache: torch.Tensor | None = None,
+                                    layer_slot_mapping: torch.Tensor | None = None) -> None:
         """Signature of triton_attn.py:836-848.  ``query`` / ``key`` ``[T, H * D]`` or ``[T, H, D]`` are rotated in
-        place, the rotated ``key`` and ``value`` quantised into ``kv_cache``."""
+        place, the rotated ``key`` and ``value`` quantised into ``kv_cache``.  Without a step's tensors it raises
+        ``NotImplementedError``, as the reference's does."""
+        if any(t is None for t in (query, key, value, positions, cos_sin_cache, kv_cache, layer_slot_mapping)):
+            raise NotImplementedError("do_rope_and_kv_cache_update needs query, key, value, positions, cos_sin_cache, "
+                                      "kv_cache and layer_slot_mapping")
         if self.attn_type in (AttentionType.ENCODER_ONLY, AttentionType.ENCODER):
             return
         key_cache, value_cache = self._pth_key_value_caches(kv_cache)
@@ -427,9 +433,6 @@ class Int8AttentionImpl(_ImplBase):
         self._ensure_scale_caches(kv_cache)
         geom = self._geometry
         _C.binding().cache_update(key, value, kv_cache, slot_mapping, geom.struct_addr, geom.base_ptr)
-
-    def do_rope_and_kv_cache_update(self, *args, **kwargs):
-        raise NotImplementedError("fused rope + cache update is not built (the reference raises here too)")
 
     def forward(self, layer, query: torch.Tensor, key: torch.Tensor, value: torch.Tensor, kv_cache: torch.Tensor,
                 attn_metadata: Int8AttentionMetadata | None, output: torch.Tensor,
