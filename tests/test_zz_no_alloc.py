@@ -145,3 +145,37 @@ def test_static_scratch_captured_and_replayed(gpu_device):
         assert torch.equal(lse.view(torch.int32), want_lse.view(torch.int32)), f"replay {it}: lse differs"
         ref = oracle.paged_attn(qh, T.storage_bytes(kv_cpu), lay, bt, sl_cpu, cu, scale)
         T.assert_close_attn(out, ref, what=f"static scratch graph replay {it}")
+
+
+@pytest.mark.parametrize("qlen,fits", [(2, True), (4, False)])
+def test_static_scratch_serves_short_runs_where_their_states_fit(gpu_device, qlen, fits):
+    """The op with ``static_scratch``: a batch of short runs takes the launch for them if the array holds what that
+    launch asks for at these head counts, else the decode and prefill kernels; the bits are those of the same launch in
+    a workspace."""
+    dev, hq, hkv, d, bs, scale = gpu_device, 32, 8, 128, 16, 0.09
+    ctx = [1500, 33, 640, qlen, 300]
+    g = torch.Generator().manual_seed(qlen)
+    kv_cpu, _, lay = T.cpu_cache(200, bs, hkv, d, "HND")
+    bt = T.make_block_tables(ctx, bs, 200, g)
+    rows = [torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in ctx]
+    T.fill_cache_from_sources(kv_cpu, lay, bt, ctx, bs, rows, [r.flip(0) for r in rows])
+    kv = T.to_device_cache(kv_cpu, dev, "HND")
+    k, v = L.key_value_views(kv)
+    ks, vs = L.scale_views(kv)
+    q = torch.randn((len(ctx) * qlen, hq, d), generator=g).to(torch.bfloat16)
+    sl = torch.tensor(ctx, dtype=torch.int32)
+    cu = torch.arange(0, len(ctx) * qlen + 1, qlen, dtype=torch.int32)
+    short = ops.short_runs_workspace_bytes(len(ctx), hq, hkv, d, qlen)
+    assert (short <= _C.load().kvq_paged_attn_static_scratch_bytes()) is fits
+
+    def call(**kw):
+        out = torch.full(q.shape, float("nan"), dtype=torch.bfloat16, device=dev)
+        ops.unified_attention(q.to(dev), k, v, out, cu.to(dev), qlen, sl.to(dev), max(ctx), scale, True,
+                              block_table=bt.to(dev), k_scale_cache=ks, v_scale_cache=vs, **kw)
+        torch.cuda.synchronize()
+        return out
+
+    got = call(static_scratch=True)
+    same = torch.equal(got, call(workspace=torch.empty(short, dtype=torch.uint8, device=dev), short_runs=fits))
+    assert same, "not the launch that was expected"
+    T.assert_close_attn(got, oracle.paged_attn(q, T.storage_bytes(kv_cpu), lay, bt, sl, cu, scale), what="static scratch")

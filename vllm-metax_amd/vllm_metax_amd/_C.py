@@ -17,6 +17,7 @@ BINDING_PATH = os.path.join(_LIB_DIR, "kvq_torch.so")   # csrc/kvq_torch.cpp
 KVQ_F32, KVQ_BF16, KVQ_F16 = 0, 1, 2
 KVQ_CODE_INT8, KVQ_CODE_FP8_E4M3, KVQ_CODE_INT4 = 0, 1, 2
 KVQ_ATTN_CAUSAL, KVQ_ATTN_NO_DECODE_ROWS, KVQ_ATTN_SHORT_RUNS = 1, 2, 4
+KVQ_STATIC_SCRATCH_BYTES = 24 << 20
 ABI_VERSION = 21
 
 

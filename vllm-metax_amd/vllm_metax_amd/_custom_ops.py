@@ -269,6 +269,13 @@ def _default_workspace(dev: torch.device, nbytes: int) -> torch.Tensor:
     return cur
 
 
+def _short_runs_room(dev: torch.device, num_seqs: int, num_q_heads: int, geom: CacheGeometry, max_seqlen_q: int) -> int:
+    """Bytes with which the launch for short runs serves this batch on this cache; 0 where it does not."""
+    if max_seqlen_q < 2 or geom.stride_slot != geom.record_bytes:
+        return 0
+    return short_runs_workspace_bytes(num_seqs, num_q_heads, geom.num_kv_heads, geom.head_size, max_seqlen_q, dev)
+
+
 def _attention_workspace(dev: torch.device, num_seqs: int, num_rows: int, num_q_heads: int, geom: CacheGeometry,
                          max_seqlen_q: int, prefill_splits: int) -> tuple[torch.Tensor, bool]:
     """Scratch for an attention call that brought none, and whether the call is one of short runs (for which it then has
@@ -277,9 +284,7 @@ def _attention_workspace(dev: torch.device, num_seqs: int, num_rows: int, num_q_
     if max_seqlen_q == 1:
         return _default_workspace(dev, paged_attn_workspace_bytes(num_seqs, num_q_heads, geom.head_size, dev)), False
     need = split_prefill_workspace_bytes(num_seqs, num_q_heads, geom.head_size, num_rows, prefill_splits, dev)
-    short = 0
-    if geom.stride_slot == geom.record_bytes:
-        short = short_runs_workspace_bytes(num_seqs, num_q_heads, geom.num_kv_heads, geom.head_size, max_seqlen_q, dev)
+    short = _short_runs_room(dev, num_seqs, num_q_heads, geom, max_seqlen_q)
     have = _ws_cache.get(dev)
     if short > need and (have is None or have.numel() < short) and torch.cuda.is_current_stream_capturing():
         short = 0
@@ -345,7 +350,7 @@ def unified_attention(
     speculative-decoding step) is served by one launch over all its sequences, on a head-major cache.  The workspace
     must then hold ``short_runs_workspace_bytes(...)``; a smaller one is refused.  Other batches are served as without
     it.  Without a workspace such a batch takes that launch (inside a stream capture: if the default workspace has
-    grown to its size before)."""
+    grown to its size before; with ``static_scratch``: if the library's array is as large as it asks for)."""
     code_type = code_type_of(kv_quant_mode)
     if output_scale is not None or mm_prefix_range is not None:
         raise NotImplementedError("fused output quantisation and mm-prefix ranges are not built")
@@ -382,7 +387,8 @@ def unified_attention(
         raise RuntimeError("q/out must be [num_tokens, num_q_heads, head_size] matching the cache head size")
     num_seqs = seqused_k.shape[0]
     if static_scratch:
-        workspace, prefill_splits, short_runs = None, 1, False
+        workspace, prefill_splits = None, 1
+        short_runs = 0 < _short_runs_room(dev, max(num_seqs, 1), q.shape[1], geom, int(max_seqlen_q)) <= _C.KVQ_STATIC_SCRATCH_BYTES
     elif workspace is None and num_seqs > 0 and q.shape[0] > 0:
         workspace, short_runs = _attention_workspace(dev, num_seqs, q.shape[0], q.shape[1], geom, int(max_seqlen_q),
                                                      prefill_splits)
