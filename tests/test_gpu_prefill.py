@@ -468,3 +468,49 @@ def test_short_runs_are_asked_for_and_do_not_depend_on_the_workspace(gpu_device,
         assert same, f"the bits depend on the workspace's size {kw}"
         with pytest.raises(RuntimeError, match="workspace"):
             call(exact - 1, **kw)
+
+
+@pytest.mark.parametrize("hq,hkv,d,bs,layout,code,shift", [
+    (32, 8, 128, 16, "HND", "int8", 0),
+    (28, 4, 128, 48, "NHD", "int8", 4),      # a block that is no whole number of tiles; records 4 bytes off
+    (32, 8, 128, 48, "HND", "fp8", 4),
+    (16, 2, 128, 32, "HND", "int4", 0),
+    (8, 8, 64, 16, "NHD", "fp8", 0),
+    (8, 2, 64, 64, "HND", "int4", 4),        # 72-byte records: one load covers a half tile
+    (16, 1, 64, 16, "HND", "int8", 0),
+])
+def test_shared_tile_at_its_edges(gpu_device, hq, hkv, d, bs, layout, code, shift):
+    """The workgroup-shared tile where lengths end at, before and behind a tile, a half tile and a column block, on caches
+    whose base is only 4-byte aligned, with NaN scales and codes in every slot that holds no token."""
+    from vllm_metax_amd.kv_cache_interface import KVQuantMode
+    dev = gpu_device
+    ct = {"int8": oracle.CODE_INT8, "fp8": oracle.CODE_FP8, "int4": oracle.CODE_INT4}[code]
+    ctx = [64, 65, 96, 31, 700, 129, 16, 450]
+    qls = [64, 33, 95, 31, 128, 2, 16, 450]
+    g = torch.Generator().manual_seed(hq + d + bs)
+    nb = sum((c + bs - 1) // bs for c in ctx) + 5
+    kv_cpu, _, lay = T.cpu_cache(nb, bs, hkv, d, layout, code_type=ct)
+    T.storage_bytes(kv_cpu).fill_(0xFF)
+    bt = T.make_block_tables(ctx, bs, nb, g)
+    src = [[torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in ctx] for _ in range(2)]
+    T.fill_cache_from_sources(kv_cpu, lay, bt, ctx, bs, *src, code_type=ct)
+    q = torch.randn((sum(qls), hq, d), generator=g).to(torch.bfloat16)
+    sl = torch.tensor(ctx, dtype=torch.int32)
+    cu = torch.tensor([0] + torch.tensor(qls).cumsum(0).tolist(), dtype=torch.int32)
+    scale = 1 / math.sqrt(d)
+    want, want_lse = oracle.paged_attn(q, T.storage_bytes(kv_cpu), lay, bt, sl, cu, scale, return_lse=True, code_type=ct)
+    kv = T.to_device_cache(kv_cpu, dev, layout, code_type=ct)
+    flat = torch.full((T.storage_bytes(kv).numel() + 16,), 0xFF, dtype=torch.uint8, device=dev)
+    flat[shift:shift + T.storage_bytes(kv).numel()] = T.storage_bytes(kv)
+    kv = flat.view(kv.dtype).as_strided(kv.shape, kv.stride(), shift // kv.element_size())
+    k, v = L.key_value_views(kv)
+    ks, vs = L.scale_views(kv)
+    for splits in (1, 3):
+        out = torch.full(q.shape, float("nan"), dtype=torch.bfloat16, device=dev)
+        lse = torch.full(q.shape[:2], float("nan"), dtype=torch.float32, device=dev)
+        ops.unified_attention(q.to(dev), k, v, out, cu.to(dev), max(qls), sl.to(dev), max(ctx), scale, True,
+                              block_table=bt.to(dev), k_scale_cache=ks, v_scale_cache=vs, lse=lse, prefill_splits=splits,
+                              kv_quant_mode=getattr(KVQuantMode, code.upper() + "_PER_TOKEN_HEAD"))
+        torch.cuda.synchronize()
+        T.assert_close_attn(out, want, what=f"shared tile {code} d{d}, {splits} ranges")
+        torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)

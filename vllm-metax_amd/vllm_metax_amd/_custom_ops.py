@@ -411,11 +411,11 @@ def split_prefill_workspace_bytes(max_num_seqs: int, num_q_heads: int, head_size
 
 
 def prefill_context_splits(query_lens, max_seq_len: int, num_q_heads: int, num_kv_heads: int, num_cus: int = 256,
-                           max_split_tokens: int = 4096) -> int:
+                           max_split_tokens: int = 4096, places_per_cu: int = 2) -> int:
     """How many context splits a launch should ask for, from what a metadata builder knows on the host: the query
     run lengths of the batch (``query_lens``: a list or CPU tensor; one-token runs do not count), the longest
     sequence, the head counts.  A run of q tokens makes ceil(q / (128 / group)) x Hkv workgroups of the
-    workgroup-shared tile; when the launch's workgroups do not fill the chip's two per compute unit and the context
+    workgroup-shared tile; when the launch's workgroups do not fill ``places_per_cu`` per compute unit and the context
     is long, the context is cut so that they do -- as long as the partial states stay small (splits x run tokens
     <= ``max_split_tokens``)."""
     group = max(1, num_q_heads // max(1, num_kv_heads))
@@ -425,7 +425,7 @@ def prefill_context_splits(query_lens, max_seq_len: int, num_q_heads: int, num_k
         return 1
     q_tokens = max(1, 128 // group)
     wgs = sum((x + q_tokens - 1) // q_tokens for x in runs) * num_kv_heads
-    splits = min(8, (2 * num_cus) // max(1, wgs), max_split_tokens // max(1, sum(runs)), max_seq_len // 2048)
+    splits = min(8, (places_per_cu * num_cus) // max(1, wgs), max_split_tokens // max(1, sum(runs)), max_seq_len // 2048)
     return max(1, splits)
 
 

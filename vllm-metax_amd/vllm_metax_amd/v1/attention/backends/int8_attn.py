@@ -164,9 +164,10 @@ class Int8AttentionMetadataBuilder(_BuilderBase):
             qlens = qsl_cpu[1:] - qsl_cpu[:-1]
             has_decode_rows = bool((qlens == 1).any())
             # a launch whose long runs make too few workgroups for the chip walks a long context in context splits;
-            # the partial states are indexed by the query row, so every row of the batch counts against the room
+            # the partial states are indexed by the query row, so every row of the batch counts against the room.
+            # Three workgroups of that tile share a compute unit (512 tokens on 32k cached ones: four ranges 370 us, six 351)
             prefill_splits = ops.prefill_context_splits(qlens, int(c.max_seq_len), self.num_heads_q, self.num_heads_kv,
-                                                        max_split_tokens=self.MAX_SPLIT_TOKENS)
+                                                        max_split_tokens=self.MAX_SPLIT_TOKENS, places_per_cu=3)
             while prefill_splits > 1 and prefill_splits * int(c.num_actual_tokens) > self.MAX_SPLIT_TOKENS:
                 prefill_splits -= 1
         workspace = self._get_workspace()
