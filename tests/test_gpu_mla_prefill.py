@@ -70,6 +70,33 @@ def test_varlen_attention_matches_fp32_statement(gpu_device, dtype, H, nope, rop
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("nope,rope,dv", [(128, 64, 128), (64, 32, 64), (128, 0, 128)])
+@pytest.mark.parametrize("causal,qlens,klens", [
+    (True, [1, 31, 32, 33, 127, 129, 300], None),
+    (False, [1, 31, 32, 33, 127, 129, 300], [64, 33, 1, 0, 31, 95, 32]),    # keys that end at, before and behind a tile
+])
+def test_a_launch_that_fills_the_chip_has_the_bits_of_a_small_one(gpu_device, dtype, nope, rope, dv, causal, qlens, klens):
+    """128 heads take the kernel with three workgroups per compute unit, eight of the same heads the one with two: the fp32
+    statement for both, and the same bits in the rows and LSE they share."""
+    dev, H, few = gpu_device, 128, 8
+    klens = klens or qlens
+    q, kv, kpe = _inputs(qlens, klens, H, nope, rope, dv, dtype, seed=17)
+    scale = 1.0 / math.sqrt(nope + rope)
+    cu_q, cu_k = _cu(qlens), _cu(klens)
+    qd, kvd, kped = q.to(dev), kv.to(dev), kpe.to(dev) if rope else None
+    cq, ck = (torch.tensor(x, dtype=torch.int32, device=dev) for x in (cu_q, cu_k))
+    out, lse = ops.mla_prefill_attention(qd, kvd[..., :nope], kped, kvd[..., nope:], cq, ck, max(qlens), scale, causal,
+                                         return_softmax_lse=True)
+    some, some_lse = ops.mla_prefill_attention(qd[:, :few].contiguous(), kvd[:, :few, :nope], kped, kvd[:, :few, nope:], cq, ck,
+                                               max(qlens), scale, causal, return_softmax_lse=True)
+    torch.cuda.synchronize()
+    assert torch.equal(out[:, :few].contiguous().view(torch.int16), some.view(torch.int16))
+    assert torch.equal(lse[:few], some_lse)
+    want, want_lse = TR.varlen_attn_lse(q[:, :few], kv[:, :few, :nope], kpe, kv[:, :few, nope:], cu_q, cu_k, scale, causal)
+    _check(some, some_lse, want, want_lse, "varlen attention, few heads")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("H,nope,rope,dv", [(16, 128, 64, 128), (4, 64, 32, 64)])
 @pytest.mark.parametrize("causal", [False, True])
 def test_merge_into_a_given_state(gpu_device, dtype, H, nope, rope, dv, causal):
