@@ -28,8 +28,9 @@ extern "C" {
 #endif
 
 /* 20: kvq_mla_prefill_attn takes `causal` as a set of flags (any non-zero value meant causal up to 18; 2 is a flag of
- * its own since 19, which other builds of 19 may not know).  21: KVQ_ATTN_SHORT_RUNS and its workspace query. */
-#define KVQ_ABI_VERSION 21
+ * its own since 19, which other builds of 19 may not know).  21: KVQ_ATTN_SHORT_RUNS and its workspace query.  22:
+ * KVQ_ATTN_SHORT_CONTEXT and the fused write's form with flags. */
+#define KVQ_ABI_VERSION 22
 
 #define KVQ_OK 0
 #define KVQ_EINVAL (-22)
@@ -93,6 +94,9 @@ typedef struct kvq_cache_geom {
 #define KVQ_ATTN_CAUSAL 1
 #define KVQ_ATTN_NO_DECODE_ROWS 2
 #define KVQ_ATTN_SHORT_RUNS 4
+#define KVQ_ATTN_SHORT_CONTEXT 16
+/* tokens up to which a caller sets it */
+#define KVQ_SHORT_CONTEXT 1024
 
 /* Byte geometry of the int8 MLA latent cache: per block, block_size code rows
  * of (kv_lora_rank + rope_dim) bytes followed by block_size fp32 scales. */
@@ -233,6 +237,11 @@ KVQ_API int kvq_rope_and_cache_int8(const int64_t* positions, void* query, int64
  * For any other batch the flag changes nothing.  Without it such a batch goes through the decode and prefill
  * kernels, whatever the workspace's size; the results agree within the tolerance, not bit for bit.
  *
+ * KVQ_ATTN_SHORT_CONTEXT (16): the caller takes the batch's sequences to be no longer than KVQ_SHORT_CONTEXT tokens.
+ * The one-row sequences of a small batch (num_seqs x kv heads <= compute units) are then computed by a workgroup per
+ * (sequence, kv head), which leaves no partial states to merge.  It decides the launch, never the result: longer
+ * sequences -- a captured launch replayed later in the conversation -- come out right as well, only slower.
+ *
  * Value range: the weights enter the second product as fp16 numbers
  * p * v_scale * 2^8, so a V row whose scale exceeds 255.8 (int8 codes: absmax
  * above 32 500; fp8 codes: above 114 000) is attended as if its scale were 255.8.
@@ -304,6 +313,19 @@ KVQ_API int kvq_paged_attn_int8_fused_write(void* out, int out_dtype, int64_t ou
                         int num_seqs, int num_q_heads, float scale, int window_size,
                         float softcap, const float* sinks, const float* alibi_slopes, float* lse, void* workspace, size_t workspace_bytes,
                         kvq_stream_t stream);
+
+/* The same with flags: 0 or KVQ_ATTN_SHORT_CONTEXT. */
+KVQ_API int kvq_paged_attn_int8_fused_write_flags(void* out, int out_dtype, int64_t out_stride_t, int64_t out_stride_h,
+                        const void* q, int q_dtype, int64_t q_stride_t, int64_t q_stride_h,
+                        const void* key, const void* value, int src_dtype,
+                        int64_t key_stride_t, int64_t key_stride_h,
+                        int64_t value_stride_t, int64_t value_stride_h, float eps,
+                        void* cache, const kvq_cache_geom* geom,
+                        const int32_t* block_table, int64_t bt_stride, const int32_t* seq_lens,
+                        const int64_t* slot_mapping,
+                        int num_seqs, int num_q_heads, float scale, int window_size,
+                        float softcap, const float* sinks, const float* alibi_slopes, float* lse, void* workspace, size_t workspace_bytes,
+                        int flags, kvq_stream_t stream);
 
 /*
  * kvq_paged_attn_int8 for callers that cannot hand over a workspace they allocated:

@@ -354,3 +354,49 @@ def test_value_magnitudes_far_from_one(gpu_device, vmag, ctx, rel):
     got = run_unified(gpu_device, kv, "NHD", bt, q, sl, cu, scale, out_dtype=torch.float32)
     mag = float(want.abs().max())
     assert float((got.cpu() - want).abs().max()) <= rel * mag, (float((got.cpu() - want).abs().max()), mag)
+
+
+@pytest.mark.parametrize("form,layout,hq,hkv,d,ctx,window,softcap,stated", [
+    ("int8", "NHD", 32, 8, 128, [1, 0, 31, 32, 33, 255, 256, 257, 1024], 0, 0.0, None),   # a tile per wave, one more, the last allowed
+    ("int8", "HND", 28, 4, 128, [512] * 63 + [7], 0, 0.0, None),                          # 256 workgroups, one per compute unit
+    ("int8", "HND", 28, 4, 128, [300] * 65, 0, 0.0, None),                                # 260: the sequences are cut again
+    ("fp8", "HND", 16, 8, 256, [500, 3, 999], 100, 50.0, None),
+    ("int4", "HND", 16, 1, 128, [288, 290, 64, 1000], 0, 0.0, None),
+    ("int8", "NHD", 16, 2, 64, [700, 40, 2500], 1024, 0.0, None),                         # the window bounds the work, not the length
+    ("int8", "HND", 32, 8, 128, [3000, 20], 0, 0.0, 1024),                                # longer than the call says
+])
+def test_whole_sequences(gpu_device, form, layout, hq, hkv, d, ctx, window, softcap, stated):
+    """Short sequences of a small batch: a workgroup per (sequence, kv head), no partial states.  The workspace is
+    filled with NaN bytes, so a merge would show."""
+    from vllm_metax_amd.kv_cache_interface import KVQuantMode
+    g = torch.Generator().manual_seed(d + len(ctx))
+    bs = 16
+    nb = sum((c + bs - 1) // bs for c in ctx) + 5
+    code = {"int8": oracle.CODE_INT8, "fp8": oracle.CODE_FP8, "int4": oracle.CODE_INT4}[form]
+    mode = {"int8": KVQuantMode.INT8_PER_TOKEN_HEAD, "fp8": KVQuantMode.FP8_PER_TOKEN_HEAD,
+            "int4": KVQuantMode.INT4_PER_TOKEN_HEAD}[form]
+    kv, _, lay = T.cpu_cache(nb, bs, hkv, d, layout, code_type=code)
+    T.storage_bytes(kv).fill_(0xFF)
+    bt = T.make_block_tables(ctx, bs, nb, g)
+    ks = [torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in ctx]
+    vs = [torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in ctx]
+    T.fill_cache_from_sources(kv, lay, bt, ctx, bs, ks, vs, code_type=code)
+    q = torch.randn((len(ctx), hq, d), generator=g).to(torch.bfloat16)
+    sl, cu = torch.tensor(ctx, dtype=torch.int32), torch.arange(len(ctx) + 1, dtype=torch.int32)
+    want, want_lse = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, 1 / math.sqrt(d), return_lse=True,
+                                       sliding_window=window, soft_cap=softcap, code_type=code)
+    dev = gpu_device
+    kvd = T.to_device_cache(kv, dev, layout, code_type=code)
+    kd, vd = L.key_value_views(kvd)
+    ksd, vsd = L.scale_views(kvd)
+    out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=dev)
+    lse = torch.full(q.shape[:2], float("nan"), dtype=torch.float32, device=dev)
+    ws = torch.full((ops.paged_attn_workspace_bytes(len(ctx), hq, d, dev),), 0xFF, dtype=torch.uint8, device=dev)
+    ops.unified_attention(q.to(dev), kd, vd, out, cu.to(dev), 1, sl.to(dev), stated or max(ctx), 1 / math.sqrt(d), True,
+                          window_size=(window - 1, 0) if window else (-1, -1), softcap=softcap, block_table=bt.to(dev),
+                          k_scale_cache=ksd, v_scale_cache=vsd, lse=lse, workspace=ws, kv_quant_mode=mode)
+    torch.cuda.synchronize()
+    T.assert_close_attn(out, want, atol=2e-3, rtol=2e-3, what=f"{form} ctx={ctx[:5]}")
+    torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)
+    if len(ctx) * hkv <= 256:
+        assert bool((ws == 0xFF).all()), "the launch left partial states"

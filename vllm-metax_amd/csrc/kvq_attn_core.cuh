@@ -1057,6 +1057,7 @@ struct StreamKArgs {
   // != 0: the batch-invariant cutting (every sequence cut by its own length alone); the partial states then take
   // kFixedSpans slots per sequence and wg_info / seq_first_unit are not used
   int fixed_spans;
+  int whole;         // != 0: no cutting, a workgroup per (sequence, kv head) (whole_sequences)
   int setup_units;   // units a sequence is charged on the balanced work line before its tiles
 };
 

@@ -15,6 +15,7 @@ int launch_decode_streamk(const StreamKArgs& a, int q_dtype, int out_dtype, hipS
 size_t streamk_workspace_bytes(int max_num_seqs, int num_q_heads, int head_size, int num_wg);
 size_t streamk_slots(int max_num_seqs, int num_wg);
 int decode_streamk_num_wg(int num_kv_heads);
+bool whole_sequences(int num_seqs, int num_kv_heads, int num_cus, bool short_context);
 int validate_common(const char* op, const void* q, const void* cache, const kvq_cache_geom* geom,
                     const int32_t* block_table, const int32_t* seq_lens, int num_seqs, int num_q_heads);
 int launch_prefill(const AttnIO& io, const int32_t* seq_lens, const int32_t* cu_seqlens_q, int num_seqs,
@@ -81,10 +82,12 @@ static int paged_attn_launch(const char* op, void* out, int out_dtype, int64_t o
                              int num_tokens = 0) {
   int rc0 = validate_common(op, q, cache, geom, block_table, seq_lens, num_seqs, num_q_heads);
   if (rc0) return rc0;
-  KVQ_REQUIRE((causal & ~(KVQ_ATTN_CAUSAL | KVQ_ATTN_NO_DECODE_ROWS | KVQ_ATTN_SHORT_RUNS)) == 0,
+  KVQ_REQUIRE((causal & ~(KVQ_ATTN_CAUSAL | KVQ_ATTN_NO_DECODE_ROWS | KVQ_ATTN_SHORT_RUNS | KVQ_ATTN_SHORT_CONTEXT)) == 0,
               "%s: unknown flag in causal (%d)", op, causal);
   const bool no_decode_rows = (causal & KVQ_ATTN_NO_DECODE_ROWS) != 0;
   const bool want_short_runs = (causal & KVQ_ATTN_SHORT_RUNS) != 0;
+  // (a window bounds a decode row's tokens as well as the sequence's length does)
+  const bool short_context = (causal & KVQ_ATTN_SHORT_CONTEXT) != 0 || (window_size > 0 && window_size <= KVQ_SHORT_CONTEXT);
   causal &= KVQ_ATTN_CAUSAL;
   KVQ_REQUIRE(out != nullptr, "%s: out is NULL", op);
   KVQ_REQUIRE(max_query_len >= 1, "%s: max_query_len must be >= 1", op);
@@ -144,6 +147,7 @@ static int paged_attn_launch(const char* op, void* out, int out_dtype, int64_t o
   a.num_wg = num_wg;
   const size_t slots = streamk_slots(num_seqs, num_wg);
   a.fixed_spans = batch_invariant() ? 1 : 0;
+  a.whole = whole_sequences(num_seqs, g.num_kv_heads, num_wg, short_context) ? 1 : 0;
   a.part_o = static_cast<float*>(workspace);
   a.part_ml = a.part_o + slots * (size_t)num_q_heads * (size_t)g.head_size;
   // 8-byte aligned: a slot's (D + 2) floats are a multiple of 8 bytes
@@ -236,6 +240,27 @@ extern "C" int kvq_paged_attn_int8_split_prefill(void* out, int out_dtype, int64
                                 prefill_splits, num_tokens);
 }
 
+extern "C" int kvq_paged_attn_int8_fused_write_flags(void* out, int out_dtype, int64_t out_stride_t, int64_t out_stride_h,
+                                               const void* q, int q_dtype, int64_t q_stride_t, int64_t q_stride_h,
+                                               const void* key, const void* value, int src_dtype,
+                                               int64_t key_stride_t, int64_t key_stride_h, int64_t value_stride_t,
+                                               int64_t value_stride_h, float eps, void* cache,
+                                               const kvq_cache_geom* geom, const int32_t* block_table,
+                                               int64_t bt_stride, const int32_t* seq_lens,
+                                               const int64_t* slot_mapping, int num_seqs,
+                                               int num_q_heads, float scale, int window_size, float softcap,
+                                               const float* sinks, const float* alibi_slopes, float* lse, void* workspace, size_t workspace_bytes,
+                                               int flags, kvq_stream_t stream) {
+  using namespace kvq;
+  KVQ_REQUIRE((flags & ~KVQ_ATTN_SHORT_CONTEXT) == 0, "paged_attn_int8_fused_write: unknown flag in flags (%d)", flags);
+  const kvq::NewTokens fresh{key, value, src_dtype, key_stride_t, key_stride_h, value_stride_t, value_stride_h, eps,
+                             slot_mapping};
+  return kvq::paged_attn_launch("paged_attn_int8_fused_write", out, out_dtype, out_stride_t, out_stride_h, q, q_dtype,
+                                q_stride_t, q_stride_h, cache, geom, block_table, bt_stride, seq_lens, nullptr, num_seqs,
+                                num_q_heads, 1, scale, KVQ_ATTN_CAUSAL | flags, window_size, softcap, sinks, alibi_slopes, lse, workspace, workspace_bytes,
+                                "workspace", stream, &fresh);
+}
+
 extern "C" int kvq_paged_attn_int8_fused_write(void* out, int out_dtype, int64_t out_stride_t, int64_t out_stride_h,
                                                const void* q, int q_dtype, int64_t q_stride_t, int64_t q_stride_h,
                                                const void* key, const void* value, int src_dtype,
@@ -247,12 +272,11 @@ extern "C" int kvq_paged_attn_int8_fused_write(void* out, int out_dtype, int64_t
                                                int num_q_heads, float scale, int window_size, float softcap,
                                                const float* sinks, const float* alibi_slopes, float* lse, void* workspace, size_t workspace_bytes,
                                                kvq_stream_t stream) {
-  const kvq::NewTokens fresh{key, value, src_dtype, key_stride_t, key_stride_h, value_stride_t, value_stride_h, eps,
-                             slot_mapping};
-  return kvq::paged_attn_launch("paged_attn_int8_fused_write", out, out_dtype, out_stride_t, out_stride_h, q, q_dtype,
-                                q_stride_t, q_stride_h, cache, geom, block_table, bt_stride, seq_lens, nullptr, num_seqs,
-                                num_q_heads, 1, scale, 1, window_size, softcap, sinks, alibi_slopes, lse, workspace, workspace_bytes,
-                                "workspace", stream, &fresh);
+  return kvq_paged_attn_int8_fused_write_flags(out, out_dtype, out_stride_t, out_stride_h, q, q_dtype, q_stride_t, q_stride_h,
+                                               key, value, src_dtype, key_stride_t, key_stride_h, value_stride_t,
+                                               value_stride_h, eps, cache, geom, block_table, bt_stride, seq_lens,
+                                               slot_mapping, num_seqs, num_q_heads, scale, window_size, softcap, sinks,
+                                               alibi_slopes, lse, workspace, workspace_bytes, 0, stream);
 }
 
 // Also the set-up hook: resolves the array's address on the current device, so that a first call of the

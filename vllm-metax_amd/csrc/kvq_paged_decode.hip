@@ -177,6 +177,19 @@ size_t streamk_workspace_bytes(int max_num_seqs, int num_q_heads, int head_size,
 
 int decode_streamk_num_wg(int num_kv_heads) { return streamk_num_wg(num_kv_heads); }
 
+// Whether a launch's decode sequences are each computed by one workgroup per kv head (paged_decode_whole_kernel) and not
+// cut.  Measured on MI355X through the op, 32 q heads / 8 kv heads of 128, int8 codes, cut / whole:
+//   length        1 sequence of 100: 17.5 / 9.6 us, 337: 17.2 / 12.1, 600: 17.0 / 13.4, 1000: 18.1 / 15.7, 1500: 17.7 / 18.3,
+//                 2000: 18.1 / 20.8 -- a wave's tiles are a serial chain of 1.7 us each, the reduce a fixed cost of 4 - 5;
+//   workgroups    32 sequences of 100 .. 1000: 22.5 / 17.5, 32 of 1000: 26.1 / 20.4 (256 workgroups), but 40: 29.6 / 30.9,
+//                 64 of 100 .. 500: 22.4 / 23.1, 250 of 100 .. 500: 46 / 71 -- past one workgroup per compute unit they
+//                 queue, and the balanced cut has every unit busy as it is.
+// Other forms, same order, 256 workgroups of 100 .. 1000 tokens: head size 256, fp8 codes 40.8 / 29.3; 4 kv heads 22.8 / 17.1; 1 kv head
+// 29.4 / 19.7.  The batch-invariant cutting has its own spans whatever the batch.
+bool whole_sequences(int num_seqs, int num_kv_heads, int num_cus, bool short_context) {
+  return short_context && !batch_invariant() && (int64_t)num_seqs * num_kv_heads <= num_cus;
+}
+
 }  // namespace kvq
 
 extern "C" {

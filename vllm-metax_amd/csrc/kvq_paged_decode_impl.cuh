@@ -313,6 +313,52 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
   }
 }
 
+// A workgroup per (kv head, sequence): its eight waves take the sequence's tiles in turn, their states meet in LDS and
+// the output row is written there and then -- no partial states, no scan of the lengths, no second launch.  For short
+// contexts in a batch that leaves the chip room (whole_sequences): such a step is a chain of latencies, of which the
+// second launch with its round trips to the partial states was the longest link (one sequence of 337 tokens: a step
+// 15.4 -> 11.6 us).  Any length comes out right: a wave goes on until the sequence ends.
+template <int D, int QDT, bool CAP, int CODE, bool STREAM>
+__global__ __launch_bounds__(512) void paged_decode_whole_kernel(StreamKArgs a) {
+  using DTile = DecodeTile<D, QDT, kRuntimeDtype, CODE, STREAM>;
+  constexpr int NSUB = 8;
+  __shared__ __align__(16) uint8_t lds[NSUB][DTile::LDS_WAVE];
+  const int lane = threadIdx.x & 63;
+  const int sub = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hkv = blockIdx.x, seq = blockIdx.y;
+  const LaneOffsets off = DTile::lane_offsets(a.io.g, lane);   // (while the length is on its way)
+  const SeqRow cur = load_seq(a, seq);
+  if (cur.q1 - cur.q0 != 1) return;
+  const int64_t row = cur.q0;
+  if (cur.len <= 0) {   // empty sequence: defined output (zeros, lse = -inf)
+    for (int i = threadIdx.x; i < a.io.group * D; i += kWave * NSUB) {
+      const int head = hkv * a.io.group + i / D;
+      store_act_rt(a.io.out_dtype, a.io.out, row * a.io.out_stride_t + (int64_t)head * a.io.out_stride_h + i % D, 0.f);
+    }
+    if (a.io.lse != nullptr && (int)threadIdx.x < a.io.group)
+      a.io.lse[row * a.io.num_q_heads + hkv * a.io.group + threadIdx.x] = -INFINITY;
+    return;
+  }
+  if (a.k_new != nullptr) {
+    const bool padding = a.new_slots != nullptr && a.new_slots[row] < 0;   // uniform: a scalar load
+    if (sub == 0 && !padding) write_new_token<D>(a, seq, row, cur.len, hkv, lane);
+    // the record is in memory before any wave of the workgroup loads the tile that holds it
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    lds_barrier();
+  }
+  const int first = window_first(cur.len, a.io.window);
+  const int t0 = first / kTile, t_end = t0 + decode_tiles(cur.len, a.io.window);
+  typename DTile::State st;
+  DTile::template run<CAP>(a.io, off, seq, row, cur.len, first, t0, t_end, hkv, lane, lds[sub], st, sub, NSUB);
+  if (sub != 0) DTile::dump_state(st, lane, lds[sub]);
+  lds_barrier();
+  if (sub != 0) return;
+#pragma unroll
+  for (int j = 1; j < NSUB; ++j)
+    if (t0 + j < t_end) DTile::fold_state(st, lane, lds[j]);   // wave j owned a tile
+  DTile::emit_final(a.io, row, hkv, lane, st);
+}
+
 // The merge of the batch-invariant cutting: grid (num_seqs, ceil(Hq / 4)), a wave per q head, a lane owns D / 64
 // dims.  Lane j takes span j's (m, l); the wave agrees on the maximum and the weights; the spans' outputs are added
 // in span order.  Empty decode sequences get their defined output here as well.
@@ -846,6 +892,28 @@ int launch_streamk(const StreamKArgs& args, hipStream_t s) {
   const int hkv = args.io.g.num_kv_heads;
   const int hpw = heads_per_wg(hkv);
   StreamKArgs a = args;
+  // a head's records of a block back to back (HND order): the tile loads may stream past the caches
+  const bool stream = a.io.g.stride_slot == 2 * (code_bytes(a.io.g) + 4) && a.io.g.block_size >= 16;
+  const bool extras = a.io.cap_c != 0.f || a.io.alibi != nullptr;   // the instantiation with soft cap and ALiBi
+  if (a.whole) {
+    const dim3 wgrid(hkv, a.num_seqs);
+#define KVQ_WHOLE_FORM(C, CODE)                                                                                     \
+  do {                                                                                                              \
+    if (stream) hipLaunchKernelGGL((paged_decode_whole_kernel<D, QDT, C, CODE, true>), wgrid, dim3(512), 0, s, a);  \
+    else hipLaunchKernelGGL((paged_decode_whole_kernel<D, QDT, C, CODE, false>), wgrid, dim3(512), 0, s, a);        \
+  } while (0)
+#define KVQ_WHOLE(CODE)                      \
+  do {                                       \
+    if (extras) KVQ_WHOLE_FORM(true, CODE);  \
+    else KVQ_WHOLE_FORM(false, CODE);        \
+  } while (0)
+    if (a.io.g.code_type == KVQ_CODE_FP8_E4M3) KVQ_WHOLE(KVQ_CODE_FP8_E4M3);
+    else if (a.io.g.code_type == KVQ_CODE_INT4) KVQ_WHOLE(KVQ_CODE_INT4);
+    else KVQ_WHOLE(KVQ_CODE_INT8);
+#undef KVQ_WHOLE
+#undef KVQ_WHOLE_FORM
+    return check_hip(hipGetLastError(), "paged_attn_int8 decode launch");
+  }
   a.setup_units = setup_units_for(8 / hpw);
   dim3 grid(a.num_wg, (hkv + hpw - 1) / hpw);
 #define KVQ_SK_FORM(H, C, CODE, S)                                                                                \
@@ -866,9 +934,7 @@ int launch_streamk(const StreamKArgs& args, hipStream_t s) {
     else if (a.io.g.code_type == KVQ_CODE_INT4) KVQ_SK_CODE(H, C, KVQ_CODE_INT4);                                 \
     else KVQ_SK_CODE(H, C, KVQ_CODE_INT8);                                                                        \
   } while (0)
-  // a head's records of a block back to back (HND order): the tile loads may stream past the caches
-  const bool stream = a.io.g.stride_slot == 2 * (code_bytes(a.io.g) + 4) && a.io.g.block_size >= 16;
-  if (a.io.cap_c != 0.f || a.io.alibi != nullptr) {   // the instantiation with the extras: soft cap and ALiBi
+  if (extras) {
     switch (hpw) {
       case 8: KVQ_SK(8, true); break;
       case 4: KVQ_SK(4, true); break;

@@ -190,6 +190,9 @@ PyObject* cache_update(Args& in) {
   Py_RETURN_NONE;
 }
 
+// The flag that tells the library of a batch of short sequences.
+int short_context(int64_t max_k) { return max_k <= KVQ_SHORT_CONTEXT ? KVQ_ATTN_SHORT_CONTEXT : 0; }
+
 // (q, out, rows, num_q_heads, cache, geom, base, cu_seqlens_q, seqused_k, block_table, max_seqlen_q, max_seqlen_k, scale,
 //  flags, window, softcap, sinks, alibi, lse, workspace, splits); rows < 0: all rows of q; num_q_heads: of flat q / out
 PyObject* paged_attention(Args& in) {
@@ -201,7 +204,7 @@ PyObject* paged_attention(Args& in) {
   const at::Tensor &cu = in.ten(), &lens = in.ten(), &table = in.ten();
   const int64_t max_q = in.num(), max_k = in.num();
   const double scale = in.real();
-  const int flags = (int)in.num(), window = (int)in.num();
+  const int flags = (int)in.num() | short_context(max_k), window = (int)in.num();
   const double softcap = in.real();
   const Ten sinks = in.opt(), alibi = in.opt(), lse = in.opt(), ws = in.opt();
   const int splits = (int)in.num();
@@ -298,12 +301,12 @@ PyObject* decode_with_update(Args& in) {
   check_heads(sinks, rq.heads, dev, "sinks");
   check_heads(alibi, rq.heads, dev, "alibi_slopes");
   const int odt = dtype_code(out, "out"), qdt = dtype_code(q, "q"), kdt = dtype_code(key, "key");
-  call(dev, "decode_attention_with_cache_update", kvq_paged_attn_int8_fused_write, ptr(out), odt, ro.stride_t, ro.stride_h,
+  call(dev, "decode_attention_with_cache_update", kvq_paged_attn_int8_fused_write_flags, ptr(out), odt, ro.stride_t, ro.stride_h,
        ptr(q), qdt, rq.stride_t, rq.stride_h, ptr(key), ptr(value), kdt, rk.stride_t, rk.stride_h, rv.stride_t, rv.stride_h,
        eps_of(kdt), const_cast<void*>(base), g, static_cast<const int32_t*>(ptr(table)), table.stride(0),
        static_cast<const int32_t*>(ptr(lens)), static_cast<const int64_t*>(ptr(slots)), (int)B, (int)rq.heads, (float)scale,
        window, (float)softcap, static_cast<const float*>(ptr(sinks)), static_cast<const float*>(ptr(alibi)),
-       static_cast<float*>(ptr(lse)), ptr(ws), ws.nbytes());
+       static_cast<float*>(ptr(lse)), ptr(ws), ws.nbytes(), short_context(max_k));
   Py_RETURN_NONE;
 }
 
