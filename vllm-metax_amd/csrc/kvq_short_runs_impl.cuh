@@ -3,12 +3,12 @@
 //
 // The decode kernel's work split for runs of more than one token: the 32-token tiles of all items -- an item is up to
 // 16 NT columns of one sequence -- form one line that is cut into equal shares, a workgroup of eight waves per compute
-// unit takes a share, a wave a kv head (or, with fewer than eight kv heads, every 8 / HPW-th tile of one).  Head sizes 64 and 128.  A run of
+// unit takes a share, 8 / HPW waves of which share a kv head's tiles (HPW = 1, 2 or 4 kv heads).  Head sizes 64 and 128.  A run of
 // tiles that covers its item writes the rows, any other leaves partial states for the reduce kernel.  One-token
 // sequences of the batch are items like any other, so the launch needs neither the decode kernels nor the plan.
 // With a workgroup per (sequence, kv head), whatever the sequence's length, a batch was as slow as its longest one:
 // 24 sequences of 1k-8k tokens with 2-6 query tokens each took 97 us in that kernel, 2.4 TB/s; the step they are part
-// of went from 105.8 to 71.3 us.
+// of went from 105.8 to 71.3 us (now 70.1).
 #pragma once
 
 #include "kvq_prefill_tile.cuh"
@@ -339,7 +339,19 @@ static int launch_one(const ShortRunArgs& a, dim3 grid, hipStream_t s) {
 template <int D>
 int launch_short_runs_d(const ShortRunArgs& args, hipStream_t s) {
   ShortRunArgs a = args;
-  const int hkv = a.io.g.num_kv_heads, hpw = heads_per_wg(hkv);
+  const int hkv = a.io.g.num_kv_heads;
+  // Kv heads per workgroup: fewer of them cut the line into fewer, longer shares (the waves of a head meet in LDS), so
+  // that an item leaves fewer partial states -- a state is up to 32 columns of D floats per head, and with a cut per 8 heads
+  // a batch wrote and read 27 MB of them beside 173 MB of cache.  Four rather than eight (MI355X, a step, 8 kv heads of 128,
+  // 2 - 6 query tokens on 1k - 8k): 24 sequences 73.5 -> 71.1 us, 40: 83.4 -> 79.8, 64: 125.2 -> 119.7; 90 short ones
+  // 55.0 -> 54.7.  Below four a share's start weighs more than the states saved (24 sequences, 4 kv heads: 2 per
+  // workgroup 50.6 for 47.9 us) until an item is cut dozens of times: one sequence of 16k tokens 34.5 -> 24.9 us, 5 of
+  // 8k - 16k on 16 kv heads 62.8 -> 60.3; 12 on 4 kv heads (21 cuts each) would lose, 38.9 -> 41.1.
+  int hpw = heads_per_wg(hkv);
+  while (hpw > 4 || (hpw > 1 && a.num_wg > 24 * a.num_seqs * a.blocks)) {
+    hpw /= 2;
+    a.num_wg /= 2;
+  }
   a.setup_units = setup_units_for(8 / hpw);
   dim3 grid(a.num_wg, (hkv + hpw - 1) / hpw);
   const bool ext = a.io.cap_c != 0.f || a.io.alibi != nullptr;
@@ -357,7 +369,6 @@ int launch_short_runs_d(const ShortRunArgs& args, hipStream_t s) {
 #define KVQ_SR_HPW(NT)          \
   do {                          \
     switch (hpw) {              \
-      case 8: KVQ_SR(NT, 8); break; \
       case 4: KVQ_SR(NT, 4); break; \
       case 2: KVQ_SR(NT, 2); break; \
       default: KVQ_SR(NT, 1); break; \
