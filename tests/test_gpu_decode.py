@@ -400,3 +400,18 @@ def test_whole_sequences(gpu_device, form, layout, hq, hkv, d, ctx, window, soft
     torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)
     if len(ctx) * hkv <= 256:
         assert bool((ws == 0xFF).all()), "the launch left partial states"
+
+
+@pytest.mark.parametrize("layout,hq,hkv,d,ctx", [
+    ("HND", 32, 8, 128, [3001]), ("NHD", 32, 8, 128, [1100, 5000, 33]), ("HND", 28, 4, 128, [2000, 1, 0, 4097, 700]),
+    ("NHD", 32, 16, 128, [2048] * 5), ("HND", 32, 16, 64, [2048] * 6), ("HND", 24, 12, 128, [1500, 1025]),
+    ("HND", 9, 3, 64, [40000])])
+def test_a_handful_of_sequences(gpu_device, layout, hq, hkv, d, ctx):
+    """Batches around the size (48 cuts per sequence on 256 compute units) below which a workgroup serves fewer kv
+    heads than it could, with kv head counts that do not divide into them and a sequence of hundreds of shares."""
+    kv, lay, bt, q, sl, cu = build_case(ctx, hq, hkv, d, 16, layout, hkv + len(ctx))
+    scale = 1 / math.sqrt(d)
+    want, want_lse = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, scale, return_lse=True)
+    got, lse = run_unified(gpu_device, kv, layout, bt, q, sl, cu, scale, out_dtype=torch.float32, want_lse=True)
+    T.assert_close_attn(got, want, atol=2e-3, rtol=2e-3, what=f"{hq}/{hkv} d{d} ctx={ctx}")
+    torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)

@@ -890,8 +890,20 @@ __global__ __launch_bounds__(WPW * 64) void paged_decode_v2_kernel(V2Args a) {
 template <int D, int QDT>
 int launch_streamk(const StreamKArgs& args, hipStream_t s) {
   const int hkv = args.io.g.num_kv_heads;
-  const int hpw = heads_per_wg(hkv);
+  int hpw = heads_per_wg(hkv);
   StreamKArgs a = args;
+  // A handful of sequences: fewer kv heads per workgroup cut each of them into fewer, longer shares -- the waves of a head
+  // meet in LDS instead of in the reduce's slots.  From 48 cuts per sequence on (5 sequences, 256 compute units); at
+  // 24 the gain is gone (10 sequences of 1k - 8k: 31.1 us both ways, 2 of 20k with the fewest heads 27.8 for 26.9 us).
+  // A step on MI355X, 8 kv heads of 128, before / after: 1 sequence of 2000 tokens 16.9 / 15.8 us, 16k 22.1 / 21.1,
+  // 100k 49.5 / 47.0; 4 of 1k - 8k 24.5 / 22.6; 3 on 4 kv heads 21.0 / 18.5; token-major cache, 4 of 1k - 8k: 26.2 / 22.9.
+  // Not at head size 256 (2 of 1k - 8k: 31.5 / 33.6), whose states are twice as long to fold.
+  if constexpr (D <= 128) {
+    while (!a.fixed_spans && hpw > 1 && a.num_wg > 48 * a.num_seqs) {
+      hpw /= 2;
+      a.num_wg /= 2;
+    }
+  }
   // a head's records of a block back to back (HND order): the tile loads may stream past the caches
   const bool stream = a.io.g.stride_slot == 2 * (code_bytes(a.io.g) + 4) && a.io.g.block_size >= 16;
   const bool extras = a.io.cap_c != 0.f || a.io.alibi != nullptr;   // the instantiation with soft cap and ALiBi
