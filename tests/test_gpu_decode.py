@@ -415,3 +415,22 @@ def test_a_handful_of_sequences(gpu_device, layout, hq, hkv, d, ctx):
     got, lse = run_unified(gpu_device, kv, layout, bt, q, sl, cu, scale, out_dtype=torch.float32, want_lse=True)
     T.assert_close_attn(got, want, atol=2e-3, rtol=2e-3, what=f"{hq}/{hkv} d{d} ctx={ctx}")
     torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("n", [64, 65, 128, 191, 256, 257, 300])
+@pytest.mark.parametrize("hq,hkv,layout", [(8, 2, "HND"), (8, 8, "NHD")])
+def test_batches_around_the_sequences_a_lane_holds(gpu_device, hq, hkv, layout, n):
+    """64 and 256 sequences are the most that the prologue holds in one and in four per lane; lengths 0 at both ends and
+    on the 64-sequence edges, one sequence of dozens of shares at the end."""
+    g = torch.Generator().manual_seed(n)
+    ctx = torch.randint(1, 120, (n,), generator=g).tolist()
+    for i in (0, 63, 64, 127, n - 2):
+        if i < n:
+            ctx[i] = 0
+    ctx[n - 1] = 3000
+    kv, lay, bt, q, sl, cu = build_case(ctx, hq, hkv, 64, 16, layout, n)
+    scale = 1 / math.sqrt(64)
+    want, want_lse = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, scale, return_lse=True)
+    got, lse = run_unified(gpu_device, kv, layout, bt, q, sl, cu, scale, out_dtype=torch.float32, want_lse=True)
+    T.assert_close_attn(got, want, atol=2e-3, rtol=2e-3, what=f"{n} sequences {hq}/{hkv}")
+    torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)

@@ -1040,8 +1040,9 @@ struct StreamKArgs {
   float* part_o;                // [(P + B), Hq, D]
   float* part_ml;               // [(P + B), Hq, 2]
   // [2 P + 2], what the main kernel leaves for the reduce kernel, whose waves would otherwise each rescan all
-  // sequence lengths: [0] = length of the work line; [2 w + 2], [2 w + 3] = the sequence that holds workgroup w's
-  // first unit and that sequence's own first unit (workgroups without a share write nothing).
+  // sequence lengths: [0] = length of the work line; [2 w + 2] = the sequence that holds workgroup w's first unit and, in
+  // the high half, its row; [2 w + 3] = the first and the last workgroup that hold a tile of it (workgroups without a
+  // share write nothing).
   int64_t* wg_info;
   int64_t* seq_first_unit;      // [B]: the first unit of every decode sequence that has a tile (same purpose)
   int num_seqs;

@@ -142,48 +142,68 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
   const LaneOffsets off = DTile::lane_offsets(a.io.g, lane);   // (while the lengths are on their way)
 
   // the balanced cutting: total units of the work line (each wave redoes this tiny scan; no LDS, no barrier)
-  const bool one_chunk = B <= kWave;
   int64_t total = 0, lo = 0, hi = 0;
+  int num_wg = 0;
   int seq = 0;
   int64_t seq_start = 0;  // global index of the sequence's first unit
   SeqRow cur{};           // the sequence's length and row
-  {
-    SeqRow mine{};
-    int n = 0, incl = 0;
-    if (one_chunk) {   // a sequence per lane: one trip to memory for the whole line
-      mine = load_seq(a, min(lane, B - 1));
-      n = lane < B ? seq_line_units<fixed>(mine, a.io.window, a.setup_units) : 0;
-      incl = wave_incl_scan(n);
-      total = __builtin_amdgcn_readlane(incl, 63);
-    } else {
-      total = scan_total<fixed>(a, lane);
-    }
+  auto take_share = [&]() __attribute__((always_inline)) {
     // (the batch-invariant line is short -- a unit is a span of at least kMinSpanTiles tiles -- and is always shared
     // out over every workgroup there is a unit for)
-    const int num_wg = fixed ? (total < a.num_wg ? (total < 1 ? 1 : (int)total) : a.num_wg) : active_workgroups(total, a.num_wg);
-    if (w >= num_wg) return;
+    num_wg = fixed ? (total < a.num_wg ? (total < 1 ? 1 : (int)total) : a.num_wg) : active_workgroups(total, a.num_wg);
+    if (w >= num_wg) return false;
     lo = wg_tile_begin(w, total, num_wg);
     hi = wg_tile_begin(w + 1, total, num_wg);
     if (lo >= hi) {   // an empty work line: workgroup 0 still reports its length
       if (!fixed && w == 0 && blockIdx.y == 0 && wave == 0 && lane == 0) a.wg_info[0] = total;
-      return;
+      return false;
     }
-    // the sequence that holds unit `lo`
-    if (one_chunk) {
-      const uint64_t hit = __builtin_amdgcn_ballot_w64(n > 0 && incl - n <= lo && lo < incl);
-      seq = __builtin_ctzll(hit);   // (lo < total: there is one)
-      seq_start = __builtin_amdgcn_readlane(incl - n, seq);
-      cur = {__builtin_amdgcn_readlane(mine.len, seq), __builtin_amdgcn_readlane(mine.q0, seq), __builtin_amdgcn_readlane(mine.q1, seq)};
-    } else {
-      scan_locate<fixed>(a, lane, lo, seq, seq_start);
-      seq = __builtin_amdgcn_readfirstlane(seq);
-      cur = load_seq(a, seq);
+    return true;
+  };
+  // Up to 64 N sequences: each lane keeps N of them, and one trip to memory serves the total, the place of the share and
+  // the sequence it begins in (200 sequences, 4 kv heads, int4 codes: the three trips one after another cost a step 1 us).
+  auto scan_held = [&](auto n_tag) __attribute__((always_inline)) {
+    constexpr int N = decltype(n_tag)::value;
+    SeqRow mine[N];
+    int n[N], incl[N], sum = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j) mine[j] = load_seq(a, min(kWave * j + lane, B - 1));
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      n[j] = kWave * j + lane < B ? seq_line_units<fixed>(mine[j], a.io.window, a.setup_units) : 0;
+      incl[j] = wave_incl_scan(n[j]) + sum;
+      sum = __builtin_amdgcn_readlane(incl[j], 63);
     }
+    total = sum;
+    if (!take_share()) return false;
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      const uint64_t hit = __builtin_amdgcn_ballot_w64(n[j] > 0 && incl[j] - n[j] <= lo && lo < incl[j]);
+      if (N == 1 || hit != 0) {   // (lo < total: there is one)
+        const int src = __builtin_ctzll(hit);
+        seq = kWave * j + src;
+        seq_start = __builtin_amdgcn_readlane(incl[j] - n[j], src);
+        cur = {__builtin_amdgcn_readlane(mine[j].len, src), __builtin_amdgcn_readlane(mine[j].q0, src),
+               __builtin_amdgcn_readlane(mine[j].q1, src)};
+      }
+    }
+    return true;
+  };
+  if (B <= kWave) {
+    if (!scan_held(std::integral_constant<int, 1>{})) return;
+  } else if (B <= kWave * kScanBatch) {
+    if (!scan_held(std::integral_constant<int, kScanBatch>{})) return;
+  } else {
+    total = scan_total<fixed>(a, lane);
+    if (!take_share()) return;
+    scan_locate<fixed>(a, lane, lo, seq, seq_start);
+    seq = __builtin_amdgcn_readfirstlane(seq);
+    cur = load_seq(a, seq);
   }
   // Where the share begins (the reduce kernel's key to the span): noted in the first round of the loop, stored
   // after the last.  A store ahead of the tile loads would sit before them in the wave's in-order memory
   // counter, and the first tile would wait for the store's acknowledgement (measured: 0.6 us per launch).
-  int info_seq = -1;
+  int info_seq = -1, info_row = 0, info_tiles = 0;
   int64_t info_start = 0;
 
   // One run of tiles [t_begin, t_end) of sequence `cur` (ntiles tiles from tile t0 on), its state to `slot` unless
@@ -286,6 +306,8 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
     const int64_t row = cur.q0;
     if (info_seq < 0) {
       info_seq = seq;
+      info_row = cur.q0;
+      info_tiles = ntiles;
       info_start = seq_start;
     }
     const int first = window_first(len, a.io.window);  // tokens before it are outside the window
@@ -307,8 +329,9 @@ __global__ __launch_bounds__(512) void paged_decode_streamk_kernel(StreamKArgs a
   if (blockIdx.y == 0 && wave == 0 && lane == 0) {   // this lane leaves the reduce kernel its notes
     if (w == 0) a.wg_info[0] = total;
     if (info_seq >= 0) {
-      a.wg_info[2 * w + 2] = info_seq;
-      a.wg_info[2 * w + 3] = info_start;
+      const uint32_t first = wg_of_unit(info_start + setup, total, num_wg), last = wg_of_unit(info_start + setup + info_tiles - 1, total, num_wg);
+      a.wg_info[2 * w + 2] = (int64_t)((uint64_t)(uint32_t)info_row << 32 | (uint32_t)info_seq);
+      a.wg_info[2 * w + 3] = (int64_t)((uint64_t)last << 32 | first);
     }
   }
 }
@@ -428,7 +451,7 @@ __global__ __launch_bounds__(256) void paged_decode_fixed_spans_reduce_kernel(St
 // lane D/16 dims.
 // A sequence is cut only where a workgroup's share begins inside it, so the grid runs over the P workgroups of
 // the main kernel, not over the sequences: block w looks at the sequence in which share w begins (the main
-// kernel left its number and its place on the work line) and merges it if share w is the
+// kernel left its number, its row and its shares) and merges it if share w is the
 // FIRST to begin inside it; a sequence cut several times is thus merged once, and one that is not cut costs a
 // block one round trip.  (A grid over the sequences, every wave scanning all sequence lengths for its place on
 // the line, took 44 us at 512 sequences; with one q head per wave the P x Hq waves of this grid, 8192 at 32
@@ -447,9 +470,8 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_kernel(Stream
   const int B = a.num_seqs;
   // the loads that depend on nothing but the arguments go out before the first branch
   const int64_t total = a.wg_info[0];
-  // (the share's sequence is undefined for a workgroup without a share: clamped here, looked at only if w < P)
-  const int seq = min(max((int)a.wg_info[2 * w + 2], 0), B - 1);
-  const int64_t start = a.wg_info[2 * w + 3];
+  // (undefined for a workgroup without a share: looked at only if w < P)
+  const uint64_t info0 = (uint64_t)a.wg_info[2 * w + 2], info1 = (uint64_t)a.wg_info[2 * w + 3];
   auto store_dims = [&](int64_t r, const float (&x)[V]) __attribute__((always_inline)) {
     if (!head_ok) return;
     const int64_t at = r * a.io.out_stride_t + (int64_t)head * a.io.out_stride_h + sub * V;
@@ -470,13 +492,8 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_kernel(Stream
   }
   const int P = active_workgroups(total, a.num_wg);
   if (w == 0 || w >= P) return;
-  const int len = a.seq_lens[seq];
-  const int64_t row = a.cu_seqlens_q ? a.cu_seqlens_q[seq] : seq;
-  const int ntiles = decode_tiles(len, a.io.window);   // a decode sequence with tiles
-  // workgroup holding unit x: the largest w with floor(w*T/P) <= x; the sequence's tiles are units
-  // start + setup_units .. start + setup_units + ntiles - 1
-  const int w_first = (int)(((start + a.setup_units + 1) * P - 1) / total);
-  const int w_last = (int)(((start + a.setup_units + ntiles) * P - 1) / total);
+  const int seq = (int)(uint32_t)info0, w_first = (int)(uint32_t)info1, w_last = (int)(info1 >> 32);
+  const int64_t row = (int64_t)(info0 >> 32);
   if (w_first == w_last) return;  // not cut
   const int span = w_last - w_first + 1;
   if (span > 16) {
@@ -491,7 +508,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_kernel(Stream
     for (int i = 0; i < V2; ++i) acc[i] = 0.f;
     for (int wb = w_first; wb <= w_last; wb += kWave) {
       const int wj = wb + lane;
-      const bool live = wj <= w_last && wg_tile_begin(wj, total, P) < wg_tile_begin(wj + 1, total, P);
+      const bool live = wj <= w_last;
       // loads are unconditional (clamped to the sequence's last workgroup) and what they return is removed with
       // a bit mask where the slot holds nothing
       const int64_t slot = (int64_t)min(wj, w_last) + seq;
@@ -560,7 +577,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_kernel(Stream
   auto pass = [&](int wb, auto n_tag) __attribute__((always_inline)) {
     constexpr int N = decltype(n_tag)::value;   // <= 16
     const int wj = wb + sub;
-    const bool live = sub < N && wj <= w_last && wg_tile_begin(wj, total, P) < wg_tile_begin(wj + 1, total, P);
+    const bool live = sub < N && wj <= w_last;
     const int64_t slot = (int64_t)min(wj, w_last) + seq;
     const float mj_raw = ml_head[slot * Hq * 2 + 0];
     const float lj_raw = ml_head[slot * Hq * 2 + 1];
@@ -636,10 +653,9 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_by_seq_kernel
     return;
   }
   const int P = active_workgroups(total, a.num_wg);
-  // workgroup holding unit x: the largest w with floor(w*T/P) <= x; the sequence's tiles are units
-  // start + setup_units .. start + setup_units + ntiles - 1
-  const int w_first = (int)(((start + a.setup_units + 1) * P - 1) / total);
-  const int w_last = (int)(((start + a.setup_units + ntiles) * P - 1) / total);
+  // the sequence's tiles are units start + setup_units .. start + setup_units + ntiles - 1
+  const int w_first = wg_of_unit(start + a.setup_units, total, P);
+  const int w_last = wg_of_unit(start + a.setup_units + ntiles - 1, total, P);
   if (w_first == w_last) return;  // written directly by the main kernel
 
   // pass 1: every lane takes one workgroup's (m, l); the wave agrees on the max and the weights
@@ -656,7 +672,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_by_seq_kernel
   auto merge_few = [&](auto n_tag) __attribute__((always_inline)) {
     constexpr int N = decltype(n_tag)::value;
     const int w = w_first + lane;
-    const bool live = w <= w_last && wg_tile_begin(w, total, P) < wg_tile_begin(w + 1, total, P);
+    const bool live = w <= w_last;
     const int64_t slot = (int64_t)min(w, w_last) + seq;
     const uint32_t keep = live ? 0xffffffffu : 0u;
     const float mj_raw = a.part_ml[(slot * a.io.num_q_heads + head) * 2 + 0];
@@ -692,7 +708,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_by_seq_kernel
   } else
   for (int wb = w_first; wb <= w_last; wb += kWave) {
     const int w = wb + lane;
-    const bool live = w <= w_last && wg_tile_begin(w, total, P) < wg_tile_begin(w + 1, total, P);
+    const bool live = w <= w_last;
     // loads are unconditional (clamped to the sequence's last workgroup) and what they return is
     // removed with a bit mask where the slot holds nothing: a select on the loaded value becomes a
     // branch around the load, and the loads of successive slots would then run one after another
@@ -773,8 +789,8 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_split4_kernel
     return;
   }
   const int P = active_workgroups(total, a.num_wg);
-  const int w_first = (int)(((start + a.setup_units + 1) * P - 1) / total);
-  const int w_last = (int)(((start + a.setup_units + ntiles) * P - 1) / total);
+  const int w_first = wg_of_unit(start + a.setup_units, total, P);
+  const int w_last = wg_of_unit(start + a.setup_units + ntiles - 1, total, P);
   if (w_first == w_last) return;  // written directly by the main kernel
   // this wave's slots: w_first + part + 4 i, i = 0 .. n - 1 (n = 0 for a span shorter than its number)
   const int span = w_last - w_first + 1;
@@ -789,7 +805,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_split4_kernel
     constexpr int N = decltype(n_tag)::value;   // <= 64
     const int i = i0 + lane;
     const int wj = w_first + part + 4 * i;
-    const bool live = lane < N && i < n && wg_tile_begin(wj, total, P) < wg_tile_begin(wj + 1, total, P);
+    const bool live = lane < N && i < n;
     const int64_t slot = (int64_t)min(wj, w_last) + seq;
     const float mj_raw = a.part_ml[(slot * Hq + head) * 2 + 0];
     const float lj_raw = a.part_ml[(slot * Hq + head) * 2 + 1];

@@ -278,8 +278,8 @@ __global__ __launch_bounds__(256) void short_runs_reduce_kernel(ShortRunArgs a) 
   const int ntiles = it.t1 - it.t0;
   if (ntiles > 0) {
     const int P = active_workgroups(total, a.num_wg);
-    const int w_first = (int)(((start + a.setup_units + 1) * P - 1) / total);
-    const int w_last = (int)(((start + a.setup_units + ntiles) * P - 1) / total);
+    const int w_first = wg_of_unit(start + a.setup_units, total, P);
+    const int w_last = wg_of_unit(start + a.setup_units + ntiles - 1, total, P);
     if (w_first == w_last) return;  // written by the main kernel
     const int hkv = head / io.group, n = qt * io.group + head - hkv * io.group;
     const int64_t stride = (int64_t)io.g.num_kv_heads * a.rows;   // rows between two slots
@@ -288,7 +288,7 @@ __global__ __launch_bounds__(256) void short_runs_reduce_kernel(ShortRunArgs a) 
     auto pass = [&](int wb, auto n_tag) __attribute__((always_inline)) {
       constexpr int N = decltype(n_tag)::value;
       const int wj = wb + lane;
-      const bool live = lane < N && wj <= w_last && wg_tile_begin(wj, total, P) < wg_tile_begin(wj + 1, total, P);
+      const bool live = lane < N && wj <= w_last;
       const int64_t mine = at0 + (2 * (int64_t)min(wj, w_last) + (wj == w_first ? 1 : 0)) * stride;
       const float mj_raw = a.part_ml[2 * mine], lj_raw = a.part_ml[2 * mine + 1];
       float po[N][V];
