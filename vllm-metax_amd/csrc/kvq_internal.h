@@ -94,11 +94,6 @@ __device__ __forceinline__ void store_act_rt(int dtype, void* p, int64_t i, floa
   else store_act<KVQ_F16>(p, i, v);
 }
 
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, kWave));
-  return v;
-}
 // Reductions over the four lanes l, l ^ 16, l ^ 32, l ^ 48 (one lane of each quarter-wave), result in
 // all four: two register swaps (v_permlane32_swap / v_permlane16_swap exchange half-waves / odd and
 // even rows of 16 between two registers), no trip through LDS.  The instruction swaps between TWO
@@ -136,12 +131,59 @@ __device__ __forceinline__ float sum_over_quarters(float v) {
   swap_halves(__builtin_bit_cast(uint32_t, v), true, a, b);
   return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
 }
+// The same over the 2, 4, 8 or 16 neighbouring lanes of a group, by data-parallel moves: lane ^ 1 and ^ 2 of a quad, then
+// the mirror images of 8 and of 16 lanes, which by then hold their group's value.  A move is an operand of the next
+// instruction; a shuffle through LDS is a trip of over a hundred cycles, and the small kernels around a decode step (cache write,
+// reduce) chain up to twelve of them (a step of 4 verification runs 19.4 -> 18.6 us, 37 sequences at head size 256 104.0 -> 103.1).
+// Every lane of the wave must take part.
+template <int CTRL>
+__device__ __forceinline__ float lane_move(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+template <int LANES>
+__device__ __forceinline__ float group_max(float v) {
+  static_assert(LANES == 8 || LANES == 16 || LANES == 32, "");
+  v = fmaxf(v, lane_move<0xb1>(v));    // quad_perm 1 0 3 2
+  v = fmaxf(v, lane_move<0x4e>(v));    // quad_perm 2 3 0 1
+  v = fmaxf(v, lane_move<0x141>(v));   // row_half_mirror
+  if constexpr (LANES >= 16) v = fmaxf(v, lane_move<0x140>(v));   // row_mirror
+  if constexpr (LANES == 32) {
+    uint32_t a, b;
+    swap_halves(__builtin_bit_cast(uint32_t, v), true, a, b);
+    v = fmaxf(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+  }
+  return v;
+}
+__device__ __forceinline__ float row16_sum(float v) {
+  v += lane_move<0xb1>(v);
+  v += lane_move<0x4e>(v);
+  v += lane_move<0x141>(v);
+  return v + lane_move<0x140>(v);
+}
+__device__ __forceinline__ float wave_max(float v) { return max_over_quarters(group_max<16>(v)); }
+__device__ __forceinline__ float wave_sum(float v) { return sum_over_quarters(row16_sum(v)); }
+// Lane `l`'s value (uniform l), to every lane.
+__device__ __forceinline__ float lane_value(float v, int l) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+}
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every global
 // load in flight (vmcnt(0)), which would drain the tile prefetch issued just before it; here the
 // loads stay in flight and the compiler's own wait before their first use still applies.
 // Code bytes of one half (K or V) of a record.
 __host__ __device__ inline int code_bytes(const kvq_cache_geom& g) {
   return g.code_type == KVQ_CODE_INT4 ? g.head_size / 2 : g.head_size;
+}
+
+// A slot's block and its place in it (a 64-bit division is a routine of over a hundred instructions).
+__device__ __forceinline__ void split_slot(int64_t slot, int block_size, int64_t& blk, int64_t& off) {
+  if ((uint64_t)slot <= 0xffffffffull) {
+    const uint32_t b32 = (uint32_t)slot / (uint32_t)block_size;
+    blk = b32;
+    off = (uint32_t)slot - b32 * (uint32_t)block_size;
+  } else {
+    blk = slot / block_size;
+    off = slot - blk * block_size;
+  }
 }
 
 // One cache row's quantisation with 8 elements per lane and LPR lanes per row (every lane of the wave takes
@@ -154,9 +196,7 @@ __device__ __forceinline__ void quant_row8(const float (&x)[8], float eps, int c
   float amax = 0.f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(x[i]));
-#pragma unroll
-  for (int o = LPR / 2; o >= 1; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, kWave));
-  amax = fmaxf(amax, eps);  // eps may be 0 for fp16 sources (1e-10 underflows)
+  amax = fmaxf(group_max<LPR>(amax), eps);  // eps may be 0 for fp16 sources (1e-10 underflows)
   scale = code_type == KVQ_CODE_FP8_E4M3 ? amax / 448.0f : (code_type == KVQ_CODE_INT4 ? amax / 7.0f : amax / 127.0f);
   pk[0] = 0u;
   pk[1] = 0u;
@@ -289,9 +329,7 @@ __device__ __forceinline__ float mla_row_scale(const MlaRowPieces& r, float eps)
   for (int j = 0; j < 2; ++j)
 #pragma unroll
     for (int i = 0; i < 8; ++i) amax = fmaxf(amax, r.have[j] ? fabsf(r.x[j][i]) : 0.f);
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) amax = fmaxf(amax, __shfl_xor(amax, o, kWave));
-  return fmaxf(amax, eps) / 127.0f;
+  return fmaxf(wave_max(amax), eps) / 127.0f;
 }
 __device__ __forceinline__ void mla_row_store(const MlaRowPieces& r, float scale, uint8_t* row, float* scale_ptr, int lane) {
   const bool pos = scale > 0.f;   // scale == 0: an all-zero row with eps 0
@@ -329,11 +367,6 @@ __device__ __forceinline__ int wave_incl_scan(int v) {
   v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
   v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 onto rows 1 and 3
   v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 onto rows 2 and 3
-  return v;
-}
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, kWave);
   return v;
 }
 

@@ -20,8 +20,8 @@ __global__ __launch_bounds__(256) void mla_quant_write_kernel(const void* __rest
   if (t >= num_tokens) return;
   const int64_t slot = slot_mapping[t];
   if (slot < 0) return;  // padding token
-  const int64_t blk = slot / g.block_size;
-  const int64_t off = slot - blk * g.block_size;
+  int64_t blk, off;
+  split_slot(slot, g.block_size, blk, off);
   const int R = g.kv_lora_rank, W = g.kv_lora_rank + g.rope_dim;
   constexpr int kMaxPerLane = 16;  // rows up to 1024 wide stay in registers
   float x[kMaxPerLane];
@@ -68,8 +68,8 @@ __global__ __launch_bounds__(256) void mla_quant_write_rows8_kernel(const void* 
   mla_row_load(kv_c, k_pe, dt, t * kv_c_stride, t * k_pe_stride, rp, np, lane, r);
   const float scale = mla_row_scale(r, eps);
   if (!live || slot < 0) return;  // padding token (after the shuffles: every lane took part)
-  const int64_t blk = slot / g.block_size;
-  const int64_t off = slot - blk * g.block_size;
+  int64_t blk, off;
+  split_slot(slot, g.block_size, blk, off);
   mla_row_store(r, scale, cache + blk * g.stride_block + off * g.stride_row,
                 reinterpret_cast<float*>(cache + blk * g.stride_block + g.scale_off + off * 4), lane);
 }
@@ -127,8 +127,8 @@ __global__ __launch_bounds__(256) void mla_rope_quant_write_kernel(
   }
   amax = fmaxf(wave_max(amax), eps);
   const float scale = amax / 127.0f;
-  const int64_t blk = slot / g.block_size;
-  const int64_t off = slot - blk * g.block_size;
+  int64_t blk, off;
+  split_slot(slot, g.block_size, blk, off);
   int8_t* row = reinterpret_cast<int8_t*>(cache + blk * g.stride_block + off * g.stride_row);
   auto code = [&](float v) {
     float r = scale > 0.f ? rintf(v / scale) : 0.f;

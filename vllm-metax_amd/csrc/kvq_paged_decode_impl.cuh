@@ -432,7 +432,7 @@ __global__ __launch_bounds__(256) void paged_decode_fixed_spans_reduce_kernel(St
     }
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const float wk = k0 + k < spans ? __shfl(ej, k0 + k, kWave) : 0.f;
+      const float wk = k0 + k < spans ? lane_value(ej, k0 + k) : 0.f;
       const uint32_t kk = wk != 0.f ? 0xffffffffu : 0u;
 #pragma unroll
       for (int i = 0; i < V; ++i) acc[i] += as_f32(as_u32(po[k][i]) & kk) * wk;
@@ -538,7 +538,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_kernel(Stream
         }
 #pragma unroll
         for (int k = 0; k < kBatch; ++k) {
-          const float wk = (k0 + k) < count ? __shfl(ej, (k0 + k) & (kWave - 1), kWave) : 0.f;  // unnormalised sums
+          const float wk = (k0 + k) < count ? lane_value(ej, (k0 + k) & (kWave - 1)) : 0.f;  // unnormalised sums
           const uint32_t kk = wk != 0.f ? 0xffffffffu : 0u;
 #pragma unroll
           for (int i = 0; i < V2; ++i) acc[i] += as_f32(as_u32(pv[k][i]) & kk) * wk;
@@ -555,16 +555,6 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_kernel(Stream
   }
   if (w != w_first + 1) return;  // another block's to merge
 
-  auto group_max = [&](float x) __attribute__((always_inline)) {
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) x = fmaxf(x, __shfl_xor(x, o, kWave));
-    return x;
-  };
-  auto group_sum = [&](float x) __attribute__((always_inline)) {
-#pragma unroll
-    for (int o = 8; o >= 1; o >>= 1) x += __shfl_xor(x, o, kWave);
-    return x;
-  };
   const float* po_head = a.part_o + (int64_t)head * D + sub * V;
   const float* ml_head = a.part_ml + (int64_t)head * 2;
   // lane `sub` of a group takes slot wb + sub's (m, l); the group agrees on the maximum and the weights, then
@@ -595,10 +585,10 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_kernel(Stream
     const uint32_t keep = live ? 0xffffffffu : 0u;
     const float mj = live ? as_f32(as_u32(mj_raw) & keep) : -INFINITY;
     const float lj = as_f32(as_u32(lj_raw) & keep);
-    const float m_new = fmaxf(m, group_max(mj));
+    const float m_new = fmaxf(m, group_max<16>(mj));
     const float ca = __builtin_amdgcn_exp2f(m - m_new);  // first pass: exp2(-inf) = 0
     const float ej = live ? __builtin_amdgcn_exp2f(mj - m_new) : 0.f;
-    l = l * ca + group_sum(lj * ej);
+    l = l * ca + row16_sum(lj * ej);
     m = m_new;
 #pragma unroll
     for (int i = 0; i < V; ++i) acc[i] *= ca;
@@ -692,7 +682,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_by_seq_kernel
     l = wave_sum(lj * ej);
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      const float wk = __shfl(ej, k, kWave);  // 0 for slots past the last and for empty ones
+      const float wk = lane_value(ej, k);  // 0 for slots past the last and for empty ones
       const uint32_t kk = wk != 0.f ? 0xffffffffu : 0u;
 #pragma unroll
       for (int i = 0; i < V; ++i) acc[i] += as_f32(as_u32(po[k][i]) & kk) * wk;
@@ -742,7 +732,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_by_seq_kernel
       }
 #pragma unroll
       for (int k = 0; k < kBatch; ++k) {
-        const float wk = (k0 + k) < count ? __shfl(ej, (k0 + k) & (kWave - 1), kWave) : 0.f;  // unnormalised sums
+        const float wk = (k0 + k) < count ? lane_value(ej, (k0 + k) & (kWave - 1)) : 0.f;  // unnormalised sums
         const uint32_t kk = wk != 0.f ? 0xffffffffu : 0u;
 #pragma unroll
         for (int i = 0; i < V; ++i) acc[i] += as_f32(as_u32(pv[k][i]) & kk) * wk;
@@ -829,7 +819,7 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_split4_kernel
     for (int x = 0; x < V; ++x) acc[x] *= ca;
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-      const float wk = __shfl(ej, k, kWave);
+      const float wk = lane_value(ej, k);
       const uint32_t kk = wk != 0.f ? 0xffffffffu : 0u;
 #pragma unroll
       for (int x = 0; x < V; ++x) acc[x] += as_f32(as_u32(po[k][x]) & kk) * wk;

@@ -47,14 +47,7 @@ __global__ __launch_bounds__(256) void quant_write_kernel(
   }
   if (slot < 0) return;  // padding token
   int64_t blk, off;
-  if ((uint64_t)slot <= 0xffffffffull) {
-    const uint32_t b32 = (uint32_t)slot / (uint32_t)g.block_size;
-    blk = b32;
-    off = (uint32_t)slot - b32 * (uint32_t)g.block_size;
-  } else {
-    blk = slot / g.block_size;
-    off = slot - blk * g.block_size;
-  }
+  split_slot(slot, g.block_size, blk, off);
   uint8_t* rec = cache + blk * g.stride_block + off * g.stride_slot + (int64_t)h * g.stride_head;
   int8_t* codes = reinterpret_cast<int8_t*>(rec + (is_v ? g.v_off : g.k_off));
   float* scale_ptr = reinterpret_cast<float*>(rec + (is_v ? g.vs_off : g.ks_off));
@@ -178,14 +171,7 @@ __global__ __launch_bounds__(256) void quant_write_rows_kernel(
   quant_row8<LPR>(x, eps, g.code_type, pk, scale);
   if (!live || slot < 0) return;  // padding token (after the shuffles: every lane took part)
   int64_t blk, off;
-  if ((uint64_t)slot <= 0xffffffffull) {
-    const uint32_t b32 = (uint32_t)slot / (uint32_t)g.block_size;
-    blk = b32;
-    off = (uint32_t)slot - b32 * (uint32_t)g.block_size;
-  } else {
-    blk = slot / g.block_size;
-    off = slot - blk * g.block_size;
-  }
+  split_slot(slot, g.block_size, blk, off);
   uint8_t* rec = cache + blk * g.stride_block + off * g.stride_slot + (int64_t)h * g.stride_head;
   if (g.code_type == KVQ_CODE_INT4) *reinterpret_cast<uint32_t*>(rec + (is_v ? g.v_off : g.k_off) + li * 4) = pk[0];
   else *reinterpret_cast<u32x2_a4*>(rec + (is_v ? g.v_off : g.k_off) + li * 8) = (u32x2){pk[0], pk[1]};
@@ -227,8 +213,8 @@ __global__ __launch_bounds__(256) void rope_quant_write_kernel(
   // ---- key / value rows
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
   const int D = g.head_size;
-  const int64_t blk = slot / g.block_size;
-  const int64_t off = slot - blk * g.block_size;
+  int64_t blk, off;
+  split_slot(slot, g.block_size, blk, off);
   constexpr int kMaxPairs = 2;   // head sizes up to 256
   for (int r = wave; r < 2 * g.num_kv_heads; r += 4) {
     const int h = r >> 1, is_v = r & 1;

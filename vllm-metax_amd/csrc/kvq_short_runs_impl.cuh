@@ -312,7 +312,7 @@ __global__ __launch_bounds__(256) void short_runs_reduce_kernel(ShortRunArgs a) 
       for (int i = 0; i < V; ++i) acc[i] *= ca;
 #pragma unroll
       for (int k = 0; k < N; ++k) {
-        const float wk = __shfl(ej, k, kWave);
+        const float wk = lane_value(ej, k);
         const uint32_t kk = wk != 0.f ? 0xffffffffu : 0u;
 #pragma unroll
         for (int i = 0; i < V; ++i) acc[i] += as_f32(as_u32(po[k][i]) & kk) * wk;
