@@ -528,3 +528,22 @@ def test_short_run_shares_by_kv_heads(gpu_device, hq, hkv, n):
     got, lse = run(gpu_device, kv, "HND", bt, q, sl, cu, 4, scale, want_lse=True)
     T.assert_close_attn(got, want, what=f"{n} short runs, {hq}/{hkv}")
     torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("hq,hkv,splits", [(32, 8, 6), (32, 8, 3), (16, 4, 2), (16, 4, 3), (12, 3, 8), (16, 2, 4), (9, 1, 8)])
+def test_context_ranges_on_their_xcd(gpu_device, hq, hkv, splits):
+    """(kv head, range) pairs that can and that cannot be dealt out to eight XCDs evenly, two runs of different
+    numbers of query blocks: every row comes from every range once."""
+    ctx, qls = [5000, 4300], [150, 40]
+    kv, lay, bt, q, sl, cu = build(ctx, qls, hq, hkv, 128, 16, layout="HND", seed=hkv + splits)
+    scale = 1 / math.sqrt(128)
+    want = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, scale)
+    dev = gpu_device
+    kvd = T.to_device_cache(kv, dev, "HND")
+    k, v = L.key_value_views(kvd)
+    ks, vs = L.scale_views(kvd)
+    out = torch.full(q.shape, float("nan"), dtype=q.dtype, device=dev)
+    ops.unified_attention(q.to(dev), k, v, out, cu.to(dev), max(qls), sl.to(dev), max(ctx), scale, True, block_table=bt.to(dev),
+                          k_scale_cache=ks, v_scale_cache=vs, prefill_splits=splits)
+    torch.cuda.synchronize()
+    T.assert_close_attn(out, want, what=f"{splits} ranges, {hq}/{hkv}")
