@@ -516,11 +516,13 @@ def test_shared_tile_at_its_edges(gpu_device, hq, hkv, d, bs, layout, code, shif
         torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)
 
 
-@pytest.mark.parametrize("hq,hkv,n", [(32, 8, 5), (32, 8, 6), (32, 8, 2), (28, 4, 10), (28, 4, 11), (24, 12, 3), (9, 3, 1), (32, 16, 1)])
+@pytest.mark.parametrize("hq,hkv,n", [(32, 8, 5), (32, 8, 6), (32, 8, 2), (28, 4, 10), (28, 4, 11), (24, 12, 3), (9, 3, 1), (32, 16, 1),
+                                      (8, 2, 64), (8, 2, 65)])
 def test_short_run_shares_by_kv_heads(gpu_device, hq, hkv, n):
     """The batch sizes around which a workgroup of the short-run launch serves fewer kv heads (24 cuts per item, on
-    256 compute units), kv head counts that do not divide into them, and a single item: against the oracle."""
-    ctx = [4000 - 331 * (i % 7) + i for i in range(n)]
+    256 compute units), kv head counts that do not divide into them, and a single item; 64 items, the most that the prologue holds, and
+    one more: against the oracle."""
+    ctx = [(4000 if n < 64 else 400) - (331 if n < 64 else 33) * (i % 7) + i for i in range(n)]
     qls = [2 + i % 3 for i in range(n - 1)] + [4]
     kv, lay, bt, q, sl, cu = build(ctx, qls, hq, hkv, 128, 16, layout="HND", seed=hkv + n)
     scale = 1 / math.sqrt(128)

@@ -76,12 +76,16 @@ __global__ __launch_bounds__(512) void short_runs_streamk_kernel(ShortRunArgs a)
   const int w = blockIdx.x;
   const int items = a.num_seqs * a.blocks;
 
-  // the share [lo, hi) of the line, and the item that holds its first unit (each wave redoes the scan)
+  // the share [lo, hi) of the line, and the item that holds its first unit (each wave redoes the scan; up to 64 items are
+  // held from the first pass, without the second trip for their lengths: 12 sequences on an int4 cache 32.4 -> 31.8 us)
   int64_t total = 0;
+  int n0 = 0, incl0 = 0;   // the last 64 items' units and their running sum: of up to 64 items, all there is to know
   for (int base = 0; base < items; base += kWave) {
     const int i = base + lane;
     const int n = short_units(short_item(a, min(i, items - 1)), a.setup_units);
-    total += __builtin_amdgcn_readlane(wave_incl_scan(i < items ? n : 0), 63);
+    n0 = i < items ? n : 0;
+    incl0 = wave_incl_scan(n0);
+    total += __builtin_amdgcn_readlane(incl0, 63);
   }
   const int num_wg = active_workgroups(total, a.num_wg);
   if (w == 0 && blockIdx.y == 0 && wave == 0 && lane == 0) a.line[0] = total;
@@ -90,7 +94,11 @@ __global__ __launch_bounds__(512) void short_runs_streamk_kernel(ShortRunArgs a)
   if (lo >= hi) return;
   int item = 0;
   int64_t start = 0;   // the item's first unit
-  {
+  if (items <= kWave) {
+    const int src = __builtin_ctzll(__builtin_amdgcn_ballot_w64(n0 > 0 && incl0 - n0 <= lo && lo < incl0));   // lo < total: there is one
+    item = src;
+    start = __builtin_amdgcn_readlane(incl0 - n0, src);
+  } else {
     int64_t cum = 0;
     for (int base = 0; base < items; base += kWave) {
       const int i = base + lane;
