@@ -549,3 +549,40 @@ def test_context_ranges_on_their_xcd(gpu_device, hq, hkv, splits):
                           k_scale_cache=ks, v_scale_cache=vs, prefill_splits=splits)
     torch.cuda.synchronize()
     T.assert_close_attn(out, want, what=f"{splits} ranges, {hq}/{hkv}")
+
+
+@pytest.mark.parametrize("d,window,cap", [(128, 0, 0.0), (64, 0, 0.0), (128, 200, 30.0), (64, 200, 30.0), (256, 0, 0.0)])
+@pytest.mark.parametrize("code", ["int8", "fp8", "int4"])
+def test_negative_softmax_scale(gpu_device, code, d, window, cap):
+    """A softmax scale below zero turns the weights round, in every kernel that one call can take: decode rows, short
+    runs, long runs whole and in context ranges."""
+    from vllm_metax_amd.kv_cache_interface import KVQuantMode
+    hq, hkv, bs, dev = 16, 4, 16, gpu_device
+    ct = {"int8": oracle.CODE_INT8, "fp8": oracle.CODE_FP8, "int4": oracle.CODE_INT4}[code]
+    ctx, qls = [900, 300, 450, 65], [1, 5, 300, 65]
+    g = torch.Generator().manual_seed(d)
+    nb = sum((c + bs - 1) // bs for c in ctx) + 5
+    kv_cpu, _, lay = T.cpu_cache(nb, bs, hkv, d, "HND", code_type=ct)
+    T.storage_bytes(kv_cpu).fill_(0xFF)
+    bt = T.make_block_tables(ctx, bs, nb, g)
+    src = [[torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in ctx] for _ in range(2)]
+    T.fill_cache_from_sources(kv_cpu, lay, bt, ctx, bs, *src, code_type=ct)
+    q = torch.randn((sum(qls), hq, d), generator=g).to(torch.bfloat16)
+    sl = torch.tensor(ctx, dtype=torch.int32)
+    cu = torch.tensor([0] + torch.tensor(qls).cumsum(0).tolist(), dtype=torch.int32)
+    scale = -1 / math.sqrt(d)
+    want, want_lse = oracle.paged_attn(q, T.storage_bytes(kv_cpu), lay, bt, sl, cu, scale, return_lse=True, code_type=ct,
+                                       sliding_window=window, soft_cap=cap)
+    kv = T.to_device_cache(kv_cpu, dev, "HND", code_type=ct)
+    k, v = L.key_value_views(kv)
+    ks, vs = L.scale_views(kv)
+    for splits in (1, 3):
+        out = torch.full(q.shape, float("nan"), dtype=torch.bfloat16, device=dev)
+        lse = torch.full(q.shape[:2], float("nan"), dtype=torch.float32, device=dev)
+        ops.unified_attention(q.to(dev), k, v, out, cu.to(dev), max(qls), sl.to(dev), max(ctx), scale, True,
+                              window_size=(window - 1, 0) if window else (-1, -1), softcap=cap, block_table=bt.to(dev),
+                              k_scale_cache=ks, v_scale_cache=vs, lse=lse, prefill_splits=splits,
+                              kv_quant_mode=getattr(KVQuantMode, code.upper() + "_PER_TOKEN_HEAD"))
+        torch.cuda.synchronize()
+        T.assert_close_attn(out, want, what=f"negative scale {code} d{d}, {splits} ranges")
+        torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)

@@ -165,7 +165,8 @@ struct SharedTile {
   }
   // The tile's scales; one wave does it.
   __device__ static __forceinline__ void expand_scales(float sc, uint8_t* buf, int lane, float sc_mul) {
-    const float val = fminf(fmaxf(sc * sc_mul, 0.f), 65504.f);   // (a slot that holds no token: anything, made finite)
+    // a slot that holds no token: anything, made finite; the softmax scale, and with it the K side, may be negative
+    const float val = fminf(fmaxf(sc * sc_mul, -65504.f), 65504.f);
     float* out = reinterpret_cast<float*>(buf + K_BYTES + V_BYTES);
     out[lane] = val;
     // how far a logit may exceed a column's reference maximum in this tile before the maximum has to move:
