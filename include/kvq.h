@@ -240,7 +240,9 @@ KVQ_API int kvq_rope_and_cache_int8(const int64_t* positions, void* query, int64
  * KVQ_ATTN_SHORT_CONTEXT (16): the caller takes the batch's sequences to be no longer than KVQ_SHORT_CONTEXT tokens.
  * The one-row sequences of a small batch (num_seqs x kv heads <= compute units) are then computed by a workgroup per
  * (sequence, kv head), which leaves no partial states to merge.  It decides the launch, never the result: longer
- * sequences -- a captured launch replayed later in the conversation -- come out right as well, only slower.
+ * sequences come out right as well, but on one compute unit per (sequence, kv head), in time proportional to their
+ * length.  A launch captured into a graph takes it along to every replay: set it there only if no replay will see
+ * longer sequences (the Python op layer does so only if the block table cannot hold any).
  *
  * Value range: the weights enter the second product as fp16 numbers
  * p * v_scale * 2^8, so a V row whose scale exceeds 255.8 (int8 codes: absmax

@@ -97,6 +97,69 @@ def test_decode_step_replays_correctly(gpu_device, one_launch):
         assert torch.equal(eager, out), f"replay {it}: graph and eager outputs differ"
 
 
+@pytest.mark.parametrize("one_launch", [False, True], ids=["attention", "one_launch_step"])
+@pytest.mark.parametrize("capacity", [4096, 1024])
+def test_a_step_captured_on_short_lengths_serves_long_ones(gpu_device, capacity, one_launch):
+    """Captured with the lengths of a dummy batch, replayed later in the conversation.  The launch is the one that suits
+    any length the block table holds: where that is more than a short context, it cuts the sequences -- the partial
+    states are in the workspace, which is filled with 0xFF bytes before each replay."""
+    dev = gpu_device
+    hq, hkv, d, bs, B = 32, 8, 128, 16, 2
+    g = torch.Generator().manual_seed(6)
+    nb = B * capacity // bs + 3
+    bt = T.make_block_tables([capacity] * B, bs, nb, g)
+    kv_cpu, _, lay = T.cpu_cache(nb, bs, hkv, d, "HND")
+    rows = [[torch.randn((capacity, hkv, d), generator=g).to(torch.bfloat16) for _ in range(B)] for _ in range(2)]
+    T.fill_cache_from_sources(kv_cpu, lay, bt, [capacity] * B, bs, *rows)
+    kv = T.to_device_cache(kv_cpu, dev, "HND")
+    k, v = L.key_value_views(kv)
+    ksc, vsc = L.scale_views(kv)
+    q = torch.randn((B, hq, d), generator=g).to(torch.bfloat16)
+    q_d, out, bt_d = q.to(dev), torch.zeros((B, hq, d), dtype=torch.bfloat16, device=dev), bt.to(dev)
+    new = [torch.zeros((B, hkv, d), dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    seq_lens = torch.ones((B,), dtype=torch.int32, device=dev)
+    cu = torch.arange(B + 1, dtype=torch.int32, device=dev)
+    ws = torch.empty(ops.paged_attn_workspace_bytes(B, hq, d), dtype=torch.uint8, device=dev)
+
+    def step(stated):
+        if one_launch:
+            ops.decode_attention_with_cache_update(q_d, new[0], new[1], k, v, out, seq_lens, stated, 0.09, bt_d, ksc, vsc,
+                                                   workspace=ws)
+        else:
+            ops.unified_attention(q_d, k, v, out, cu, 1, seq_lens, stated, 0.09, True, block_table=bt_d, k_scale_cache=ksc,
+                                  v_scale_cache=vsc, workspace=ws)
+
+    def load(lens):   # the step's new token is the one that the cache holds at that place
+        seq_lens.copy_(torch.tensor(lens, dtype=torch.int32))
+        for x, r in zip(new, rows):
+            x.copy_(torch.stack([r[i][lens[i] - 1] for i in range(B)]))
+
+    load([40, 9])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step(40)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        step(40)
+    for lens in ([capacity, 900], [40, 33], [700, capacity - 5]):
+        load(lens)
+        ws.fill_(0xFF)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = oracle.paged_attn(q, T.storage_bytes(kv_cpu), lay, bt, torch.tensor(lens, dtype=torch.int32),
+                                 torch.arange(B + 1, dtype=torch.int32), 0.09)
+        T.assert_close_attn(out, want, what=f"replay at {lens}")
+        assert bool((ws == 0xFF).all()) == (capacity <= 1024), f"{lens}: not the launch for the lengths the table holds"
+        out.zero_()                       # eager work between the replays
+        step(max(lens))
+        torch.cuda.synchronize()
+        T.assert_close_attn(out, want, what=f"eager at {lens}")
+
+
 @pytest.mark.parametrize("one_launch", [False, True], ids=["write_then_decode", "one_launch_step"])
 def test_mla_decode_replays_correctly(gpu_device, one_launch):
     dev = gpu_device
