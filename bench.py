@@ -597,7 +597,8 @@ def mixed_main(args, cfg, dev, ops):
     scale = 1.0 / math.sqrt(d)
 
     # context splits of the long runs, as the metadata builder proposes them from the run lengths
-    splits = ops.prefill_context_splits(qls, max(ctx), hq, hkv, places_per_cu=3) if cfg.get("chunk") else 1
+    places = ops.prefill_tile_places(d, False)
+    splits = ops.prefill_context_splits(qls, max(ctx), hq, hkv, places_per_cu=places) if cfg.get("chunk") else 1
     if splits > 1:
         ws = torch.empty(ops.split_prefill_workspace_bytes(B, hq, d, n_tok, splits), dtype=torch.uint8, device=dev)
     # a batch of short runs: the launch that serves it, as the layer asks for it with the builder's workspace

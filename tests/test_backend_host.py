@@ -8,7 +8,7 @@ import types
 import pytest
 import torch
 
-from vllm_metax_amd import _C, platform as P
+from vllm_metax_amd import _C, layout, platform as P
 from vllm_metax_amd.kv_cache_interface import KVQuantMode, get_kv_quant_mode, kv_cache_uses_per_token_head_scales
 from vllm_metax_amd.v1.attention.backends.int8_attn import (
     AttentionType, Int8AttentionBackend, Int8AttentionImpl, Int8AttentionMetadataBuilder, MultipleOf)
@@ -358,6 +358,30 @@ def test_context_split_proposal_follows_the_launch_shape():
     assert f([2048], 131072, 32, 8, max_split_tokens=4096) == 1
     assert f([1024], 131072, 32, 8, max_split_tokens=4096) == 2    # 256 workgroups: two ranges fill the chip's 512 places
     assert f(torch.tensor([300, 1, 1]), 8192, 28, 4) == 4          # the context allows one split per 2048 tokens
+
+
+@pytest.mark.parametrize("head_size,kw,splits", [
+    (128, {}, 6), (128, dict(sliding_window=4096), 4), (128, dict(logits_soft_cap=50.0), 4),
+    (128, dict(alibi_slopes=[0.5] * 32), 4), (64, {}, 6), (64, dict(logits_soft_cap=50.0), 6)])
+def test_layers_ask_for_the_context_splits_their_tile_has_room_for(monkeypatch, head_size, kw, splits):
+    """A 512-token chunk on 32k is 128 workgroups: the builder's metadata holds an answer for layers whose tile fits three
+    workgroups on a compute unit and for those whose tile fits two, and the layer takes its own."""
+    spec = types.SimpleNamespace(block_size=16, num_kv_heads=8, head_size=head_size, num_q_heads=32)
+    cfg = types.SimpleNamespace(scheduler_config=types.SimpleNamespace(max_num_seqs=4))
+    cu = torch.tensor([0, 512], dtype=torch.int32)
+    md = Int8AttentionMetadataBuilder(spec, ["l0"], cfg, "cpu").build(0, types.SimpleNamespace(
+        num_reqs=1, num_actual_tokens=512, max_query_len=512, max_seq_len=32768, query_start_loc=cu, query_start_loc_cpu=cu,
+        seq_lens=torch.tensor([32768], dtype=torch.int32), block_table_tensor=torch.zeros((1, 2048), dtype=torch.int32),
+        slot_mapping=torch.zeros(512, dtype=torch.int64), causal=True))
+    md.workspace = torch.empty(16, dtype=torch.uint8)
+    asked = []
+    stub = types.SimpleNamespace(is_cache=lambda *a: False, cache_ref=lambda c: c,
+                                 paged_attention=lambda *a: asked.append(a[-1]))
+    monkeypatch.setattr(_C, "binding", lambda: stub)
+    impl = Int8AttentionImpl(32, head_size, 0.1, 8, kv_cache_dtype="int8_per_token_head", **kw)
+    q = torch.zeros((512, 32 * head_size), dtype=torch.bfloat16)
+    impl.forward(None, q, None, None, layout.allocate_kv_cache(4, 16, 8, head_size, device="cpu"), md, torch.empty_like(q))
+    assert asked == [splits]
 
 
 def test_native_op_layer_refuses_tensors_without_storage():

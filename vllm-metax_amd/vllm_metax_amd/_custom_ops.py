@@ -410,13 +410,23 @@ def split_prefill_workspace_bytes(max_num_seqs: int, num_q_heads: int, head_size
                                                                          num_tokens, prefill_splits))
 
 
+def prefill_tile_places(head_size: int, extras: bool) -> int:
+    """Workgroups of the prefill tile on a compute unit that context splits should count on (``places_per_cu`` of
+    ``prefill_context_splits``).  ``extras``: the layer has a sliding window, a soft cap or ALiBi; their tile fits two
+    workgroups at head size 128, the plain one three.  512 tokens on 32k cached ones, 32 / 8 heads, four splits (two
+    places) / six (three): plain 384 / 351 us, soft cap 515 / 535, window of 4096 tokens 70.1 / 81.1, of 20000 218 / 236,
+    int4 codes and soft cap 578 / 591.  Head size 64 fits four, and three is the better count: 512 tokens 244 us with six
+    splits, 240 with eight, but 700 tokens on 50k 515 us with four splits and 523 with five."""
+    return 2 if extras and head_size > 64 else 3
+
+
 def prefill_context_splits(query_lens, max_seq_len: int, num_q_heads: int, num_kv_heads: int, num_cus: int = 256,
                            max_split_tokens: int = 4096, places_per_cu: int = 2) -> int:
     """How many context splits a launch should ask for, from what a metadata builder knows on the host: the query
     run lengths of the batch (``query_lens``: a list or CPU tensor; one-token runs do not count), the longest
     sequence, the head counts.  A run of q tokens makes ceil(q / (128 / group)) x Hkv workgroups of the
-    workgroup-shared tile; when the launch's workgroups do not fill ``places_per_cu`` per compute unit and the context
-    is long, the context is cut so that they do -- as long as the partial states stay small (splits x run tokens
+    workgroup-shared tile; when the launch's workgroups do not fill ``places_per_cu`` per compute unit
+    (``prefill_tile_places`` of the layer; the default holds for every layer) and the context is long, the context is cut so that they do -- as long as the partial states stay small (splits x run tokens
     <= ``max_split_tokens``)."""
     group = max(1, num_q_heads // max(1, num_kv_heads))
     lens = [int(x) for x in (query_lens.tolist() if hasattr(query_lens, "tolist") else query_lens)]

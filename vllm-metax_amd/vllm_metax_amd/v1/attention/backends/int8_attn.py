@@ -81,6 +81,8 @@ class Int8AttentionMetadata:
     workspace: torch.Tensor | None
     causal: bool = True
     prefill_splits: int = 1      # context splits of the long query runs (the builder's proposal for this launch)
+    # the same for layers with a sliding window, a soft cap or ALiBi, where it differs (None: prefill_splits)
+    prefill_splits_extras: int | None = None
     use_cascade: bool = False
     common_prefix_len: int = 0
     # False when the builder KNOWS (from the host copy of query_start_loc) that no sequence has exactly one query
@@ -158,22 +160,29 @@ class Int8AttentionMetadataBuilder(_BuilderBase):
         if c.num_reqs > self.max_num_seqs:
             raise RuntimeError(f"batch of {c.num_reqs} sequences exceeds max_num_seqs={self.max_num_seqs}")
         has_decode_rows = True
-        prefill_splits = 1
+        prefill_splits, prefill_splits_extras = 1, None
         qsl_cpu = getattr(c, "query_start_loc_cpu", None)
         if qsl_cpu is not None and c.max_query_len > 1 and qsl_cpu.numel() > 1:
             qlens = qsl_cpu[1:] - qsl_cpu[:-1]
             has_decode_rows = bool((qlens == 1).any())
             # a launch whose long runs make too few workgroups for the chip walks a long context in context splits;
-            # the partial states are indexed by the query row, so every row of the batch counts against the room.
-            # Three workgroups of that tile share a compute unit (512 tokens on 32k cached ones: four ranges 370 us, six 351)
-            prefill_splits = ops.prefill_context_splits(qlens, int(c.max_seq_len), self.num_heads_q, self.num_heads_kv,
-                                                        max_split_tokens=self.MAX_SPLIT_TOKENS, places_per_cu=3)
-            while prefill_splits > 1 and prefill_splits * int(c.num_actual_tokens) > self.MAX_SPLIT_TOKENS:
-                prefill_splits -= 1
+            # the partial states are indexed by the query row, so every row of the batch counts against the room
+            def propose(extras: bool) -> int:
+                n = ops.prefill_context_splits(qlens, int(c.max_seq_len), self.num_heads_q, self.num_heads_kv,
+                                               max_split_tokens=self.MAX_SPLIT_TOKENS,
+                                               places_per_cu=ops.prefill_tile_places(self.headdim, extras))
+                while n > 1 and n * int(c.num_actual_tokens) > self.MAX_SPLIT_TOKENS:
+                    n -= 1
+                return n
+
+            prefill_splits = propose(False)
+            if prefill_splits > 1:
+                prefill_splits_extras = propose(True)
         workspace = self._get_workspace()
         return Int8AttentionMetadata(
             has_decode_rows=has_decode_rows,
             prefill_splits=prefill_splits,
+            prefill_splits_extras=prefill_splits_extras,
             short_runs=self._short_runs,
             num_actual_tokens=c.num_actual_tokens,
             max_query_len=c.max_query_len,
@@ -453,14 +462,17 @@ class Int8AttentionImpl(_ImplBase):
         workspace, short_runs = md.workspace, getattr(md, "short_runs", False)
         if workspace is None:
             workspace, short_runs = self._own_workspace(query, md)
+        splits = getattr(md, "prefill_splits", 1)
+        if splits > 1 and (self._window > 0 or self.logits_soft_cap > 0 or self.alibi_slopes is not None):
+            own = getattr(md, "prefill_splits_extras", None)
+            splits = splits if own is None else own
         flags = (_C.KVQ_ATTN_CAUSAL if md.causal else 0) | (_C.KVQ_ATTN_SHORT_RUNS if short_runs else 0) \
             | (0 if getattr(md, "has_decode_rows", True) else _C.KVQ_ATTN_NO_DECODE_ROWS)
         _C.binding().paged_attention(
             query, output, md.num_actual_tokens, self.num_heads, kv_cache, geom.struct_addr, geom.base_ptr,
             md.query_start_loc, md.seq_lens, md.block_table, md.max_query_len, md.max_seq_len, self.scale, flags, self._window,
             self.logits_soft_cap, self._sinks_on(query.device) if self.sinks is not None else None,
-            self._alibi_on(query.device) if self.alibi_slopes is not None else None, None, workspace,
-            getattr(md, "prefill_splits", 1))
+            self._alibi_on(query.device) if self.alibi_slopes is not None else None, None, workspace, splits)
         return output
 
     def _own_workspace(self, query, md):
