@@ -405,7 +405,7 @@ def test_whole_sequences(gpu_device, form, layout, hq, hkv, d, ctx, window, soft
 @pytest.mark.parametrize("layout,hq,hkv,d,ctx", [
     ("HND", 32, 8, 128, [3001]), ("NHD", 32, 8, 128, [1100, 5000, 33]), ("HND", 28, 4, 128, [2000, 1, 0, 4097, 700]),
     ("NHD", 32, 16, 128, [2048] * 5), ("HND", 32, 16, 64, [2048] * 6), ("HND", 24, 12, 128, [1500, 1025]),
-    ("HND", 9, 3, 64, [40000])])
+    ("HND", 9, 3, 64, [40000]), ("HND", 24, 12, 128, [4000]), ("NHD", 32, 32, 128, [3000, 40]), ("HND", 40, 40, 64, [900, 2500, 7])])
 def test_a_handful_of_sequences(gpu_device, layout, hq, hkv, d, ctx):
     """Batches around the size (48 cuts per sequence on 256 compute units) below which a workgroup serves fewer kv
     heads than it could, with kv head counts that do not divide into them and a sequence of hundreds of shares."""
@@ -415,6 +415,27 @@ def test_a_handful_of_sequences(gpu_device, layout, hq, hkv, d, ctx):
     got, lse = run_unified(gpu_device, kv, layout, bt, q, sl, cu, scale, out_dtype=torch.float32, want_lse=True)
     T.assert_close_attn(got, want, atol=2e-3, rtol=2e-3, what=f"{hq}/{hkv} d{d} ctx={ctx}")
     torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (28, 4, 128), (24, 12, 128), (32, 16, 64), (32, 32, 128)])
+def test_a_handful_of_sequences_is_one_round_of_workgroups(gpu_device, hq, hkv, d):
+    """One sequence of 125 tiles with fewer kv heads per workgroup: a workgroup per (share, kv head), and no more of them
+    than compute units.  The shares are counted by the partial states that they leave ([share + sequence][q head][dim] at
+    the workspace's start)."""
+    kv, lay, bt, q, sl, cu = build_case([4000], hq, hkv, d, 16, "HND", hkv)
+    dev = gpu_device
+    kvd = T.to_device_cache(kv, dev, "HND")
+    k, v = L.key_value_views(kvd)
+    ks, vs = L.scale_views(kvd)
+    ws = torch.full((ops.paged_attn_workspace_bytes(1, hq, d, dev),), 0xFF, dtype=torch.uint8, device=dev)
+    out = torch.empty_like(q, device=dev)
+    ops.unified_attention(q.to(dev), k, v, out, cu.to(dev), 1, sl.to(dev), 4000, 0.1, True, block_table=bt.to(dev),
+                          k_scale_cache=ks, v_scale_cache=vs, workspace=ws)
+    torch.cuda.synchronize()
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    states = ws[:(cus + 1) * hq * d * 4].view(cus + 1, -1)
+    shares = int((states != 0xFF).any(1).sum())
+    assert 1 < shares and shares * hkv <= max(cus, hkv), f"{shares} shares x {hkv} kv heads on {cus} compute units"
 
 
 @pytest.mark.parametrize("n", [64, 65, 128, 191, 256, 257, 300])

@@ -904,11 +904,16 @@ int launch_streamk(const StreamKArgs& args, hipStream_t s) {
   // A step on MI355X, 8 kv heads of 128, before / after: 1 sequence of 2000 tokens 16.9 / 15.8 us, 16k 22.1 / 21.1,
   // 100k 49.5 / 47.0; 4 of 1k - 8k 24.5 / 22.6; 3 on 4 kv heads 21.0 / 18.5; token-major cache, 4 of 1k - 8k: 26.2 / 22.9.
   // Not at head size 256 (2 of 1k - 8k: 31.5 / 33.6), whose states are twice as long to fold.
+  // One round of workgroups: more than eight kv heads would otherwise make two and more of them, of shares too short to be
+  // worth it.
   if constexpr (D <= 128) {
+    const int units = a.num_wg;
     while (!a.fixed_spans && hpw > 1 && a.num_wg > 48 * a.num_seqs) {
       hpw /= 2;
       a.num_wg /= 2;
     }
+    const int groups = (hkv + hpw - 1) / hpw;
+    if (hpw < heads_per_wg(hkv) && a.num_wg * groups > units) a.num_wg = units / groups > 1 ? units / groups : 1;
   }
   // a head's records of a block back to back (HND order): the tile loads may stream past the caches
   const bool stream = a.io.g.stride_slot == 2 * (code_bytes(a.io.g) + 4) && a.io.g.block_size >= 16;
