@@ -586,3 +586,34 @@ def test_negative_softmax_scale(gpu_device, code, d, window, cap):
         torch.cuda.synchronize()
         T.assert_close_attn(out, want, what=f"negative scale {code} d{d}, {splits} ranges")
         torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("d,window", [(128, 0), (64, 0), (128, 100), (64, 100)])
+@pytest.mark.parametrize("code", ["int8", "fp8", "int4"])
+def test_output_types_of_the_shared_tile(gpu_device, code, d, window):
+    """Long runs write bf16, fp16 or fp32 rows: the 16-bit ones are the fp32 row rounded to nearest even."""
+    from vllm_metax_amd.kv_cache_interface import KVQuantMode
+    hq, hkv, bs, dev = 14, 2, 16, gpu_device
+    ct = {"int8": oracle.CODE_INT8, "fp8": oracle.CODE_FP8, "int4": oracle.CODE_INT4}[code]
+    ctx, qls = [70, 333, 96], [70, 100, 33]
+    g = torch.Generator().manual_seed(d)
+    nb = sum((c + bs - 1) // bs for c in ctx) + 5
+    kv_cpu, _, lay = T.cpu_cache(nb, bs, hkv, d, "HND", code_type=ct)
+    bt = T.make_block_tables(ctx, bs, nb, g)
+    src = [[torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in ctx] for _ in range(2)]
+    T.fill_cache_from_sources(kv_cpu, lay, bt, ctx, bs, *src, code_type=ct)
+    q = torch.randn((sum(qls), hq, d), generator=g).to(torch.bfloat16)
+    kv = T.to_device_cache(kv_cpu, dev, "HND", code_type=ct)
+    k, v = L.key_value_views(kv)
+    ks, vs = L.scale_views(kv)
+    cu = torch.tensor([0] + torch.tensor(qls).cumsum(0).tolist(), dtype=torch.int32, device=dev)
+    outs = {}
+    for dtype in (torch.float32, torch.bfloat16, torch.float16):
+        outs[dtype] = torch.zeros(q.shape, dtype=dtype, device=dev)
+        ops.unified_attention(q.to(dev), k, v, outs[dtype], cu, max(qls), torch.tensor(ctx, dtype=torch.int32, device=dev),
+                              max(ctx), d ** -0.5, True, window_size=(window - 1, 0) if window else (-1, -1),
+                              block_table=bt.to(dev), k_scale_cache=ks, v_scale_cache=vs,
+                              kv_quant_mode=getattr(KVQuantMode, code.upper() + "_PER_TOKEN_HEAD"))
+    torch.cuda.synchronize()
+    for dtype, out in outs.items():
+        assert torch.equal(out, outs[torch.float32].to(dtype)), dtype
