@@ -570,9 +570,9 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
       step_fn(std::false_type{}, I0{}, t);
       step_fn(std::false_type{}, I1{}, t + 1);
     }
-    for (; t < t_hi; t += 2) {   // an odd end runs one step past it: every slot is masked there
+    for (; t < t_hi; t += 2) {   // (the same end for all waves, in whichever loops they have been)
       step_fn(std::true_type{}, I0{}, t);
-      step_fn(std::true_type{}, I1{}, t + 1);
+      if (t + 1 < t_hi) step_fn(std::true_type{}, I1{}, t + 1);
     }
     // no load may land in LDS after the workgroup has given it up
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
