@@ -617,3 +617,25 @@ def test_output_types_of_the_shared_tile(gpu_device, code, d, window):
     torch.cuda.synchronize()
     for dtype, out in outs.items():
         assert torch.equal(out, outs[torch.float32].to(dtype)), dtype
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(28, 4, 128), (8, 8, 64), (32, 8, 128)])
+@pytest.mark.parametrize("window", [0, 1, 20, 40, 100])
+def test_odd_ends_of_the_shared_tile(gpu_device, hq, hkv, d, window):
+    """Runs that end in an odd tile, whole and in ranges, with windows that put some waves of a workgroup into the steps at
+    its lower edge to the very end and others not: the same steps for all of them."""
+    ctx, qls = [33, 95, 161, 224, 290], [33, 95, 150, 130, 65]
+    kv, lay, bt, q, sl, cu = build(ctx, qls, hq, hkv, d, 16, layout="HND", seed=hq + window)
+    scale = 1 / math.sqrt(d)
+    want = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, scale, sliding_window=window)
+    dev = gpu_device
+    kvd = T.to_device_cache(kv, dev, "HND")
+    k, v = L.key_value_views(kvd)
+    ks, vs = L.scale_views(kvd)
+    for splits in (1, 2):
+        out = torch.full(q.shape, float("nan"), dtype=q.dtype, device=dev)
+        ops.unified_attention(q.to(dev), k, v, out, cu.to(dev), max(qls), sl.to(dev), max(ctx), scale, True,
+                              window_size=(window - 1, 0) if window else (-1, -1), block_table=bt.to(dev), k_scale_cache=ks,
+                              v_scale_cache=vs, prefill_splits=splits)
+        torch.cuda.synchronize()
+        T.assert_close_attn(out, want, what=f"odd ends, window {window}, {splits} ranges")

@@ -563,7 +563,7 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
       const int t_head = min(t_hi, ((max(wave_max_first, wg_first) + kTile - 1) / kTile + 1) & ~1);
       for (; t < t_head; t += 2) {
         step_fn(std::true_type{}, I0{}, t);
-        step_fn(std::true_type{}, I1{}, t + 1);
+        if (t + 1 < t_hi) step_fn(std::true_type{}, I1{}, t + 1);
       }
     }
     for (; t < t_plain; t += 2) {
