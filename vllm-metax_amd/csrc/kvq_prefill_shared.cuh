@@ -11,7 +11,11 @@
 // of LDS each, which is what the rest follows from: tiles go from memory into LDS without passing through registers, the
 // operands of a tile are read as they are used up, a token's scales reach the lanes by a broadcast inside the multiply
 // (one LDS read per tile instead of four 16-byte ones) and a wave loads from one half tile only (one block table entry, one
-// resource).  At three workgroups the vector unit is 60 % busy, the matrix unit 39 %, the LDS 44 %.
+// resource).  168 registers hold what a step needs and no more: lane number, column and limit, which only the masked steps
+// and the ends of the walk use, are worked out anew there.  Kept through the loops they were spilled, 11 to 14 of them, and
+// some reloaded in every step behind the next tile's loads, which the reload then waited for (16 prompts of 300 tokens 60.1
+// -> 54.5 us, one of 2000 82.9 -> 74.0, the mixed step below 447 -> 437).  One value is left, spilled outside the loops; head
+// size 64 spills up to three with the extras, at head size 128 those do not spill.  At three workgroups the vector unit is 60 % busy, the matrix unit 39 %, the LDS 44 %.
 // Measured on MI355X against two workgroups per compute unit with register loads and padded tiles: 4 x 2048 new tokens on
 // 0-6k cached ones beside 60 decode rows (28/4 heads) 525 -> 456 us for the step, a 6000-token prompt (32/8 heads)
 // 444 -> 389 us, 512 tokens on 32k in context ranges 384 -> 351 us, int4 cache 235 -> 191 us, head size 64 307 -> 255 us.
@@ -163,8 +167,16 @@ struct SharedTile {
     }
     *reinterpret_cast<u32x2*>(buf + p.v_out + b * (D / 4) * 16) = o;   // dim 4 dq + b is row b D/4 + dq
   }
+  // The lane number, worked out anew (kept from tile to tile it, and what follows from it, were spilled).
+  __device__ static __forceinline__ uint32_t lane_anew() {
+    uint32_t lane;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane));
+    return lane;
+  }
   // The tile's scales; one wave does it.
-  __device__ static __forceinline__ void expand_scales(float sc, uint8_t* buf, int lane, float sc_mul) {
+  __device__ static __forceinline__ void expand_scales(float sc, uint8_t* buf, float k_mul) {
+    const uint32_t lane = lane_anew();
+    const float sc_mul = lane < 32 ? k_mul : kPScale;
     // a slot that holds no token: anything, made finite; the softmax scale, and with it the K side, may be negative
     const float val = fminf(fmaxf(sc * sc_mul, -65504.f), 65504.f);
     float* out = reinterpret_cast<float*>(buf + K_BYTES + V_BYTES);
@@ -339,19 +351,33 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
   if (q_len <= 1 || q0 >= q_len || len <= 0) return;   // uniform over the workgroup
   if (a.route == 1 && q_len * io.group < 64) return;    // the per-wave tile's
 
-  // column of this lane: (query token q0 + n / group, head n % group), n = wave * 32 + (lane & 31)
+  // column of a lane: (query token q0 + n / group, head n % group), n = wave * 32 + (lane & 31); n / group by a
+  // reciprocal: both are small, and n + 1/2 is half a column away from every multiple
   const int ctx = len - q_len;
-  const int n = wave * 32 + (lane & 31);
-  const int qt = n / io.group;
-  const int qi = q0 + qt;
-  const bool valid = qt < a.q_tokens && qi < q_len;
-  const int head = hkv * io.group + (n - qt * io.group);
-  const int64_t row = q_begin + (valid ? qi : q0);
-  int lim = a.causal ? ctx + qi + 1 : len;
-  lim = lim < 0 ? 0 : (lim > len ? len : lim);
-  const int limit = valid ? lim : 0;
+  struct Column {
+    bool valid;
+    int qi, head;
+    int64_t row;
+  };
+  const float per_column = as_f32(__builtin_amdgcn_readfirstlane(as_u32(__builtin_amdgcn_rcpf((float)io.group))));
+  auto column = [&](int of_lane) __attribute__((always_inline)) {
+    const int n = wave * 32 + (of_lane & 31);
+    const int qt = (int)(((float)n + 0.5f) * per_column);
+    Column c;
+    c.qi = q0 + qt;
+    c.valid = qt < a.q_tokens && c.qi < q_len;
+    c.head = hkv * io.group + (n - qt * io.group);
+    c.row = q_begin + (c.valid ? c.qi : q0);
+    return c;
+  };
+  auto limit_of = [&](const Column& c) __attribute__((always_inline)) {
+    const int lim = a.causal ? ctx + c.qi + 1 : len;
+    return c.valid ? (lim < 0 ? 0 : (lim > len ? len : lim)) : 0;
+  };
+  const Column col = column(lane);
+  int limit = limit_of(col), step_lane = lane;   // of the masked steps
   const int wave_max_limit = wave_max_i32(limit);
-  const int wave_min_limit = -wave_max_i32(valid ? -lim : -0x7fffffff);
+  const int wave_min_limit = -wave_max_i32(col.valid ? -limit : -0x7fffffff);
   int wg_limit = a.causal ? ctx + min(q0 + a.q_tokens, q_len) : len;
   wg_limit = wg_limit < 0 ? 0 : (wg_limit > len ? len : wg_limit);
   const int t_end = (wg_limit + kTile - 1) / kTile;
@@ -426,16 +452,16 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
     next_place();
 
     half8_t qop[KS];
-    const int64_t elem = row * io.q_stride_t + (int64_t)(valid ? head : hkv * io.group) * io.q_stride_h;
-    if (q_dtype == KVQ_BF16) W::template load_q<KVQ_BF16>(io, elem, valid, lane, qop);
-    else if (q_dtype == KVQ_F16) W::template load_q<KVQ_F16>(io, elem, valid, lane, qop);
-    else W::template load_q<KVQ_F32>(io, elem, valid, lane, qop);
-    const float sc_mul = lane < 32 ? io.scale_log2 * DTile::kKScaleMul : kPScale;
+    const int64_t elem = col.row * io.q_stride_t + (int64_t)(col.valid ? col.head : hkv * io.group) * io.q_stride_h;
+    if (q_dtype == KVQ_BF16) W::template load_q<KVQ_BF16>(io, elem, col.valid, lane, qop);
+    else if (q_dtype == KVQ_F16) W::template load_q<KVQ_F16>(io, elem, col.valid, lane, qop);
+    else W::template load_q<KVQ_F32>(io, elem, col.valid, lane, qop);
+    const float k_mul = io.scale_log2 * DTile::kKScaleMul;
     float ali = 0.f;
     bool biased = false;
     if constexpr (EXT) {
       biased = io.alibi != nullptr;
-      ali = alibi_slope(io.alibi, valid ? head : hkv * io.group);
+      ali = alibi_slope(io.alibi, col.valid ? col.head : hkv * io.group);
     }
 
     auto fence = []() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
@@ -448,7 +474,7 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
     for (int i = 0; i < 4; ++i) W::expand_k_piece(e, places, i, bufs);
 #pragma unroll
     for (int i = 0; i < 5; ++i) W::template expand_v_piece<true>(e, places, i, bufs);
-    if (wave == 0) W::expand_scales(e.sc, bufs, lane, sc_mul);
+    if (wave == 0) W::expand_scales(e.sc, bufs, k_mul);
     tile_barrier();
     issue(raws);
     next_place();
@@ -494,7 +520,7 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
           }
         fence();
       }
-      const float d = W::template logits<MASK, EXT>(ksc, io, ali, limit, wspan, t, lane, biased, s);
+      const float d = W::template logits<MASK, EXT>(ksc, io, ali, limit, wspan, t, step_lane, biased, s);
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) read_v(buf, mt, 0);
       // The reference maximum only has to keep 2^(logit - m) in range: it stays put while no logit exceeds it by more
@@ -511,7 +537,7 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) o[mt] *= alpha;
       }
-      if (wave == 0) W::expand_scales(e.sc, nbuf, lane, sc_mul);
+      if (wave == 0) W::expand_scales(e.sc, nbuf, k_mul);
       auto weights = [&](int i) __attribute__((always_inline)) {
         float x[2];
 #pragma unroll
@@ -570,6 +596,10 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
       step_fn(std::false_type{}, I0{}, t);
       step_fn(std::false_type{}, I1{}, t + 1);
     }
+    if (t < t_hi) {   // what the plain steps did not need
+      step_lane = (int)W::lane_anew();
+      limit = limit_of(column(step_lane));
+    }
     for (; t < t_hi; t += 2) {   // (the same end for all waves, in whichever loops they have been)
       step_fn(std::true_type{}, I0{}, t);
       if (t + 1 < t_hi) step_fn(std::true_type{}, I1{}, t + 1);
@@ -578,12 +608,14 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
 
+  const int lane_end = (int)W::lane_anew();
+  const Column end = column(lane_end);
   l += __shfl_xor(l, 32, kWave);
-  if (!valid) return;
-  const int g = lane >> 5;
+  if (!end.valid) return;
+  const int g = lane_end >> 5;
   if (nsplit > 1) {
     // the range's state: the row as accumulated (without the factor the weights carry), the reference maximum, the sum
-    float* p = a.part + (((int64_t)row * io.num_q_heads + head) * nsplit + split) * (D + 2);
+    float* p = a.part + ((end.row * io.num_q_heads + end.head) * nsplit + split) * (D + 2);
     const float unit = 1.0f / DTile::kOutDiv;
 #pragma unroll
     for (int i = 0; i < D / 8; ++i) {
@@ -598,9 +630,9 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
     }
     return;
   }
-  if (l > 0.f) l += sink_term(io.sinks, head, m);   // a row without a visible key keeps its zeros
+  if (l > 0.f) l += sink_term(io.sinks, end.head, m);   // a row without a visible key keeps its zeros
   const float mul = l > 0.f ? 1.0f / (l * DTile::kOutDiv) : 0.f;
-  const int64_t base = row * io.out_stride_t + (int64_t)head * io.out_stride_h;
+  const int64_t base = end.row * io.out_stride_t + (int64_t)end.head * io.out_stride_h;
   // One straight run of stores per output type: a short prompt's launch fetches all of this for the first time (asked for
   // the type and branching on NaN element by element it was 2300 instructions: 70 tokens, 8 kv heads of 128, captured, a step
   // 15.9 us in the kernel that knew its type at compile time, 17.6 so, 15.2 now).
@@ -621,7 +653,7 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
   else if (out_dtype == KVQ_F16) store_row(std::integral_constant<int, KVQ_F16>{});
   else store_row(std::integral_constant<int, KVQ_F32>{});
   if (io.lse != nullptr && g == 0)
-    io.lse[row * io.num_q_heads + head] = l > 0.f ? (m + __builtin_amdgcn_logf(l)) * kLn2 : -INFINITY;
+    io.lse[end.row * io.num_q_heads + end.head] = l > 0.f ? (m + __builtin_amdgcn_logf(l)) * kLn2 : -INFINITY;
 }
 
 // The merge of the context splits: grid (query rows, ceil(Hq / 4)), a wave per (row of a run, q head), a lane D / 64 dims.
