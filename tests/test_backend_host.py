@@ -362,10 +362,12 @@ def test_context_split_proposal_follows_the_launch_shape():
 
 @pytest.mark.parametrize("head_size,kw,splits", [
     (128, {}, 6), (128, dict(sliding_window=4096), 4), (128, dict(logits_soft_cap=50.0), 4),
-    (128, dict(alibi_slopes=[0.5] * 32), 4), (64, {}, 6), (64, dict(logits_soft_cap=50.0), 6)])
+    (128, dict(alibi_slopes=[0.5] * 32), 4), (64, {}, 6), (64, dict(logits_soft_cap=50.0), 6),
+    (64, dict(sliding_window=4096), 6), (64, dict(sliding_window=1024), 4), (128, dict(sliding_window=100), 1)])
 def test_layers_ask_for_the_context_splits_their_tile_has_room_for(monkeypatch, head_size, kw, splits):
     """A 512-token chunk on 32k is 128 workgroups: the builder's metadata holds an answer for layers whose tile fits three
-    workgroups on a compute unit and for those whose tile fits two, and the layer takes its own."""
+    workgroups on a compute unit and for those whose tile fits two, and the layer takes its own, or as many as its window
+    leaves tokens for."""
     spec = types.SimpleNamespace(block_size=16, num_kv_heads=8, head_size=head_size, num_q_heads=32)
     cfg = types.SimpleNamespace(scheduler_config=types.SimpleNamespace(max_num_seqs=4))
     cu = torch.tensor([0, 512], dtype=torch.int32)
