@@ -517,7 +517,7 @@ def test_shared_tile_at_its_edges(gpu_device, hq, hkv, d, bs, layout, code, shif
 
 
 @pytest.mark.parametrize("hq,hkv,n", [(32, 8, 5), (32, 8, 6), (32, 8, 2), (28, 4, 10), (28, 4, 11), (24, 12, 3), (9, 3, 1), (32, 16, 1),
-                                      (8, 2, 64), (8, 2, 65)])
+                                      (8, 2, 64), (8, 2, 65), (32, 32, 1), (40, 40, 7), (32, 16, 30)])
 def test_short_run_shares_by_kv_heads(gpu_device, hq, hkv, n):
     """The batch sizes around which a workgroup of the short-run launch serves fewer kv heads (24 cuts per item, on
     256 compute units), kv head counts that do not divide into them, and a single item; 64 items, the most that the prologue holds, and
@@ -530,6 +530,26 @@ def test_short_run_shares_by_kv_heads(gpu_device, hq, hkv, n):
     got, lse = run(gpu_device, kv, "HND", bt, q, sl, cu, 4, scale, want_lse=True)
     T.assert_close_attn(got, want, what=f"{n} short runs, {hq}/{hkv}")
     torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (24, 12, 128), (32, 32, 128), (40, 40, 64)])
+def test_short_runs_are_one_round_of_workgroups(gpu_device, hq, hkv, d):
+    """One run of three tokens on 125 tiles: a workgroup per (share, group of kv heads), one kv head each here, and no more
+    of them than compute units.  A share leaves its states in slots 2 w and 2 w + 1 ([slot][kv head][row][dim])."""
+    kv, lay, bt, q, sl, cu = build([4000], [3], hq, hkv, d, 16, layout="HND", seed=hkv)
+    dev = gpu_device
+    kvd = T.to_device_cache(kv, dev, "HND")
+    k, v = L.key_value_views(kvd)
+    ks, vs = L.scale_views(kvd)
+    ws = torch.full((ops.short_runs_workspace_bytes(1, hq, hkv, d, 3, dev),), 0xFF, dtype=torch.uint8, device=dev)
+    out = torch.empty_like(q, device=dev)
+    ops.unified_attention(q.to(dev), k, v, out, cu.to(dev), 3, sl.to(dev), 4000, 0.1, True, block_table=bt.to(dev),
+                          k_scale_cache=ks, v_scale_cache=vs, workspace=ws, short_runs=True)
+    torch.cuda.synchronize()
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    states = ws[:2 * cus * hq * 3 * d * 4].view(cus, -1)
+    shares = int((states != 0xFF).any(1).sum())
+    assert 1 < shares and shares * hkv <= max(cus, hkv), f"{shares} shares x {hkv} kv heads on {cus} compute units"
 
 
 @pytest.mark.parametrize("hq,hkv,splits", [(32, 8, 6), (32, 8, 3), (16, 4, 2), (16, 4, 3), (12, 3, 8), (16, 2, 4), (9, 1, 8)])
