@@ -29,8 +29,8 @@ extern "C" {
 
 /* 20: kvq_mla_prefill_attn takes `causal` as a set of flags (any non-zero value meant causal up to 18; 2 is a flag of
  * its own since 19, which other builds of 19 may not know).  21: KVQ_ATTN_SHORT_RUNS and its workspace query.  22:
- * KVQ_ATTN_SHORT_CONTEXT and the fused write's form with flags. */
-#define KVQ_ABI_VERSION 22
+ * KVQ_ATTN_SHORT_CONTEXT and the fused write's form with flags.  23: kvq_short_context_tokens. */
+#define KVQ_ABI_VERSION 23
 
 #define KVQ_OK 0
 #define KVQ_EINVAL (-22)
@@ -95,7 +95,7 @@ typedef struct kvq_cache_geom {
 #define KVQ_ATTN_NO_DECODE_ROWS 2
 #define KVQ_ATTN_SHORT_RUNS 4
 #define KVQ_ATTN_SHORT_CONTEXT 16
-/* tokens up to which a caller sets it */
+/* tokens up to which a caller sets it at most; kvq_short_context_tokens() knows the batch */
 #define KVQ_SHORT_CONTEXT 1024
 
 /* Byte geometry of the int8 MLA latent cache: per block, block_size code rows
@@ -237,7 +237,8 @@ KVQ_API int kvq_rope_and_cache_int8(const int64_t* positions, void* query, int64
  * For any other batch the flag changes nothing.  Without it such a batch goes through the decode and prefill
  * kernels, whatever the workspace's size; the results agree within the tolerance, not bit for bit.
  *
- * KVQ_ATTN_SHORT_CONTEXT (16): the caller takes the batch's sequences to be no longer than KVQ_SHORT_CONTEXT tokens.
+ * KVQ_ATTN_SHORT_CONTEXT (16): the caller takes the batch's sequences to be no longer than KVQ_SHORT_CONTEXT tokens
+ * (kvq_short_context_tokens(): the length up to which it pays for the batch at hand).
  * The one-row sequences of a small batch (num_seqs x kv heads <= compute units) are then computed by a workgroup per
  * (sequence, kv head), which leaves no partial states to merge.  It decides the launch, never the result: longer
  * sequences come out right as well, but on one compute unit per (sequence, kv head), in time proportional to their
@@ -315,6 +316,10 @@ KVQ_API int kvq_paged_attn_int8_fused_write(void* out, int out_dtype, int64_t ou
                         int num_seqs, int num_q_heads, float scale, int window_size,
                         float softcap, const float* sinks, const float* alibi_slopes, float* lse, void* workspace, size_t workspace_bytes,
                         kvq_stream_t stream);
+
+/* Tokens up to which KVQ_ATTN_SHORT_CONTEXT pays for a batch of num_seqs sequences on such a cache, at most
+ * KVQ_SHORT_CONTEXT. */
+KVQ_API int kvq_short_context_tokens(const kvq_cache_geom* geom, int num_seqs);
 
 /* The same with flags: 0 or KVQ_ATTN_SHORT_CONTEXT. */
 KVQ_API int kvq_paged_attn_int8_fused_write_flags(void* out, int out_dtype, int64_t out_stride_t, int64_t out_stride_h,

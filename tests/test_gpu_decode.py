@@ -455,3 +455,39 @@ def test_batches_around_the_sequences_a_lane_holds(gpu_device, hq, hkv, layout, 
     got, lse = run_unified(gpu_device, kv, layout, bt, q, sl, cu, scale, out_dtype=torch.float32, want_lse=True)
     T.assert_close_attn(got, want, atol=2e-3, rtol=2e-3, what=f"{n} sequences {hq}/{hkv}")
     torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("form,hq,hkv,d,n,length,window,whole", [
+    ("int8", 16, 1, 128, 3, 512, 0, True), ("int8", 16, 1, 128, 3, 513, 0, False), ("int8", 16, 1, 128, 33, 1000, 0, True),
+    ("fp8", 16, 2, 128, 16, 768, 0, True), ("fp8", 16, 2, 128, 16, 769, 0, False), ("int8", 28, 4, 128, 8, 1000, 0, False),
+    ("int8", 28, 4, 128, 9, 1000, 0, True), ("int8", 32, 8, 128, 1, 1024, 0, True), ("int8", 32, 8, 128, 1, 1025, 0, False),
+    ("int8", 16, 2, 256, 4, 256, 0, True), ("int8", 16, 2, 256, 4, 257, 0, False), ("int8", 16, 2, 256, 16, 1000, 0, True),
+    ("int4", 16, 2, 256, 4, 512, 0, True), ("int4", 16, 2, 256, 4, 513, 0, False), ("int8", 8, 1, 64, 1, 1024, 0, True),
+    ("int8", 16, 2, 256, 4, 3000, 300, False), ("int8", 16, 2, 256, 4, 3000, 200, True)])
+def test_length_up_to_which_sequences_are_not_cut(gpu_device, form, hq, hkv, d, n, length, window, whole):
+    """The rule follows kv heads, head size, codes and batch, by the stated length or by the window; cut sequences leave
+    partial states in the workspace.  Either way the oracle's rows, also of an empty and of a one-token sequence."""
+    from vllm_metax_amd.kv_cache_interface import KVQuantMode
+    ctx = [length] * n if n < 3 else [length, 0, 1] + [length - 7 * (i % 9) for i in range(n - 3)]
+    g = torch.Generator().manual_seed(d + n)
+    code = {"int8": oracle.CODE_INT8, "fp8": oracle.CODE_FP8, "int4": oracle.CODE_INT4}[form]
+    kv, _, lay = T.cpu_cache(sum((c + 15) // 16 for c in ctx) + 5, 16, hkv, d, "HND", code_type=code)
+    T.storage_bytes(kv).fill_(0xFF)
+    bt = T.make_block_tables(ctx, 16, kv.shape[0], g)
+    src = [[torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in ctx] for _ in range(2)]
+    T.fill_cache_from_sources(kv, lay, bt, ctx, 16, *src, code_type=code)
+    q = torch.randn((n, hq, d), generator=g).to(torch.bfloat16)
+    sl, cu = torch.tensor(ctx, dtype=torch.int32), torch.arange(n + 1, dtype=torch.int32)
+    want = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, 0.09, sliding_window=window, code_type=code)
+    dev = gpu_device
+    kvd = T.to_device_cache(kv, dev, "HND", code_type=code)
+    k, v = L.key_value_views(kvd)
+    ks, vs = L.scale_views(kvd)
+    out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=dev)
+    ws = torch.full((ops.paged_attn_workspace_bytes(n, hq, d, dev),), 0xFF, dtype=torch.uint8, device=dev)
+    ops.unified_attention(q.to(dev), k, v, out, cu.to(dev), 1, sl.to(dev), length, 0.09, True,
+                          window_size=(window - 1, 0) if window else (-1, -1), block_table=bt.to(dev), k_scale_cache=ks,
+                          v_scale_cache=vs, workspace=ws, kv_quant_mode=getattr(KVQuantMode, form.upper() + "_PER_TOKEN_HEAD"))
+    torch.cuda.synchronize()
+    T.assert_close_attn(out, want, atol=2e-3, rtol=2e-3, what=f"{form} {hq}/{hkv} d{d} n={n} length {length}")
+    assert bool((ws == 0xFF).all()) == whole

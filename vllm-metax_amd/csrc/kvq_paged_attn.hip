@@ -15,6 +15,7 @@ int launch_decode_streamk(const StreamKArgs& a, int q_dtype, int out_dtype, hipS
 size_t streamk_workspace_bytes(int max_num_seqs, int num_q_heads, int head_size, int num_wg);
 size_t streamk_slots(int max_num_seqs, int num_wg);
 int decode_streamk_num_wg(int num_kv_heads);
+int short_context_tokens(const kvq_cache_geom& g, int num_seqs);
 bool whole_sequences(int num_seqs, int num_kv_heads, int num_cus, bool short_context);
 int validate_common(const char* op, const void* q, const void* cache, const kvq_cache_geom* geom,
                     const int32_t* block_table, const int32_t* seq_lens, int num_seqs, int num_q_heads);
@@ -87,7 +88,8 @@ static int paged_attn_launch(const char* op, void* out, int out_dtype, int64_t o
   const bool no_decode_rows = (causal & KVQ_ATTN_NO_DECODE_ROWS) != 0;
   const bool want_short_runs = (causal & KVQ_ATTN_SHORT_RUNS) != 0;
   // (a window bounds a decode row's tokens as well as the sequence's length does)
-  const bool short_context = (causal & KVQ_ATTN_SHORT_CONTEXT) != 0 || (window_size > 0 && window_size <= KVQ_SHORT_CONTEXT);
+  const bool short_context = (causal & KVQ_ATTN_SHORT_CONTEXT) != 0 ||
+                             (window_size > 0 && window_size <= short_context_tokens(*geom, num_seqs));
   causal &= KVQ_ATTN_CAUSAL;
   KVQ_REQUIRE(out != nullptr, "%s: out is NULL", op);
   KVQ_REQUIRE(max_query_len >= 1, "%s: max_query_len must be >= 1", op);

@@ -177,6 +177,23 @@ size_t streamk_workspace_bytes(int max_num_seqs, int num_q_heads, int head_size,
 
 int decode_streamk_num_wg(int num_kv_heads) { return streamk_num_wg(num_kv_heads); }
 
+// Tokens up to which that form pays.  With a few kv heads the cut has the waves of a workgroup share a head's tiles as well,
+// and a small batch leaves it the units it needs; wide heads make the serial chain longer.  MI355X, a step, captured, cut / whole:
+//   head size 128, int8: 1 kv head, 1 sequence of 512 tokens 12.0 / 12.2 us, 768: 12.1 / 13.1, 1024: 12.1 / 14.7; 2 kv heads, 4 of 768
+//     12.5 / 13.9 (13.8 before that cut served fewer heads), 1024: 12.5 / 15.3; 4 kv heads, 8 of 768 14.0 / 14.3, 1024: 14.4 / 15.7,
+//     16 of 1024 15.3 / 15.9;
+//   head size 256, int8: 1 kv head, 1 of 256 17.7 / 18.4, 1024: 17.7 / 24.7; 2, 4 of 256 19.6 / 19.2, 384: 19.9 / 20.9, 1024: 20.7 / 25.7;
+//     4, 4 of 512 22.5 / 22.0, 768: 23.3 / 24.0, 8 of 1024 27.1 / 26.9; int4: 1 kv head, 1 of 512 16.3 / 19.1; 2, 4 of 512 19.4 / 19.9,
+//     768: 19.8 / 21.6; 4, 4 of 1024 23.6 / 23.1.
+int short_context_tokens(const kvq_cache_geom& g, int num_seqs) {
+  const int hkv = g.num_kv_heads;
+  const bool int4 = g.code_type == KVQ_CODE_INT4;
+  if (hkv > 4 || (int64_t)num_seqs * hkv > (g.head_size == 256 ? 31 : 32)) return KVQ_SHORT_CONTEXT;
+  if (g.head_size == 256) return (int4 ? 256 : 128) * hkv;
+  if (g.head_size == 128 && !int4) return hkv == 1 ? 512 : 768;
+  return KVQ_SHORT_CONTEXT;
+}
+
 // Whether a launch's decode sequences are each computed by one workgroup per kv head (paged_decode_whole_kernel) and not
 // cut.  Measured on MI355X through the op, 32 q heads / 8 kv heads of 128, int8 codes, cut / whole:
 //   length        1 sequence of 100: 17.5 / 9.6 us, 337: 17.2 / 12.1, 600: 17.0 / 13.4, 1000: 18.1 / 15.7, 1500: 17.7 / 18.3,
@@ -193,6 +210,10 @@ bool whole_sequences(int num_seqs, int num_kv_heads, int num_cus, bool short_con
 }  // namespace kvq
 
 extern "C" {
+
+int kvq_short_context_tokens(const kvq_cache_geom* geom, int num_seqs) {
+  return geom == nullptr || num_seqs <= 0 ? 0 : kvq::short_context_tokens(*geom, num_seqs);
+}
 
 size_t kvq_paged_attn_workspace_bytes(int max_num_seqs, int num_q_heads, int head_size) {
   if (max_num_seqs <= 0 || num_q_heads <= 0 || head_size <= 0) return 0;

@@ -194,9 +194,11 @@ PyObject* cache_update(Args& in) {
 // lengths the buffers hold then, and a replay cannot change the launch: there only what the block table can hold counts
 // (one sequence captured at 300 tokens, 8 kv heads: replayed at 4000 26.8 us with a workgroup per kv head, 12.0 cut, at
 // 100 000 483 and 40 us; replayed at 300 8.5 and 9.4).
-int short_context(int64_t max_k, const at::Tensor& table, int block_size, int device) {
+int short_context(int64_t max_k, const at::Tensor& table, const kvq_cache_geom* g, int64_t num_seqs, int device) {
   if (max_k > KVQ_SHORT_CONTEXT) return 0;
-  if (table.size(1) * block_size > KVQ_SHORT_CONTEXT) {
+  const int limit = kvq_short_context_tokens(g, (int)num_seqs);
+  if (max_k > limit) return 0;
+  if (table.size(1) * g->block_size > limit) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(c10::hip::getCurrentHIPStream(device).stream(), &status) != hipSuccess) {
       (void)hipGetLastError();   // the legacy stream while another one captures: no capture of this call
@@ -250,7 +252,7 @@ PyObject* paged_attention(Args& in) {
   const auto *sk = static_cast<const float*>(ptr(sinks)), *al = static_cast<const float*>(ptr(alibi));
   auto* ls = static_cast<float*>(ptr(lse));
   const char* op = "unified_attention";
-  const int flags = asked | short_context(max_k, table, g->block_size, dev);
+  const int flags = asked | short_context(max_k, table, g, B, dev);
   if (ws == nullptr)   // the states live in the library's own array
     call(dev, op, kvq_paged_attn_int8_static_scratch, ptr(out), odt, ro.stride_t, ro.stride_h, ptr(q), qdt, rq.stride_t,
          rq.stride_h, base, g, bt, table.stride(0), sl, cq, (int)B, (int)rq.heads, (int)max_q, (float)scale, flags, window,
@@ -321,7 +323,7 @@ PyObject* decode_with_update(Args& in) {
        eps_of(kdt), const_cast<void*>(base), g, static_cast<const int32_t*>(ptr(table)), table.stride(0),
        static_cast<const int32_t*>(ptr(lens)), static_cast<const int64_t*>(ptr(slots)), (int)B, (int)rq.heads, (float)scale,
        window, (float)softcap, static_cast<const float*>(ptr(sinks)), static_cast<const float*>(ptr(alibi)),
-       static_cast<float*>(ptr(lse)), ptr(ws), ws.nbytes(), short_context(max_k, table, g->block_size, dev));
+       static_cast<float*>(ptr(lse)), ptr(ws), ws.nbytes(), short_context(max_k, table, g, B, dev));
   Py_RETURN_NONE;
 }
 

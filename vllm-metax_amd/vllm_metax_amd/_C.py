@@ -18,7 +18,7 @@ KVQ_F32, KVQ_BF16, KVQ_F16 = 0, 1, 2
 KVQ_CODE_INT8, KVQ_CODE_FP8_E4M3, KVQ_CODE_INT4 = 0, 1, 2
 KVQ_ATTN_CAUSAL, KVQ_ATTN_NO_DECODE_ROWS, KVQ_ATTN_SHORT_RUNS, KVQ_ATTN_SHORT_CONTEXT = 1, 2, 4, 16
 KVQ_STATIC_SCRATCH_BYTES = 24 << 20
-ABI_VERSION = 22
+ABI_VERSION = 23
 
 
 class CacheGeom(ctypes.Structure):
@@ -63,6 +63,7 @@ SIGNATURES = {
     "kvq_paged_attn_int8_fused_write": (_i, [_vp, _i, _i64, _i64, _vp, _i, _i64, _i64, _vp, _vp, _i, _i64, _i64, _i64, _i64,
                                              _f, _vp, _geom_p, _vp, _i64, _vp, _vp, _i, _i, _f, _i, _f, _vp, _vp, _vp, _vp, _sz,
                                              _vp]),
+    "kvq_short_context_tokens": (_i, [_geom_p, _i]),
     "kvq_paged_attn_int8_fused_write_flags": (_i, [_vp, _i, _i64, _i64, _vp, _i, _i64, _i64, _vp, _vp, _i, _i64, _i64, _i64, _i64,
                                              _f, _vp, _geom_p, _vp, _i64, _vp, _vp, _i, _i, _f, _i, _f, _vp, _vp, _vp, _vp, _sz,
                                              _i, _vp]),
