@@ -24,30 +24,33 @@ def _last_slots(bt, ctx, bs):
 
 
 def _both_ways(dev, kv_cpu, layout, bt, q, sl, ctx, key, value, scale, mode=KVQuantMode.INT8_PER_TOKEN_HEAD,
-               window=(-1, -1), softcap=0.0, out_dtype=torch.bfloat16, padding=()):
-    """`padding`: rows whose slot mapping entry is -1 (cudagraph padding): neither way may write them."""
-    bs = L.key_value_views(T.to_device_cache(kv_cpu, dev, layout))[0].shape[1]
+               window=(-1, -1), softcap=0.0, out_dtype=torch.bfloat16, padding=(), stated=None, code_type=oracle.CODE_INT8):
+    """`padding`: rows whose slot mapping entry is -1 (cudagraph padding): neither way may write them.  `stated`: the longest
+    sequence as the call states it; above a short context the sequences are cut whatever their lengths."""
+    bs = L.key_value_views(T.to_device_cache(kv_cpu, dev, layout, code_type=code_type))[0].shape[1]
     slots = _last_slots(bt, ctx, bs)
     for i in padding:
         slots[i] = -1
     res = []
     for fused in (False, True):
-        kv = T.to_device_cache(kv_cpu, dev, layout)
+        kv = T.to_device_cache(kv_cpu, dev, layout, code_type=code_type)
         k, v = L.key_value_views(kv)
         ks, vs = L.scale_views(kv)
         out = torch.full(q.shape, float("nan"), dtype=out_dtype, device=dev)
         lse = torch.full(q.shape[:2], float("nan"), dtype=torch.float32, device=dev)
-        common = dict(block_table=bt.to(dev), k_scale_cache=ks, v_scale_cache=vs, lse=lse, softcap=softcap,
+        longest = stated or int(sl.max())
+        table = torch.nn.functional.pad(bt, (0, max(0, longest // bs + 1 - bt.shape[1])))
+        common = dict(block_table=table.to(dev), k_scale_cache=ks, v_scale_cache=vs, lse=lse, softcap=softcap,
                       window_size=window, kv_quant_mode=mode)
         if fused:
             ops.decode_attention_with_cache_update(q.to(dev), key.to(dev), value.to(dev), k, v, out, sl.to(dev),
-                                                   int(sl.max()), scale, **common,
+                                                   longest, scale, **common,
                                                    slot_mapping=slots.to(dev) if padding else None)
         else:
             ops.reshape_and_cache_flash_per_token_head_quant(key.to(dev), value.to(dev), k, v, ks, vs,
                                                              slots.to(dev), kv_quant_mode=mode)
             cu = torch.arange(len(ctx) + 1, dtype=torch.int32, device=dev)
-            ops.unified_attention(q.to(dev), k, v, out, cu, 1, sl.to(dev), int(sl.max()), scale, True, **common)
+            ops.unified_attention(q.to(dev), k, v, out, cu, 1, sl.to(dev), longest, scale, True, **common)
         torch.cuda.synchronize()
         res.append((T.storage_bytes(kv).cpu(), out.cpu(), lse.cpu()))
     return res
@@ -98,6 +101,44 @@ def test_fused_write_skips_padding_rows(gpu_device, hkv):
     assert torch.equal(cache_a, cache_b), "a padding row was written (or a live one was not)"
     assert not torch.equal(cache_b, before)
     assert torch.equal(out_a.view(torch.int16), out_b.view(torch.int16))
+
+
+@pytest.mark.parametrize("code", ["int8", "fp8", "int4"])
+@pytest.mark.parametrize("hq,hkv,d,ctx,padding,window", [
+    (32, 8, 128, [300, 48, 1000, 17, 64], (1, 4), 0),       # a wave per kv head
+    (16, 2, 128, [300, 48, 1000, 17, 64], (1, 4), 0),       # four waves per kv head
+    (16, 1, 128, [777, 1, 48], (0,), 0),                    # eight
+    (16, 8, 256, [260, 15, 1024, 700], (3,), 0),
+    (32, 8, 64, [200, 1, 900, 31], (), 0),
+    (32, 8, 128, [0, 40, 0, 1], (), 0),                     # empty sequences next to live ones
+    (16, 8, 256, [900, 33, 1000], (1,), 1100),              # a window past every sequence
+])
+def test_fused_write_of_short_contexts_cut_and_not_cut(gpu_device, code, hq, hkv, d, ctx, padding, window):
+    """Short contexts take a workgroup per (sequence, kv head) or, where the call states a longer context, are cut: either
+    way the write kernel's bytes, padding rows untouched, and the oracle's rows."""
+    mode = getattr(KVQuantMode, code.upper() + "_PER_TOKEN_HEAD")
+    ct = {"int8": oracle.CODE_INT8, "fp8": oracle.CODE_FP8, "int4": oracle.CODE_INT4}[code]
+    g = torch.Generator().manual_seed(d + hkv)
+    nb = sum((c + 15) // 16 for c in ctx) + 5
+    kv, _, lay = T.cpu_cache(nb, 16, hkv, d, "HND", code_type=ct)
+    bt = T.make_block_tables(ctx, 16, nb, g)
+    src = [[torch.randn((c, hkv, d), generator=g).to(torch.bfloat16) for c in ctx] for _ in range(2)]
+    T.fill_cache_from_sources(kv, lay, bt, ctx, 16, *src, code_type=ct)
+    q = torch.randn((len(ctx), hq, d), generator=g).to(torch.bfloat16)
+    key, value = (torch.randn((len(ctx), hkv, d), generator=g).to(torch.bfloat16) for _ in range(2))
+    sl, cu = torch.tensor(ctx, dtype=torch.int32), torch.arange(len(ctx) + 1, dtype=torch.int32)
+    ref = T.storage_bytes(kv).clone()
+    rows = [i for i, c in enumerate(ctx) if c > 0 and i not in padding]
+    oracle.cache_write(key[rows], value[rows], ref, lay, _last_slots(bt, ctx, 16)[rows], code_type=ct)
+    want = oracle.paged_attn(q, ref, lay, bt, sl, cu, 0.09, code_type=ct, sliding_window=window)
+    live = torch.tensor([i for i, c in enumerate(ctx) if c > 0])
+    for stated in (None, 1500):
+        ways = _both_ways(gpu_device, kv, "HND", bt, q, sl, ctx, key, value, 0.09, mode=mode, padding=padding, stated=stated,
+                          window=(window - 1, 0) if window else (-1, -1), code_type=ct)
+        for cache, out, _ in ways:
+            assert torch.equal(cache, ref), f"cache bytes, stated {stated}"
+            T.assert_close_attn(out[live], want[live], what=f"{code} {hq}/{hkv} d{d} stated {stated}")
+        assert torch.equal(ways[0][1].view(torch.int16), ways[1][1].view(torch.int16)), f"stated {stated}"
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.float32])

@@ -60,11 +60,26 @@ def test_decode_head_shapes(gpu_device, hq, hkv, d, bs):
 
 
 def test_decode_many_sequences_long_window(gpu_device):
-    """More sequences than a wave scans at once, each a few tiles of window inside a long context:
-    the tile line is built from the windows, not from the sequence lengths."""
+    """More sequences than a wave scans at once, each a few tiles of window inside a long context: a workgroup per sequence
+    and kv head (test_cut_decode_with_a_window has the batches that are cut)."""
     g = torch.Generator().manual_seed(1)
     ctx = torch.randint(200, 1500, (70,), generator=g).tolist()
     check(gpu_device, ctx, [1] * len(ctx), 8, 2, 128, 16, 100, None, seed=11, what="decode b70")
+
+
+@pytest.mark.parametrize("layout", ["NHD", "HND"])
+@pytest.mark.parametrize("hq,hkv,d,n,window,cap", [
+    (8, 8, 64, 40, 100, None), (8, 8, 64, 40, 33, 50.0),       # 320 (sequence, kv head) pairs: cut, whatever the window
+    (8, 4, 128, 70, 256, 50.0), (8, 4, 128, 300, 20, None),    # more sequences than a lane holds, more than four per lane
+    (32, 8, 128, 9, 1025, None), (16, 8, 256, 5, 1500, 30.0),  # windows past a short context
+    (16, 8, 256, 37, 1400, 50.0), (16, 1, 128, 4, 1100, None)])
+def test_cut_decode_with_a_window(gpu_device, hq, hkv, d, n, window, cap, layout):
+    """Batches whose sequences are cut although a window bounds them: the line is made of the windows' tiles, with windows
+    that start inside a tile and sequences shorter than the window beside ones far longer."""
+    g = torch.Generator().manual_seed(n + window)
+    ctx = torch.randint(1, 3 * window + 200, (n,), generator=g).tolist()
+    ctx[0], ctx[-1] = window + 31, 1
+    check(gpu_device, ctx, [1] * n, hq, hkv, d, 16, window, cap, seed=n, what=f"cut {hq}/{hkv} d{d} n={n}", layout=layout)
 
 
 @pytest.mark.parametrize("window", [None, 1, 20, 64, 256, 3000])
