@@ -131,10 +131,10 @@ __device__ __forceinline__ float sum_over_quarters(float v) {
   swap_halves(__builtin_bit_cast(uint32_t, v), true, a, b);
   return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b);
 }
-// The same over the 2, 4, 8 or 16 neighbouring lanes of a group, by data-parallel moves: lane ^ 1 and ^ 2 of a quad, then
-// the mirror images of 8 and of 16 lanes, which by then hold their group's value.  A move is an operand of the next
+// The maximum over the 8, 16 or 32 neighbouring lanes of a group, the sum over 16, by data-parallel moves: lane ^ 1 and
+// ^ 2 of a quad, then the mirror images of 8 and of 16 lanes, which by then hold their group's value.  A move is an operand of the next
 // instruction; a shuffle through LDS is a trip of over a hundred cycles, and the small kernels around a decode step (cache write,
-// reduce) chain up to twelve of them (a step of 4 verification runs 19.4 -> 18.6 us, 37 sequences at head size 256 104.0 -> 103.1).
+// reduce) chain up to twelve of them (a step of 4 verification runs 19.4 -> 18.6 us).
 // Every lane of the wave must take part.
 template <int CTRL>
 __device__ __forceinline__ float lane_move(float v) {

@@ -23,7 +23,8 @@ __device__ __forceinline__ int64_t line_div(int64_t a, int64_t b) {
   return (((uint64_t)a | (uint64_t)b) >> 32) == 0 ? (int64_t)((uint32_t)a / (uint32_t)b) : a / b;
 }
 
-// A share is never empty unless the line is: active_workgroups leaves at least kMinUnitsPerWg units to each.
+// A line of units is shared out over at most as many workgroups as it has units (active_workgroups, and the batch-invariant
+// line's own count), so no share of a line that is not empty is empty; the reduces rely on it.
 __device__ __forceinline__ int64_t wg_tile_begin(int w, int64_t total, int num_wg) {
   return line_div((int64_t)w * total, num_wg);
 }
