@@ -9,9 +9,9 @@
 // tile ahead, double-buffered (one barrier per tile), and every wave feeds its two row blocks from there, so a K or V byte
 // is fetched from L2 once per 128 rows.  Which bytes a load's lanes bring is chosen so that the operand reads of K (chunks
 // xor-swizzled by the row) and of V (successive rows from different loads, 32 bytes apart) meet no bank twice.
-// What bounds it: latency -- matrix unit 43 % busy, vector unit 36 %, LDS 21 %.  Hence no registers between memory and LDS
+// What bounds it: latency -- matrix unit 40 % busy, vector unit 40 %, LDS 20 %.  Hence no registers between memory and LDS
 // (they took 20 of them and a fifth of the tile's instructions) and three workgroups per compute unit where the launch has
-// that many: 4 requests with 300-1500 new tokens on 1000-2300 cached ones, 128 heads, a layer step 1320 -> 1178 us
+// that many: 4 requests with 300-1500 new tokens on 1000-2300 cached ones, 128 heads, a layer step 1335 -> 1192 us
 // (of which 484 us are the two kv_b_proj products), 16 heads 249 -> 227, one request of 2500 tokens at 32 heads 164 -> 153.
 // Both products are computed transposed so that every per-row quantity is lane-local:
 //   S^T = K Q^T   A = K rows (lane = key, 8 consecutive d), B = Q (lane = query row): 16x16x32 MFMA of the

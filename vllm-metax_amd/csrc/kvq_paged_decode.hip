@@ -195,7 +195,7 @@ int short_context_tokens(const kvq_cache_geom& g, int num_seqs) {
 }
 
 // Whether a launch's decode sequences are each computed by one workgroup per kv head (paged_decode_whole_kernel) and not
-// cut.  Measured on MI355X through the op, 32 q heads / 8 kv heads of 128, int8 codes, cut / whole:
+// cut.  Measured on MI355X through the op, 32 q heads / 8 kv heads of 128, int8 codes, cut (by eight heads per workgroup) / whole:
 //   length        1 sequence of 100: 17.5 / 9.6 us, 337: 17.2 / 12.1, 600: 17.0 / 13.4, 1000: 18.1 / 15.7, 1500: 17.7 / 18.3,
 //                 2000: 18.1 / 20.8 -- a wave's tiles are a serial chain of 1.7 us each, the reduce a fixed cost of 4 - 5;
 //   workgroups    32 sequences of 100 .. 1000: 22.5 / 17.5, 32 of 1000: 26.1 / 20.4 (256 workgroups), but 40: 29.6 / 30.9,

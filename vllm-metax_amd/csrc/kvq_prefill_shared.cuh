@@ -15,10 +15,11 @@
 // and the ends of the walk use, are worked out anew there.  Kept through the loops they were spilled, 11 to 14 of them, and
 // some reloaded in every step behind the next tile's loads, which the reload then waited for (16 prompts of 300 tokens 60.1
 // -> 54.5 us, one of 2000 82.9 -> 74.0, the mixed step below 447 -> 437).  One value is left, spilled outside the loops; head
-// size 64 spills up to three with the extras, at head size 128 those do not spill.  At three workgroups the vector unit is 60 % busy, the matrix unit 39 %, the LDS 44 %.
+// size 64 spills up to three with the extras, at head size 128 those do not spill.  At three workgroups the vector unit is 65 % busy, the matrix unit 45 %, the LDS 51 %.
 // Measured on MI355X against two workgroups per compute unit with register loads and padded tiles: 4 x 2048 new tokens on
-// 0-6k cached ones beside 60 decode rows (28/4 heads) 525 -> 456 us for the step, a 6000-token prompt (32/8 heads)
-// 444 -> 389 us, 512 tokens on 32k in context ranges 384 -> 351 us, int4 cache 235 -> 191 us, head size 64 307 -> 255 us.
+// 0-6k cached ones beside 60 decode rows (28/4 heads) 534 -> 442 us for the step, 512 tokens on 32k in context ranges (32/8 heads)
+// 395 -> 341 us; captured: a 2000-token prompt 98.7 -> 74.0 us, with int4 codes 103.7 -> 79.7, head size 64 77.4 -> 60.5, one of 70
+// tokens 15.8 -> 14.0, a window of 1500 tokens in the mixed step 320 -> 271, with a soft cap 736 -> 653.
 // One wave per SIMD with 64 columns each (half the operand reads and expansion work) reached 334 us for the 512 tokens,
 // but 497 us for the mixed step: a wave alone issues an instruction every 5.6 cycles, two or more waves one every 2 to 4.
 #pragma once
@@ -297,7 +298,8 @@ struct SharedTile {
 // With a.ksplit > 1 the grid's x dimension carries that many context ranges per query block; a workgroup takes one range
 // of its item's tiles and writes a partial state instead of the rows.
 // Waves per SIMD: the extras need 190 registers at head size 128 (at 168 they spill inside the loop: a window of 2000
-// tokens 331 us against 285), head size 64 fits 128 (mixed batch 264 us at three waves, 255 at four).
+// tokens 331 us against 285), head size 64 fits 128 (mixed batch 264 us at three waves, 255 at four; with a soft cap 314 at three,
+// 358 at four, but with a window alone 129 and 120).
 template <int D, bool EXT>
 constexpr int kSharedWaves = D == 64 ? 4 : EXT ? 2 : 3;
 

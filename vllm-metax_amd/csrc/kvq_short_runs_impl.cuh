@@ -352,7 +352,8 @@ int launch_short_runs_d(const ShortRunArgs& args, hipStream_t s) {
   // that an item leaves fewer partial states -- a state is up to 32 columns of D floats per head, and with a cut per 8 heads
   // a batch wrote and read 27 MB of them beside 173 MB of cache.  Four rather than eight (MI355X, a step, 8 kv heads of 128,
   // 2 - 6 query tokens on 1k - 8k): 24 sequences 73.5 -> 71.1 us, 40: 83.4 -> 79.8, 64: 125.2 -> 119.7; 90 short ones
-  // 55.0 -> 54.7.  Below four a share's start weighs more than the states saved (24 sequences, 4 kv heads: 2 per
+  // 55.0 -> 54.7.  Head size 64, 24 sequences 43.7 -> 41.2; int4 codes 54.9 -> 53.7, 64: 102.8 -> 102.3; 2 kv heads, 64 sequences
+  // 76.7 -> 77.8, with int4 codes 66.3 -> 66.5, fewer of them gain.  Below four a share's start weighs more than the states saved (24 sequences, 4 kv heads: 2 per
   // workgroup 50.6 for 47.9 us) until an item is cut dozens of times: one sequence of 16k tokens 34.5 -> 24.9 us, 5 of
   // 8k - 16k on 16 kv heads 62.8 -> 60.3; 12 on 4 kv heads (21 cuts each) would lose, 38.9 -> 41.1.
   int hpw = heads_per_wg(hkv);
