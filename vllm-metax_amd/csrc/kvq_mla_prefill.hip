@@ -9,10 +9,16 @@
 // tile ahead, double-buffered (one barrier per tile), and every wave feeds its two row blocks from there, so a K or V byte
 // is fetched from L2 once per 128 rows.  Which bytes a load's lanes bring is chosen so that the operand reads of K (chunks
 // xor-swizzled by the row) and of V (successive rows from different loads, 32 bytes apart) meet no bank twice.
-// What bounds it: latency -- matrix unit 40 % busy, vector unit 40 %, LDS 20 %.  Hence no registers between memory and LDS
-// (they took 20 of them and a fifth of the tile's instructions) and three workgroups per compute unit where the launch has
-// that many: 4 requests with 300-1500 new tokens on 1000-2300 cached ones, 128 heads, a layer step 1335 -> 1192 us
-// (of which 484 us are the two kv_b_proj products), 16 heads 249 -> 227, one request of 2500 tokens at 32 heads 164 -> 153.
+// What bounds it: latency -- matrix unit 47 % busy, vector unit 36 %, LDS 25 %.  Hence no registers between memory and LDS
+// (they took 20 of them and a fifth of the tile's instructions), three workgroups per compute unit where the launch has
+// that many, and operands of either product requested four ahead of their use: K from the step's start, the first V while the
+// softmax runs.  The reference maximum moves only when a product exceeds it by 2^7 or more, so that most steps reduce
+// nothing over lanes and rescale nothing.  Lane numbers, limits and the K addresses of a step are worked out anew for it:
+// kept, they were 18 registers more than the 168 there are at three workgroups.
+// Measured: 4 requests with 300-1500 new tokens on 1000-2300 cached ones, 128 heads, a layer step 1335 us with tiles through
+// registers, 1181 with two operand reads under way, a wait for the next tile's loads in front of the V reads and a maximum
+// taken in every step, 1099 now (of which 484 us are the two kv_b_proj products); one request of 200 tokens on 4900 cached
+// ones at 16 heads 219 -> 186, three of 500-1500 at 64 heads 221 -> 201.
 // Both products are computed transposed so that every per-row quantity is lane-local:
 //   S^T = K Q^T   A = K rows (lane = key, 8 consecutive d), B = Q (lane = query row): 16x16x32 MFMA of the
 //                 input type; a lane ends up with 8 keys of ITS query row, so the row maximum is a
@@ -103,6 +109,14 @@ struct VarlenTile {
   }
 };
 
+template <int FROM, int TO, class F>
+__device__ __forceinline__ void static_for(F f) {
+  if constexpr (FROM < TO) {
+    f(std::integral_constant<int, FROM>{});
+    static_for<FROM + 1, TO>(f);
+  }
+}
+
 // WAVES: waves per SIMD, i.e. workgroups per compute unit, that the kernel is compiled for (see launch_varlen).
 template <int DT, int NOPE, int ROPE, int DV, int WAVES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void varlen_attn_kernel(VarlenArgs a) {
@@ -112,6 +126,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   constexpr int RB = 2;                                             // row blocks of 16 per wave
   // fp16 weights are kept 2^8 larger so that small ones stay normal; l carries the same factor
   constexpr float kShift = DT == KVQ_F16 ? 8.f : 0.f;
+  // how far, in base 2, a logit may exceed its row's reference maximum: 2^(kShift + kAllow) must stay inside fp16
+  constexpr float kAllow = DT == KVQ_F16 ? 7.f : 8.f;
+  constexpr int AHEAD = 4 < 2 * KS ? 4 : 2 * KS, AHEAD_V = 4 < DPL ? 4 : DPL;   // K and V operands requested ahead of their products
   __shared__ __align__(16) uint8_t lds[2][VT::BYTES];
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -143,8 +160,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   const int num_tiles = (wg_k_end + 31) / 32;
   if (a.merge && num_tiles == 0) return;   // nothing to add to the rows (uniform over the workgroup)
 
+  // the lane number, worked out anew (kept from tile to tile it, and what follows from it, take registers)
+  auto lane_anew = []() __attribute__((always_inline)) {
+    uint32_t n;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(n));
+    return (int)n;
+  };
   // ---- the wave's rows
-  int q0[RB], my_limit[RB], blk_k_end[RB];
+  int q0[RB], blk_k_end[RB], min_limit = k_len;
+  auto limit_of = [&](int rb, int row) __attribute__((always_inline)) {   // keys that row `row` of a row block sees
+    return a.causal ? max(0, min(k_len, q0[rb] + row + diag + 1)) : k_len;
+  };
   u32x4 qop[RB][KS];
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
@@ -153,20 +179,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
     const uint16_t* qp = static_cast<const uint16_t*>(a.q) + (int64_t)(q_begin + qrow) * a.q_st + (int64_t)head * a.q_sh + 8 * g;
 #pragma unroll
     for (int s = 0; s < KS; ++s) qop[rb][s] = *reinterpret_cast<const u32x4*>(qp + 32 * s);
-    my_limit[rb] = a.causal ? max(0, min(k_len, q0[rb] + c + diag + 1)) : k_len;
+    min_limit = min(min_limit, limit_of(rb, 0));
     blk_k_end[rb] = q0[rb] >= q_len ? 0 : (a.causal ? max(0, min(k_len, q0[rb] + 15 + diag + 1)) : k_len);
   }
   const int wave_tiles = (max(blk_k_end[0], blk_k_end[1]) + 31) / 32;   // tiles this wave has anything to do in
   // the smallest limit among the wave's rows: tiles that end at or below it are visible to every row
-  const int wave_min_limit = -wave_max_i32(-min(my_limit[0], my_limit[1]));
+  const int wave_min_limit = min_limit;
 
   floatx4 oacc[RB][DPL];
-  float m[RB], l[RB];   // maximum, lane's sum of weights
+  float off[RB], thr[RB], l[RB];   // kShift - reference maximum; product above which it moves; lane's sum of weights
+  const float allow = kAllow / a.scale_log2;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
 #pragma unroll
     for (int i = 0; i < DPL; ++i) oacc[rb][i] = (floatx4){0.f, 0.f, 0.f, 0.f};
-    m[rb] = -INFINITY;
+    off[rb] = kShift;
+    thr[rb] = -INFINITY;
     l[rb] = 0.f;
   }
 
@@ -207,99 +235,124 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   // every load into LDS of this wave has landed, every LDS read is done, and so for the other waves
   auto tile_barrier = []() __attribute__((always_inline)) { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
-  // operand places of the lane: K row c, chunk g of a k-step (a k-step is four chunks); V rows 4 g + c / 4
-  uint32_t kn_read[KSN], kr_read[KSR > 0 ? KSR : 1];
-#pragma unroll
-  for (int s = 0; s < KSN; ++s) kn_read[s] = (uint32_t)(c * NOPE * 2 + ((4 * s + g) ^ VT::template swizzle<NOPE>(c)) * 16);
-#pragma unroll
-  for (int s = 0; s < KSR; ++s) kr_read[s] = (uint32_t)(VT::KN_BYTES + c * ROPE * 2 + ((4 * s + g) ^ VT::template swizzle<ROPE>(c)) * 16);
+  // operand places of the lane: K row c, chunk g of a k-step (a k-step is four chunks); V rows 4 g + c / 4.  The chunk of
+  // k-step s is that of the first one xor 4 s: worked out anew in every step, a register per part is all that is kept.
+  uint32_t kn_read = (uint32_t)(c * NOPE * 2 + (g ^ VT::template swizzle<NOPE>(c)) * 16);
+  uint32_t kr_read = ROPE > 0 ? (uint32_t)(VT::KN_BYTES + c * ROPE * 2 + (g ^ VT::template swizzle<ROPE>(c)) * 16) : 0;
   const uint32_t v_read = (uint32_t)(VT::V_AT + VT::v_at(4 * g + (c >> 2)) + 8 * (c & 3));
+
+  // V^T operand of output block i, half h (keys 4 g .. + 3 and 16 + 4 g ..): the LDS's transposing read.  Lane s of a
+  // quarter-wave names the 8 bytes [key kb + s / 4][dims 16 i + 4 (s % 4) .. + 3] and receives [keys kb .. kb + 3][dim 16 i + s].
+  // In assembly because the compiler waits for every load under way, the next tile's too, in front of the builtin; so the
+  // waits for what these read are written out as well.
+  struct VOperand {
+    u32x2 half[2];
+  };
+  auto read_v = [&](uint32_t at, auto block, VOperand& o) __attribute__((always_inline)) {
+    constexpr int I = decltype(block)::value;
+    asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%3\n\tds_read_b64_tr_b16 %1, %2 offset:%4"
+                 : "=&v"(o.half[0]), "=&v"(o.half[1]) : "v"(at), "n"(32 * I), "n"(VT::v_at(16) + 32 * I));
+  };
+  auto wait_v = [&](auto behind, VOperand& o) __attribute__((always_inline)) {   // `behind`: operands requested after this one
+    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(o.half[0]), "+v"(o.half[1]) : "n"(2 * decltype(behind)::value));
+  };
+  auto fence = []() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
 
   auto step_fn = [&](int t, const uint8_t* buf) __attribute__((always_inline)) {
     // a wave at its products and softmax outranks the waves of its SIMD that wait at the barrier
     __builtin_amdgcn_s_setprio(1);
     // ---- S^T = K Q^T for the tile's two blocks of 16 keys, both row blocks off one operand read
     floatx4 sacc[RB][2];
+    u32x4 ka[2 * KS];
+    asm volatile("" : "+v"(kn_read), "+v"(kr_read));   // (what follows from them is not to be kept either)
+    auto read_k = [&](int i) __attribute__((always_inline)) {
+      const int blk = i / KS, s = i % KS;
+      const uint8_t* p = s < KSN ? buf + (kn_read ^ (64 * s)) + blk * 16 * NOPE * 2 : buf + (kr_read ^ (64 * (s - KSN))) + blk * 16 * ROPE * 2;
+      ka[i] = *reinterpret_cast<const u32x4*>(p);
+    };
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
+    for (int i = 0; i < AHEAD; ++i) read_k(i);
+    fence();
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const uint8_t* p = s < KSN ? buf + kn_read[s < KSN ? s : 0] + blk * 16 * NOPE * 2
-                                   : buf + kr_read[s < KSN ? 0 : s - KSN] + blk * 16 * ROPE * 2;
-        const u32x4 ka = *reinterpret_cast<const u32x4*>(p);
+    for (int i = 0; i < 2 * KS; ++i) {
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb)
-          sacc[rb][blk] = mfma16<DT>(ka, qop[rb][s], s == 0 ? (floatx4){0.f, 0.f, 0.f, 0.f} : sacc[rb][blk]);
-      }
+      for (int rb = 0; rb < RB; ++rb)
+        sacc[rb][i / KS] = mfma16<DT>(ka[i], qop[rb][i % KS], i % KS == 0 ? (floatx4){0.f, 0.f, 0.f, 0.f} : sacc[rb][i / KS]);
+      if (i + AHEAD < 2 * KS) read_k(i + AHEAD);
+      fence();
     }
+    // the first V operands come in while the softmax runs
+    VOperand va[DPL];
+    const uint32_t v_at = v_read + (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)buf;
+    static_for<0, AHEAD_V>([&](auto i) __attribute__((always_inline)) { read_v(v_at, i, va[i]); });
+    fence();
     // ---- online softmax in base 2, per row block
-    u32x4 pk[RB];
     // only a tile that reaches past some row's limit (the causal diagonal, the end of the keys) is masked: a uniform
     // branch round the compares and selects, which work on the products where they lie
     if ((t + 1) * 32 > wave_min_limit) {
+      const int of = lane_anew();
 #pragma unroll
-      for (int rb = 0; rb < RB; ++rb)
+      for (int rb = 0; rb < RB; ++rb) {
+        const int visible = limit_of(rb, of & 15) - t * 32 - 4 * (of >> 4);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int key = t * 32 + 16 * (j >> 2) + 4 * g + (j & 3);
-          sacc[rb][j >> 2][j & 3] = key < my_limit[rb] ? sacc[rb][j >> 2][j & 3] : -INFINITY;
-        }
+        for (int j = 0; j < 8; ++j)
+          sacc[rb][j >> 2][j & 3] = 16 * (j >> 2) + (j & 3) < visible ? sacc[rb][j >> 2][j & 3] : -INFINITY;
+      }
     }
-    float alpha[RB];
-    bool moved[RB];
+    // The reference maximum only has to keep 2^(logit - m) in range: it stays put while no product exceeds thr, the
+    // reference plus kAllow, and then neither the reduction over a row's four lanes nor any rescaling is due.
+    float mx[RB];
+    bool over = false;
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
       // the maximum is taken over the raw products (the scale is positive and the same for every key), so that
-      // scale and maximum enter each logit in ONE multiply-add
-      float mx = -INFINITY;
+      // scale and reference enter each logit in ONE multiply-add
+      mx[rb] = -INFINITY;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) mx = fmaxf(mx, sacc[rb][j >> 2][j & 3]);
-      mx = max_over_quarters(mx) * a.scale_log2;
-      const float m_new = fmaxf(m[rb], mx);
-      const float m_use = m_new == -INFINITY ? 0.f : m_new;
-      alpha[rb] = __builtin_amdgcn_exp2f(m[rb] - m_use);
-      moved[rb] = m_new > m[rb];
-      m[rb] = m_new;
-      const float off = kShift - m_use;
+      for (int j = 0; j < 8; ++j) mx[rb] = fmaxf(mx[rb], sacc[rb][j >> 2][j & 3]);
+      over = over || mx[rb] > thr[rb];
+    }
+    if (__builtin_amdgcn_ballot_w64(over) != 0) {
+#pragma unroll
+      for (int rb = 0; rb < RB; ++rb) {
+        const float row_mx = max_over_quarters(mx[rb]);
+        const bool moves = row_mx > thr[rb];   // (a row's reference depends on its own products only)
+        const float new_off = moves ? kShift - row_mx * a.scale_log2 : off[rb];
+        const float alpha = thr[rb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(new_off - off[rb]);
+        thr[rb] = moves ? row_mx + allow : thr[rb];
+        off[rb] = new_off;
+        l[rb] *= alpha;
+#pragma unroll
+        for (int i = 0; i < DPL; ++i) oacc[rb][i] *= alpha;
+      }
+    }
+    u32x4 pk[RB];
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
       float p[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        p[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[rb][j >> 2][j & 3], a.scale_log2, off));   // a masked key: 2^-inf = 0
+        p[j] = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[rb][j >> 2][j & 3], a.scale_log2, off[rb]));   // a masked key: 2^-inf = 0
       pk[rb].x = pack2<DT>(p[0], p[1]);
       pk[rb].y = pack2<DT>(p[2], p[3]);
       pk[rb].z = pack2<DT>(p[4], p[5]);
       pk[rb].w = pack2<DT>(p[6], p[7]);
       // the row sum is that of the weights as the second product sees them (rounded to the input type): one
       // two-element dot product with ones per packed pair instead of two additions
-      float sum = l[rb] * alpha[rb];
 #pragma unroll
-      for (int w = 0; w < 4; ++w) sum = pair_sum<DT>(pk[rb][w], sum);
-      l[rb] = sum;
+      for (int w = 0; w < 4; ++w) l[rb] = pair_sum<DT>(pk[rb][w], l[rb]);
     }
-    // The accumulators of a row block are rescaled only in the tiles in which some row's maximum moved.
+    fence();
+    // ---- O^T += V^T P^T
+    static_for<0, DPL>([&](auto ic) __attribute__((always_inline)) {
+      constexpr int I = decltype(ic)::value, BEHIND = I + AHEAD_V <= DPL ? AHEAD_V - 1 : DPL - 1 - I;
+      wait_v(std::integral_constant<int, BEHIND>{}, va[I]);
+      const u32x4 vt = {va[I].half[0].x, va[I].half[0].y, va[I].half[1].x, va[I].half[1].y};
 #pragma unroll
-    for (int rb = 0; rb < RB; ++rb)
-      if (__builtin_amdgcn_ballot_w64(moved[rb]) != 0) {
-#pragma unroll
-        for (int i = 0; i < DPL; ++i) oacc[rb][i] *= alpha[rb];
-      }
-    // ---- O^T += V^T P^T.  V^T operands straight from the row-major tile with the LDS's transposing read
-    //      (ds_read_b64_tr_b16): lane s of a quarter-wave names the 8 bytes [key kb + s / 4][dims 16 i + 4 (s % 4) .. + 3]
-    //      and receives [keys kb .. kb + 3][dim 16 i + s]; two reads (kb = 4 g and 16 + 4 g, the keys of the lane's k slots)
-    //      make the A operand of output block i = dims 16 i .. 16 i + 15.
-    {
-      typedef short s4_t __attribute__((ext_vector_type(4)));
-      typedef __attribute__((address_space(3))) s4_t* lds_s4_ptr;
-      const uint8_t* v0 = buf + v_read;
-#pragma unroll
-      for (int i = 0; i < DPL; ++i) {
-        const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_ptr)(v0 + 32 * i)));
-        const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4_ptr)(v0 + VT::v_at(16) + 32 * i)));
-        const u32x4 vt = {lo.x, lo.y, hi.x, hi.y};
-#pragma unroll
-        for (int rb = 0; rb < RB; ++rb) oacc[rb][i] = mfma16<DT>(vt, pk[rb], oacc[rb][i]);
-      }
-    }
+      for (int rb = 0; rb < RB; ++rb) oacc[rb][I] = mfma16<DT>(vt, pk[rb], oacc[rb][I]);
+      if constexpr (I + AHEAD_V < DPL) read_v(v_at, std::integral_constant<int, I + AHEAD_V>{}, va[I + AHEAD_V]);
+      fence();
+    });
     __builtin_amdgcn_s_setprio(0);
   };
   if (num_tiles > 0) {
@@ -317,15 +370,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
     }
   }
 
+  const int lane_end = lane_anew(), c_end = lane_end & 15, g_end = lane_end >> 4;
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
     const float l_tot = sum_over_quarters(l[rb]);
     const bool live = l_tot > 0.f;
     float mul = live ? 1.f / l_tot : 0.f;
-    if (q0[rb] + c >= q_len) continue;
-    const int64_t tok = q_begin + q0[rb] + c;
+    if (q0[rb] + c_end >= q_len) continue;
+    const int64_t tok = q_begin + q0[rb] + c_end;
     uint16_t* op = static_cast<uint16_t*>(a.out) + tok * a.out_st + (int64_t)head * a.out_sh;
-    float lse = live ? (m[rb] - kShift) * kLn2 + __logf(l_tot) : -INFINITY;
+    float lse = live ? __logf(l_tot) - off[rb] * kLn2 : -INFINITY;
     if (a.merge) {
       // The algebra of merge_attn_states, in the epilogue: the other keys' rows are read and the sum is written once.
       // (As a launch of its own the merge read both states and wrote the rows: 46 us of 1352 for 2765 rows x 128 heads.)
@@ -339,7 +393,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
       mul *= wn / tot;
       u32x2 old[DPL];
 #pragma unroll
-      for (int i = 0; i < DPL; ++i) old[i] = *reinterpret_cast<const u32x2*>(op + 16 * i + 4 * g);
+      for (int i = 0; i < DPL; ++i) old[i] = *reinterpret_cast<const u32x2*>(op + 16 * i + 4 * g_end);
 #pragma unroll
       for (int i = 0; i < DPL; ++i) {
         float f[4];
@@ -348,9 +402,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
         u32x2 w;
         w.x = pack2<DT>(__builtin_fmaf(f[0], other, oacc[rb][i][0] * mul), __builtin_fmaf(f[1], other, oacc[rb][i][1] * mul));
         w.y = pack2<DT>(__builtin_fmaf(f[2], other, oacc[rb][i][2] * mul), __builtin_fmaf(f[3], other, oacc[rb][i][3] * mul));
-        *reinterpret_cast<u32x2*>(op + 16 * i + 4 * g) = w;
+        *reinterpret_cast<u32x2*>(op + 16 * i + 4 * g_end) = w;
       }
-      if (g == 0) *lp = __logf(tot) + mx;
+      if (g_end == 0) *lp = __logf(tot) + mx;
       continue;
     }
     // block i: the lane holds dims 16 i + 4 g .. + 3 of its row
@@ -359,9 +413,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
       u32x2 w;
       w.x = pack2<DT>(oacc[rb][i][0] * mul, oacc[rb][i][1] * mul);
       w.y = pack2<DT>(oacc[rb][i][2] * mul, oacc[rb][i][3] * mul);
-      *reinterpret_cast<u32x2*>(op + 16 * i + 4 * g) = w;
+      *reinterpret_cast<u32x2*>(op + 16 * i + 4 * g_end) = w;
     }
-    if (a.lse != nullptr && g == 0) a.lse[(int64_t)head * a.total_q + tok] = lse;
+    if (a.lse != nullptr && g_end == 0) a.lse[(int64_t)head * a.total_q + tok] = lse;
   }
 }
 
