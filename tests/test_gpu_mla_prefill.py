@@ -70,6 +70,37 @@ def test_varlen_attention_matches_fp32_statement(gpu_device, dtype, H, nope, rop
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rise", [0.02, 0.2, 0.24, 3.0, -0.2])
+@pytest.mark.parametrize("H,causal", [(2, False), (2, True), (32, False)])
+def test_logits_that_keep_rising(gpu_device, dtype, rise, H, causal):
+    """The reference maximum of a row lags behind its logits by up to an allowance (2^8, fp16 2^7).  Logits that rise by
+    ``rise`` from key to key stay inside it for many tiles, pass it inside a tile, or in every tile; every third row's are all
+    below -1000, every fifth sees them fall."""
+    dev, nope, rope, dv = gpu_device, 128, 64, 128
+    qlens, klens = [300, 70], [400, 97]
+    if causal:
+        klens = qlens
+    q, kv, kpe = _inputs(qlens, klens, H, nope, rope, dv, dtype, seed=19)
+    q.mul_(0.25)   # the rest of a logit is small beside its trend
+    at = torch.cat([torch.arange(n) for n in klens]).float()
+    n = torch.arange(sum(qlens))
+    # two channels carry the trend: position times the row's slope, and a constant per row
+    kv[..., 0] = at.to(dtype)[:, None]
+    kv[..., 1] = 1
+    scale = 1.0 / math.sqrt(nope + rope)
+    q[..., 0] = torch.where(n % 5 == 4, -rise, rise).to(dtype)[:, None] / scale
+    q[..., 1] = torch.where(n % 3 == 2, -1000.0, 0.0).to(dtype)[:, None] / scale
+    cu_q, cu_k = _cu(qlens), _cu(klens)
+    kvd = kv.to(dev)
+    out, lse = ops.mla_prefill_attention(
+        q.to(dev), kvd[..., :nope], kpe.to(dev), kvd[..., nope:], torch.tensor(cu_q, dtype=torch.int32, device=dev),
+        torch.tensor(cu_k, dtype=torch.int32, device=dev), max(qlens), scale, causal, return_softmax_lse=True)
+    torch.cuda.synchronize()
+    want, want_lse = TR.varlen_attn_lse(q, kv[..., :nope], kpe, kv[..., nope:], cu_q, cu_k, scale, causal)
+    _check(out, lse, want, want_lse, "rising logits")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("nope,rope,dv", [(128, 64, 128), (64, 32, 64), (128, 0, 128)])
 @pytest.mark.parametrize("causal,qlens,klens", [
     (True, [1, 31, 32, 33, 127, 129, 300], None),
