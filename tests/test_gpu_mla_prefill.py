@@ -127,6 +127,35 @@ def test_a_launch_that_fills_the_chip_has_the_bits_of_a_small_one(gpu_device, dt
     _check(some, some_lse, want, want_lse, "varlen attention, few heads")
 
 
+@pytest.mark.parametrize("H,qlens", [
+    (128, [600, 1, 130]),            # all pairs block by block
+    (64, [700] * 6),                 # the first pairs one after the other, the last ones block by block
+    (27, [520, 900, 641]),           # 81 pairs: no share for each XCD
+    (16, [4100, 30]),                # more blocks per pair than a round has places to share out
+])
+def test_every_block_of_a_large_causal_launch_is_taken(gpu_device, H, qlens):
+    """The order in which a causal launch's workgroups take the (sequence, head, block) items: rows and LSE have the bits of
+    launches of one sequence and four heads at a time, which go pair by pair."""
+    dev, nope, rope, dv = gpu_device, 64, 32, 64
+    q, kv, kpe = _inputs(qlens, qlens, H, nope, rope, dv, torch.bfloat16, seed=23)
+    scale = 1.0 / math.sqrt(nope + rope)
+    qd, kvd, kped = q.to(dev), kv.to(dev), kpe.to(dev)
+    cu = _cu(qlens)
+    c = torch.tensor(cu, dtype=torch.int32, device=dev)
+    out = torch.full((cu[-1], H, dv), 7.0, dtype=torch.bfloat16, device=dev)
+    lse = torch.full((H, cu[-1]), 7.0, device=dev)
+    ops.mla_prefill_attention(qd, kvd[..., :nope], kped, kvd[..., nope:], c, c, max(qlens), scale, True, out=out, lse=lse,
+                              return_softmax_lse=True)
+    for a, b in zip(cu, cu[1:]):
+        one = torch.tensor([0, b - a], dtype=torch.int32, device=dev)
+        for h in range(0, H, 4):
+            part, part_lse = ops.mla_prefill_attention(
+                qd[a:b, h:h + 4].contiguous(), kvd[a:b, h:h + 4, :nope], kped[a:b], kvd[a:b, h:h + 4, nope:], one, one, b - a, scale,
+                True, return_softmax_lse=True)
+            assert torch.equal(out[a:b, h:h + 4].contiguous().view(torch.int16), part.view(torch.int16)), (a, h)
+            assert torch.equal(lse[h:h + 4, a:b], part_lse), (a, h)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("H,nope,rope,dv", [(16, 128, 64, 128), (4, 64, 32, 64)])
 @pytest.mark.parametrize("causal", [False, True])

@@ -135,17 +135,32 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   // Workgroups go to the eight XCDs in turn by their linear number, and every XCD has its own L2.  The query
   // blocks of one (sequence, head) all stream the same keys: numbered so that they land on ONE XCD (possible when
   // the (sequence, head) pairs divide by eight), its L2 serves all but the first reader of a tile.
-  int seq = blockIdx.z, head = blockIdx.y, qb = blockIdx.x;
+  // Under the causal mask a pair's blocks differ in length, and one pair after the other, longest block first, the launch
+  // ends on the long blocks of the last pairs.  So the last pairs, of two rounds of workgroups, are taken block by block
+  // over all of them (four requests of 430-1220 new tokens at 128 heads: the causal launch's longest place 95 tiles, now 76 of 70;
+  // the layer step 1095 -> 1075 us, one of 1400 tokens at 32 heads, a grid of 352, 113 -> 105, three of 500-1500 at 64 heads 207 -> 196).
+  // Not with a grid of 320 or less, nor with four blocks or fewer, which hardly differ: a pair's blocks side by side find its
+  // keys in L2 (requests of 490 and 1190 tokens at 16 heads, a grid of 320: 112 us so, 113.5 otherwise; four of 67-240 at 128
+  // heads 120, 123).
+  int seq, head, qb;
   {
-    const unsigned pairs = gridDim.y * gridDim.z;
-    if ((pairs & 7u) == 0) {
-      const unsigned lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
-      const unsigned j = lin >> 3;                             // the XCD's j-th workgroup
-      const unsigned pair = (j / gridDim.x) * 8 + (lin & 7u);  // every eighth pair is this XCD's
-      qb = (int)(j % gridDim.x);
-      head = (int)(pair % gridDim.y);
-      seq = (int)(pair / gridDim.y);
+    const unsigned pairs = gridDim.y * gridDim.z, blocks = gridDim.x;
+    const unsigned xcd_bits = (pairs & 7u) == 0 ? 3 : 0;
+    const unsigned lin = blockIdx.x + blocks * (blockIdx.y + gridDim.y * blockIdx.z);
+    const unsigned j = lin >> xcd_bits, per_xcd = pairs >> xcd_bits;   // the XCD's j-th workgroup
+    unsigned pair = j / blocks;
+    qb = (int)(j - pair * blocks);
+    if (a.causal && blocks > 4 && pairs * blocks > 320) {
+      const unsigned last = min(per_xcd, ((2 * WAVES * 256) >> xcd_bits) / blocks + 1);
+      if (pair >= per_xcd - last) {
+        const unsigned r = j - (per_xcd - last) * blocks;
+        qb = (int)(r / last);
+        pair = per_xcd - last + (r - (unsigned)qb * last);
+      }
     }
+    pair = (pair << xcd_bits) + (lin & ((1u << xcd_bits) - 1));   // every eighth pair is this XCD's
+    seq = (int)(pair / gridDim.y);
+    head = (int)(pair - (unsigned)seq * gridDim.y);
   }
   const int q_begin = a.cu_q[seq], q_len = a.cu_q[seq + 1] - q_begin;
   const int k_begin = a.cu_k[seq], k_len = a.cu_k[seq + 1] - k_begin;
