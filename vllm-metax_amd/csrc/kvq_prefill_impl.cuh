@@ -51,7 +51,7 @@ struct PrefillArgs {
 // 1k-8k tokens with 2 or 4 query tokens each: 280 us per call that way against 118 us for one query token).
 template <int D, int QDT, int ODT, int NT, int WPW, int CODE = KVQ_CODE_INT8, bool SPLIT = false>
 __global__ __launch_bounds__(WPW * 64) void paged_prefill_kernel(PrefillArgs a) {
-  using PT = PrefillTile<D, QDT, ODT, NT, CODE>;
+  using PT = PrefillTile<D, QDT, ODT, NT, CODE, false, D == 256 && WPW == 8>;
   using DTile = typename PT::DTile;
   __shared__ __align__(16) uint8_t lds_all[WPW][DTile::LDS_WAVE];
   const int lane = threadIdx.x & 63;
@@ -200,9 +200,12 @@ static int launch_prefill_cfg(const PrefillArgs& a, int max_query_len, hipStream
   // (not in the batch-invariant mode: how an item is cut would depend on what else the launch holds)
   if (!batch_invariant() && (int64_t)blocks * a.num_seqs * a.io.g.num_kv_heads <= kSplitItems &&
       a.io.g.num_kv_heads <= 65535) {
-    // waves per item: eight with one column tile per wave; four with two (their accumulators need the registers
-    // of a 256-thread workgroup)
-    constexpr int SW = NT == 1 ? 8 : 4;
+    // waves per item: eight with one column tile per wave; four with two, and for 8-bit codes of head size 256 (their
+    // accumulators, and there a tile in flight beside them, need the registers of a 256-thread workgroup.  In eight waves of
+    // head size 256 up to 42 words went to scratch and came back in every tile, each time behind a wait for the tile in
+    // flight: 24 sequences of 1k-8k tokens with 2-6 query tokens, 16/8 heads, 527 us a step, 254 with the eight waves' steps
+    // in order and 142 with four; one of 512 tokens on 16k 1852, 755, 471.  int4 tiles are half the registers: 295, 81, 103.)
+    constexpr int SW = NT == 1 && (D < 256 || CODE == KVQ_CODE_INT4) ? 8 : 4;
     dim3 grid(blocks, a.num_seqs, a.io.g.num_kv_heads);
     hipLaunchKernelGGL((paged_prefill_kernel<D, QDT, ODT, NT, SW, CODE, true>), grid, dim3(SW * 64), 0, s, a);
     return check_hip(hipGetLastError(), "paged_prefill launch");

@@ -6,7 +6,7 @@
 
 namespace kvq {
 
-template <int D, int QDT, int ODT, int NT, int CODE = KVQ_CODE_INT8, bool STREAM = false>
+template <int D, int QDT, int ODT, int NT, int CODE = KVQ_CODE_INT8, bool STREAM = false, bool SCARCE = (NT > 1 && STREAM)>
 struct PrefillTile {
   using DTile = DecodeTile<D, QDT, ODT, CODE, STREAM>;
   static constexpr bool FP8 = DTile::FP8;
@@ -16,9 +16,9 @@ struct PrefillTile {
   static constexpr int VB = DTile::VB;
   static constexpr int PITCH = DTile::PITCH;
   static constexpr int LDS_TILE = DTile::LDS_TILE;
-  // Two column tiles in an eight-wave workgroup: the steps are kept in order, since the scheduler would otherwise read and
-  // convert operands so far ahead that accumulators spill.
-  static constexpr bool kScarce = NT > 1 && STREAM;
+  // SCARCE: two column tiles, or one of head size 256, in an eight-wave workgroup.  The steps are kept in order, since the
+  // scheduler would otherwise read and convert operands so far ahead that accumulators spill.
+  static constexpr bool kScarce = SCARCE;
 
   struct State {
     floatx4 o[NT][DT];
