@@ -659,3 +659,26 @@ def test_odd_ends_of_the_shared_tile(gpu_device, hq, hkv, d, window):
                               v_scale_cache=vs, prefill_splits=splits)
         torch.cuda.synchronize()
         T.assert_close_attn(out, want, what=f"odd ends, window {window}, {splits} ranges")
+
+
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 64, 65, 100])
+@pytest.mark.parametrize("hq,hkv,d,splits", [(32, 8, 128, 1), (32, 8, 128, 3), (8, 2, 256, 1), (8, 8, 64, 2)])
+def test_runs_of_a_batch_by_its_number_of_sequences(gpu_device, n, hq, hkv, d, splits):
+    """Up to 16 sequences every workgroup finds its query run itself, beyond the decode launch lists them: runs between decode
+    rows and sequences without tokens, several of one length.  The oracle decides, within the bounds of the other tests."""
+    lens = [(90, 90, 40, 200)[i % 4] + (i % 3) * 16 for i in range(n)]
+    qls = [(70, 1, 33, 90)[i % 4] if n > 2 else 70 for i in range(n)]
+    kv, lay, bt, q, sl, cu = build(lens, qls, hq, hkv, d, 16, seed=n + d)
+    if n > 2:
+        sl[n - 3] = 0   # its rows are left alone: not compared
+    scale = 1 / math.sqrt(d)
+    want = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, scale)
+    kvd = T.to_device_cache(kv, gpu_device, "NHD")
+    k, v = L.key_value_views(kvd)
+    ks, vs = L.scale_views(kvd)
+    out = torch.full(q.shape, float("nan"), dtype=q.dtype, device=gpu_device)
+    ops.unified_attention(q.to(gpu_device), k, v, out, cu.to(gpu_device), max(qls), sl.to(gpu_device), int(sl.max()), scale,
+                          True, block_table=bt.to(gpu_device), k_scale_cache=ks, v_scale_cache=vs, prefill_splits=splits)
+    torch.cuda.synchronize()
+    rows = [r for i in range(n) if int(sl[i]) > 0 for r in range(int(cu[i]), int(cu[i + 1]))]
+    T.assert_close_attn(out[rows], want[rows], what=f"{n} sequences d{d} splits {splits}")

@@ -1040,6 +1040,51 @@ struct DecodeTile {
   }
 };
 
+// One wave lists the sequences that have work for the prefill kernels, where the workgroups do not find them by
+// themselves (find_run).  A mixed batch is mostly decode rows; a grid over all sequences would spend most of its workgroups
+// finding that out one by one, in between the ones that have work.  plan: [1 + num_seqs], their number, then they.
+__device__ __forceinline__ void write_prefill_plan(const int32_t* seq_lens, const int32_t* cu_seqlens_q, int num_seqs, int32_t* plan) {
+  const int lane = threadIdx.x & 63;
+  // Up to 64 of them are put longest sequence first: their workgroups start in the plan's order, and the longest
+  // sequence's are the ones that should not start last.
+  auto rank_in = [&](uint64_t mask, int key) __attribute__((always_inline)) {   // `key` among those of the mask's lanes
+    int rank = 0;
+    for (uint64_t left = mask; left != 0; left &= left - 1) {
+      const int j = __builtin_ctzll(left), kj = __builtin_amdgcn_readlane(key, j);
+      rank += (kj > key || (kj == key && j < lane)) ? 1 : 0;
+    }
+    return rank;
+  };
+  auto run_mask = [&](int base, int& len) __attribute__((always_inline)) {
+    const int s = min(base + lane, num_seqs - 1);
+    len = seq_lens[s];
+    return __builtin_amdgcn_ballot_w64(base + lane < num_seqs && cu_seqlens_q[s + 1] - cu_seqlens_q[s] > 1 && len > 0);
+  };
+  int len;
+  uint64_t mask = run_mask(0, len);
+  if (num_seqs <= kWave) {
+    const int rank = rank_in(mask, len);
+    if ((mask >> lane) & 1) plan[1 + rank] = lane;
+    if (lane == 0) plan[0] = __builtin_popcountll(mask);
+    return;
+  }
+  int count = 0;
+  for (int base = 0;;) {
+    if ((mask >> lane) & 1) plan[1 + count + __builtin_popcountll(mask & ((1ull << lane) - 1))] = base + lane;
+    count += __builtin_popcountll(mask);
+    base += kWave;
+    if (base >= num_seqs) break;
+    mask = run_mask(base, len);
+  }
+  if (lane == 0) plan[0] = count;
+  if (count > 1 && count <= kWave) {
+    __threadfence_block();
+    const int id = plan[1 + (lane < count ? lane : 0)];
+    const int rank = rank_in(count < kWave ? (1ull << count) - 1 : ~0ull, seq_lens[id]);
+    if (lane < count) plan[1 + rank] = id;
+  }
+}
+
 // Arguments of the balanced split-K decode launch (main kernel + reduce).
 struct StreamKArgs {
   AttnIO io;
@@ -1068,6 +1113,7 @@ struct StreamKArgs {
   int fixed_spans;
   int whole;         // != 0: no cutting, a workgroup per (sequence, kv head) (whole_sequences)
   int setup_units;   // units a sequence is charged on the balanced work line before its tiles
+  int32_t* plan;     // the prefill kernels' plan for the reduce kernel to write, or nullptr
 };
 
 // The decode kernel's fused cache update: the wave that owns kv head `hkv` of the run that holds a sequence's

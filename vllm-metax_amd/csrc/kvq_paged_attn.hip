@@ -20,8 +20,9 @@ bool whole_sequences(int num_seqs, int num_kv_heads, int num_cus, bool short_con
 int validate_common(const char* op, const void* q, const void* cache, const kvq_cache_geom* geom,
                     const int32_t* block_table, const int32_t* seq_lens, int num_seqs, int num_q_heads);
 int launch_prefill(const AttnIO& io, const int32_t* seq_lens, const int32_t* cu_seqlens_q, int num_seqs,
-                   int max_query_len, int causal, int q_dtype, int out_dtype, int32_t* plan, hipStream_t s,
-                   int ksplit, int num_tokens, float* part);
+                   int max_query_len, int causal, int q_dtype, int out_dtype, int32_t* plan, bool planned,
+                   hipStream_t s, int ksplit, int num_tokens, float* part);
+bool prefill_needs_plan(int num_seqs, int head_size, int max_query_len, int group);
 
 // Where the context splits' partial states begin in a workspace, and how many bytes they take.
 static size_t split_part_offset(size_t streamk_bytes) { return (streamk_bytes + 255) & ~(size_t)255; }
@@ -188,14 +189,19 @@ static int paged_attn_launch(const char* op, void* out, int out_dtype, int64_t o
     r.q_dtype = q_dtype;
     return launch_short_runs(r, workspace, out_dtype, s);
   }
+  // the list of the sequences that have a query run sits behind the decode kernels' notes in the workspace; the decode
+  // launch writes it where it ends in a reduce kernel over cut sequences
+  int32_t* plan = reinterpret_cast<int32_t*>(a.seq_first_unit + num_seqs);
   // a batch that the caller knows to hold no one-row sequence has nothing for the decode kernel and its reduce
-  if (!(no_decode_rows && max_query_len > 1)) rc = launch_decode_streamk(a, q_dtype, out_dtype, s);
+  const bool decodes = !(no_decode_rows && max_query_len > 1);
+  const bool planned = decodes && max_query_len > 1 && !a.whole && !a.fixed_spans &&
+                       prefill_needs_plan(num_seqs, g.head_size, max_query_len, a.io.group);
+  if (planned) a.plan = plan;
+  if (decodes) rc = launch_decode_streamk(a, q_dtype, out_dtype, s);
   if (rc) return rc;
   if (max_query_len > 1) {
-    // the list of the sequences that have a query run sits behind the decode kernels' notes in the workspace
-    int32_t* plan = reinterpret_cast<int32_t*>(a.seq_first_unit + num_seqs);
     // (the batch-invariant mode keeps one cut of the context whatever the caller proposes for this launch)
-    rc = launch_prefill(a.io, seq_lens, cu_seqlens_q, num_seqs, max_query_len, causal, q_dtype, out_dtype, plan, s,
+    rc = launch_prefill(a.io, seq_lens, cu_seqlens_q, num_seqs, max_query_len, causal, q_dtype, out_dtype, plan, planned, s,
                         batch_invariant() ? 1 : prefill_splits, num_tokens,
                         reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + part_at));
   }

@@ -446,9 +446,17 @@ __global__ __launch_bounds__(256) void paged_decode_fixed_spans_reduce_kernel(St
   if (a.io.lse != nullptr && lane == 0) a.io.lse[row * Hq + head] = (m + __builtin_amdgcn_logf(lt)) * kLn2;
 }
 
-// Merge the partial states of every decode sequence that more than one workgroup touched, and give empty decode
-// sequences their defined output.  grid (P, ceil(Hq / 16)), 4 waves; a wave takes four q heads, 16 lanes each, a
-// lane D/16 dims.
+// The prefill plan of a mixed batch rides on the reduce launch, one more block of it (PLAN: the last of the grid's first row;
+// the rest of its column leaves).  As a launch of its own between the two it cost the step 2 - 3 us (30 decode rows beside 4
+// runs of 60 - 300 tokens 77.5 us for 74.8, 30 beside 3 of 300 - 600 at head size 256 with fp8 codes 255.8 for 248.7; the mixed step of 60
+// rows and 4 x 2048 tokens 436.7 for 435.1).  An instantiation of its own, since a look at a.plan in front of a decode
+// step's reduce took 0.2 us of it.
+__device__ __forceinline__ bool plan_block(const StreamKArgs& a) {
+  if (blockIdx.x + 1 != gridDim.x) return false;
+  if (blockIdx.y == 0 && threadIdx.x < kWave) write_prefill_plan(a.seq_lens, a.cu_seqlens_q, a.num_seqs, a.plan);
+  return true;
+}
+
 // A sequence is cut only where a workgroup's share begins inside it, so the grid runs over the P workgroups of
 // the main kernel, not over the sequences: block w looks at the sequence in which share w begins (the main
 // kernel left its number, its row and its shares) and merges it if share w is the
@@ -456,8 +464,10 @@ __global__ __launch_bounds__(256) void paged_decode_fixed_spans_reduce_kernel(St
 // block one round trip.  (A grid over the sequences, every wave scanning all sequence lengths for its place on
 // the line, took 44 us at 512 sequences; with one q head per wave the P x Hq waves of this grid, 8192 at 32
 // heads, did not fit the chip at once and took 11-13 us.)
-template <int D>
+template <int D, bool PLAN>
 __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_kernel(StreamKArgs a) {
+  if constexpr (PLAN)
+    if (plan_block(a)) return;
   constexpr int V = D / 16;
   const int lane = threadIdx.x & 63;
   const int sub = lane & 15;           // lane within the head's group of 16
@@ -620,8 +630,10 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_kernel(Stream
 // The same merge with a grid over the sequences, for batches of few sequences (every one of which is cut, most
 // of them several times): grid (num_seqs, ceil(Hq / 4)), 4 waves, one wave per q head, lane owns D/64 dims.  The
 // sequence's place on the work line comes from the main kernel (seq_first_unit).
-template <int D>
+template <int D, bool PLAN>
 __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_by_seq_kernel(StreamKArgs a) {
+  if constexpr (PLAN)
+    if (plan_block(a)) return;
   constexpr int V = D / 64;
   const int lane = threadIdx.x & 63;
   const int head = blockIdx.y * 4 + (threadIdx.x >> 6);
@@ -752,8 +764,10 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_by_seq_kernel
 // (num_seqs, Hq), the block's four waves share ONE q head's span -- wave p takes the span's slots p, p + 4, ... --
 // and their four states meet in LDS.  (With a wave per head a 256-slot span was a chain of eight round trips:
 // 20.8 us for one 128k-token sequence, next to a 48 us main kernel.)
-template <int D>
+template <int D, bool PLAN>
 __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_split4_kernel(StreamKArgs a) {
+  if constexpr (PLAN)
+    if (plan_block(a)) return;
   constexpr int V = D / 64;
   __shared__ float sh_acc[3][V][kWave];
   __shared__ float sh_ml[3][2];
@@ -985,16 +999,23 @@ int launch_streamk(const StreamKArgs& args, hipStream_t s) {
   // a sequence is cut where a share begins inside it: a batch of few sequences has most of them cut several
   // times (grid over the sequences, a wave per q head), a large batch has at most one cut per share and many
   // sequences with none (grid over the shares, four q heads per wave)
+#define KVQ_REDUCE(K)                                                                      \
+  do {                                                                                     \
+    if (plan_blocks > 0) hipLaunchKernelGGL((K<D, true>), rgrid, dim3(256), 0, s, a);      \
+    else hipLaunchKernelGGL((K<D, false>), rgrid, dim3(256), 0, s, a);                     \
+  } while (0)
+  const int plan_blocks = a.plan != nullptr ? 1 : 0;
   if (16 * a.num_seqs <= a.num_wg) {   // a handful of sequences, each cut many times: four waves per q head
-    dim3 rgrid(a.num_seqs, a.io.num_q_heads);
-    hipLaunchKernelGGL((paged_decode_streamk_reduce_split4_kernel<D>), rgrid, dim3(256), 0, s, a);
+    dim3 rgrid(a.num_seqs + plan_blocks, a.io.num_q_heads);
+    KVQ_REDUCE(paged_decode_streamk_reduce_split4_kernel);
   } else if (8 * a.num_seqs <= 3 * a.num_wg) {
-    dim3 rgrid(a.num_seqs, (a.io.num_q_heads + 3) / 4);
-    hipLaunchKernelGGL((paged_decode_streamk_reduce_by_seq_kernel<D>), rgrid, dim3(256), 0, s, a);
+    dim3 rgrid(a.num_seqs + plan_blocks, (a.io.num_q_heads + 3) / 4);
+    KVQ_REDUCE(paged_decode_streamk_reduce_by_seq_kernel);
   } else {
-    dim3 rgrid(a.num_wg, (a.io.num_q_heads + 15) / 16);
-    hipLaunchKernelGGL((paged_decode_streamk_reduce_kernel<D>), rgrid, dim3(256), 0, s, a);
+    dim3 rgrid(a.num_wg + plan_blocks, (a.io.num_q_heads + 15) / 16);
+    KVQ_REDUCE(paged_decode_streamk_reduce_kernel);
   }
+#undef KVQ_REDUCE
   return check_hip(hipGetLastError(), "paged_attn_int8 reduce launch");
 }
 

@@ -17,6 +17,7 @@
 namespace kvq {
 
 constexpr int kMaxKSplit = 8;   // context splits of a launch at most
+constexpr int kRunsInKernel = 16;   // sequences of a launch up to which the shared tile needs no plan (find_run)
 
 struct PrefillArgs {
   AttnIO io;
@@ -25,8 +26,9 @@ struct PrefillArgs {
   int num_seqs;
   int causal;
   int q_tokens;  // query tokens per block: (16 * NT) / group
-  // [1 + B]: how many sequences of the batch have a query run (q_len > 1, len > 0), then their numbers in batch
-  // order; written by prefill_plan_kernel ahead of the attention kernel of the same call.
+  // [1 + B]: how many sequences of the batch have a query run (q_len > 1, len > 0), then their numbers; written by
+  // prefill_plan_kernel ahead of the attention kernel of the same call; nullptr where the workgroup-shared tile
+  // finds the runs itself (find_run).
   const int32_t* plan;
   // Context splits of the workgroup-shared tile (1 = none).  With S > 1 an item's tiles are cut into S ranges, each
   // range is a workgroup of its own that leaves a partial state per (query row, q head) in `part`
@@ -219,6 +221,9 @@ static int launch_prefill_cfg(const PrefillArgs& a, int max_query_len, hipStream
 template <int D>
 int launch_prefill_shared(PrefillArgs& a, int max_query_len, int q_dtype, int out_dtype, hipStream_t s);
 
+// Runs that fill the workgroup-shared tile's columns take it.
+inline bool takes_shared_tile(int head_size, int max_query_len, int group) { return head_size <= 128 && max_query_len * group >= 64; }
+
 template <int D, int QDT, int ODT>
 static int launch_prefill_nt(PrefillArgs& a, int max_query_len, hipStream_t s);
 
@@ -228,7 +233,7 @@ static int launch_prefill_nt(PrefillArgs& a, int max_query_len, hipStream_t s);
 template <int D, int QDT, int ODT>
 static int launch_prefill_invariant(PrefillArgs& a, int max_query_len, hipStream_t s) {
   const int group = a.io.group;
-  if (D <= 128 && max_query_len * group >= 64) {
+  if (takes_shared_tile(D, max_query_len, group)) {
     a.route = 1;
     if (int e = launch_prefill_nt<D, QDT, ODT>(a, max_query_len, s)) return e;
     a.route = 2;
@@ -247,7 +252,7 @@ static int launch_prefill_nt(PrefillArgs& a, int max_query_len, hipStream_t s) {
   const bool int4 = a.io.g.code_type == KVQ_CODE_INT4;
   // long runs: the workgroup-shared fp16 tile (compute-bound shape), for every kind of code
   if constexpr (D <= 128) {
-    if (max_query_len * a.io.group >= 64 && a.route != 2) return launch_prefill_shared<D>(a, max_query_len, QDT, ODT, s);
+    if (takes_shared_tile(D, max_query_len, a.io.group) && a.route != 2) return launch_prefill_shared<D>(a, max_query_len, QDT, ODT, s);
   }
   if (fp8) {  // short runs of fp8 codes: the per-wave tile, one column tile per wave
     a.q_tokens = 16 / a.io.group;

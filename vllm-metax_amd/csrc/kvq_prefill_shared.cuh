@@ -294,6 +294,33 @@ struct SharedTile {
   }
 };
 
+// The sequence of workgroup `lin` of a launch with `per_seq` workgroups per query run (-1: there are not as many runs),
+// longest sequence first: workgroups start in this order, and the longest sequence's are the ones that should not start last.
+// Up to kRunsInKernel sequences: a lane for each, one trip to memory, ranked by lane moves inside the row of 16.  With the
+// plan kernel in front of them too, a step with a prompt of 70 tokens (32/8 heads of 128) took 14.0 us for 12.0, one of 2000
+// 71.7 for 69.2.  Beyond, and for the per-wave tile, the plan kernel lists them once: ranked in every workgroup, 64 prompts of
+// 200 - 400 tokens took 193 us for 180.
+// (PLANNED: an instantiation of its own, since choosing at run time cost launches with a plan up to 1 %.)
+template <bool PLANNED>
+__device__ __forceinline__ int find_run(const PrefillArgs& a, unsigned lin, unsigned per_seq) {
+  if constexpr (PLANNED) {
+    return lin >= per_seq * (unsigned)a.plan[0] ? -1 : a.plan[1 + lin / per_seq];
+  }
+  static_assert(kRunsInKernel == 16, "a lane of one row for every sequence");
+  const int lane = threadIdx.x & 63, s = min(lane, a.num_seqs - 1);
+  const int q_len = a.cu_seqlens_q[s + 1] - a.cu_seqlens_q[s], len = a.seq_lens[s];
+  const bool has = lane < a.num_seqs && q_len > 1 && len > 0;
+  if (lin >= per_seq * (unsigned)__builtin_popcountll(__builtin_amdgcn_ballot_w64(has))) return -1;
+  // distinct; of sequences of the same length the first
+  const uint32_t key = has ? (uint32_t)min(len, (1 << 27) - 1) * 16u + (uint32_t)(15 - lane) : 0u;
+  unsigned rank = 0;
+#define KVQ_RANK(N) rank += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key, 0x120 + N, 0xf, 0xf, true) > key ? 1u : 0u;   // row_ror:N
+  KVQ_RANK(1) KVQ_RANK(2) KVQ_RANK(3) KVQ_RANK(4) KVQ_RANK(5) KVQ_RANK(6) KVQ_RANK(7) KVQ_RANK(8)
+  KVQ_RANK(9) KVQ_RANK(10) KVQ_RANK(11) KVQ_RANK(12) KVQ_RANK(13) KVQ_RANK(14) KVQ_RANK(15)
+#undef KVQ_RANK
+  return __builtin_ctzll(__builtin_amdgcn_ballot_w64(has && rank == lin / per_seq));
+}
+
 // EXT adds the sliding window, the logits soft cap and ALiBi; the plain causal kernel carries none of them.
 // With a.ksplit > 1 the grid's x dimension carries that many context ranges per query block; a workgroup takes one range
 // of its item's tiles and writes a partial state instead of the rows.
@@ -303,7 +330,7 @@ struct SharedTile {
 template <int D, bool EXT>
 constexpr int kSharedWaves = D == 64 ? 4 : EXT ? 2 : 3;
 
-template <int D, bool EXT, int CODE>
+template <int D, bool EXT, int CODE, bool PLANNED>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kSharedWaves<D, EXT>, kSharedWaves<D, EXT>)))
 void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
   using W = SharedTile<D, CODE>;
@@ -315,7 +342,7 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // Which sequence, kv head and query block this workgroup takes.  Workgroups start in the order of their linear
   // number and go to the eight XCDs in turn by it.  The number is read over the sequences that HAVE a query run
-  // (the plan; the surplus workgroups of the grid, which is sized for every sequence of the batch, come last and
+  // (find_run; the surplus workgroups of the grid, which is sized for every sequence of the batch, come last and
   // leave at once), sequence by sequence, and inside a sequence query-block-major over its kv heads, longest block
   // first: the heads of a sequence then walk the same tokens at the same time (their records are neighbours in
   // memory, and what one head's workgroup brought into L2 is there for the next), and the head is shifted by the
@@ -327,15 +354,14 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
   // with long contexts (the mixed batch 959 us: sixteen streams of keys at once, six times the HBM fetches).
   const unsigned nsplit = (unsigned)a.ksplit;
   const unsigned nqb = gridDim.x / nsplit, hk = gridDim.z, per_seq = nqb * hk;
-  const unsigned nseq = (unsigned)a.plan[0];
   const unsigned lin_all = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
   const unsigned lin = lin_all / nsplit;
-  if (lin >= per_seq * nseq) return;   // uniform over the workgroup
+  const int seq = find_run<PLANNED>(a, lin, per_seq);
+  if (seq < 0) return;   // uniform over the workgroup
   unsigned split = lin_all % nsplit;   // the splits of an item are neighbours in launch order
   const unsigned rem = lin % per_seq;
   int qb = (int)(rem / hk);
   int hkv = (int)((rem % hk + (unsigned)qb) % hk);
-  const int seq = a.plan[1 + lin / per_seq];
   // Context ranges: all query blocks of a (kv head, range) pair go to ONE XCD, whose L2 then serves the range's records to
   // all but the first of them, where the pairs can be dealt out to the eight evenly (512 tokens on 32k, 8 kv heads, 6 ranges:
   // a step 388 -> 366 us, 1000 on 50k 1097 -> 1032, 4 kv heads 352 -> 342).
@@ -659,8 +685,9 @@ void paged_prefill_shared_kernel(PrefillArgs a, int q_dtype, int out_dtype) {
 }
 
 // The merge of the context splits: grid (query rows, ceil(Hq / 4)), a wave per (row of a run, q head), a lane D / 64 dims.
-// The rows are counted over the plan's runs, a handful where a launch is split (over every sequence of a mixed batch,
-// most of the blocks would find a decode row: 153 us of 330 beside 91 of them).  out = sum_s w_s o_s / sum_s w_s l_s with w_s = 2^(m_s - max m): the algebra of
+// The rows are counted over the runs (over every sequence of a mixed batch, most of the blocks would find a decode row:
+// 153 us of 330 beside 91 of them): a few sequences by a lane each, more over the plan's, a handful where a launch is split.
+// out = sum_s w_s o_s / sum_s w_s l_s with w_s = 2^(m_s - max m): the algebra of
 // merge_attn_states over the splits' states; the sink's term and the row's lse as in the unsplit kernel.
 // A stream of the states, 520 bytes per split at D = 128: every load of a row leaves before the first is used (splits past
 // the last reread it and weigh 0).  One block per row whose four waves went through the heads, and a head's splits, one
@@ -675,14 +702,24 @@ __global__ __launch_bounds__(256) void prefill_split_merge_kernel(PrefillArgs a,
   if (head >= io.num_q_heads) return;
   int qi = blockIdx.x;
   int64_t row = -1;
-  for (int i = 0; i < a.plan[0]; ++i) {   // uniform: scalar loads
-    const int seq = a.plan[1 + i];
-    const int q_begin = a.cu_seqlens_q[seq], q_len = a.cu_seqlens_q[seq + 1] - q_begin;
-    if (qi < q_len) {
-      row = q_begin + qi;
-      break;
+  if (a.plan == nullptr) {
+    const int i = min(lane, a.num_seqs - 1);   // (kRunsInKernel of them at most)
+    const int q_begin = a.cu_seqlens_q[i], q_len = a.cu_seqlens_q[i + 1] - q_begin;
+    const int n = lane < a.num_seqs && q_len > 1 && a.seq_lens[i] > 0 ? q_len : 0;
+    const int end = wave_incl_scan(n);
+    const uint64_t hit = __builtin_amdgcn_ballot_w64(qi < end && qi >= end - n);
+    if (hit == 0) return;
+    row = __builtin_amdgcn_readlane(q_begin + qi - (end - n), __builtin_ctzll(hit));
+  } else {
+    for (int i = 0; i < a.plan[0]; ++i) {   // uniform: scalar loads
+      const int seq = a.plan[1 + i];
+      const int q_begin = a.cu_seqlens_q[seq], q_len = a.cu_seqlens_q[seq + 1] - q_begin;
+      if (qi < q_len) {
+        row = q_begin + qi;
+        break;
+      }
+      qi -= q_len;
     }
-    qi -= q_len;
   }
   if (row < 0) return;
   const int S = a.ksplit;
@@ -727,7 +764,10 @@ static int launch_shared_code(PrefillArgs& a, int max_query_len, int q_dtype, in
   if (a.num_seqs > 65535 || a.io.g.num_kv_heads > 65535) return fail(KVQ_EINVAL, "paged_attn_int8: prefill grid out of range");
   if (a.ksplit < 1) a.ksplit = 1;
   dim3 grid(blocks * a.ksplit, a.num_seqs, a.io.g.num_kv_heads);
-  hipLaunchKernelGGL((paged_prefill_shared_kernel<D, EXT, CODE>), grid, dim3(256), 0, s, a, q_dtype, out_dtype);
+  if (a.plan != nullptr)
+    hipLaunchKernelGGL((paged_prefill_shared_kernel<D, EXT, CODE, true>), grid, dim3(256), 0, s, a, q_dtype, out_dtype);
+  else
+    hipLaunchKernelGGL((paged_prefill_shared_kernel<D, EXT, CODE, false>), grid, dim3(256), 0, s, a, q_dtype, out_dtype);
   if (int e = check_hip(hipGetLastError(), "paged_prefill_shared launch")) return e;
   if (a.ksplit == 1) return KVQ_OK;
   dim3 mgrid(a.num_tokens, (a.io.num_q_heads + 3) / 4);
