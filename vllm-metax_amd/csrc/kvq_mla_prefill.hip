@@ -12,13 +12,13 @@
 // What bounds it: latency -- matrix unit 47 % busy, vector unit 36 %, LDS 25 %.  Hence no registers between memory and LDS
 // (they took 20 of them and a fifth of the tile's instructions), three workgroups per compute unit where the launch has
 // that many, and operands of either product requested four ahead of their use: K from the step's start, the first V while the
-// softmax runs.  The reference maximum moves only when a product exceeds it by 2^7 or more, so that most steps reduce
-// nothing over lanes and rescale nothing.  Lane numbers, limits and the K addresses of a step are worked out anew for it:
-// kept, they were 18 registers more than the 168 there are at three workgroups.
+// softmax runs.  A step in which no product exceeds its row's maximum reduces nothing over lanes and rescales nothing.  Lane
+// numbers, limits and the K addresses of a step are worked out anew for it: kept, they were 18 registers more than the 168
+// there are at three workgroups.
 // Measured: 4 requests with 300-1500 new tokens on 1000-2300 cached ones, 128 heads, a layer step 1335 us with tiles through
 // registers, 1181 with two operand reads under way, a wait for the next tile's loads in front of the V reads and a maximum
-// taken in every step, 1099 now (of which 484 us are the two kv_b_proj products); one request of 200 tokens on 4900 cached
-// ones at 16 heads 219 -> 186, three of 500-1500 at 64 heads 221 -> 201.
+// reduced in every step, 1135 now (of which 484 us are the two kv_b_proj products); one request of 200 tokens on 4900 cached
+// ones at 16 heads 215 -> 200, three of 500-1500 at 64 heads 157 -> 140, one of 1400 in fp16 at 32 heads 98 -> 84.
 // Both products are computed transposed so that every per-row quantity is lane-local:
 //   S^T = K Q^T   A = K rows (lane = key, 8 consecutive d), B = Q (lane = query row): 16x16x32 MFMA of the
 //                 input type; a lane ends up with 8 keys of ITS query row, so the row maximum is a
@@ -126,8 +126,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   constexpr int RB = 2;                                             // row blocks of 16 per wave
   // fp16 weights are kept 2^8 larger so that small ones stay normal; l carries the same factor
   constexpr float kShift = DT == KVQ_F16 ? 8.f : 0.f;
-  // how far, in base 2, a logit may exceed its row's reference maximum: 2^(kShift + kAllow) must stay inside fp16
-  constexpr float kAllow = DT == KVQ_F16 ? 7.f : 8.f;
   constexpr int AHEAD = 4 < 2 * KS ? 4 : 2 * KS, AHEAD_V = 4 < DPL ? 4 : DPL;   // K and V operands requested ahead of their products
   __shared__ __align__(16) uint8_t lds[2][VT::BYTES];
   const int tid = threadIdx.x;
@@ -138,7 +136,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   // Under the causal mask a pair's blocks differ in length, and one pair after the other, longest block first, the launch
   // ends on the long blocks of the last pairs.  So the last pairs, of two rounds of workgroups, are taken block by block
   // over all of them (four requests of 430-1220 new tokens at 128 heads: the causal launch's longest place 95 tiles, now 76 of 70;
-  // the layer step 1095 -> 1075 us, one of 1400 tokens at 32 heads, a grid of 352, 113 -> 105, three of 500-1500 at 64 heads 207 -> 196).
+  // the layer step 20 us less of 1095, one of 1400 tokens at 32 heads, a grid of 352, 113 -> 105, three of 500-1500 at 64 heads 207 -> 196).
   // Not with a grid of 320 or less, nor with four blocks or fewer, which hardly differ: a pair's blocks side by side find its
   // keys in L2 (requests of 490 and 1190 tokens at 16 heads, a grid of 320: 112 us so, 113.5 otherwise; four of 67-240 at 128
   // heads 120, 123).
@@ -202,14 +200,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   const int wave_min_limit = min_limit;
 
   floatx4 oacc[RB][DPL];
-  float off[RB], thr[RB], l[RB];   // kShift - reference maximum; product above which it moves; lane's sum of weights
-  const float allow = kAllow / a.scale_log2;
+  float off[RB], top[RB], l[RB];   // kShift - row maximum; the largest product; lane's sum of weights
 #pragma unroll
   for (int rb = 0; rb < RB; ++rb) {
 #pragma unroll
     for (int i = 0; i < DPL; ++i) oacc[rb][i] = (floatx4){0.f, 0.f, 0.f, 0.f};
     off[rb] = kShift;
-    thr[rb] = -INFINITY;
+    top[rb] = -INFINITY;
     l[rb] = 0.f;
   }
 
@@ -314,27 +311,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
           sacc[rb][j >> 2][j & 3] = 16 * (j >> 2) + (j & 3) < visible ? sacc[rb][j >> 2][j & 3] : -INFINITY;
       }
     }
-    // The reference maximum only has to keep 2^(logit - m) in range: it stays put while no product exceeds thr, the
-    // reference plus kAllow, and then neither the reduction over a row's four lanes nor any rescaling is due.
-    float mx[RB];
-    bool over = false;
+    // A row's maximum moves where some lane's product exceeds it; in a step without such a lane neither the reduction over a
+    // row's four lanes nor any rescaling is due.  It is the true maximum, whose weight is then exactly 1: a maximum that stays
+    // put until exceeded by 2^8 saves more (four requests at 128 heads 1086 us, 1135 so) but has that weight rounded like any
+    // other, and the error against float64 was 2 to 16 % larger.
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) {
       // the maximum is taken over the raw products (the scale is positive and the same for every key), so that
-      // scale and reference enter each logit in ONE multiply-add
-      mx[rb] = -INFINITY;
+      // scale and maximum enter each logit in ONE multiply-add
+      float mx = -INFINITY;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) mx[rb] = fmaxf(mx[rb], sacc[rb][j >> 2][j & 3]);
-      over = over || mx[rb] > thr[rb];
-    }
-    if (__builtin_amdgcn_ballot_w64(over) != 0) {
-#pragma unroll
-      for (int rb = 0; rb < RB; ++rb) {
-        const float row_mx = max_over_quarters(mx[rb]);
-        const bool moves = row_mx > thr[rb];   // (a row's reference depends on its own products only)
-        const float new_off = moves ? kShift - row_mx * a.scale_log2 : off[rb];
-        const float alpha = thr[rb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(new_off - off[rb]);
-        thr[rb] = moves ? row_mx + allow : thr[rb];
+      for (int j = 0; j < 8; ++j) mx = fmaxf(mx, sacc[rb][j >> 2][j & 3]);
+      if (__builtin_amdgcn_ballot_w64(mx > top[rb]) != 0) {
+        const float new_top = fmaxf(top[rb], max_over_quarters(mx));
+        const float new_off = new_top == -INFINITY ? off[rb] : kShift - new_top * a.scale_log2;
+        const float alpha = top[rb] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(new_off - off[rb]);
+        top[rb] = new_top;
         off[rb] = new_off;
         l[rb] *= alpha;
 #pragma unroll
