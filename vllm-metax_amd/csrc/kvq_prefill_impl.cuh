@@ -26,8 +26,8 @@ struct PrefillArgs {
   int num_seqs;
   int causal;
   int q_tokens;  // query tokens per block: (16 * NT) / group
-  // [1 + B]: how many sequences of the batch have a query run (q_len > 1, len > 0), then their numbers; written by
-  // prefill_plan_kernel ahead of the attention kernel of the same call; nullptr where the workgroup-shared tile
+  // [1 + B]: how many sequences of the batch have a query run (q_len > 1, len > 0), then their numbers; written
+  // ahead of the attention kernel of the same call (write_prefill_plan); nullptr where the workgroup-shared tile
   // finds the runs itself (find_run).
   const int32_t* plan;
   // Context splits of the workgroup-shared tile (1 = none).  With S > 1 an item's tiles are cut into S ranges, each
