@@ -73,9 +73,9 @@ def test_varlen_attention_matches_fp32_statement(gpu_device, dtype, H, nope, rop
 @pytest.mark.parametrize("rise", [0.02, 0.2, 0.24, 3.0, -0.2])
 @pytest.mark.parametrize("H,causal", [(2, False), (2, True), (32, False)])
 def test_logits_that_keep_rising(gpu_device, dtype, rise, H, causal):
-    """The reference maximum of a row lags behind its logits by up to an allowance (2^8, fp16 2^7).  Logits that rise by
-    ``rise`` from key to key stay inside it for many tiles, pass it inside a tile, or in every tile; every third row's are all
-    below -1000, every fifth sees them fall."""
+    """A row's sums are rescaled in the tiles in which its maximum moves.  Logits that rise by ``rise`` from key to key move it in
+    every tile, by a little or by more than fp16's range; every third row's are all below -1000, every fifth sees them fall, so
+    that rows of one wave differ in whether theirs moves."""
     dev, nope, rope, dv = gpu_device, 128, 64, 128
     qlens, klens = [300, 70], [400, 97]
     if causal:
