@@ -661,24 +661,66 @@ def test_odd_ends_of_the_shared_tile(gpu_device, hq, hkv, d, window):
         T.assert_close_attn(out, want, what=f"odd ends, window {window}, {splits} ranges")
 
 
-@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 64, 65, 100])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 64, 65, 100, 257, 300])
 @pytest.mark.parametrize("hq,hkv,d,splits", [(32, 8, 128, 1), (32, 8, 128, 3), (8, 2, 256, 1), (8, 8, 64, 2)])
 def test_runs_of_a_batch_by_its_number_of_sequences(gpu_device, n, hq, hkv, d, splits):
     """Up to 16 sequences every workgroup finds its query run itself, beyond the decode launch lists them: runs between decode
-    rows and sequences without tokens, several of one length.  The oracle decides, within the bounds of the other tests."""
+    rows and sequences without tokens, several of one length.  The oracle decides, within the bounds of the other tests; an empty
+    sequence's one row is zeros with lse -inf, its several rows are left alone."""
     lens = [(90, 90, 40, 200)[i % 4] + (i % 3) * 16 for i in range(n)]
     qls = [(70, 1, 33, 90)[i % 4] if n > 2 else 70 for i in range(n)]
+    empty = [n - 3] if n > 2 else []
+    if n > 256:
+        qls[256] = 1
+        empty.append(256)
     kv, lay, bt, q, sl, cu = build(lens, qls, hq, hkv, d, 16, seed=n + d)
-    if n > 2:
-        sl[n - 3] = 0   # its rows are left alone: not compared
+    sl[empty] = 0
     scale = 1 / math.sqrt(d)
-    want = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, scale)
+    want, want_lse = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, scale, return_lse=True)
     kvd = T.to_device_cache(kv, gpu_device, "NHD")
     k, v = L.key_value_views(kvd)
     ks, vs = L.scale_views(kvd)
     out = torch.full(q.shape, float("nan"), dtype=q.dtype, device=gpu_device)
+    lse = torch.full(q.shape[:2], float("nan"), dtype=torch.float32, device=gpu_device)
     ops.unified_attention(q.to(gpu_device), k, v, out, cu.to(gpu_device), max(qls), sl.to(gpu_device), int(sl.max()), scale,
-                          True, block_table=bt.to(gpu_device), k_scale_cache=ks, v_scale_cache=vs, prefill_splits=splits)
+                          True, block_table=bt.to(gpu_device), k_scale_cache=ks, v_scale_cache=vs, prefill_splits=splits, lse=lse)
     torch.cuda.synchronize()
-    rows = [r for i in range(n) if int(sl[i]) > 0 for r in range(int(cu[i]), int(cu[i + 1]))]
-    T.assert_close_attn(out[rows], want[rows], what=f"{n} sequences d{d} splits {splits}")
+    out, lse = out.cpu(), lse.cpu()
+    written = torch.ones(q.shape[0], dtype=torch.bool)
+    for i in empty:
+        at = slice(int(cu[i]), int(cu[i + 1]))
+        if qls[i] == 1:
+            assert (out[at] == 0).all() and (lse[at] == -math.inf).all(), f"sequence {i} of {n}: empty, one row"
+        else:
+            assert out[at].isnan().all() and lse[at].isnan().all(), f"sequence {i} of {n}: empty, {qls[i]} rows"
+        written[at] = False
+    T.assert_close_attn(out[written], want[written], what=f"{n} sequences d{d} splits {splits}")
+    torch.testing.assert_close(lse[written], want_lse[written], atol=5e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("hq,hkv,d", [(8, 2, 64), (32, 8, 128), (4, 4, 256)])
+@pytest.mark.parametrize("run", [9, 70])
+def test_empty_decode_rows_of_a_mixed_batch_of_any_size(gpu_device, hq, hkv, d, run):
+    """One-row sequences of length 0 anywhere in a batch of more sequences than the chip has compute units, next to query runs:
+    zeros, lse -inf.  What the rows held before is NaN, so a row that no workgroup takes shows."""
+    n = 2 * torch.cuda.get_device_properties(gpu_device).multi_processor_count + 20
+    qls = [run if i % 50 == 7 else 1 for i in range(n)]
+    lens = [max(qls[i], 1 + 3 * (i % 11)) for i in range(n)]
+    kv, lay, bt, q, sl, cu = build(lens, qls, hq, hkv, d, 16, seed=run + d)
+    for i in range(n):
+        if qls[i] == 1 and (i % 3 == 0 or i > n // 2 - 12):
+            sl[i] = 0
+    scale = 1 / math.sqrt(d)
+    want, want_lse = oracle.paged_attn(q, T.storage_bytes(kv), lay, bt, sl, cu, scale, return_lse=True)
+    kvd = T.to_device_cache(kv, gpu_device, "NHD")
+    k, v = L.key_value_views(kvd)
+    ks, vs = L.scale_views(kvd)
+    out = torch.full(q.shape, float("nan"), dtype=torch.float32, device=gpu_device)
+    lse = torch.full(q.shape[:2], float("nan"), dtype=torch.float32, device=gpu_device)
+    ops.unified_attention(q.to(gpu_device), k, v, out, cu.to(gpu_device), max(qls), sl.to(gpu_device), int(sl.max()), scale,
+                          True, block_table=bt.to(gpu_device), k_scale_cache=ks, v_scale_cache=vs, lse=lse)
+    torch.cuda.synchronize()
+    left = [i for i in range(n) if out[int(cu[i])].isnan().any() or lse[int(cu[i])].isnan().any()]
+    assert not left, f"rows that nobody wrote: sequences {left} of {n}"
+    T.assert_close_attn(out, want, what=f"empty decode rows d{d}")
+    torch.testing.assert_close(lse.cpu(), want_lse, atol=5e-3, rtol=1e-3)

@@ -457,6 +457,9 @@ __device__ __forceinline__ bool plan_block(const StreamKArgs& a) {
   return true;
 }
 
+// Merge the partial states of every decode sequence that more than one workgroup touched, and give empty decode
+// sequences their defined output.  grid (num_wg, ceil(Hq / 16)), with PLAN (num_wg + 1, ...); 4 waves; a wave takes four
+// q heads, 16 lanes each, a lane D/16 dims.
 // A sequence is cut only where a workgroup's share begins inside it, so the grid runs over the P workgroups of
 // the main kernel, not over the sequences: block w looks at the sequence in which share w begins (the main
 // kernel left its number, its row and its shares) and merges it if share w is the
@@ -488,8 +491,9 @@ __global__ __launch_bounds__(256) void paged_decode_streamk_reduce_kernel(Stream
 #pragma unroll
     for (int i = 0; i < V; ++i) store_act_rt(a.io.out_dtype, a.io.out, at + i, x[i]);
   };
-  // empty decode sequences (no tile: length 0): zeros, lse = -inf; the blocks share them out
-  for (int s = w; s < B; s += (int)gridDim.x) {
+  // empty decode sequences (no tile: length 0): zeros, lse = -inf; the merging blocks share them out (the grid may hold one
+  // more, the plan's)
+  for (int s = w; s < B; s += a.num_wg) {
     const int q0e = a.cu_seqlens_q ? a.cu_seqlens_q[s] : s;
     const int q1e = a.cu_seqlens_q ? a.cu_seqlens_q[s + 1] : s + 1;
     if (q1e - q0e == 1 && a.seq_lens[s] <= 0) {
