@@ -132,6 +132,9 @@ def test_a_launch_that_fills_the_chip_has_the_bits_of_a_small_one(gpu_device, dt
     (64, [700] * 6),                 # the first pairs one after the other, the last ones block by block
     (27, [520, 900, 641]),           # 81 pairs: no share for each XCD
     (16, [4100, 30]),                # more blocks per pair than a round has places to share out
+    (64, [500, 450]),                # four blocks per pair, the fewest that are taken so
+    (16, [100] * 7 + [1500]),        # most places of the grid without rows: pair by pair
+    (16, [90, 3000, 70, 800]),       # the same with two rounds of workgroups that have rows
 ])
 def test_every_block_of_a_large_causal_launch_is_taken(gpu_device, H, qlens):
     """The order in which a causal launch's workgroups take the (sequence, head, block) items: rows and LSE have the bits of

@@ -48,6 +48,7 @@ struct VarlenArgs {
   int64_t q_st, q_sh, kn_st, kn_sh, kpe_st, v_st, v_sh, out_st, out_sh, total_q;
   int causal;
   int merge;   // out and lse hold the rows' state over other keys: this launch's is merged into it
+  int last_pairs;   // (sequence, head) pairs of an XCD, the last ones, whose blocks are taken in turn (by_block_pairs)
   float scale_log2;
 };
 
@@ -117,6 +118,9 @@ __device__ __forceinline__ void static_for(F f) {
   }
 }
 
+// log2 of the XCDs that a launch's (sequence, head) pairs are dealt out to, every eighth pair to one of eight; 0: not at all.
+__host__ __device__ constexpr unsigned xcd_bits_of(unsigned pairs) { return (pairs & 7u) == 0 ? 3 : 0; }
+
 // WAVES: waves per SIMD, i.e. workgroups per compute unit, that the kernel is compiled for (see launch_varlen).
 template <int DT, int NOPE, int ROPE, int DV, int WAVES>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void varlen_attn_kernel(VarlenArgs a) {
@@ -134,27 +138,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   // blocks of one (sequence, head) all stream the same keys: numbered so that they land on ONE XCD (possible when
   // the (sequence, head) pairs divide by eight), its L2 serves all but the first reader of a tile.
   // Under the causal mask a pair's blocks differ in length, and one pair after the other, longest block first, the launch
-  // ends on the long blocks of the last pairs.  So the last pairs, of two rounds of workgroups, are taken block by block
-  // over all of them (four requests of 430-1220 new tokens at 128 heads: the causal launch's longest place 95 tiles, now 76 of 70;
-  // the layer step 20 us less of 1095, one of 1400 tokens at 32 heads, a grid of 352, 113 -> 105, three of 500-1500 at 64 heads 207 -> 196).
-  // Not with a grid of 320 or less, nor with four blocks or fewer, which hardly differ: a pair's blocks side by side find its
-  // keys in L2 (requests of 490 and 1190 tokens at 16 heads, a grid of 320: 112 us so, 113.5 otherwise; four of 67-240 at 128
-  // heads 120, 123).
+  // ends on the long blocks of the last pairs: the last a.last_pairs of an XCD's pairs are taken block by block over all of
+  // them (by_block_pairs says when and how many).
   int seq, head, qb;
   {
     const unsigned pairs = gridDim.y * gridDim.z, blocks = gridDim.x;
-    const unsigned xcd_bits = (pairs & 7u) == 0 ? 3 : 0;
+    const unsigned xcd_bits = xcd_bits_of(pairs);
     const unsigned lin = blockIdx.x + blocks * (blockIdx.y + gridDim.y * blockIdx.z);
     const unsigned j = lin >> xcd_bits, per_xcd = pairs >> xcd_bits;   // the XCD's j-th workgroup
     unsigned pair = j / blocks;
     qb = (int)(j - pair * blocks);
-    if (a.causal && blocks > 4 && pairs * blocks > 320) {
-      const unsigned last = min(per_xcd, ((2 * WAVES * 256) >> xcd_bits) / blocks + 1);
-      if (pair >= per_xcd - last) {
-        const unsigned r = j - (per_xcd - last) * blocks;
-        qb = (int)(r / last);
-        pair = per_xcd - last + (r - (unsigned)qb * last);
-      }
+    const unsigned last = (unsigned)a.last_pairs;
+    if (pair >= per_xcd - last) {
+      const unsigned r = j - (per_xcd - last) * blocks;
+      qb = (int)(r / last);
+      pair = per_xcd - last + (r - (unsigned)qb * last);
     }
     pair = (pair << xcd_bits) + (lin & ((1u << xcd_bits) - 1));   // every eighth pair is this XCD's
     seq = (int)(pair / gridDim.y);
@@ -433,9 +431,34 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
 // The lengths are device data; rows and sequences give the number of workgroups to within half of one per sequence.
 constexpr int64_t kTwoPerUnit = 512;
 
+// How many of an XCD's last pairs a causal launch takes block by block: those of two rounds of workgroups, or none.  `live`
+// counts the workgroups that have rows, as far as the host knows.  What the order changes, the launch alone, us on MI355X,
+// pair by pair / so:
+//   up to one live workgroup per compute unit there is no second round to even out, and a pair's blocks side by side find its
+//   keys in L2: 16 heads, requests of 490 and 1190 tokens (224 live) 36.9 / 38.2, of 1700 and 300 (256) 49.8 / 53.0, of 2000
+//   (256) 55.7 / 55.7; but 16 heads x 2560 (336) 75.8 / 74.1, 20 x 2000 (320) 73.6 / 58.8, 32 x 1280 (352) 46.5 / 43.0, 64 x 1000
+//   (512) 45.4 / 38.7, 128 x 1000 (1024) 76.8 / 63.2, 128 heads, 4 requests of 430 - 1220 (2944) 156.6 / 149.1;
+//   up to three blocks hardly differ in length: 128 heads, 4 of 200 28.8 / 30.1, 4 of 300 44.5 / 47.3, 64 heads, 8 of 380
+//   56.2 / 56.4; with four 128 heads, 4 of 500 96.7 / 83.7, 16 heads, 8 of 500 30.0 / 26.1;
+//   where most of the grid has no rows, a long request's blocks lie a fixed number of places apart and pile up on part of an
+//   XCD (with the places rotated from block to block they do not); two rounds of live ones even that out.  16 heads, 7 of
+//   100 and one of 1500 (336 live of 1536) 47.7 / 66.2, but 7 of 100 and one of 3000 (512 of 3072) 104.9 / 99.5, 32 heads, 4 of
+//   150 and one of 1300 (544 of 1760) 63.2 / 50.5, 15 of 100 and one of 2000 (1120 of 8192) 104.1 / 95.3.
+static int by_block_pairs(dim3 grid, int64_t live, int max_seqlen_q, int64_t total_q, int per_unit) {
+  const int64_t units = num_cus();
+  const bool half_live = 2 * total_q >= (int64_t)max_seqlen_q * grid.z;
+  if (grid.x < 4 || live <= units || !(half_live || live >= 2 * units)) return 0;
+  const unsigned pairs = grid.y * grid.z, bits = xcd_bits_of(pairs);
+  const int64_t last = ((2 * per_unit * units) >> bits) / grid.x + 1;
+  return (int)(last < (pairs >> bits) ? last : (pairs >> bits));
+}
+
 template <int NOPE, int ROPE, int DV>
-static int launch_varlen(int dtype, const VarlenArgs& a, dim3 grid, hipStream_t s) {
-  const bool few = (a.total_q / 128 + (grid.z + 1) / 2) * (int64_t)grid.y <= kTwoPerUnit;
+static int launch_varlen(int dtype, const VarlenArgs& args, int max_seqlen_q, dim3 grid, hipStream_t s) {
+  VarlenArgs a = args;
+  const int64_t live = (a.total_q / 128 + (grid.z + 1) / 2) * (int64_t)grid.y;
+  const bool few = live <= kTwoPerUnit;
+  a.last_pairs = a.causal ? by_block_pairs(grid, live, max_seqlen_q, a.total_q, few ? 2 : 3) : 0;
   if (dtype == KVQ_F16) {
     if (few) hipLaunchKernelGGL((varlen_attn_kernel<KVQ_F16, NOPE, ROPE, DV, 2>), grid, dim3(256), 0, s, a);
     else hipLaunchKernelGGL((varlen_attn_kernel<KVQ_F16, NOPE, ROPE, DV, 3>), grid, dim3(256), 0, s, a);
@@ -486,9 +509,9 @@ extern "C" int kvq_mla_prefill_attn(const void* q, int dtype, int64_t q_stride_t
   a.scale_log2 = scale * kLog2e;
   const dim3 grid((unsigned)((max_seqlen_q + 127) / 128), (unsigned)num_heads, (unsigned)num_seqs);
   hipStream_t s = as_stream(stream);
-  if (nope_dim == 128 && rope_dim == 64 && v_dim == 128) return launch_varlen<128, 64, 128>(dtype, a, grid, s);
-  if (nope_dim == 64 && rope_dim == 32 && v_dim == 64) return launch_varlen<64, 32, 64>(dtype, a, grid, s);
-  if (nope_dim == 128 && rope_dim == 0 && v_dim == 128) return launch_varlen<128, 0, 128>(dtype, a, grid, s);
+  if (nope_dim == 128 && rope_dim == 64 && v_dim == 128) return launch_varlen<128, 64, 128>(dtype, a, max_seqlen_q, grid, s);
+  if (nope_dim == 64 && rope_dim == 32 && v_dim == 64) return launch_varlen<64, 32, 64>(dtype, a, max_seqlen_q, grid, s);
+  if (nope_dim == 128 && rope_dim == 0 && v_dim == 128) return launch_varlen<128, 0, 128>(dtype, a, max_seqlen_q, grid, s);
   return fail(KVQ_EINVAL, "%s: head dims (nope %d, rope %d, v %d) are not built; built: (128, 64, 128), (64, 32, 64), (128, 0, 128)",
               op, nope_dim, rope_dim, v_dim);
 }
