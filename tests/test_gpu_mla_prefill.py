@@ -107,8 +107,8 @@ def test_logits_that_keep_rising(gpu_device, dtype, rise, H, causal):
     (False, [1, 31, 32, 33, 127, 129, 300], [64, 33, 1, 0, 31, 95, 32]),    # keys that end at, before and behind a tile
 ])
 def test_a_launch_that_fills_the_chip_has_the_bits_of_a_small_one(gpu_device, dtype, nope, rope, dv, causal, qlens, klens):
-    """128 heads take the kernel with three workgroups per compute unit, eight of the same heads the one with two: the fp32
-    statement for both, and the same bits in the rows and LSE they share."""
+    """128 heads put three workgroups on a compute unit, eight of the same heads one: the fp32 statement for both, and the same
+    bits in the rows and LSE they share."""
     dev, H, few = gpu_device, 128, 8
     klens = klens or qlens
     q, kv, kpe = _inputs(qlens, klens, H, nope, rope, dv, dtype, seed=17)

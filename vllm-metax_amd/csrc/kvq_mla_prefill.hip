@@ -121,9 +121,13 @@ __device__ __forceinline__ void static_for(F f) {
 // log2 of the XCDs that a launch's (sequence, head) pairs are dealt out to, every eighth pair to one of eight; 0: not at all.
 __host__ __device__ constexpr unsigned xcd_bits_of(unsigned pairs) { return (pairs & 7u) == 0 ? 3 : 0; }
 
-// WAVES: waves per SIMD, i.e. workgroups per compute unit, that the kernel is compiled for (see launch_varlen).
-template <int DT, int NOPE, int ROPE, int DV, int WAVES>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void varlen_attn_kernel(VarlenArgs a) {
+// Three waves per SIMD, i.e. workgroups per compute unit.  Two, of the same instructions, are no better where a launch has no more
+// (launch alone, two / three per unit: 128 heads, 300 new tokens on 4000, 384 workgroups, 139.8 / 140.2 us, 500, 512, 168.0 / 169.7) and
+// worse beyond (600, 640, 244.4 / 212.3; 64 heads, 1500 on 3000, 768, 194.0 / 173.8).
+constexpr int kPerUnit = 3;
+
+template <int DT, int NOPE, int ROPE, int DV>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kPerUnit, kPerUnit))) void varlen_attn_kernel(VarlenArgs a) {
   using VT = VarlenTile<NOPE, ROPE, DV>;
   constexpr int KSN = NOPE / 32, KSR = ROPE / 32, KS = KSN + KSR;   // k-steps of the QK product
   constexpr int DPL = DV / 16;                                      // dims per lane and output block
@@ -424,13 +428,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(WAVES, WAVE
   }
 }
 
-// Three workgroups per compute unit where the launch has work for them, two -- with operands read further ahead -- where it
-// does not.  Measured on MI355X, two against three, us per layer step at 128 heads unless stated: 512 workgroups (500 new
-// tokens on 4000) 394 / 409, 384 (16 heads, 2765 new tokens of four requests) 227 / 255, 640 (600 on 4000) 542 / 497,
-// 768 (64 heads, 1500 on 3000) 424 / 390, 1536 (1500 on 2000) 591 / 561, 3072 (2765 of four requests) 1230 / 1178.
-// The lengths are device data; rows and sequences give the number of workgroups to within half of one per sequence.
-constexpr int64_t kTwoPerUnit = 512;
-
 // How many of an XCD's last pairs a causal launch takes block by block: those of two rounds of workgroups, or none.  `live`
 // counts the workgroups that have rows, as far as the host knows.  What the order changes, the launch alone, us on MI355X,
 // pair by pair / so:
@@ -444,28 +441,23 @@ constexpr int64_t kTwoPerUnit = 512;
 //   XCD (with the places rotated from block to block they do not); two rounds of live ones even that out.  16 heads, 7 of
 //   100 and one of 1500 (336 live of 1536) 47.7 / 66.2, but 7 of 100 and one of 3000 (512 of 3072) 104.9 / 99.5, 32 heads, 4 of
 //   150 and one of 1300 (544 of 1760) 63.2 / 50.5, 15 of 100 and one of 2000 (1120 of 8192) 104.1 / 95.3.
-static int by_block_pairs(dim3 grid, int64_t live, int max_seqlen_q, int64_t total_q, int per_unit) {
+static int by_block_pairs(dim3 grid, int64_t live, int max_seqlen_q, int64_t total_q) {
   const int64_t units = num_cus();
   const bool half_live = 2 * total_q >= (int64_t)max_seqlen_q * grid.z;
   if (grid.x < 4 || live <= units || !(half_live || live >= 2 * units)) return 0;
   const unsigned pairs = grid.y * grid.z, bits = xcd_bits_of(pairs);
-  const int64_t last = ((2 * per_unit * units) >> bits) / grid.x + 1;
+  const int64_t last = ((2 * kPerUnit * units) >> bits) / grid.x + 1;
   return (int)(last < (pairs >> bits) ? last : (pairs >> bits));
 }
 
 template <int NOPE, int ROPE, int DV>
 static int launch_varlen(int dtype, const VarlenArgs& args, int max_seqlen_q, dim3 grid, hipStream_t s) {
   VarlenArgs a = args;
+  // the lengths are device data; rows and sequences give the number of workgroups to within half of one per sequence
   const int64_t live = (a.total_q / 128 + (grid.z + 1) / 2) * (int64_t)grid.y;
-  const bool few = live <= kTwoPerUnit;
-  a.last_pairs = a.causal ? by_block_pairs(grid, live, max_seqlen_q, a.total_q, few ? 2 : 3) : 0;
-  if (dtype == KVQ_F16) {
-    if (few) hipLaunchKernelGGL((varlen_attn_kernel<KVQ_F16, NOPE, ROPE, DV, 2>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((varlen_attn_kernel<KVQ_F16, NOPE, ROPE, DV, 3>), grid, dim3(256), 0, s, a);
-  } else {
-    if (few) hipLaunchKernelGGL((varlen_attn_kernel<KVQ_BF16, NOPE, ROPE, DV, 2>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((varlen_attn_kernel<KVQ_BF16, NOPE, ROPE, DV, 3>), grid, dim3(256), 0, s, a);
-  }
+  a.last_pairs = a.causal ? by_block_pairs(grid, live, max_seqlen_q, a.total_q) : 0;
+  if (dtype == KVQ_F16) hipLaunchKernelGGL((varlen_attn_kernel<KVQ_F16, NOPE, ROPE, DV>), grid, dim3(256), 0, s, a);
+  else hipLaunchKernelGGL((varlen_attn_kernel<KVQ_BF16, NOPE, ROPE, DV>), grid, dim3(256), 0, s, a);
   return check_hip(hipGetLastError(), "mla_prefill_attn launch");
 }
 
