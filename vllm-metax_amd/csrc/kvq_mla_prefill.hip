@@ -258,7 +258,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kPerUnit, k
   // V^T operand of output block i, half h (keys 4 g .. + 3 and 16 + 4 g ..): the LDS's transposing read.  Lane s of a
   // quarter-wave names the 8 bytes [key kb + s / 4][dims 16 i + 4 (s % 4) .. + 3] and receives [keys kb .. kb + 3][dim 16 i + s].
   // In assembly because the compiler waits for every load under way, the next tile's too, in front of the builtin; so the
-  // waits for what these read are written out as well.
+  // waits for what these read are written out as well.  To the compiler a read's registers hold their values at once:
+  // tests/test_lds_read_waits.py follows the compiled code for a copy, a spill or a reuse before the wait.
   struct VOperand {
     u32x2 half[2];
   };
