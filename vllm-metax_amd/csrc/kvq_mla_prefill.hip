@@ -9,16 +9,16 @@
 // tile ahead, double-buffered (one barrier per tile), and every wave feeds its two row blocks from there, so a K or V byte
 // is fetched from L2 once per 128 rows.  Which bytes a load's lanes bring is chosen so that the operand reads of K (chunks
 // xor-swizzled by the row) and of V (successive rows from different loads, 32 bytes apart) meet no bank twice.
-// What bounds it: latency -- matrix unit 47 % busy, vector unit 36 %, LDS 25 %.  Hence no registers between memory and LDS
-// (they took 20 of them and a fifth of the tile's instructions), three workgroups per compute unit where the launch has
-// that many, and operands of either product requested four ahead of their use: K from the step's start, the first V while the
-// softmax runs.  A step in which no product exceeds its row's maximum reduces nothing over lanes and rescales nothing.  Lane
+// What bounds it: latency -- matrix unit 44 % busy, vector unit 39 %, LDS 22 %.  Hence no registers between memory and LDS
+// (they took 20 of them and a fifth of the tile's instructions), three workgroups per compute unit, and operands of either
+// product requested four ahead of their use: K from the step's start, the first V while the softmax runs.  A step in which no product exceeds its row's maximum reduces nothing over lanes and rescales nothing.  Lane
 // numbers, limits and the K addresses of a step are worked out anew for it: kept, they were 18 registers more than the 168
 // there are at three workgroups.
-// Measured: 4 requests with 300-1500 new tokens on 1000-2300 cached ones, 128 heads, a layer step 1335 us with tiles through
-// registers, 1181 with two operand reads under way, a wait for the next tile's loads in front of the V reads and a maximum
-// reduced in every step, 1135 now (of which 484 us are the two kv_b_proj products); one request of 200 tokens on 4900 cached
-// ones at 16 heads 215 -> 200, three of 500-1500 at 64 heads 157 -> 140, one of 1400 in fp16 at 32 heads 98 -> 84.
+// Measured: 4 requests with 300-1500 new tokens on 1000-2300 cached ones, 128 heads, a layer step 1335 -> 1192 us without the
+// registers; then, side by side, with two operand reads under way, a wait for the next tile's loads in front of the V reads, a
+// maximum reduced in every step and pairs of a causal launch one after the other / now: 1215 / 1176 (of which 484 us are the
+// two kv_b_proj products); one request of 200 tokens on 4900 cached ones at 16 heads 215 / 200, three of 500-1500 at 64 heads
+// 161 / 144, one of 1400 in fp16 at 32 heads 98 / 84.
 // Both products are computed transposed so that every per-row quantity is lane-local:
 //   S^T = K Q^T   A = K rows (lane = key, 8 consecutive d), B = Q (lane = query row): 16x16x32 MFMA of the
 //                 input type; a lane ends up with 8 keys of ITS query row, so the row maximum is a
@@ -121,9 +121,9 @@ __device__ __forceinline__ void static_for(F f) {
 // log2 of the XCDs that a launch's (sequence, head) pairs are dealt out to, every eighth pair to one of eight; 0: not at all.
 __host__ __device__ constexpr unsigned xcd_bits_of(unsigned pairs) { return (pairs & 7u) == 0 ? 3 : 0; }
 
-// Three waves per SIMD, i.e. workgroups per compute unit.  Two, of the same instructions, are no better where a launch has no more
-// (launch alone, two / three per unit: 128 heads, 300 new tokens on 4000, 384 workgroups, 139.8 / 140.2 us, 500, 512, 168.0 / 169.7) and
-// worse beyond (600, 640, 244.4 / 212.3; 64 heads, 1500 on 3000, 768, 194.0 / 173.8).
+// Three waves per SIMD, i.e. workgroups per compute unit.  Two, of the same instructions, are no better where a launch has no
+// more (launch alone, two / three per unit: 128 heads, 300 new tokens on 4000, 384 workgroups, 139.8 / 140.2 us, 500, 512,
+// 168.0 / 169.7) and worse beyond (600, 640, 244.4 / 212.3; 64 heads, 1500 on 3000, 768, 194.0 / 173.8).
 constexpr int kPerUnit = 3;
 
 template <int DT, int NOPE, int ROPE, int DV>

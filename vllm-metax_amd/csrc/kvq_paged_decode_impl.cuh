@@ -448,8 +448,8 @@ __global__ __launch_bounds__(256) void paged_decode_fixed_spans_reduce_kernel(St
 
 // The prefill plan of a mixed batch rides on the reduce launch, one more block of it (PLAN: the last of the grid's first row;
 // the rest of its column leaves).  As a launch of its own between the two it cost the step 2 - 3 us (30 decode rows beside 4
-// runs of 60 - 300 tokens 77.5 us for 74.8, 30 beside 3 of 300 - 600 at head size 256 with fp8 codes 255.8 for 248.7; the mixed step of 60
-// rows and 4 x 2048 tokens 436.7 for 435.1).  An instantiation of its own, since a look at a.plan in front of a decode
+// runs of 60 - 300 tokens 77.5 us for 74.8, 12 beside 4 of those 37.4 for 34.6, 200 beside 8 of 60 - 100 70.6 for 68.6; in a step of 60
+// rows and 4 x 2048 tokens, 473 us, no more than its runs differ).  An instantiation of its own, since a look at a.plan in front of a decode
 // step's reduce took 0.2 us of it.
 __device__ __forceinline__ bool plan_block(const StreamKArgs& a) {
   if (blockIdx.x + 1 != gridDim.x) return false;
